@@ -5,14 +5,14 @@
 // whatever M is, so that logits do not depend on how a step was cut: K goes in segments of SEG; a
 // segment's sum runs k ascending from zero, one fused multiply-add a step; the segments' sums are
 // added in ascending order, starting from zero.  Two kernels keep to it.  Many rows (M > 64): 64 x 64
-// tiles, a workgroup walks all of K.  Few rows: a tile of 8 to 64 rows x 64 columns, and where the
+// tiles on the matrix cores, a workgroup walks all of K.  Few rows: a tile of 8 to 64 rows x 64 columns, and where the
 // column tiles alone do not fill the chip every segment is a workgroup of its own, which asks for its
 // whole share of W (64 x 128: 32 KB) at once and leaves its sum in a workspace; a second kernel adds
 // the segments' sums in order and ends with the epilogue.  (Few rows used to run in the many-rows
 // kernel: a hundred workgroups, each walking all of K alone.)
 // ---------------------------------------------------------------------------------------
 namespace plain {
-constexpr int BM = 64, BN = 64, BK = 16, PAD = 4;
+constexpr int BM = 64, BN = 64, PAD = 4;
 constexpr int SEG = 128;
 
 template <typename TC>
@@ -27,90 +27,134 @@ __device__ __forceinline__ void finish(float v, int m, int n, const float* bias,
   }
 }
 
-// WHOLE: K is a multiple of 4, so a thread's four elements along K are all inside or all outside
-template <typename TI, typename TC, bool WHOLE>
-__global__ __launch_bounds__(256) void gemm_kernel(const TI* __restrict__ A, int lda, const TI* __restrict__ W,
-                                                    const float* __restrict__ bias, TC* __restrict__ C, int ldc,
-                                                    float* __restrict__ resid, int ldr, int M, int N, int K,
-                                                    int epi) {
-  __shared__ float As[BK][BM + PAD];
-  __shared__ float Ws[BK][BN + PAD];
-  const int t = threadIdx.x;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int lrow = t / 4, lk = (t % 4) * 4;   // loader: 64 rows x 4 groups of 4 k
-  const int tx = t % 16, ty = t / 16;         // computer: 4x4 outputs
-  float acc[4][4], tot[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = tot[i][j] = 0.f;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    {
-      int m = m0 + lrow, k = k0 + lk;
-      float v[4] = {0.f, 0.f, 0.f, 0.f};
-      if (m < M && k < K) {
-        const TI* p = A + static_cast<size_t>(m) * lda + k;
-        if (WHOLE || k + 4 <= K) {
+// Many rows.  v_mfma_f32_32x32x2_f32 adds its two products to the sum one after the other, k ascending, each with one
+// rounding, subnormals kept: the same bits as the chain of fused multiply-adds that `rows_kernel` runs, at twice the rate of
+// the vector unit's single 32-bit multiply-adds (157 against 79 TFLOP/s on the card), which bounded this kernel while it used
+// them: the 97 products of a GPT-2 Medium step of 2,048 rows took 242 us on average and take 142 now (62 -> 105 TFLOP/s; the
+// matrix cores are busy three quarters of the largest one's time, the rest is waits for operands at the barriers).
+// A workgroup's tile is 64 x 64, a wave's 32 x 32: small, because operands are cheap here (two numbers a lane for 64
+// cycles of matrix work) and with four workgroups a CU a product of 1,024 columns still gives every CU two tiles.
+// Slabs of 32 along K wait in registers while the slab before is multiplied, and lie in LDS with every eight k of a row in
+// the order 0 2 4 6 1 3 5 7: a lane (row l % 32, k = 2 s + l / 32) then reads its four steps' numbers in one 16-byte load;
+// rows 36 floats apart meet the banks evenly.  (Slabs of 16 in three buffers, the next one's operands read ahead: 149 us.)
+// WHOLE: K is a multiple of 4, so four elements along K are all inside or all outside.
+constexpr int LK = 32, LLD = LK + 4;
+
+// Eight numbers along K of a row.  What lies beyond K is read from inside the row instead (a load behind a condition would be
+// waited for where the paths meet, before the matrix instructions and not behind them) and zeroed by `lay8`.
+template <typename TI, bool WHOLE>
+__device__ __forceinline__ void load8(const TI* __restrict__ row, int k, int K, TI* v) {
+  if (WHOLE) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = to_float(p[i]);
-        } else {                                        // (K need be no multiple of 4: zeros beyond it)
+    for (int h = 0; h < 2; ++h) {
+      const TI* p = row + min(k + 4 * h, K - 4);
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (k + i < K) v[i] = to_float(p[i]);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) As[lk + i][lrow] = v[i];
-      int n = n0 + lrow;
-      float w[4] = {0.f, 0.f, 0.f, 0.f};
-      if (n < N && k < K) {
-        const TI* p = W + static_cast<size_t>(n) * K + k;
-        if (WHOLE || k + 4 <= K) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) w[i] = to_float(p[i]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (k + i < K) w[i] = to_float(p[i]);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) Ws[lk + i][lrow] = w[i];
+      for (int i = 0; i < 4; ++i) v[4 * h + i] = p[i];
     }
-    __syncthreads();
+  } else {
 #pragma unroll
-    for (int k = 0; k < BK; ++k) {
-      float a[4], w[4];
+    for (int i = 0; i < 8; ++i) v[i] = row[min(k + i, K - 1)];
+  }
+}
+
+template <typename TI>
+__device__ __forceinline__ void lay8(float* at, const TI* v, int inside) {
+  float f[8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[k][ty * 4 + i];
+  for (int i = 0; i < 8; ++i) f[i] = i < inside ? to_float(v[i]) : 0.f;
+  *reinterpret_cast<float4*>(at) = float4{f[0], f[2], f[4], f[6]};
+  *reinterpret_cast<float4*>(at + 4) = float4{f[1], f[3], f[5], f[7]};
+}
+
+template <typename TI, typename TC, bool WHOLE>
+__global__ __launch_bounds__(256, 4) void gemm_kernel(const TI* __restrict__ A, int lda, const TI* __restrict__ W,
+                                                       const float* __restrict__ bias, TC* __restrict__ C, int ldc,
+                                                       float* __restrict__ resid, int ldr, int M, int N, int K,
+                                                       int epi, int mtiles, int tiles, int per_xcd) {
+  __shared__ __attribute__((aligned(16))) float As[2][BM * LLD];
+  __shared__ __attribute__((aligned(16))) float Ws[2][BN * LLD];
+  // each of the 8 XCDs, among which workgroups go round, takes a run of tiles, rows first: its L2 then serves a few column
+  // tiles' weights and the rows
+  const int tile = static_cast<int>(blockIdx.x % 8) * per_xcd + static_cast<int>(blockIdx.x / 8);
+  if (tile >= tiles) return;
+  const int t = threadIdx.x, lane = t % 64, wave = t / 64;
+  const int m0 = tile % mtiles * BM, n0 = tile / mtiles * BN;
+  const int lrow = t / 4, lk = (t % 4) * 8;             // loader: 64 rows x 4 groups of 8 k
+  // (rows beyond M and N: the last one again; what they give is not stored)
+  const TI* arow = A + static_cast<size_t>(min(m0 + lrow, M - 1)) * lda;
+  const TI* wrow = W + static_cast<size_t>(min(n0 + lrow, N - 1)) * K;
+  const int wm = wave / 2 * 32, wn = wave % 2 * 32;
+  const int fa = (wm + lane % 32) * LLD + 4 * (lane / 32), fw = (wn + lane % 32) * LLD + 4 * (lane / 32);
+  f32x16 acc, tot;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = Ws[k][tx * 4 + j];
+  for (int r = 0; r < 16; ++r) acc[r] = tot[r] = 0.f;
+  TI av[8], wv[8];
+  load8<TI, WHOLE>(arow, lk, K, av);
+  load8<TI, WHOLE>(wrow, lk, K, wv);
+  lay8(&As[0][lrow * LLD + lk], av, K - lk);
+  lay8(&Ws[0][lrow * LLD + lk], wv, K - lk);
+  load8<TI, WHOLE>(arow, LK + lk, K, av);
+  load8<TI, WHOLE>(wrow, LK + lk, K, wv);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += LK, buf ^= 1) {
+    // a slab's operands are read at once; in the middle of its matrix instructions the next slab is laid down and the one
+    // after it asked for, so that only the barrier stands between two slabs' matrix instructions
+    float4 a[LK / 8], w[LK / 8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
+    for (int g = 0; g < LK / 8; ++g) {
+      a[g] = *reinterpret_cast<const float4*>(&As[buf][fa + 8 * g]);
+      w[g] = *reinterpret_cast<const float4*>(&Ws[buf][fw + 8 * g]);
     }
-    if ((k0 + BK) % SEG == 0 || k0 + BK >= K) {     // a segment ends: its sum joins the others'
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int g = 0; g < LK / 8; ++g) {
+      if (g == LK / 16) {
+        __builtin_amdgcn_sched_barrier(0);
+        const int inside = k0 + 2 * LK <= K ? 8 : K - (k0 + LK + lk);
+        lay8(&As[buf ^ 1][lrow * LLD + lk], av, inside);      // (behind the last slab: zeros that nobody reads)
+        lay8(&Ws[buf ^ 1][lrow * LLD + lk], wv, inside);
+        load8<TI, WHOLE>(arow, k0 + 2 * LK + lk, K, av);
+        load8<TI, WHOLE>(wrow, k0 + 2 * LK + lk, K, wv);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].x, w[g].x, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].y, w[g].y, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].z, w[g].z, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].w, w[g].w, acc, 0, 0, 0);
+    }
+    if ((k0 + LK) % SEG == 0 || k0 + LK >= K) {         // a segment ends: its sum joins the others'
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          tot[i][j] += acc[i][j];
-          acc[i][j] = 0.f;
-        }
+      for (int r = 0; r < 16; ++r) {
+        tot[r] += acc[r];
+        acc[r] = 0.f;
+      }
     }
     __syncthreads();
   }
+  // a lane holds column lane % 32 of the rows 8 (r / 4) + 4 (lane / 32) + r % 4
+  const int n = n0 + wn + lane % 32;
+  if (n >= N) return;
+  const float b = bias ? bias[n] : 0.f;
+  const int mb = m0 + wm + 4 * (lane / 32);
+  if (resid) {
+    float old[16];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
+    for (int r = 0; r < 16; ++r) {
+      const int m = mb + 8 * (r / 4) + r % 4;
+      old[r] = m < M ? resid[static_cast<size_t>(m) * ldr + n] : 0.f;
+    }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
-      finish<TC>(tot[i][j], m, n, bias, C, ldc, resid, ldr, epi);
+    for (int r = 0; r < 16; ++r) {
+      const int m = mb + 8 * (r / 4) + r % 4;
+      if (m < M) resid[static_cast<size_t>(m) * ldr + n] = old[r] + (bias ? tot[r] + b : tot[r]);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int m = mb + 8 * (r / 4) + r % 4;
+      if (m < M) C[static_cast<size_t>(m) * ldc + n] = from_float<TC>(apply_epilogue(bias ? tot[r] + b : tot[r], epi));
     }
   }
 }
@@ -311,13 +355,16 @@ static int run(const void* A, int lda, const void* W, const float* bias, void* C
   TC* c = static_cast<TC*>(C);
   if (!few_rows_take<TI>(A, lda, W, M, K)) {
     if (kv.slot_map) return DN_ERR_SHAPE;
-    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+    const int mtiles = (M + BM - 1) / BM;
+    const long all = static_cast<long>(mtiles) * ((N + BN - 1) / BN);
+    if (all > (1 << 30)) return DN_ERR_SHAPE;
+    const int tiles = static_cast<int>(all), per_xcd = (tiles + 7) / 8;
     if (K % 4 == 0)
-      hipLaunchKernelGGL((gemm_kernel<TI, TC, true>), grid, dim3(256), 0, stream, a, lda, w, bias, c, ldc, resid, ldr, M, N,
-                         K, epi);
+      hipLaunchKernelGGL((gemm_kernel<TI, TC, true>), dim3(per_xcd * 8), dim3(256), 0, stream, a, lda, w, bias, c, ldc, resid,
+                         ldr, M, N, K, epi, mtiles, tiles, per_xcd);
     else
-      hipLaunchKernelGGL((gemm_kernel<TI, TC, false>), grid, dim3(256), 0, stream, a, lda, w, bias, c, ldc, resid, ldr, M, N,
-                         K, epi);
+      hipLaunchKernelGGL((gemm_kernel<TI, TC, false>), dim3(per_xcd * 8), dim3(256), 0, stream, a, lda, w, bias, c, ldc, resid,
+                         ldr, M, N, K, epi, mtiles, tiles, per_xcd);
     return 0;
   }
   const long need = work_floats(M, N, K);

@@ -1,0 +1,44 @@
+"""The 32-bit kernels on the matrix cores against the kernels that run the same sums as chains of fused multiply-adds:
+the same bits, whichever of them a step takes."""
+import math
+
+import pytest
+import torch
+
+from test_kernels_gpu import i32, ops, paged_case, rnd
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(65, 64, 128), (65, 1, 4), (129, 63, 1), (200, 65, 127), (64 * 9, 257, 129), (130, 200, 1600),
+                                   (67, 130, 250), (300, 96, 34)])
+def test_a_product_of_many_rows_has_the_few_rows_bits(dtype, M, N, K):
+    """Numbers of very different sizes, so that another order or another rounding shows; ends of tiles, of slabs, of segments."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = (torch.randn(M, K, generator=g) * torch.exp2(torch.randint(-12, 13, (M, K), generator=g).float())).to(dtype).to(DEV)
+    w = (torch.randn(N, K, generator=g) * torch.exp2(torch.randint(-12, 13, (N, K), generator=g).float())).to(dtype).to(DEV)
+    bias = rnd(N, seed=1)
+    many = torch.zeros(M, N, device=DEV)
+    ops().linear(a, w, bias, out=many)
+    stream, few_stream = rnd(M, N, seed=2), rnd(M, N, seed=2)
+    ops().linear(a, w, bias, residual=stream)
+    # one order of summation, spelled out: segments of 128 with one rounding a step (64-bit products are exact)
+    rows = torch.tensor(sorted({0, 1, 31, 32, 63, 64, M - 1}))
+    a64, w64 = a[rows].double().cpu(), w.double().cpu()
+    total = torch.zeros(len(rows), N)
+    for seg in range(0, K, 128):
+        acc = torch.zeros(len(rows), N)
+        for k in range(seg, min(K, seg + 128)):
+            acc = (a64[:, k:k + 1] * w64[None, :, k] + acc.double()).float()
+        total = total + acc
+    want = total + bias.cpu()
+    # (64 bits round the sum once before 32 bits do: two roundings differ from one in a few of a thousand million cases)
+    assert (many[rows].cpu() != want).float().mean() < 1e-4, (M, N, K)
+    if K % 4 == 0:      # the kernel for few rows takes these
+        few = torch.zeros(M, N, device=DEV)
+        for m in range(0, M, 64):
+            ops().linear(a[m:m + 64], w, bias, out=few[m:m + 64])
+            ops().linear(a[m:m + 64], w, bias, residual=few_stream[m:m + 64])
+        assert torch.equal(many, few) and torch.equal(stream, few_stream), (M, N, K)
