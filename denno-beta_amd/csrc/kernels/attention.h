@@ -49,6 +49,14 @@ int dn_attention_rows_extras(const void* q, int ldq, void* out, int ldo, const v
                              int window, int chunk, const float* bias, int span, int sink, const float* sink_at, int keep, float cap,
                              int dtype, hipStream_t stream);
 
+// dn_attention_extras in 32-bit over tiles of up to 128 rows, on the matrix cores: the same bits (head sizes that are
+// multiples of 16 up to 128, pages of a multiple of 16 keys, pools and out 16-byte aligned, ldo a multiple of 4)
+int dn_attention_portions(const void* q, int ldq, void* out, int ldo, const void* k_pool, const void* v_pool,
+                          const int32_t* block_tables, int max_blocks, const int32_t* tile_seq, const int32_t* tile_row0,
+                          const int32_t* tile_nrows, const int32_t* tile_pos0, int n_tiles, int H, int Hkv, int dh,
+                          int page_size, float scale, int window, int chunk, const float* bias, int span, int sink,
+                          const float* sink_at, int keep, float cap, hipStream_t stream);
+
 // the same kernels' arithmetic for a step of single rows (tile s = request s = row s), every tile of keys a
 // workgroup of its own; part: n_tiles * H * ceil(max_context / dn_attention_rows_tile(dh)) * (dh + 2) floats
 int dn_attention_rows_tile(int dh);

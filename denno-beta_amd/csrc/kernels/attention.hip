@@ -296,6 +296,209 @@ __global__ __launch_bounds__(THREADS) void attention_kernel(
   }
 }
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// The value of the lane 16 away inside each half of the wave (an exchange through the LDS crossbar, no memory).
+__device__ __forceinline__ float other_row(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x401F));
+}
+
+// Portions, 32-bit, on the matrix cores: the sums of attention_kernel in the same order, so the same bits.
+// v_mfma_f32_16x16x4_f32 adds its four products one after the other, k ascending, each with one rounding and subnormals
+// kept: exactly key_dot's chain over the dims and dim_sum's over the keys.  attention_kernel reads two numbers from LDS a
+// multiply-add, which bounds it: two portions of 1,024 rows with 16 heads of 64 take it 778 us a layer and this one 129.
+// A workgroup is 64 rows of a wide tile (half = which 64), a wave 16 of them.  K . Q^T puts a row's scores on the four lanes
+// row, row + 16, row + 32, row + 48; the keys of a run of 16 go to the product's rows in the order 0 4 8 12 1 5 9 13 ..., so
+// that lane row + 16 q holds the keys 4 r + q in its register r: just what V^T . P^T wants as its second operand in step r.
+// Both operands wait in LDS with every 16 numbers that a product walks through turned 4 x 4, so that a lane reads its four
+// steps in one 16-byte load.  The next tile's keys and values wait in registers, the pages of the one after it too.
+// NDIM: head size / 16 (up to 8); the keys of a tile: tile_keys(head size).
+template <int NDIM>
+__global__ __launch_bounds__(256, 2) void portion_kernel(
+    const float* __restrict__ q, int ldq, float* __restrict__ out, int ldo, const float* __restrict__ k_pool,
+    const float* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks,
+    const int32_t* __restrict__ tile_seq, const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ tile_nrows,
+    const int32_t* __restrict__ tile_pos0, int H, int Hkv, int page_size, float scale, int window, ScoreExtras ex) {
+  constexpr int DH = 16 * NDIM, BK = NDIM <= 4 ? 64 : 32, NC = BK / 16, KLD = DH + 4, VLD = BK + 4;
+  __shared__ __attribute__((aligned(16))) float Ks[BK * KLD];
+  __shared__ __attribute__((aligned(16))) float Vs[DH * VLD];
+  const int tile = blockIdx.x / 2, half = 1 - blockIdx.x % 2, h = blockIdx.y;     // (the half with more keys first)
+  const int seq = tile_seq[tile];
+  const int nrows = min(64, tile_nrows[tile] - 64 * half);
+  if (seq < 0 || nrows <= 0) return;
+  const int row0 = tile_row0[tile] + 64 * half, pos0 = tile_pos0[tile] + 64 * half;
+  const int hk = h / (H / Hkv);
+  const int32_t* bt = block_tables + static_cast<size_t>(seq) * max_blocks;
+  const int t = threadIdx.x, lane = t % 64, w0 = t / 64 * 16;
+  const int i16 = lane % 16, quarter = lane / 16;
+  const bool row_ok = w0 + i16 < nrows;
+  const int pos = pos0 + w0 + i16;
+  const int lo = first_key(pos, window, ex.chunk);
+  const int last_pos = pos0 + nrows - 1;
+  const int wave_last = pos0 + min(w0 + 16, nrows) - 1;      // (a wave without rows: below its own first)
+  const bool wave_ok = w0 < nrows;
+  const float* bias = ex.bias ? ex.bias + static_cast<size_t>(h) * ex.span : nullptr;
+  const float NEG_INF = -INFINITY;
+
+  // the wave's queries: step s of the product over the dims reads dim 4 s + quarter
+  float qv[4 * NDIM];
+  {
+    const float* qr = q + static_cast<size_t>(row0 + (row_ok ? w0 + i16 : 0)) * ldq + h * DH + quarter;
+#pragma unroll
+    for (int s = 0; s < 4 * NDIM; ++s) qv[s] = row_ok ? qr[4 * s] : 0.f;
+  }
+
+  // loader: 16 dims of a key, and 16 keys of a dim (one page: pages hold a multiple of 16 keys)
+  const bool loads = t < BK * NDIM;
+  const int k_key = t / NDIM, k_a = t % NDIM, v_dim = t / NC, v_c = t % NC;
+  const TileWalk walk(BK, first_key(pos0, window, ex.chunk), ex.keep);
+  auto page_of = [&](int key) { return loads && key <= last_pos ? bt[key / page_size] : -1; };
+  float4 kr[4], vr[4];
+  auto ask = [&](int kt, int k_page, int v_page) {
+    const int kkey = kt + k_key, vkey = kt + 16 * v_c;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) kr[b] = vr[b] = float4{0.f, 0.f, 0.f, 0.f};
+    if (k_page >= 0) {
+      const float* p = k_pool + ((static_cast<size_t>(k_page) * Hkv + hk) * page_size + kkey % page_size) * DH + 16 * k_a;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) kr[b] = *reinterpret_cast<const float4*>(p + 4 * b);
+    }
+    if (v_page >= 0) {
+      const float* p = v_pool + ((static_cast<size_t>(v_page) * Hkv + hk) * DH + v_dim) * page_size + vkey % page_size;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) vr[b] = *reinterpret_cast<const float4*>(p + 4 * b);
+    }
+  };
+  auto lay = [&](int kt) {
+    if (!loads) return;
+    float* kd = &Ks[k_key * KLD + 16 * k_a];
+    *reinterpret_cast<float4*>(kd) = float4{kr[0].x, kr[1].x, kr[2].x, kr[3].x};
+    *reinterpret_cast<float4*>(kd + 4) = float4{kr[0].y, kr[1].y, kr[2].y, kr[3].y};
+    *reinterpret_cast<float4*>(kd + 8) = float4{kr[0].z, kr[1].z, kr[2].z, kr[3].z};
+    *reinterpret_cast<float4*>(kd + 12) = float4{kr[0].w, kr[1].w, kr[2].w, kr[3].w};
+    const int over = last_pos - (kt + 16 * v_c);             // keys beyond the last row: zeros
+    float* vd = &Vs[v_dim * VLD + 16 * v_c];
+    float e[16];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) e[4 * b] = vr[b].x, e[4 * b + 1] = vr[b].y, e[4 * b + 2] = vr[b].z, e[4 * b + 3] = vr[b].w;
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      if (j > over) e[j] = 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) *reinterpret_cast<float4*>(vd + 4 * g) = float4{e[g], e[4 + g], e[8 + g], e[12 + g]};
+  };
+
+  float m = NEG_INF, l = 0.f;
+  f32x4 acc[NDIM];
+#pragma unroll
+  for (int d = 0; d < NDIM; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  int kt = walk.first(), next = walk.next(kt);
+  ask(kt, page_of(kt + k_key), page_of(kt + 16 * v_c));
+  int k_page = page_of(next + k_key), v_page = page_of(next + 16 * v_c);
+  while (kt <= last_pos) {
+    __syncthreads();
+    lay(kt);
+    __syncthreads();
+    const int after = walk.next(next);
+    if (next <= last_pos) {
+      ask(next, k_page, v_page);
+      k_page = page_of(after + k_key), v_page = page_of(after + 16 * v_c);
+    }
+    if (wave_ok && kt <= wave_last) {
+      f32x4 s[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) s[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const float* kf = &Ks[(4 * (i16 % 4) + i16 / 4) * KLD + 4 * quarter];
+#pragma unroll
+      for (int a = 0; a < NDIM; ++a)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const float4 k4 = *reinterpret_cast<const float4*>(kf + 16 * c * KLD + 16 * a);
+          s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.x, qv[4 * a], s[c], 0, 0, 0);
+          s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.y, qv[4 * a + 1], s[c], 0, 0, 0);
+          s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.z, qv[4 * a + 2], s[c], 0, 0, 0);
+          s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.w, qv[4 * a + 3], s[c], 0, 0, 0);
+        }
+      float m_t = NEG_INF;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = kt + 16 * c + 4 * r + quarter;
+          const bool ok = row_ok && reads_key(key, lo, pos, ex.keep);
+          s[c][r] = ok ? score_of(s[c][r], scale, ex.cap, bias, pos - key, ex.span) : NEG_INF;
+          m_t = fmaxf(m_t, s[c][r]);
+        }
+      m_t = fmaxf(m_t, other_row(m_t));
+      m_t = fmaxf(m_t, other_half(m_t));
+      // the sum of p over the keys g, g + 16, ... for each g = 4 r + quarter, then the sixteen sums as group_reduce<16> joins them
+      float four[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float psum = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          s[c][r] = s[c][r] > NEG_INF ? expf(s[c][r] - m_t) : 0.f;
+          psum += s[c][r];
+        }
+        psum += other_row(psum);
+        psum += other_half(psum);
+        four[r] = psum;
+      }
+      const float l_t = (four[0] + four[1]) + (four[2] + four[3]);
+      f32x4 a_t[NDIM];
+#pragma unroll
+      for (int d = 0; d < NDIM; ++d) a_t[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const bool edge = kt + BK - 1 > wave_last;             // keys that other waves' rows read and these do not: no values
+      const float* vf = &Vs[i16 * VLD + 4 * quarter];
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int d = 0; d < NDIM; ++d) {
+          float4 v4 = *reinterpret_cast<const float4*>(vf + 16 * d * VLD + 16 * c);
+          if (edge) {
+            const int over = wave_last - (kt + 16 * c + quarter);
+            if (over < 0) v4.x = 0.f;
+            if (over < 4) v4.y = 0.f;
+            if (over < 8) v4.z = 0.f;
+            if (over < 12) v4.w = 0.f;
+          }
+          a_t[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.x, s[c][0], a_t[d], 0, 0, 0);
+          a_t[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.y, s[c][1], a_t[d], 0, 0, 0);
+          a_t[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.z, s[c][2], a_t[d], 0, 0, 0);
+          a_t[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.w, s[c][3], a_t[d], 0, 0, 0);
+        }
+      if (m_t > NEG_INF) {                                   // the same for the four lanes of a row: join_tile
+        if (!(m > NEG_INF)) {
+          m = m_t;
+          l = l_t;
+#pragma unroll
+          for (int d = 0; d < NDIM; ++d) acc[d] = a_t[d];
+        } else {
+          const float m_new = fmaxf(m, m_t);
+          const float alpha = expf(m - m_new), beta = expf(m_t - m_new);
+          l = fmaf(l_t, beta, l * alpha);
+#pragma unroll
+          for (int d = 0; d < NDIM; ++d)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[d][r] = fmaf(a_t[d][r], beta, acc[d][r] * alpha);
+          m = m_new;
+        }
+      }
+    }
+    kt = next;
+    next = after;
+  }
+  if (row_ok) {
+    const float inv = 1.0f / (ex.sink ? l + expf(sink_score(ex, h) - m) : l);
+    float* o = out + static_cast<size_t>(row0 + w0 + i16) * ldo + h * DH + 4 * quarter;
+#pragma unroll
+    for (int d = 0; d < NDIM; ++d)
+      *reinterpret_cast<float4*>(o + 16 * d) = float4{acc[d][0] * inv, acc[d][1] * inv, acc[d][2] * inv, acc[d][3] * inv};
+  }
+}
+
 // A step of single rows (request s = tile s = row s): every tile of keys is a workgroup of its own, so
 // that a context of a thousand keys is sixteen workgroups side by side and not sixteen steps of one.  It
 // leaves (m_T, l_T, a_T) in part[((tile * H + h) * n_key_tiles + key tile) * (dh + 2)]; m_T = -inf: the
@@ -552,6 +755,44 @@ extern "C" int dn_attention_extras(const void* q, int ldq, void* out, int ldo, c
                        tile_nrows, tile_pos0, H, Hkv, dh, page_size, BK, scale, window, ex);
   else
     return DN_ERR_DTYPE;
+  return dn_launch_status();
+}
+
+// The 32-bit kernel for portions on the matrix cores, over the wide tiles (up to 128 rows): the same bits as
+// dn_attention_extras gives over the narrow ones.  Head sizes that are multiples of 16 up to 128, pages of a multiple of 16
+// keys; everything else is refused here and takes that kernel.
+extern "C" int dn_attention_portions(const void* q, int ldq, void* out, int ldo, const void* k_pool, const void* v_pool,
+                                     const int32_t* block_tables, int max_blocks, const int32_t* tile_seq,
+                                     const int32_t* tile_row0, const int32_t* tile_nrows, const int32_t* tile_pos0,
+                                     int n_tiles, int H, int Hkv, int dh, int page_size, float scale, int window, int chunk,
+                                     const float* bias, int span, int sink, const float* sink_at, int keep, float cap,
+                                     hipStream_t stream) {
+  if (n_tiles <= 0) return 0;
+  if (chunk < 0 || !(cap >= 0.f) || (bias && span < 1) || !keep_ok(keep, window, chunk)) return DN_ERR_SHAPE;
+  if (dh < 16 || dh > 128 || dh % 16 != 0 || Hkv < 1 || H % Hkv != 0 || page_size < 16 || page_size % 16 != 0 || max_blocks < 1)
+    return DN_ERR_SHAPE;
+  if (ldo % 4 != 0 || reinterpret_cast<uintptr_t>(out) % 16 != 0 || reinterpret_cast<uintptr_t>(k_pool) % 16 != 0 ||
+      reinterpret_cast<uintptr_t>(v_pool) % 16 != 0)
+    return DN_ERR_SHAPE;
+  const ScoreExtras ex{chunk, bias, span, sink, sink_at, keep, cap};
+#define DN_PORTION(ND)                                                                                                \
+  case ND:                                                                                                            \
+    hipLaunchKernelGGL((plain::portion_kernel<ND>), dim3(2 * n_tiles, H), dim3(256), 0, stream,                       \
+                       static_cast<const float*>(q), ldq, static_cast<float*>(out), ldo,                              \
+                       static_cast<const float*>(k_pool), static_cast<const float*>(v_pool), block_tables, max_blocks, \
+                       tile_seq, tile_row0, tile_nrows, tile_pos0, H, Hkv, page_size, scale, window, ex);             \
+    break
+  switch (dh / 16) {
+    DN_PORTION(1);
+    DN_PORTION(2);
+    DN_PORTION(3);
+    DN_PORTION(4);
+    DN_PORTION(5);
+    DN_PORTION(6);
+    DN_PORTION(7);
+    DN_PORTION(8);
+  }
+#undef DN_PORTION
   return dn_launch_status();
 }
 

@@ -118,6 +118,7 @@ def _declare(name, lib):
         },
         "attention": {
             "dn_attention": [P, I, P, I, P, P, P, I, P, P, P, P, I, I, I, I, I, F, I, I, P],
+            "dn_attention_portions": [P, I, P, I, P, P, P, I, P, P, P, P, I, I, I, I, I, F, I, I, P, I, I, P, I, F, P],
             "dn_attention_rows": [P, I, P, I, P, P, P, I, P, P, I, P, I, I, I, I, I, F, I, I, P],
             "dn_attention_rows_tile": [I],
             "dn_attention_extras": [P, I, P, I, P, P, P, I, P, P, P, P, I, I, I, I, I, F, I, I, P, I, I, P, I, F, I, P],
@@ -761,6 +762,19 @@ def attention(q, out, k_pool, v_pool, block_tables, tiles, n_heads, scale, windo
             block_tables.shape[1], base, base + 12 * n_tiles, n_tiles, part.data_ptr(), int(max_context), n_heads, Hkv,
             dh, ps, float(scale), int(window), int(chunk), _ptr(bias), span, int(sink), _ptr(sink_at), keep_first, float(softcap),
             _CODE[q.dtype], _stream()), "attention (single rows)")
+        return out
+    if (q.dtype == torch.float32 and tiles_wide is not None and dh % 16 == 0 and dh <= 128 and ps % 16 == 0 and ldo % 4 == 0
+            and out.data_ptr() % 16 == 0 and k_pool.data_ptr() % 16 == 0 and v_pool.data_ptr() % 16 == 0):
+        # the same sums on the matrix cores (two portions of 1,024 rows with 16 heads of 64: 778 -> 129 us a layer); what it does not take goes on below
+        _dev(tiles_wide, "tiles_wide", _I32, 2)
+        _need(tiles_wide.is_contiguous() and tiles_wide.shape[0] == 4, "attention: tiles_wide")
+        n_tiles = tiles_wide.shape[1]
+        base = tiles_wide.data_ptr()
+        _ok(lib.dn_attention_portions(
+            q.data_ptr(), ldq, out.data_ptr(), ldo, k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),
+            block_tables.shape[1], base, base + 4 * n_tiles, base + 8 * n_tiles, base + 12 * n_tiles, n_tiles,
+            n_heads, Hkv, dh, ps, float(scale), int(window), int(chunk), _ptr(bias), span, int(sink), _ptr(sink_at), keep_first,
+            float(softcap), _stream()), "attention (32-bit portions)")
         return out
     _ok(lib.dn_attention_extras(
         q.data_ptr(), ldq, out.data_ptr(), ldo, k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),

@@ -42,3 +42,32 @@ def test_a_product_of_many_rows_has_the_few_rows_bits(dtype, M, N, K):
             ops().linear(a[m:m + 64], w, bias, out=few[m:m + 64])
             ops().linear(a[m:m + 64], w, bias, residual=few_stream[m:m + 64])
         assert torch.equal(many, few) and torch.equal(stream, few_stream), (M, N, K)
+
+
+@pytest.mark.parametrize("H,Hkv,dh,ps,kw", [
+    (2, 2, 16, 16, {}), (3, 1, 32, 16, {}), (2, 2, 48, 48, {}), (4, 2, 64, 16, {}), (2, 2, 64, 64, dict(window=70)), (2, 1, 80, 32, {}),
+    (2, 2, 96, 16, dict(window=33)), (1, 1, 112, 16, {}), (2, 1, 128, 32, {}), (2, 2, 64, 16, dict(chunk=50, sink=True)),
+    (2, 2, 64, 32, dict(window=40, keep_first=5, softcap=20.0)), (2, 2, 32, 16, dict(bias=True))])
+def test_portions_have_the_narrow_kernels_bits(H, Hkv, dh, ps, kw):
+    """Portions that end at every place in a tile of rows and start at every place in a tile of keys; the cache holds NaN
+    beyond a request's tokens and in pages that no request has, and infinities in tokens that come later."""
+    seq_lens, new_rows = [300, 64, 133, 1, 430, 129, 65], [1, 64, 21, 1, 300, 129, 16]
+    q, k, v, bt, tiles, T = paged_case(seq_lens, new_rows, H, Hkv, dh, ps, torch.float32, seed=H + dh)
+    used = torch.zeros(k.shape[0], ps, dtype=torch.bool)
+    for s, n in enumerate(seq_lens):
+        for p in range(n):
+            used[int(bt[s, p // ps]), p % ps] = True
+    spare = ~used.to(DEV)
+    k.masked_fill_(spare[:, None, :, None], math.nan), v.masked_fill_(spare[:, None, None, :], math.nan)
+    last = int(bt[4, 429 // ps])
+    v[last, :, :, 429 % ps] = math.inf
+    kw = dict(kw)
+    window = kw.pop("window", 0)
+    if kw.get("bias"):
+        kw["bias"] = rnd(H, 100, seed=3)
+    args = (k, v, bt, tiles, H, 1 / math.sqrt(dh), window)
+    narrow, wide = torch.zeros(T, H * dh, device=DEV), torch.zeros(T, H * dh, device=DEV)
+    ops().attention(q[:, H * dh:2 * H * dh], narrow, *args, **kw)
+    ops().attention(q[:, H * dh:2 * H * dh], wide, *args, tiles_wide=paged_case.wide, **kw)
+    assert torch.equal(narrow.nan_to_num(nan=7e30), wide.nan_to_num(nan=7e30)), (narrow - wide).abs().nan_to_num().max()
+    assert torch.isfinite(wide[:-17]).float().mean() > 0.9
