@@ -57,8 +57,29 @@ __device__ __forceinline__ void wait_loads() {      // until at most N of this w
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// WM x WN waves, each TM x TN blocks of 16 x 16: the tile is 16 WM TM rows x 16 WN TN columns
-template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1>
+// Tiles in the order in which a run of them shares most: bands of about 1,024 rows, a band column by column.  Each of the 8 XCDs,
+// among which workgroups go round, takes a run of that order, so that the 32 tiles that its CUs work on at a time are some four by
+// eight and its L2 fetches their rows and columns once.  (With whole columns of tiles one after the other an XCD fetched all rows of A
+// for every column: 8,192 x 1,280 x 5,120 brought 685 MB into the L2s, now 220; 112 -> 103 us, 8,192 x 6,400 x 1,600 222 -> 197.)
+__device__ __forceinline__ void tile_at(int pid, int tiles_m, int tiles_n, int band, int& tm, int& tn) {
+  const int total = tiles_m * tiles_n, each = total / XCDS, more = total % XCDS, x = pid % XCDS;
+  pid = x * each + min(x, more) + pid / XCDS;
+  if (tiles_m <= band) {      // (few rows: one band, and a division less in front of a short kernel)
+    tm = pid % tiles_m;
+    tn = pid / tiles_m;
+    return;
+  }
+  const int in_band = band * tiles_n, b = pid / in_band, first = b * band, rows = min(band, tiles_m - first), i = pid - b * in_band;
+  tm = first + i % rows;
+  tn = i / rows;
+}
+
+// WM x WN waves, each TM x TN blocks of 16 x 16: the tile is 16 WM TM rows x 16 WN TN columns.
+// PING: eight waves, two a SIMD, that take turns: while one reads a stage's operands from LDS and asks for a later stage, the other
+// multiplies (the second half of the waves runs a barrier behind the first).  Without it all waves read at the same time and multiply at the same
+// time, and neither LDS nor the matrix cores are busy for more than half of a stage: 256 x 160 tiles took 0.91 us a stage of 64
+// along K with sixteen waves in step and take 0.76 with eight in turns.
+template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __restrict__ A, int lda,
                                                            const bf16_t* __restrict__ W, const float* __restrict__ bias,
                                                            TC* __restrict__ C, int ldc, float* __restrict__ resid, int ldr,
@@ -73,10 +94,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   constexpr int HI = (PER + NW - 1) / NW, REM = PER % NW;   // waves below REM load HI blocks, the others HI - 1
   static_assert((STAGES - 2) * HI < 64, "vmcnt has six bits");
   extern __shared__ u32x4 lds[];
-  const int total = tiles_m * tiles_n;
-  int pid = blockIdx.x;
-  if (total % XCDS == 0) pid = (pid % XCDS) * (total / XCDS) + pid / XCDS;   // an XCD walks down a column of tiles
-  const int tm = pid % tiles_m, tn = pid / tiles_m;
+  int tm, tn;
+  tile_at(blockIdx.x, tiles_m, tiles_n, 1024 / BM, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -92,6 +111,18 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   // (a packed A is in the operand's order already: lane l reads at 16 l)
   const int aslot = (packed & PACKED_A) ? lane : 16 * (lane % 4) + 4 * ((lane % 16) / 4) + ((lane / 16) ^ (lane % 4));
 
+  // the tokens' slots, which the epilogue reads, are asked for before everything else: the row's, and those of the quad's four tokens
+  // (8,192 rows of fused projections of 4,800 and 3,840 columns: 166 -> 160 and 115 -> 108 us)
+  int kslot[KV ? TM : 1], vslot[KV ? TM : 1][4];
+  if constexpr (KV) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int m = m0 + (wmb + i) * 16 + lane % 16, mq = m - lane % 4;
+      kslot[i] = m < M ? kv.slot_map[m] : -1;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vslot[i][e] = mq + e < M ? kv.slot_map[mq + e] : -1;
+    }
+  }
   floatx4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -135,32 +166,73 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < ksteps) issue(s);
-  for (int kt = 0; kt < ksteps; ++kt) {
-    // slab kt of this wave has landed when only the loads of the STAGES - 2 slabs after it are out
-    if (kt + STAGES - 2 < ksteps) {
-      if (REM == 0 || wave < REM)
-        wait_loads<(STAGES - 2) * HI>();
-      else
-        wait_loads<(STAGES - 2) * (HI - 1)>();
-    } else {
+  // this wave's share of a stage has landed when only its loads of the STAGES - 2 stages after it are out
+  auto landed = [&](bool more) {
+    if (!more)
       wait_loads<0>();
+    else if (REM == 0 || wave < REM)
+      wait_loads<(STAGES - 2) * HI>();
+    else
+      wait_loads<(STAGES - 2) * (HI - 1)>();
+  };
+  if constexpr (PING) {
+    static_assert(NW == 8, "two waves a SIMD");
+    const bool late = wave >= NW / 2;
+    landed(ksteps >= STAGES - 1);
+    __builtin_amdgcn_s_barrier();
+    if (late) __builtin_amdgcn_s_barrier();
+    for (int kt = 0; kt < ksteps; ++kt) {
+      // (a stage is read a barrier after every wave has waited for its share of it, and its place is asked for again two barriers
+      // after its last reader was done)
+      const u32x4* slab = lds + (kt % STAGES) * SLAB;
+      bf16x8 af[KB][TM], wf[KB][TN];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const u32x4* sl = slab + kb * (AB + WB) * 64;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) af[kb][i] = __builtin_bit_cast(bf16x8, sl[(wmb + i) * 64 + aslot]);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) wf[kb][j] = __builtin_bit_cast(bf16x8, sl[(AB + wnb + j) * 64 + lane]);
+      }
+      const bool more = kt + STAGES - 1 < ksteps;
+      if (more) issue(kt + STAGES - 1);
+      landed(more);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[kb][j], af[kb][i], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();      // every wave's share of slab kt is there, and slab kt - 1 has been read
-    if (kt + STAGES - 1 < ksteps) issue(kt + STAGES - 1);
-    const u32x4* slab = lds + (kt % STAGES) * SLAB;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      const u32x4* sl = slab + kb * (AB + WB) * 64;
-      bf16x8 af[TM], wf[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = __builtin_bit_cast(bf16x8, sl[(wmb + i) * 64 + aslot]);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) wf[j] = __builtin_bit_cast(bf16x8, sl[(AB + wnb + j) * 64 + lane]);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
+    if (!late) __builtin_amdgcn_s_barrier();
+  } else {
+    for (int kt = 0; kt < ksteps; ++kt) {
+      landed(kt + STAGES - 2 < ksteps);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();      // every wave's share of slab kt is there, and slab kt - 1 has been read
+      if (kt + STAGES - 1 < ksteps) issue(kt + STAGES - 1);
+      const u32x4* slab = lds + (kt % STAGES) * SLAB;
+  #pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const u32x4* sl = slab + kb * (AB + WB) * 64;
+        bf16x8 af[TM], wf[TN];
+  #pragma unroll
+        for (int i = 0; i < TM; ++i) af[i] = __builtin_bit_cast(bf16x8, sl[(wmb + i) * 64 + aslot]);
+  #pragma unroll
+        for (int j = 0; j < TN; ++j) wf[j] = __builtin_bit_cast(bf16x8, sl[(AB + wnb + j) * 64 + lane]);
+  #pragma unroll
+        for (int i = 0; i < TM; ++i)
+  #pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
+      }
     }
   }
   // acc[i][j][r]: row m0 + 16 (wmb + i) + lane % 16, column n0 + 16 (wnb + j) + 4 (lane / 16) + r
@@ -172,23 +244,16 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   // multiple of 4 are 8 bytes side by side for one dim: the four lanes of a quad, which hold four
   // tokens x four dims, exchange them (a 4 x 4 turn), and each stores four tokens of one dim.
   int kpage[KV ? TM : 1], koff[KV ? TM : 1], vpage[KV ? TM : 1], voff[KV ? TM : 1];
-  int vslot[KV ? TM : 1][4];      // the quad's four tokens' slots, for values that do not lie side by side (decoded tokens)
   if constexpr (KV) {
 #pragma clang loop unroll(full)
     for (int i = 0; i < TM; ++i) {
-      const int m = m0 + (wmb + i) * 16 + lane % 16, mq = m - lane % 4;
-      const int slot = m < M ? kv.slot_map[m] : -1;
-      page_and_offset(kv, max(slot, 0), kpage[i], koff[i]);
-      if (slot < 0) kpage[i] = -1, koff[i] = 0;
-      int sq[4];
-#pragma clang loop unroll(full)
-      for (int e = 0; e < 4; ++e) sq[e] = mq + e < M ? kv.slot_map[mq + e] : -1;
+      page_and_offset(kv, max(kslot[i], 0), kpage[i], koff[i]);
+      if (kslot[i] < 0) kpage[i] = -1, koff[i] = 0;
+      const int* sq = vslot[i];
       const bool run = kv.page_size % 4 == 0 && sq[0] >= 0 && sq[0] % 4 == 0 && sq[1] == sq[0] + 1 && sq[2] == sq[0] + 2 &&
                        sq[3] == sq[0] + 3;
       page_and_offset(kv, max(sq[0], 0), vpage[i], voff[i]);
       if (!run) vpage[i] = -1, voff[i] = 0;
-#pragma clang loop unroll(full)
-      for (int e = 0; e < 4; ++e) vslot[i][e] = sq[e];
     }
   }
   if (part) {
@@ -294,7 +359,7 @@ bool takes(const void* A, int lda, const void* W, const float* bias, const void*
 }
 
 
-template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1>
+template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false>
 static int launch(const Args& a, hipStream_t stream) {
   constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
@@ -302,13 +367,13 @@ static int launch(const Args& a, hipStream_t stream) {
   if (a.K % (32 * KB) != 0) return DN_ERR_SHAPE;
   static bool raised = false;      // more than 64 KB of LDS has to be asked for once per kernel
   if (lds > 65536 && !raised) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     if (e != hipSuccess) return static_cast<int>(e);
     raised = true;
   }
   const int split_slabs = (a.K / (32 * KB) + a.splits - 1) / a.splits;
-  hipLaunchKernelGGL((gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB>), dim3(tiles_m * tiles_n, a.part ? a.splits : 1),
+  hipLaunchKernelGGL((gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING>), dim3(tiles_m * tiles_n, a.part ? a.splits : 1),
                      dim3(WM * WN * 64), lds, stream, static_cast<const bf16_t*>(a.A), a.lda,
                      static_cast<const bf16_t*>(a.W), a.bias, static_cast<TC*>(a.C), a.ldc, a.resid, a.ldr, a.M, a.N, a.K,
                      a.epi, a.packed, tiles_m, tiles_n, a.kv ? *a.kv : KVScatter{}, a.part, split_slabs);
@@ -323,10 +388,10 @@ static int launch_as(const Args& a, hipStream_t stream) {
 }
 
 // (for tiles that never write the cache: the variant with the cache write is not built)
-template <int WM, int WN, int TM, int TN, int STAGES, int KB = 1>
+template <int WM, int WN, int TM, int TN, int STAGES, int KB = 1, bool PING = false>
 static int launch_without_kv(const Args& a, hipStream_t stream) {
-  if (a.out_dtype == DN_BF16 && !a.resid) return launch<bf16_t, WM, WN, TM, TN, STAGES, false, KB>(a, stream);
-  return launch<float, WM, WN, TM, TN, STAGES, false, KB>(a, stream);
+  if (a.out_dtype == DN_BF16 && !a.resid) return launch<bf16_t, WM, WN, TM, TN, STAGES, false, KB, PING>(a, stream);
+  return launch<float, WM, WN, TM, TN, STAGES, false, KB, PING>(a, stream);
 }
 
 // The tiles that `pick` chooses among: rows x columns, and the slabs in flight that its model counts LDS with.
@@ -434,7 +499,12 @@ int run(const Args& a, hipStream_t stream) {
       return launch_as<2, 2, 2, 4, 4>(a, stream);
     case 1: return sixteen && two ? launch_as<4, 4, 2, 2, 3, 2>(a, stream) : launch_as<4, 2, 2, 4, 4>(a, stream);
     case 2: return sixteen && two ? launch_as<8, 2, 2, 4, 3, 2>(a, stream) : launch_as<4, 2, 4, 4, 4>(a, stream);
-    case 3: return sixteen && two ? launch_as<8, 2, 2, 5, 3, 2>(a, stream) : launch_as<4, 2, 4, 5, 4>(a, stream);
+    case 3:
+      if (!sixteen || !two) return launch_as<4, 2, 4, 5, 4>(a, stream);
+      // (the cache write's epilogue is the longer the more blocks a wave has: 2,048 x 4,800 x 1,600 46.8 us with sixteen waves
+      // in step, 54.9 with eight in turns)
+      if (a.kv) return launch<bf16_t, 8, 2, 2, 5, 3, true, 2>(a, stream);
+      return launch_without_kv<4, 2, 4, 5, 3, 2, true>(a, stream);
     case 4:
       if (!sixteen) return launch_as<4, 2, 4, 6, 4>(a, stream);
       return two && short_k ? launch_as<8, 2, 2, 6, 2, 2>(a, stream) : launch_as<8, 2, 2, 6, 3>(a, stream);
