@@ -21,3 +21,19 @@ def test_every_tile_is_made_once(M, N, K):
     x = stream.clone()
     ops().linear(a, wp, bias, residual=x)
     assert (x - (stream + want)).abs().max().item() < 1e-3
+
+
+@pytest.mark.parametrize("M,N,K", [(257, 1280, 5120), (320, 1280, 1280), (384, 1024, 4096), (512, 1280, 5120), (511, 96, 4096)])
+def test_sums_left_for_the_norm_beyond_256_rows(M, N, K):
+    o = ops()
+    a, w, bias = rnd(M, K, seed=M, dtype=torch.bfloat16), rnd(N, K, seed=N, dtype=torch.bfloat16, scale=0.05), rnd(N, seed=3)
+    wp, x0, gamma, beta = o.pack_matrix(w), rnd(M, N, seed=4), rnd(N, seed=5), rnd(N, seed=6)
+    shares = o.linear_deferred_shares(M, wp, rows_max=512)
+    assert shares >= 2
+    part = o.linear_deferred(a, wp)
+    assert part.shape == (shares, M, N)
+    x, out = x0.clone(), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    o.layernorm_join(x, part, bias, gamma, beta, 1e-5, out)
+    want = (x0.double() + a.double() @ w.double().t() + bias.double()).float()
+    assert torch.allclose(x, want, atol=2e-3, rtol=1e-4)
+    assert torch.equal(out, o.layernorm(x, gamma, beta, 1e-5, torch.empty_like(out)))
