@@ -733,6 +733,7 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
   constexpr int NL = DK >= 64 ? DK / 64 : 1;
   // TB: rows asked for at a time (a trip to memory is paid once per TB rows, not per row; all TB places are worked on,
   // so steps of single rows take a small TB).  A row's sums are the same for every TB.
+  constexpr int GR = KQ <= 4 ? (TB < 4 ? TB : 4) : KQ <= 8 ? 2 : 1;      // rows whose operands are read at a time
   constexpr int N4 = TB * DK / 4, NV = N4 >= 64 ? N4 / 64 : 1;      // VEC: groups of four numbers per array, per lane
   __shared__ __attribute__((aligned(16))) float sh[TB][PARTS * DK];
   __shared__ __attribute__((aligned(16))) float shv[TB][CW];
@@ -741,6 +742,7 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
   const int s = blockIdx.z, h = blockIdx.y, lane = threadIdx.x;
   const int hq = h / (a.H / a.G);                     // the head of r and k that this head reads
   const float wh = a.w_head ? a.w_head[h] : 1.0f;     // one decay for the head, where w is none
+  const bool w_wide = !a.w_head && !a.w_rows;         // a decay per key channel
   const int kg = lane % KG, j0 = blockIdx.x * CW, j = j0 + lane / KG;
   const int slot = a.slots[s];
   if (slot < 0) return;
@@ -749,33 +751,58 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
   const bool live = j < a.dv;
   const int dk = a.dk, dv = a.dv;
   // the state lies [head][value column][key channel]: a lane's channels side by side, a column's lanes too
-  float* sp = a.state + static_cast<size_t>(slot) * a.slot_stride + (static_cast<size_t>(h) * dv + j) * dk + kg * KQ;
+  const size_t at_head = static_cast<size_t>(slot) * a.slot_stride + static_cast<size_t>(h) * dv * dk;
   float S[KQ];
 #pragma unroll
-  for (int q = 0; q < KQ; ++q) S[q] = (live && kg * KQ + q < dk) ? sp[q] : 0.f;
+  for (int q = 0; q < KQ; ++q) S[q] = a.state[at_head + static_cast<size_t>(min(j, dv - 1)) * dk + min(kg * KQ + q, dk - 1)];
+#pragma unroll
+  for (int q = 0; q < KQ; ++q) S[q] = (live && kg * KQ + q < dk) ? S[q] : 0.f;
   for (int i = lane; i < DK; i += 64) shu[i] = (a.u && i < dk) ? a.u[h * dk + i] : 0.f;
   // what a fetch brings: (not VEC) a lane's own numbers row by row; (VEC: every size a multiple of 4 and every row at a
   // multiple of 16 bytes) 16 bytes a lane and load, eight rows of r, k or w in DK / 32 loads: a row then costs a wave
-  // 7 / 8 of a vector load where it cost four, and those loads, not the arithmetic, were what a row waited for
+  // 7 / 8 of a vector load where it cost four, and those loads, not the arithmetic, were what a row waited for.  Every
+  // load is made, from the nearest place there is, and what lies beyond the rows is put right on the way into LDS: a load behind a
+  // condition was waited for by itself (1,024 rows of 8 heads of 64 x 128, delta rule 212 -> 190 us, one decay a row 232 -> 156).
   float nr[VEC ? 1 : TB][NL], nk[VEC ? 1 : TB][NL], nw[VEC ? 1 : TB][NL], nv[VEC ? 1 : TB], nb[VEC ? 1 : TB], nd[VEC ? 1 : TB];
   f32x4 r4[VEC ? NV : 1], k4[VEC ? NV : 1], w4[VEC ? NV : 1], v4;
+  float w1[VEC ? NV : 1];
   auto beta_of = [&](float z) { return a.beta_logits ? 1.0f / (1.0f + expf(-z)) : z; };      // (beta given as it is, or as sigmoid's argument)
   auto decay_of = [&](float z) { return a.w_rate ? expf(-a.w_rate[h] * softplus_f(z + (a.w_bias ? a.w_bias[h] : 0.f))) : z; };
   auto fetch = [&](int t0) {
     if constexpr (VEC) {
-      const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
+      // (32-bit factors: a product of 64-bit numbers is three instructions of four times the length, and a lane makes a dozen)
+      const uint32_t ldr = a.ldr, ldk = a.ldk, ldw = a.ldw;
+      uint32_t t[NV];
+      int i[NV];
 #pragma unroll
       for (int it = 0; it < NV; ++it) {
-        const int idx = it * 64 + lane, bq = idx / (DK / 4), i = (idx % (DK / 4)) * 4, t = t0 + bq;
-        const bool ok = idx < N4 && t < row1 && i < dk;
-        r4[it] = ok ? *reinterpret_cast<const f32x4*>(a.r + t * a.ldr + hq * dk + i) : zero;
-        k4[it] = (ok && !a.key_from_decay) ? *reinterpret_cast<const f32x4*>(a.k + t * a.ldk + hq * dk + i) : zero;
-        if constexpr (!ROWS) w4[it] = !ok ? one : a.w_head ? one * wh : a.w_rows ? one * a.w[t * a.ldw + h] : *reinterpret_cast<const f32x4*>(a.w + t * a.ldw + h * dk + i);
+        const int idx = it * 64 + lane;
+        t[it] = min(t0 + idx / (DK / 4), row1 - 1);
+        i[it] = min((idx % (DK / 4)) * 4, dk - 4);
       }
-      if constexpr (DELTA) nb[0] = (lane < TB && t0 + lane < row1) ? beta_of(a.beta[(t0 + lane) * a.ldb + h]) : 0.f;
-      if constexpr (ROWS) nd[0] = (lane < TB && t0 + lane < row1) ? decay_of(a.w[(t0 + lane) * a.ldw + h]) : 1.f;
-      const int bq = lane / (CW / 4), col = j0 + (lane % (CW / 4)) * 4, t = t0 + bq;
-      v4 = (lane < TB * CW / 4 && t < row1 && col < dv) ? *reinterpret_cast<const f32x4*>(a.v + t * a.ldv + h * dv + col) : zero;
+#pragma unroll
+      for (int it = 0; it < NV; ++it) r4[it] = *reinterpret_cast<const f32x4*>(a.r + static_cast<uint64_t>(t[it]) * ldr + (hq * dk + i[it]));
+      if (!a.key_from_decay) {
+#pragma unroll
+        for (int it = 0; it < NV; ++it) k4[it] = *reinterpret_cast<const f32x4*>(a.k + static_cast<uint64_t>(t[it]) * ldk + (hq * dk + i[it]));
+      }
+      if constexpr (!ROWS) {
+        if (w_wide) {
+#pragma unroll
+          for (int it = 0; it < NV; ++it) w4[it] = *reinterpret_cast<const f32x4*>(a.w + static_cast<uint64_t>(t[it]) * ldw + (h * dk + i[it]));
+        } else {
+          // (one a row, or the same one for every row)
+          const float* wr = a.w_rows ? a.w + h : a.w_head + h;
+          const uint32_t step = a.w_rows ? ldw : 0;
+#pragma unroll
+          for (int it = 0; it < NV; ++it) w1[it] = wr[static_cast<uint64_t>(t[it]) * step];
+        }
+      }
+      const size_t tb = min(t0 + min(lane, TB - 1), row1 - 1);
+      if constexpr (DELTA) nb[0] = a.beta[tb * a.ldb + h];
+      if constexpr (ROWS) nd[0] = a.w[tb * a.ldw + h];
+      const size_t tv = min(t0 + lane / (CW / 4), row1 - 1);
+      v4 = *reinterpret_cast<const f32x4*>(a.v + tv * a.ldv + h * dv + min(j0 + (lane % (CW / 4)) * 4, dv - 4));
     } else {
 #pragma unroll
       for (int bq = 0; bq < TB; ++bq) {
@@ -799,23 +826,33 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
   for (int t0 = row0; t0 < row1; t0 += TB) {
     float vj[TB], bj[TB], dj[TB];
     if constexpr (VEC) {
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
       if constexpr (DELTA) {
-        if (lane < TB) shb[lane] = nb[0];
+        const float b = beta_of(nb[0]);
+        if (lane < TB) shb[lane] = t0 + lane < row1 ? b : 0.f;
       }
       if constexpr (ROWS) {
-        if (lane < TB) shw[lane] = nd[0];
+        const float d = decay_of(nd[0]);
+        if (lane < TB) shw[lane] = t0 + lane < row1 ? d : 1.f;
       }
 #pragma unroll
       for (int it = 0; it < NV; ++it) {
         const int idx = it * 64 + lane, bq = idx / (DK / 4), i = (idx % (DK / 4)) * 4;
+        const bool ok = t0 + bq < row1 && i < dk;
+        f32x4 w = one;
+        if constexpr (!ROWS) {
+          w = w_wide ? w4[it] : one * w1[it];
+          w = ok ? w : one;
+        }
+        const f32x4 key = !ROWS && a.key_from_decay ? one - w : ok ? k4[it] : zero, rr = ok ? r4[it] : zero;
         if (idx < N4) {
-          const f32x4 one = {1.f, 1.f, 1.f, 1.f};
-          *reinterpret_cast<f32x4*>(&sh[bq][i]) = r4[it];
-          *reinterpret_cast<f32x4*>(&sh[bq][DK + i]) = !ROWS && a.key_from_decay ? one - w4[it] : k4[it];
-          if constexpr (!ROWS) *reinterpret_cast<f32x4*>(&sh[bq][2 * DK + i]) = w4[it];
+          *reinterpret_cast<f32x4*>(&sh[bq][i]) = rr;
+          *reinterpret_cast<f32x4*>(&sh[bq][DK + i]) = key;
+          if constexpr (!ROWS) *reinterpret_cast<f32x4*>(&sh[bq][2 * DK + i]) = w;
         }
       }
-      if (lane < TB * CW / 4) *reinterpret_cast<f32x4*>(&shv[lane / (CW / 4)][(lane % (CW / 4)) * 4]) = v4;
+      const f32x4 vv = t0 + lane / (CW / 4) < row1 && j0 + (lane % (CW / 4)) * 4 < dv ? v4 : zero;
+      if (lane < TB * CW / 4) *reinterpret_cast<f32x4*>(&shv[lane / (CW / 4)][(lane % (CW / 4)) * 4]) = vv;
     } else {
 #pragma unroll
       for (int bq = 0; bq < TB; ++bq) {
@@ -843,57 +880,85 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
       }
     }
     if (t0 + TB < row1) fetch(t0 + TB);
-    // (no branch inside the eight rows: their reads, sums and joins can then overlap)
+    // (no branch inside the rows: their sums and joins can then overlap.  The operands of some rows are read from LDS while those of the rows
+    // before them are worked on: one wave has the SIMD to itself, and each row waited for its own reads: delta rule 190 -> 183 us,
+    // fading by a constant 155 -> 140)
     float ob[TB];
+    struct Operands { float r[GR][KQ], k[GR][KQ], w[ROWS ? 1 : GR][ROWS ? 1 : KQ]; };
+    auto take = [&](int b0, Operands& x) {
 #pragma unroll
-    for (int bq = 0; bq < TB; ++bq) {
-      const float* mr = sh[bq] + kg * KQ;
-      const float* mk = mr + DK;
-      const float* mw = mk + DK;
-      const float* mu = shu + kg * KQ;
-      float o = 0.f;
-      if constexpr (DELTA) {
-        // the state fades; what it answers to the key is taken off the value; the rest, times beta, is written
-        float ans = 0.f;
+      for (int g = 0; g < GR; ++g) {
+        const float* mr = sh[b0 + g] + kg * KQ;
 #pragma unroll
         for (int q = 0; q < KQ; ++q) {
-          S[q] *= ROWS ? dj[bq] : mw[q];
-          ans = fmaf(mk[q], S[q], ans);
+          x.r[g][q] = mr[q];
+          x.k[g][q] = mr[DK + q];
+          if constexpr (!ROWS) x.w[g][q] = mr[2 * DK + q];
         }
-        ans = group_reduce<KG>(ans, SumOp());
-        const float e = bj[bq] * (vj[bq] - ans);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto work = [&](int b0, const Operands& x) {
 #pragma unroll
-        for (int q = 0; q < KQ; ++q) {
-          S[q] = fmaf(mk[q], e, S[q]);
-          o = fmaf(mr[q], S[q], o);
+      for (int g = 0; g < GR; ++g) {
+        const int bq = b0 + g;
+        float o = 0.f;
+        if constexpr (DELTA) {
+          // the state fades; what it answers to the key is taken off the value; the rest, times beta, is written
+          float ans = 0.f;
+#pragma unroll
+          for (int q = 0; q < KQ; ++q) {
+            S[q] *= ROWS ? dj[bq] : x.w[ROWS ? 0 : g][ROWS ? 0 : q];
+            ans = fmaf(x.k[g][q], S[q], ans);
+          }
+          ans = group_reduce<KG>(ans, SumOp());
+          const float e = bj[bq] * (vj[bq] - ans);
+#pragma unroll
+          for (int q = 0; q < KQ; ++q) {
+            S[q] = fmaf(x.k[g][q], e, S[q]);
+            o = fmaf(x.r[g][q], S[q], o);
+          }
+        } else {
+#pragma unroll
+          for (int q = 0; q < KQ; ++q) {
+            const float kv = x.k[g][q] * vj[bq], w = x.w[ROWS ? 0 : g][ROWS ? 0 : q];
+            if (AFTER) {
+              S[q] = fmaf(w, S[q], kv);
+              o = fmaf(x.r[g][q], S[q], o);
+            } else {
+              o = fmaf(x.r[g][q], fmaf(shu[kg * KQ + q], kv, S[q]), o);
+              S[q] = fmaf(w, S[q], kv);
+            }
+          }
         }
         ob[bq] = group_reduce<KG>(o, SumOp());
-        continue;
       }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    Operands x0, x1;
+    take(0, x0);
 #pragma unroll
-      for (int q = 0; q < KQ; ++q) {
-        const float kv = mk[q] * vj[bq];
-        if (AFTER) {
-          S[q] = fmaf(mw[q], S[q], kv);
-          o = fmaf(mr[q], S[q], o);
-        } else {
-          o = fmaf(mr[q], fmaf(mu[q], kv, S[q]), o);
-          S[q] = fmaf(mw[q], S[q], kv);
-        }
-      }
-      ob[bq] = group_reduce<KG>(o, SumOp());
+    for (int b0 = 0; b0 < TB; b0 += 2 * GR) {
+      if (b0 + GR < TB) take(b0 + GR, x1);
+      work(b0, x0);
+      if (b0 + 2 * GR < TB) take(b0 + 2 * GR, x0);
+      if (b0 + GR < TB) work(b0 + GR, x1);
     }
-    if (live && kg == 0) {
+    // (every lane of a column has its sums: lane kg stores row kg's, one store for KG rows where each took one and a branch; with the
+    // addresses of 32-bit factors above: delta rule 183 -> 146 us, fading by a constant 140 -> 110.  Asking two fetches ahead gave nothing more)
 #pragma unroll
-      for (int bq = 0; bq < TB; ++bq)
-        if (t0 + bq < row1) a.out[(t0 + bq) * a.ldo + h * dv + j] = ob[bq];
+    for (int b0 = 0; b0 < TB; b0 += KG) {
+      float o = ob[b0];
+#pragma unroll
+      for (int q = 1; q < KG && b0 + q < TB; ++q) o = kg == q ? ob[b0 + q] : o;
+      if (live && b0 + kg < TB && t0 + b0 + kg < row1) a.out[static_cast<size_t>(t0 + b0 + kg) * a.ldo + h * dv + j] = o;
     }
     __syncthreads();
   }
   if (live)
 #pragma unroll
     for (int q = 0; q < KQ; ++q)
-      if (kg * KQ + q < dk) sp[q] = S[q];
+      if (kg * KQ + q < dk) a.state[at_head + static_cast<size_t>(j) * dk + kg * KQ + q] = S[q];
 }
 
 // ---- a norm per head, with a gate ----------------------------------------------------------------------------
@@ -2336,7 +2401,7 @@ int dn_state_scan(const float* r, long long ldr, const float* k, long long ldk, 
   // (the parts of a column's sum by the head's size alone, never by the step: a row's bits are the same in every step)
   const dim3 few((dv + 15) / 16, H, S), many((dv + 3) / 4, H, S);
   auto by16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const bool vec = dk % 4 == 0 && dv % 4 == 0 && ldr % 4 == 0 && ldv % 4 == 0 && (w == nullptr || w_rows || ldw % 4 == 0) &&
+  const bool vec = dk % 4 == 0 && dv % 4 == 0 && std::max(std::max(ldr, ldk), ldw) < (1LL << 31) && ldr % 4 == 0 && ldv % 4 == 0 && (w == nullptr || w_rows || ldw % 4 == 0) &&
                    (key_from_decay || ldk % 4 == 0) && by16(r) && by16(v) && (w_rows || by16(w)) && (key_from_decay || by16(k));
   const bool few_rows = T <= 2 * S;      // (decoded tokens: a row or two a request)
 #define DN_SCAN3(DK, KG, GRID, AFTER, VEC)                                                                    \
