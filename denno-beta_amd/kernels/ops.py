@@ -656,9 +656,10 @@ def attention(q, out, k_pool, v_pool, block_tables, tiles, n_heads, scale, windo
     head h's summand is exp(sink[h]), which nothing scales; keep_first: with a window, the request's first so many keys are
     read by every row as well; softcap > 0: a scaled score s becomes softcap * tanh(s / softcap), before the bias.
 
-    Three kernels: 32-bit takes the plain one; bfloat16 takes the MFMA kernel over tiles_wide, or,
-    for a pure decode step, the split kernel (with both, out may be packed rows); a head size that
-    those do not take falls to the plain one."""
+    Four kernels: 32-bit takes the plain one, or, for portions with tiles_wide, the one on the matrix cores with the
+    same bits (head sizes that are multiples of 16 up to 128, pages of a multiple of 16 keys); bfloat16 takes the MFMA
+    kernel over tiles_wide, or, for a pure decode step, the split kernel (with both, out may be packed rows); a head
+    size that those do not take falls to the plain one."""
     out_packed = isinstance(out, PackedMatrix)
     _dev(q, "q", _FLOATS, 2)
     if not out_packed:

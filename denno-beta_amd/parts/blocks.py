@@ -40,7 +40,7 @@ class PreNormBlock:
 
     def forward(self, x, ctx, caches, runtime):
         cache = caches[0]
-        # A product into the stream may leave its sum for the kernel of the norm behind it (steps of 65 to 256
+        # A product into the stream may leave its sum for the kernel of the norm behind it (steps of 65 to 512
         # rows, few columns: parts.base.DeferredSum): the part before a norm is offered an empty one, the norm gets
         # what was put there; across blocks it travels in runtime.stream_deferred.
         came = runtime.stream_deferred
