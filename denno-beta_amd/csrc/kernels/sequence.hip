@@ -2441,7 +2441,7 @@ int dn_head_norm(const float* o, long long ld, const float* weight, int w_stride
   if (!float_kind(out_dt)) return DN_ERR_DTYPE;
   if (gate && (gate_kind < 0 || gate_kind > ACT_TANH)) return DN_ERR_SHAPE;
   if (skip && (!skip_scale || skip_dim < 1)) return DN_ERR_SHAPE;
-  if (T == 0) return 0;
+  if (T == 0 || dv < 1) return 0;      // (the kernels read a head's last column in place of those beyond it: there has to be one)
   HeadNormArgs a{o, static_cast<size_t>(ld), weight, w_stride, eps, gate, static_cast<size_t>(ldg), gate_kind, gate_first, skip,
                  static_cast<size_t>(lds), skip_scale, skip_dim, out, out_dt, static_cast<size_t>(ldo), dv};
   if (dv > 256 && dv <= 2048)
