@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const void* x, int x_dt, s
 }
 
 // N numbers of a row that a thread of 256 holds, its columns threadIdx.x, threadIdx.x + 256, ...: all asked for before the first is used,
-// those beyond the row from its last place (never a load behind a condition, which would be waited for by itself)
+// those beyond the row from its last place (never a load behind a condition of its own, which would be waited for by itself)
 template <int N>
 __device__ __forceinline__ void hold_row(const void* p, size_t at, int dt, int width, float* v) {
   if (dt == DN_F32) {
@@ -77,14 +77,18 @@ __device__ __forceinline__ void hold_row(const void* p, size_t at, int dt, int w
 
 // rmsnorm_kernel and rmsnorm_add_kernel for rows of up to 256 N numbers, held in registers: one trip to memory where the loops over columns
 // make one per 256 columns and pass (8 rows of 1,024: 4.8 -> 3.0 and 6.6 -> 3.0 us a launch).  The same sums in the same order: the same bits.
+// N is what the row needs, to the next power of two, and with N = 1 a wave beyond the row loads nothing: all N places are loaded, and where the
+// rows fill the chip those beyond the row cost as much as the others (8,192 rows of 64: rmsnorm 5.8 us in loops, 7.7 with N = 4, 5.5 with N = 1).
 template <int N>
 __global__ __launch_bounds__(256) void rmsnorm_held_kernel(const void* x, int x_dt, size_t ldx, const float* weight, void* out, int out_dt, size_t ldo,
                                                            const int* rows, int width, float eps) {
   __shared__ float sh[4];
   const int r = blockIdx.x;
-  float v[N], w[N];
-  if (weight) hold_row<N>(weight, 0, DN_F32, width, w);
-  hold_row<N>(x, static_cast<size_t>(rows ? rows[r] : r) * ldx, x_dt, width, v);
+  float v[N] = {}, w[N] = {};
+  if (N > 1 || static_cast<int>(threadIdx.x) < width) {
+    if (weight) hold_row<N>(weight, 0, DN_F32, width, w);
+    hold_row<N>(x, static_cast<size_t>(rows ? rows[r] : r) * ldx, x_dt, width, v);
+  }
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < N; ++i)
@@ -106,13 +110,15 @@ __global__ __launch_bounds__(256) void rmsnorm_add_held_kernel(const void* y, in
                                                                size_t ldn) {
   __shared__ float sh[4];
   const size_t dst = static_cast<size_t>(blockIdx.x) * ldx;
-  float v[N], g[N], w[N], sc[N], xs[N], nw[N];
-  hold_row<N>(y, static_cast<size_t>(blockIdx.x) * ldy, y_dt, width, v);
-  if (gate) hold_row<N>(gate, static_cast<size_t>(blockIdx.x) * ldg, DN_F32, width, g);
-  hold_row<N>(x, dst, DN_F32, width, xs);
-  if (weight) hold_row<N>(weight, 0, DN_F32, width, w);
-  if (scale) hold_row<N>(scale, 0, DN_F32, width, sc);
-  if (next_out && next_w) hold_row<N>(next_w, 0, DN_F32, width, nw);
+  float v[N] = {}, g[N] = {}, w[N] = {}, sc[N] = {}, xs[N] = {}, nw[N] = {};
+  if (N > 1 || static_cast<int>(threadIdx.x) < width) {
+    hold_row<N>(y, static_cast<size_t>(blockIdx.x) * ldy, y_dt, width, v);
+    if (gate) hold_row<N>(gate, static_cast<size_t>(blockIdx.x) * ldg, DN_F32, width, g);
+    hold_row<N>(x, dst, DN_F32, width, xs);
+    if (weight) hold_row<N>(weight, 0, DN_F32, width, w);
+    if (scale) hold_row<N>(scale, 0, DN_F32, width, sc);
+    if (next_out && next_w) hold_row<N>(next_w, 0, DN_F32, width, nw);
+  }
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
@@ -2213,7 +2219,11 @@ int dn_rmsnorm(const void* x, int x_dt, long long ldx, const float* weight, void
 #define DN_RMSNORM(kernel)                                                                                                    \
   hipLaunchKernelGGL(kernel, dim3(R), dim3(256), 0, stream, x, x_dt, static_cast<size_t>(ldx), weight, out, out_dt,            \
                      static_cast<size_t>(ldo), rows, width, eps)
-  if (width <= 1024)
+  if (width <= 256)
+    DN_RMSNORM(rmsnorm_held_kernel<1>);
+  else if (width <= 512)
+    DN_RMSNORM(rmsnorm_held_kernel<2>);
+  else if (width <= 1024)
     DN_RMSNORM(rmsnorm_held_kernel<4>);
   else if (width <= 2048)
     DN_RMSNORM(rmsnorm_held_kernel<8>);
@@ -2235,14 +2245,19 @@ int dn_rmsnorm_add(const void* y, int y_dt, long long ldy, const float* weight, 
   hipLaunchKernelGGL(kernel, dim3(T), dim3(256), 0, stream, y, y_dt, static_cast<size_t>(ldy), weight, scale, mult, x,          \
                      static_cast<size_t>(ldx), width, eps, gate, static_cast<size_t>(ldg), next_w, next_eps, next_out, next_dt, \
                      static_cast<size_t>(ldn))
-  if (width <= 1024)
+  // (a row that one wave holds and nothing beside it: the loops make one trip a pass too, in less code: 8,192 rows of 64 6.2 us, held 7.3)
+  if (width > 4096 || (width <= 64 && !gate && !next_out))
+    DN_RMSNORM_ADD(rmsnorm_add_kernel);
+  else if (width <= 256)
+    DN_RMSNORM_ADD(rmsnorm_add_held_kernel<1>);
+  else if (width <= 512)
+    DN_RMSNORM_ADD(rmsnorm_add_held_kernel<2>);
+  else if (width <= 1024)
     DN_RMSNORM_ADD(rmsnorm_add_held_kernel<4>);
   else if (width <= 2048)
     DN_RMSNORM_ADD(rmsnorm_add_held_kernel<8>);
-  else if (width <= 4096)
-    DN_RMSNORM_ADD(rmsnorm_add_held_kernel<16>);
   else
-    DN_RMSNORM_ADD(rmsnorm_add_kernel);
+    DN_RMSNORM_ADD(rmsnorm_add_held_kernel<16>);
 #undef DN_RMSNORM_ADD
   return dn_launch_status();
 }

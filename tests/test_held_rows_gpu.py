@@ -17,7 +17,7 @@ def rms(x, eps):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("width", [1, 255, 257, 1024, 1025, 2048, 2049, 4096, 4097])
+@pytest.mark.parametrize("width", [1, 64, 65, 255, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 4096, 4097])
 def test_rmsnorm_and_the_sum_behind_it(width, dtype):
     o, R = ops(), 3
     wide = rnd(R + 2, width + 5, seed=width).to(dtype)
@@ -38,6 +38,17 @@ def test_rmsnorm_and_the_sum_behind_it(width, dtype):
         assert torch.allclose(mine.double(), want, **TOL[torch.float32])
         # (the norm of the row as it was stored: a row of one column may be near zero, where its norm is steep)
         assert torch.allclose(then.double(), rms(mine.double(), 1e-6) * (1.0 if norm is None else nw.double()), **TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [1, 63, 64, 65, 256, 4097])
+def test_a_sum_with_nothing_beside_it(width, dtype):
+    o, R = ops(), 5
+    y, w, stream = rnd(R, width + 3, seed=1, dtype=dtype)[:, :width], rnd(width, seed=2), rnd(R, width + 2, seed=3)
+    mine = stream.clone()
+    o.rmsnorm_add(y, w, None, 0.37, 1e-5, mine[:, :width])
+    want = stream[:, :width].double() + 0.37 * rms(y.double(), 1e-5) * w.double()
+    assert torch.allclose(mine[:, :width].double(), want, **TOL[torch.float32]) and torch.equal(mine[:, width:], stream[:, width:])
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
