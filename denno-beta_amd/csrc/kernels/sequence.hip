@@ -1030,18 +1030,22 @@ __device__ __forceinline__ void head_norm_leave(const HeadNormArgs& a, size_t t,
   }
 }
 
-// A wave a head of up to 256 columns (the loops over columns, a trip to memory each 64 and pass: 8 rows of 16 heads of 64 to 128, 4.2 us; now 3.7)
+// A wave a head of up to 64 N columns (the loops over columns, a trip to memory each 64 and pass: 8 rows of 16 heads of 64 to 128, 4.2 us; now
+// 3.7).  N, here and in head_norm_held_kernel, is what a head needs, to the next size there is: the places beyond it are loaded and worked on
+// like the others (gated norms of 4,096 rows: 32 heads of 16 columns 38 us in loops, 47 with N = 4, 33 with N = 1; 4 heads of 300 33 us, 45
+// with eight places a thread of 256, 20 with two).
+template <int N>
 __global__ __launch_bounds__(64) void head_norm_kernel(HeadNormArgs a) {
   const int h = blockIdx.y;
   const size_t t = blockIdx.x;
-  float y[4], w[4], g[4];
-  head_norm_hold<4, 64>(a, t, h, y, w, g);
+  float y[N], w[N], g[N];
+  head_norm_hold<N, 64>(a, t, h, y, w, g);
   float ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
+  for (int k = 0; k < N; ++k)
     if (static_cast<int>(threadIdx.x) + 64 * k < a.dv) ss = fmaf(y[k], y[k], ss);
   ss = wave_sum(ss);
-  head_norm_leave<4, 64>(a, t, h, 1.0f / sqrtf(ss / static_cast<float>(a.dv) + a.eps), y, w, g);
+  head_norm_leave<N, 64>(a, t, h, 1.0f / sqrtf(ss / static_cast<float>(a.dv) + a.eps), y, w, g);
 }
 
 // The same for heads of many columns (all heads normed as one vector): a workgroup a head, the sums as in rmsnorm_kernel.
@@ -1066,9 +1070,10 @@ __global__ __launch_bounds__(256) void head_norm_wide_kernel(HeadNormArgs a) {
 }
 
 // head_norm_wide_kernel for heads of up to 256 NC columns: a thread's share of the head stays in registers between the sum and
-// the stores (one trip to memory where the kernel above makes two).  The same sums in the same order: the same bits.
+// the stores (one trip to memory where the kernel above makes two).  The same sums in the same order: the same bits.  Four workgroups a CU,
+// also with 16 places, which would take 140 registers: 1,024 gated rows of 4,096 then run at once (16.7 -> 13.7 us).
 template <int NC>
-__global__ __launch_bounds__(256) void head_norm_held_kernel(HeadNormArgs a) {
+__global__ __launch_bounds__(256, 4) void head_norm_held_kernel(HeadNormArgs a) {
   __shared__ float sh[4];
   const int h = blockIdx.y;
   const size_t t = blockIdx.x;
@@ -2459,14 +2464,17 @@ int dn_head_norm(const float* o, long long ld, const float* weight, int w_stride
   if (T == 0 || dv < 1) return 0;      // (the kernels read a head's last column in place of those beyond it: there has to be one)
   HeadNormArgs a{o, static_cast<size_t>(ld), weight, w_stride, eps, gate, static_cast<size_t>(ldg), gate_kind, gate_first, skip,
                  static_cast<size_t>(lds), skip_scale, skip_dim, out, out_dt, static_cast<size_t>(ldo), dv};
-  if (dv > 256 && dv <= 2048)
-    hipLaunchKernelGGL(head_norm_held_kernel<8>, dim3(T, H), dim3(256), 0, stream, a);
-  else if (dv > 2048 && dv <= 4096)
-    hipLaunchKernelGGL(head_norm_held_kernel<16>, dim3(T, H), dim3(256), 0, stream, a);
-  else if (dv > 256)
-    hipLaunchKernelGGL(head_norm_wide_kernel, dim3(T, H), dim3(256), 0, stream, a);
-  else
-    hipLaunchKernelGGL(head_norm_kernel, dim3(T, H), dim3(64), 0, stream, a);
+#define DN_HEAD_NORM(kernel, threads) hipLaunchKernelGGL(kernel, dim3(T, H), dim3(threads), 0, stream, a)
+  if (dv <= 64) DN_HEAD_NORM(head_norm_kernel<1>, 64);
+  else if (dv <= 128) DN_HEAD_NORM(head_norm_kernel<2>, 64);
+  else if (dv <= 256) DN_HEAD_NORM(head_norm_kernel<4>, 64);
+  else if (dv <= 512) DN_HEAD_NORM(head_norm_held_kernel<2>, 256);
+  else if (dv <= 1024) DN_HEAD_NORM(head_norm_held_kernel<4>, 256);
+  else if (dv <= 2048) DN_HEAD_NORM(head_norm_held_kernel<8>, 256);
+  else if (dv <= 3072) DN_HEAD_NORM(head_norm_held_kernel<12>, 256);
+  else if (dv <= 4096) DN_HEAD_NORM(head_norm_held_kernel<16>, 256);
+  else DN_HEAD_NORM(head_norm_wide_kernel, 256);
+#undef DN_HEAD_NORM
   return dn_launch_status();
 }
 

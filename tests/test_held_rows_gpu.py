@@ -68,7 +68,8 @@ def test_activations_over_cut_rows(n, dtype):
     assert torch.allclose(mine.double(), torch.nn.functional.silu(x), **TOL[torch.float32])
 
 
-@pytest.mark.parametrize("heads,dv", [(1, 1), (3, 63), (3, 65), (2, 256), (2, 257), (1, 2049)])
+@pytest.mark.parametrize("heads,dv", [(1, 1), (5, 16), (3, 63), (3, 64), (3, 65), (2, 128), (2, 129), (2, 256), (2, 257), (2, 512), (2, 513), (1, 1024),
+                                      (2, 1025), (1, 2048), (1, 2049), (1, 3072), (2, 3073), (1, 4096), (1, 4097)])
 @pytest.mark.parametrize("gate_first", [False, True])
 def test_head_norms_hold_their_heads(heads, dv, gate_first):
     o, T = ops(), 3
