@@ -81,3 +81,25 @@ def test_head_norms_hold_their_heads(heads, dv, gate_first):
     v = rms(v.view(T, heads, dv), 1e-5) * w.double()
     v = v.reshape(T, -1) * (1.0 if gate_first else act)
     assert torch.allclose(out.double(), v, **TOL[torch.float32])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,dim", [(1, 2), (3, 64), (25, 80)])
+def test_turned_runs_of_many_rows_and_few(heads, dim, dtype):
+    """Up to 1,024 rows a row's pairs are cut among workgroups, beyond them not: the same numbers, places beside them untouched."""
+    o, T = ops(), 1025
+    src, pos = rnd(T, 2 * heads * dim, seed=dim), torch.arange(T, device=DEV, dtype=torch.int32)
+    freq = 100.0 ** (-torch.arange(0, dim, 2, device=DEV).float() / dim)
+
+    def turned(a, b):
+        q, v = (torch.full((b - a, heads * dim + 1), 7.0, dtype=dtype, device=DEV) for _ in range(2))
+        o.rotary_runs(src[a:b], pos[a:b], freq, [(q, 0, heads, dim, dim, 0, dim), (v, heads * dim, heads, dim, 0, 0, dim)])
+        return q, v
+    many, few = turned(0, T), [torch.cat(x) for x in zip(turned(0, 1), turned(1, T))]
+    angle = (pos.double()[:, None] * freq.double()).repeat(1, heads)
+    x = src[:, :heads * dim].double()
+    even = x[:, 0::2] * torch.cos(angle) - x[:, 1::2] * torch.sin(angle)
+    # (an angle of up to 1,024 is off by up to 2^-14 in 32 bits; bfloat16 rounds numbers of up to 8 by up to 2^-6)
+    assert (many[0][:, 0:-1:2].double() - even).abs().max() < 4e-2 and bool((many[0][:, -1] == 7).all())
+    assert torch.equal(many[1][:, :-1], src[:, heads * dim:].to(dtype))
+    assert all(torch.equal(m, f) for m, f in zip(many, few))
