@@ -52,7 +52,7 @@ def test_a_sum_with_nothing_beside_it(width, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("n", [1, 257, 1023, 1024, 1025, 4097])
+@pytest.mark.parametrize("n", [1, 256, 257, 512, 513, 769, 1023, 1024, 1025, 1280, 1281, 2560, 2561, 4097])
 def test_activations_over_cut_rows(n, dtype):
     o, T = ops(), 3
     z, bias, two = rnd(T, n + 3, seed=n)[:, :n], rnd(n, seed=1), torch.tensor([0.7, 0.4], device=DEV)
