@@ -528,10 +528,10 @@ def linear(a, w, bias=None, out=None, epilogue="none", residual=None):
     return out
 
 
-def linear_deferred_shares(n_rows, w, rows_max=256):
+def linear_deferred_shares(n_rows, w):
     """How many shares of K `linear_deferred` cuts the product of n_rows rows with w into; 0: it does not take it
-    (the product then adds into the stream itself).  rows_max: up to so many rows (at most 512)."""
-    if not isinstance(w, PackedMatrix) or n_rows > rows_max:
+    (the product then adds into the stream itself)."""
+    if not isinstance(w, PackedMatrix):
         return 0
     return _lib_quiet("gemm").dn_gemm_deferred_shares(n_rows, w.shape[0], w.shape[1])
 
@@ -542,7 +542,7 @@ def linear_deferred(a, w):
     rows; w: a PackedMatrix."""
     M, K = a.shape
     lda, N, packed = _operands(a, w, "linear_deferred")
-    shares = linear_deferred_shares(M, w, rows_max=512)
+    shares = linear_deferred_shares(M, w)
     _need(shares > 0 and (packed & PACKED_W), lambda: f"linear_deferred: {M} rows x {tuple(w.shape)} is not deferred")
     part = torch.empty((shares, M, N), dtype=torch.float32, device=a.device)
     _ok(_lib("gemm").dn_gemm_deferred(a.data_ptr(), lda, w.data_ptr(), M, N, K, packed, part.data_ptr(), part.numel(), _stream()),

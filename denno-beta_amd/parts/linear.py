@@ -87,7 +87,7 @@ class Linear:
 
     def defers(self, n_rows: int) -> bool:
         """Whether a call with n_rows rows that adds into the residual stream can leave its sum for the next norm's kernel."""
-        return ops.linear_deferred_shares(n_rows, self.weight, rows_max=512) > 0
+        return ops.linear_deferred_shares(n_rows, self.weight) > 0
 
     def _fusable(self, a, out_dtype):
         """(c1, c2, eps, no_mean) if `a` is a LazyNorm that this call can run in its own kernel."""

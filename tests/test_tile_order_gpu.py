@@ -28,7 +28,7 @@ def test_sums_left_for_the_norm_beyond_256_rows(M, N, K):
     o = ops()
     a, w, bias = rnd(M, K, seed=M, dtype=torch.bfloat16), rnd(N, K, seed=N, dtype=torch.bfloat16, scale=0.05), rnd(N, seed=3)
     wp, x0, gamma, beta = o.pack_matrix(w), rnd(M, N, seed=4), rnd(N, seed=5), rnd(N, seed=6)
-    shares = o.linear_deferred_shares(M, wp, rows_max=512)
+    shares = o.linear_deferred_shares(M, wp)
     assert shares >= 2
     part = o.linear_deferred(a, wp)
     assert part.shape == (shares, M, N)
