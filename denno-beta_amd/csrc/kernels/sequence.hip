@@ -749,7 +749,9 @@ struct ScanArgs {
   size_t ldo;
 };
 
-template <int DK, int KG, int MODE, bool VEC, int TB>
+// AHEAD: the operands of some rows are read from LDS while those of the rows before them are worked on (one wave with the SIMD to itself
+// waits for its own reads otherwise).  That takes 50 to 80 registers, a wave less a SIMD or two: see dn_state_scan for where it pays.
+template <int DK, int KG, int MODE, bool VEC, int TB, bool AHEAD>
 __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
   constexpr bool AFTER = MODE == SCAN_AFTER, DELTA = MODE == SCAN_DELTA || MODE == SCAN_DELTA_ROWS;
   constexpr bool ROWS = MODE == SCAN_DELTA_ROWS;      // (a row's decay is one number: it takes no place beside r and k)
@@ -759,7 +761,7 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
   constexpr int NL = DK >= 64 ? DK / 64 : 1;
   // TB: rows asked for at a time (a trip to memory is paid once per TB rows, not per row; all TB places are worked on,
   // so steps of single rows take a small TB).  A row's sums are the same for every TB.
-  constexpr int GR = KQ <= 4 ? (TB < 4 ? TB : 4) : KQ <= 8 ? 2 : 1;      // rows whose operands are read at a time
+  constexpr int GR = !AHEAD ? 1 : KQ <= 4 ? (TB < 4 ? TB : 4) : KQ <= 8 ? 2 : 1;      // rows whose operands are read at a time
   constexpr int N4 = TB * DK / 4, NV = N4 >= 64 ? N4 / 64 : 1;      // VEC: groups of four numbers per array, per lane
   __shared__ __attribute__((aligned(16))) float sh[TB][PARTS * DK];
   __shared__ __attribute__((aligned(16))) float shv[TB][CW];
@@ -793,7 +795,8 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
   f32x4 r4[VEC ? NV : 1], k4[VEC ? NV : 1], w4[VEC ? NV : 1], v4;
   float w1[VEC ? NV : 1];
   auto beta_of = [&](float z) { return a.beta_logits ? 1.0f / (1.0f + expf(-z)) : z; };      // (beta given as it is, or as sigmoid's argument)
-  auto decay_of = [&](float z) { return a.w_rate ? expf(-a.w_rate[h] * softplus_f(z + (a.w_bias ? a.w_bias[h] : 0.f))) : z; };
+  const float w_rate = a.w_rate ? a.w_rate[h] : 0.f, w_bias = a.w_bias ? a.w_bias[h] : 0.f;
+  auto decay_of = [&](float z) { return a.w_rate ? expf(-w_rate * softplus_f(z + w_bias)) : z; };
   auto fetch = [&](int t0) {
     if constexpr (VEC) {
       // (32-bit factors: a product of 64-bit numbers is three instructions of four times the length, and a lane makes a dozen)
@@ -906,9 +909,7 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
       }
     }
     if (t0 + TB < row1) fetch(t0 + TB);
-    // (no branch inside the rows: their sums and joins can then overlap.  The operands of some rows are read from LDS while those of the rows
-    // before them are worked on: one wave has the SIMD to itself, and each row waited for its own reads: delta rule 190 -> 183 us,
-    // fading by a constant 155 -> 140)
+    // (no branch inside the rows: their sums and joins can then overlap.  AHEAD: delta rule 190 -> 183 us, fading by a constant 155 -> 140)
     float ob[TB];
     struct Operands { float r[GR][KQ], k[GR][KQ], w[ROWS ? 1 : GR][ROWS ? 1 : KQ]; };
     auto take = [&](int b0, Operands& x) {
@@ -922,7 +923,7 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
           if constexpr (!ROWS) x.w[g][q] = mr[2 * DK + q];
         }
       }
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
     };
     auto work = [&](int b0, const Operands& x) {
 #pragma unroll
@@ -959,16 +960,24 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
         }
         ob[bq] = group_reduce<KG>(o, SumOp());
       }
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
     };
     Operands x0, x1;
-    take(0, x0);
+    if constexpr (AHEAD) {
+      take(0, x0);
 #pragma unroll
-    for (int b0 = 0; b0 < TB; b0 += 2 * GR) {
-      if (b0 + GR < TB) take(b0 + GR, x1);
-      work(b0, x0);
-      if (b0 + 2 * GR < TB) take(b0 + 2 * GR, x0);
-      if (b0 + GR < TB) work(b0 + GR, x1);
+      for (int b0 = 0; b0 < TB; b0 += 2 * GR) {
+        if (b0 + GR < TB) take(b0 + GR, x1);
+        work(b0, x0);
+        if (b0 + 2 * GR < TB) take(b0 + 2 * GR, x0);
+        if (b0 + GR < TB) work(b0 + GR, x1);
+      }
+    } else {
+#pragma unroll
+      for (int b0 = 0; b0 < TB; ++b0) {
+        take(b0, x0);
+        work(b0, x0);
+      }
     }
     // (every lane of a column has its sums: lane kg stores row kg's, one store for KG rows where each took one and a branch; with the
     // addresses of 32-bit factors above: delta rule 183 -> 146 us, fading by a constant 140 -> 110.  Asking two fetches ahead gave nothing more)
@@ -2462,10 +2471,23 @@ int dn_state_scan(const float* r, long long ldr, const float* k, long long ldk, 
   const bool vec = dk % 4 == 0 && dv % 4 == 0 && std::max(std::max(ldr, ldk), ldw) < (1LL << 31) && ldr % 4 == 0 && ldv % 4 == 0 && (w == nullptr || w_rows || ldw % 4 == 0) &&
                    (key_from_decay || ldk % 4 == 0) && by16(r) && by16(v) && (w_rows || by16(w)) && (key_from_decay || by16(k));
   const bool few_rows = T <= 2 * S;      // (decoded tokens: a row or two a request)
+  // Operands read ahead cost a SIMD one of three waves (heads of up to 64 key channels) or of two (up to 128; nothing where a row has one
+  // decay, nor beyond 128, where one wave fits either way).  So they are for steps whose waves all run at once all the same, up to 2 or 1 for each
+  // of the 1,024 SIMDs; for more waves the place is worth more (us with and without, 64 x 128: 24 requests of 64 rows x 8 heads, delta rule 46 and 43, one
+  // decay a head 39 and 37; 32 of 5 rows 20 and 18, 18 and 16; 128 x 128: 3 of 400 x 16 heads 190 and 117; 64 x 63: 32 of 200 x 8 heads 254 and 152),
+  // but for long runs of rows, where more waves at a time only wait for the same memory (64 x 128: 6 requests of 300 rows x 16 heads 103 and 119, 32 of
+  // 200 x 16 312 and 350).  With key channels beyond 128 the bonus's products leave the compiler no registers to read ahead with (32 of 200 rows x
+  // 4 heads 335 and 286; delta rule 288 and 300).
+  auto ahead = [&](dim3 grid, int DK) {
+    const long long waves = static_cast<long long>(grid.x) * grid.y * grid.z;
+    if (DK <= 64) return waves <= 2048 || (vec && T > 128 * static_cast<long long>(S));
+    return waves <= 1024 ? !(vec && DK > 128 && mode == SCAN_BEFORE) : vec && (DK > 128 ? mode != SCAN_BEFORE : mode == SCAN_DELTA && w_rows);
+  };
 #define DN_SCAN3(DK, KG, GRID, AFTER, VEC)                                                                    \
   do {                                                                                                        \
-    if (few_rows) hipLaunchKernelGGL((scan_kernel<DK, KG, AFTER, VEC, 2>), GRID, dim3(64), 0, stream, a);  \
-    else hipLaunchKernelGGL((scan_kernel<DK, KG, AFTER, VEC, (VEC ? 16 : 8)>), GRID, dim3(64), 0, stream, a); \
+    if (few_rows) hipLaunchKernelGGL((scan_kernel<DK, KG, AFTER, VEC, 2, VEC>), GRID, dim3(64), 0, stream, a);  \
+    else if (ahead(GRID, DK)) hipLaunchKernelGGL((scan_kernel<DK, KG, AFTER, VEC, (VEC ? 16 : 8), true>), GRID, dim3(64), 0, stream, a); \
+    else hipLaunchKernelGGL((scan_kernel<DK, KG, AFTER, VEC, (VEC ? 16 : 8), false>), GRID, dim3(64), 0, stream, a); \
   } while (0)
 #define DN_SCAN2(DK, KG, GRID, AFTER)        \
   do {                                       \
