@@ -78,7 +78,10 @@ __device__ __forceinline__ void tile_at(int pid, int tiles_m, int tiles_n, int b
 // PING: eight waves, two a SIMD, that take turns: while one reads a stage's operands from LDS and asks for a later stage, the other
 // multiplies (the second half of the waves runs a barrier behind the first).  Without it all waves read at the same time and multiply at the same
 // time, and neither LDS nor the matrix cores are busy for more than half of a stage: 256 x 160 tiles took 0.91 us a stage of 64
-// along K with sixteen waves in step and take 0.76 with eight in turns.
+// along K with sixteen waves in step and take 0.76 with eight in turns.  `run` says from which K on that pays for the longer epilogue.  The
+// other tiles of 256 rows do not take turns: with bfloat16 results and K up to 3,200 they are level to 15 % slower so (256 x 128: 2,048 x 4,096 x 1,024
+// 26.0 -> 28.7 us; 256 x 224: 2,048 x 6,400 x 1,600 46.8 -> 52.6; 256 x 256: 8,192 x 4,096 x 1,024 79.6 -> 91.4; 192 and more columns with
+// slabs of 32 a stage, since three stages of 64 do not fit in LDS).  Left open: from K = 5,120 on they would gain 3 to 12 % (8,192 x 2,048 x 8,192 225.6 -> 199.3).
 template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __restrict__ A, int lda,
                                                            const bf16_t* __restrict__ W, const float* __restrict__ bias,
@@ -176,14 +179,15 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
       wait_loads<(STAGES - 2) * (HI - 1)>();
   };
   if constexpr (PING) {
-    static_assert(NW == 8, "two waves a SIMD");
+    static_assert(NW == 8 && STAGES >= 3, "two waves a SIMD; the stage that is read, the one that has landed, the one that is asked for");
     const bool late = wave >= NW / 2;
     landed(ksteps >= STAGES - 1);
     __builtin_amdgcn_s_barrier();
     if (late) __builtin_amdgcn_s_barrier();
     for (int kt = 0; kt < ksteps; ++kt) {
-      // (a stage is read a barrier after every wave has waited for its share of it, and its place is asked for again two barriers
-      // after its last reader was done)
+      // A stage is read a barrier after every wave has waited for its share of it.  Its place is asked for again one barrier after its last
+      // reader was done: the late half has read stage kt - 1 (lgkmcnt(0)) in front of the barrier that ends the early half's turn kt - 1,
+      // and right behind that barrier the early half asks for stage kt + STAGES - 1, which lies where kt - 1 lay.  There is none to spare.
       const u32x4* slab = lds + (kt % STAGES) * SLAB;
       bf16x8 af[KB][TM], wf[KB][TN];
 #pragma unroll
@@ -510,10 +514,13 @@ int run(const Args& a, hipStream_t stream) {
     case 2: return sixteen && two ? launch_as<8, 2, 2, 4, 3, 2>(a, stream) : launch_as<4, 2, 4, 4, 4>(a, stream);
     case 3:
       if (!sixteen || !two) return launch_as<4, 2, 4, 5, 4>(a, stream);
-      // (the cache write's epilogue is the longer the more blocks a wave has: 2,048 x 4,800 x 1,600 46.8 us with sixteen waves
-      // in step, 54.9 with eight in turns)
-      if (a.kv) return launch<bf16_t, 8, 2, 2, 5, 3, true, 2>(a, stream);
-      return launch_without_kv<4, 2, 4, 5, 3, 2, true>(a, stream);
+      // Eight waves in turns walk along K faster than sixteen in step and end slower, the more so the more the epilogue does: a wave
+      // has twice the blocks to finish.  So a long K takes turns: from 1,600 on where the results are 32-bit, from 2,560 where they
+      // are rounded to bfloat16 (time of turns over time in step, 1,500 x 6,400 with GELU: K = 64 1.29, 1,024 1.10, 1,600 1.05, 2,560 1.00, 4,096
+      // 0.97, 6,400 0.93; added into the stream: 1.16, 1.03, 1.00, 0.98, 0.95, 0.93), and the product with a cache write, whose
+      // epilogue is the longest, never does (2,048 x 4,800 x 1,600 46.8 us in step, 54.9 in turns).
+      if (!a.kv && a.K >= (a.out_dtype == DN_BF16 && !a.resid ? 2560 : 1600)) return launch_without_kv<4, 2, 4, 5, 3, 2, true>(a, stream);
+      return launch_as<8, 2, 2, 5, 3, 2>(a, stream);
     case 4:
       if (!sixteen) return launch_as<4, 2, 4, 6, 4>(a, stream);
       return two && short_k ? launch_as<8, 2, 2, 6, 2, 2>(a, stream) : launch_as<8, 2, 2, 6, 3>(a, stream);
