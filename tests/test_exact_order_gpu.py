@@ -44,6 +44,39 @@ def test_a_product_of_many_rows_has_the_few_rows_bits(dtype, M, N, K):
         assert torch.equal(many, few) and torch.equal(stream, few_stream), (M, N, K)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("a_exp,w_exp", [(-70, -70), (-64, -66), (-63, -63), (-127, 0), (0, -127), (-40, -100)])
+def test_products_below_the_smallest_normal_number(dtype, a_exp, w_exp):
+    """Operands, products or partial sums (or all) are subnormal: kept by the matrix instruction as by the multiply-adds."""
+    M, N, K = 130, 70, 260
+    g = torch.Generator().manual_seed(K)
+    a, w = ((torch.randn(n, K, generator=g).double() * 2.0 ** e).to(dtype).to(DEV) for n, e in ((M, a_exp), (N, w_exp)))
+    many, few = torch.zeros(M, N, device=DEV), torch.zeros(M, N, device=DEV)
+    ops().linear(a, w, None, out=many)
+    for m in range(0, M, 64):
+        ops().linear(a[m:m + 64], w, None, out=few[m:m + 64])
+    assert torch.equal(many, few)
+    assert ((many != 0) & (many.abs() < 2.0 ** -126)).float().mean() > 0.02
+    # (a step rounds by at most half of the smallest subnormal number, or by 2^-24 of a sum that is itself below 64 times the operands' sizes)
+    exact = a.double() @ w.double().t()
+    assert (many.double() - exact).abs().max() <= K * max(2.0 ** -150, 2.0 ** (a_exp + w_exp + 6 - 24))
+
+
+@pytest.mark.parametrize("dh,q_exp,v_exp", [(64, -130, 0), (64, 0, -130), (128, -127, -127), (48, -140, -128)])
+def test_portions_of_subnormal_queries_and_values(dh, q_exp, v_exp):
+    """Scores and weighted values below the smallest normal number: the portions' kernel and the narrow one give the same bits."""
+    q, k, v, bt, tiles, T = paged_case([300, 64, 133], [100, 64, 1], 2, 2, dh, 16, torch.float32, seed=dh)
+    q, v = (q.double() * 2.0 ** q_exp).float(), (v.double() * 2.0 ** v_exp).float()
+    narrow, wide = torch.zeros(T, 2 * dh, device=DEV), torch.zeros(T, 2 * dh, device=DEV)
+    # (a scale that brings the scores back to about 1: a dot product rounded among subnormal numbers then shows)
+    args = (q[:, 2 * dh:4 * dh], k, v, bt, tiles, 2, 2.0 ** min(-q_exp, 126) / math.sqrt(dh), 0)
+    ops().attention(args[0], narrow, *args[1:])
+    ops().attention(args[0], wide, *args[1:], tiles_wide=paged_case.wide)
+    assert torch.equal(narrow, wide) and bool(torch.isfinite(wide).all()) and (wide != 0).float().mean() > 0.9
+    if v_exp < -120:
+        assert (wide.abs() < 2.0 ** -126).float().mean() > 0.9
+
+
 @pytest.mark.parametrize("H,Hkv,dh,ps,kw", [
     (2, 2, 16, 16, {}), (3, 1, 32, 16, {}), (2, 2, 48, 48, {}), (4, 2, 64, 16, {}), (2, 2, 64, 64, dict(window=70)), (2, 1, 80, 32, {}),
     (2, 2, 96, 16, dict(window=33)), (1, 1, 112, 16, {}), (2, 1, 128, 32, {}), (2, 2, 64, 16, dict(chunk=50, sink=True)),

@@ -133,6 +133,40 @@ def test_every_cutting_at_real_layer_sizes(real_folder, shape, dtype):
         del got
 
 
+@pytest.mark.parametrize("width,heads", [(1280, 20), (1024, 16), (1600, 25)])
+def test_steps_whose_sums_the_norms_add(tmp_path, width, heads):
+    """Steps of 257 to 512 rows, decoded tokens beside portions: the products into the stream leave their shares' sums for the norms
+    behind them (across blocks and behind the last one too), and the logits stay the plain implementation's."""
+    from denno_beta_amd.engine import StepEntry
+    from denno_beta_amd.kernels import ops
+    from denno_beta_amd.weights import write_model_folder
+    cfg, folder = _cfg(3, width, heads, 5000), str(tmp_path / "model")
+    write_model_folder(folder, cfg, 31, "bfloat16")
+    seqs = [seeded_tokens(700 + i, n, 5000) for i, n in enumerate((60, 400, 700, 301))]
+    plain, shares = PlainGPT2.from_folder(folder), []
+    asked = ops.linear_deferred
+    r = runner_for(folder, "bfloat16", 2048)
+    for i in range(4):
+        r.start_request(i)
+    got, at = [[] for _ in seqs], [0] * 4
+    ops.linear_deferred = lambda a, w: shares.append((a.shape[0], ops.linear_deferred_shares(a.shape[0], w))) or asked(a, w)
+    try:
+        for portions in ((50, 399, 0, 0), (1, 1, 255, 0), (1, 0, 318, 1), (1, 0, 120, 300), (7, 0, 7, 0)):
+            live = [(i, n) for i, n in enumerate(portions) if n]
+            out = r.step([StepEntry(i, seqs[i][at[i]:at[i] + n], list(range(n))) for i, n in live]).cpu()
+            for i, n in live:
+                got[i].append(out[:n])
+                out, at[i] = out[n:], at[i] + n
+    finally:
+        ops.linear_deferred = asked
+    for i, s in enumerate(seqs):
+        check(torch.cat(got[i]), plain.logits(s)[:at[i]], "bfloat16", f"width {width} request {i}")
+    assert at == [60, 400, 700, 301]
+    # (a step of 320 rows may run as one of more, in a captured graph; 1,600 columns from 385 rows on are not cut, K = 1,600 from 321)
+    rows = {n for n, k in shares if k > 0}
+    assert 257 in rows and all(256 < n <= 512 for n in rows) and len(rows) >= (2 if width == 1600 else 4), shares
+
+
 # All 24 layers of the Medium shape: what rounding adds up to over a model's whole depth.  Measured over eight
 # sequences of 1,024 tokens in four cuttings: 0.047 of a row's spread at worst and 0.0060 on average (the 48 layers of
 # the XL shape: 0.051 and 0.0061), where two layers give 0.028 and 0.0039; the 32-bit engine stays within 3.5e-6.
