@@ -68,13 +68,16 @@ __device__ __forceinline__ void lay8(float* at, const TI* v, int inside) {
   *reinterpret_cast<float4*>(at + 4) = float4{f[1], f[3], f[5], f[7]};
 }
 
-template <typename TI, typename TC, bool WHOLE>
-__global__ __launch_bounds__(256, 4) void gemm_kernel(const TI* __restrict__ A, int lda, const TI* __restrict__ W,
+// SHORT: K of at most 64, a slab or two: nothing to overlap inside a workgroup, so a slab is loaded, laid down and multiplied, in half of the LDS, and eight
+// workgroups a CU hide each other's waits.  (With slabs asked for that are not there, and four workgroups a CU, the long walk's kernel takes 40.3 us for 2,048 x
+// 8,192 x 16 in bfloat16, 11.6 for 1 x 50,257 x 33; single multiply-adds took 32.5 and 9.0, this takes 30.9 and 9.5.)
+template <typename TI, typename TC, bool WHOLE, bool SHORT>
+__global__ __launch_bounds__(256, SHORT ? 8 : 4) void gemm_kernel(const TI* __restrict__ A, int lda, const TI* __restrict__ W,
                                                        const float* __restrict__ bias, TC* __restrict__ C, int ldc,
                                                        float* __restrict__ resid, int ldr, int M, int N, int K,
                                                        int epi, int mtiles, int tiles, int per_xcd) {
-  __shared__ __attribute__((aligned(16))) float As[2][BM * LLD];
-  __shared__ __attribute__((aligned(16))) float Ws[2][BN * LLD];
+  __shared__ __attribute__((aligned(16))) float As[SHORT ? 1 : 2][BM * LLD];
+  __shared__ __attribute__((aligned(16))) float Ws[SHORT ? 1 : 2][BN * LLD];
   // each of the 8 XCDs, among which workgroups go round, takes a run of tiles, rows first: its L2 then serves a few column
   // tiles' weights and the rows
   const int tile = static_cast<int>(blockIdx.x % 8) * per_xcd + static_cast<int>(blockIdx.x / 8);
@@ -91,47 +94,68 @@ __global__ __launch_bounds__(256, 4) void gemm_kernel(const TI* __restrict__ A, 
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = tot[r] = 0.f;
   TI av[8], wv[8];
-  load8<TI, WHOLE>(arow, lk, K, av);
-  load8<TI, WHOLE>(wrow, lk, K, wv);
-  lay8(&As[0][lrow * LLD + lk], av, K - lk);
-  lay8(&Ws[0][lrow * LLD + lk], wv, K - lk);
-  load8<TI, WHOLE>(arow, LK + lk, K, av);
-  load8<TI, WHOLE>(wrow, LK + lk, K, wv);
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += LK, buf ^= 1) {
-    // a slab's operands are read at once; in the middle of its matrix instructions the next slab is laid down and the one
-    // after it asked for, so that only the barrier stands between two slabs' matrix instructions
-    float4 a[LK / 8], w[LK / 8];
+  if constexpr (SHORT) {
+    for (int k0 = 0; k0 < K; k0 += LK) {
+      load8<TI, WHOLE>(arow, k0 + lk, K, av);
+      load8<TI, WHOLE>(wrow, k0 + lk, K, wv);
+      if (k0 > 0) __syncthreads();
+      lay8(&As[0][lrow * LLD + lk], av, K - k0 - lk);
+      lay8(&Ws[0][lrow * LLD + lk], wv, K - k0 - lk);
+      __syncthreads();
 #pragma unroll
-    for (int g = 0; g < LK / 8; ++g) {
-      a[g] = *reinterpret_cast<const float4*>(&As[buf][fa + 8 * g]);
-      w[g] = *reinterpret_cast<const float4*>(&Ws[buf][fw + 8 * g]);
-    }
-#pragma unroll
-    for (int g = 0; g < LK / 8; ++g) {
-      if (g == LK / 16) {
-        __builtin_amdgcn_sched_barrier(0);
-        const int inside = k0 + 2 * LK <= K ? 8 : K - (k0 + LK + lk);
-        lay8(&As[buf ^ 1][lrow * LLD + lk], av, inside);      // (behind the last slab: zeros that nobody reads)
-        lay8(&Ws[buf ^ 1][lrow * LLD + lk], wv, inside);
-        load8<TI, WHOLE>(arow, k0 + 2 * LK + lk, K, av);
-        load8<TI, WHOLE>(wrow, k0 + 2 * LK + lk, K, wv);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].x, w[g].x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].y, w[g].y, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].z, w[g].z, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].w, w[g].w, acc, 0, 0, 0);
-    }
-    if ((k0 + LK) % SEG == 0 || k0 + LK >= K) {         // a segment ends: its sum joins the others'
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        tot[r] += acc[r];
-        acc[r] = 0.f;
+      for (int g = 0; g < LK / 8; ++g) {
+        const float4 a = *reinterpret_cast<const float4*>(&As[0][fa + 8 * g]), w = *reinterpret_cast<const float4*>(&Ws[0][fw + 8 * g]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, w.x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, w.y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, w.z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, w.w, acc, 0, 0, 0);
       }
     }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tot[r] += acc[r];
+  } else {
+    load8<TI, WHOLE>(arow, lk, K, av);
+    load8<TI, WHOLE>(wrow, lk, K, wv);
+    lay8(&As[0][lrow * LLD + lk], av, K - lk);
+    lay8(&Ws[0][lrow * LLD + lk], wv, K - lk);
+    load8<TI, WHOLE>(arow, LK + lk, K, av);
+    load8<TI, WHOLE>(wrow, LK + lk, K, wv);
     __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < K; k0 += LK, buf ^= 1) {
+      // a slab's operands are read at once; in the middle of its matrix instructions the next slab is laid down and the one
+      // after it asked for, so that only the barrier stands between two slabs' matrix instructions
+      float4 a[LK / 8], w[LK / 8];
+#pragma unroll
+      for (int g = 0; g < LK / 8; ++g) {
+        a[g] = *reinterpret_cast<const float4*>(&As[buf][fa + 8 * g]);
+        w[g] = *reinterpret_cast<const float4*>(&Ws[buf][fw + 8 * g]);
+      }
+#pragma unroll
+      for (int g = 0; g < LK / 8; ++g) {
+        if (g == LK / 16) {
+          __builtin_amdgcn_sched_barrier(0);
+          const int inside = k0 + 2 * LK <= K ? 8 : K - (k0 + LK + lk);
+          lay8(&As[buf ^ 1][lrow * LLD + lk], av, inside);      // (behind the last slab: zeros that nobody reads)
+          lay8(&Ws[buf ^ 1][lrow * LLD + lk], wv, inside);
+          load8<TI, WHOLE>(arow, k0 + 2 * LK + lk, K, av);
+          load8<TI, WHOLE>(wrow, k0 + 2 * LK + lk, K, wv);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].x, w[g].x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].y, w[g].y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].z, w[g].z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].w, w[g].w, acc, 0, 0, 0);
+      }
+      if ((k0 + LK) % SEG == 0 || k0 + LK >= K) {         // a segment ends: its sum joins the others'
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          tot[r] += acc[r];
+          acc[r] = 0.f;
+        }
+      }
+      __syncthreads();
+    }
   }
   // a lane holds column lane % 32 of the rows 8 (r / 4) + 4 (lane / 32) + r % 4
   const int n = n0 + wn + lane % 32;
@@ -359,12 +383,21 @@ static int run(const void* A, int lda, const void* W, const float* bias, void* C
     const long all = static_cast<long>(mtiles) * ((N + BN - 1) / BN);
     if (all > (1 << 30)) return DN_ERR_SHAPE;
     const int tiles = static_cast<int>(all), per_xcd = (tiles + 7) / 8;
-    if (K % 4 == 0)
-      hipLaunchKernelGGL((gemm_kernel<TI, TC, true>), dim3(per_xcd * 8), dim3(256), 0, stream, a, lda, w, bias, c, ldc, resid,
-                         ldr, M, N, K, epi, mtiles, tiles, per_xcd);
+#define DN_MANY(WHOLE, SHORT)                                                                                                    \
+  hipLaunchKernelGGL((gemm_kernel<TI, TC, WHOLE, SHORT>), dim3(per_xcd * 8), dim3(256), 0, stream, a, lda, w, bias, c, ldc, resid, \
+                     ldr, M, N, K, epi, mtiles, tiles, per_xcd)
+    // (a short K whose tiles are two a CU at most: nobody's waits to hide, and the registers of the long walk's kernel make the shorter end:
+    // 200 x 64 x 64 in bfloat16, added into the stream, 5.9 us and 6.3)
+    const bool brief = K <= 2 * LK && tiles > 2 * 256;
+    if (K % 4 == 0 && brief)
+      DN_MANY(true, true);
+    else if (K % 4 == 0)
+      DN_MANY(true, false);
+    else if (brief)
+      DN_MANY(false, true);
     else
-      hipLaunchKernelGGL((gemm_kernel<TI, TC, false>), dim3(per_xcd * 8), dim3(256), 0, stream, a, lda, w, bias, c, ldc, resid,
-                         ldr, M, N, K, epi, mtiles, tiles, per_xcd);
+      DN_MANY(false, false);
+#undef DN_MANY
     return 0;
   }
   const long need = work_floats(M, N, K);

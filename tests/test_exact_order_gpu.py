@@ -13,7 +13,9 @@ DEV = "cuda:0"
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K", [(65, 64, 128), (65, 1, 4), (129, 63, 1), (200, 65, 127), (64 * 9, 257, 129), (130, 200, 1600),
-                                   (67, 130, 250), (300, 96, 34)])
+                                   (67, 130, 250), (300, 96, 34), (70, 66, 16), (131, 300, 32), (65, 200, 33), (194, 70, 36), (66, 129, 63), (257, 65, 64),
+                                   (66, 70, 65), (130, 64, 68),
+                                   (65, 16449, 33), (1030, 2001, 64), (1030, 2001, 20), (129, 16384, 1)])
 def test_a_product_of_many_rows_has_the_few_rows_bits(dtype, M, N, K):
     """Numbers of very different sizes, so that another order or another rounding shows; ends of tiles, of slabs, of segments."""
     g = torch.Generator().manual_seed(M + N + K)
