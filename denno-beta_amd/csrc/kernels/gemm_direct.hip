@@ -4,12 +4,16 @@
 // Many rows, bfloat16, slabs carried from memory straight into LDS (global_load_lds_dwordx4: 16
 // bytes per lane, lane l's at the wave's LDS address + 16 l, no register and no LDS store between).
 // A slab of 32 along K is a list of 1 KB blocks in the packed layout, 16 rows x 32 columns each:
-// a block of W is 1 KB of memory as it lies and is read back at 16 l by lane l; a block of A is
-// made by the load itself, in an order of its own: the vector cache looks a load's lines up per 16
-// lanes, so 16 lanes take 64 bytes from each of four rows (four lines) and not 16 bytes from each of
-// sixteen (with a lane per row the lookups, 52 per load on average, kept the cache busy for three
-// quarters of the kernel's time), and the four 16-byte pieces of a row are exchanged by the row's
-// number so that the operand read (lane l wants row l % 16, piece l / 16) meets every bank once.  STAGES
+// a block of W is 1 KB of memory as it lies and is read back at 16 l by lane l; rows of A are put in place
+// by the load itself, in an order of its own.  Where a stage has two slabs (K a multiple of 64), 1 KB of A is 8 rows x 128
+// bytes: whole cache lines.  From the L2 into LDS a CU takes 110 GB/s in pieces of 1 KB, 105 so, and 68 where a load takes 64
+// bytes from each of 16 rows, which is what a stage of one slab leaves (16 lanes then take 64 bytes from each of four rows: with a lane per row the lookups, 52 per
+// load on average, kept the vector cache busy for three quarters of the kernel's time).  With 64 bytes a row everywhere: 320 x 3,840
+// x 1,280 15.9 us, now 13.7; 3,500 x 1,280 x 5,120 88.6 -> 70.0; 8,192 x 3,840 x 1,280 110.4 -> 98.4; 8,192 x 6,400 x 1,600 201.5 -> 194; 2,048 x 4,800 x 1,600
+// 44.4 -> 42.8; two slabs a stage for tiles of 192 and more columns with a long K too (it had been one slab in more stages):
+// 8,192 x 1,600 x 6,400 169.5 -> 161.  The 16-byte pieces of a row are exchanged by the row's number so that the operand read (lane l wants
+// row l % 16, piece l / 16) meets every bank once: LDS serves lanes 0-3, 12-15 and 20-27 together, 4-11, 16-19 and 28-31, and
+// the same 32 lanes on (an order that is free of conflicts for 16 lanes in a row only was slower by 0.3 us a product of 512 rows).  STAGES
 // stages of KB slabs are in flight (vmcnt counts a wave's own loads; one barrier per stage publishes them and
 // frees the stage read before).
 //
@@ -82,7 +86,8 @@ __device__ __forceinline__ void tile_at(int pid, int tiles_m, int tiles_n, int b
 // other tiles of 256 rows do not take turns: with bfloat16 results and K up to 3,200 they are level to 15 % slower so (256 x 128: 2,048 x 4,096 x 1,024
 // 26.0 -> 28.7 us; 256 x 224: 2,048 x 6,400 x 1,600 46.8 -> 52.6; 256 x 256: 8,192 x 4,096 x 1,024 79.6 -> 91.4; 192 and more columns with
 // slabs of 32 a stage, since three stages of 64 do not fit in LDS).  Left open: from K = 5,120 on they would gain 3 to 12 % (8,192 x 2,048 x 8,192 225.6 -> 199.3).
-template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false>
+// A_IN: A comes in rows (0), packed (1), or as `packed` says (2).
+template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false, int A_IN = 2>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __restrict__ A, int lda,
                                                            const bf16_t* __restrict__ W, const float* __restrict__ bias,
                                                            TC* __restrict__ C, int ldc, float* __restrict__ resid, int ldr,
@@ -90,6 +95,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
                                                            int tiles_n, KVScatter kv, float* __restrict__ part,
                                                            int split_slabs) {
   constexpr int NW = WM * WN;
+  const bool a_packed = A_IN == 2 ? (packed & PACKED_A) != 0 : A_IN == 1;
   constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
   constexpr int AB = BM / 16, WB = BN / 16;              // 1 KB blocks per slab of 32 along K
   constexpr int PER = (AB + WB) * KB;                    // blocks per stage: KB slabs travel and are multiplied together
@@ -109,10 +115,19 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   const int kall = K / 32, nblocks = (N + 15) / 16;
   const int first = part ? blockIdx.y * split_slabs : 0;
   const int ksteps = part ? min(split_slabs, kall / KB - first) : kall / KB;
-  // where the 16 bytes of row lane % 16, columns 8 (lane / 16) .. of a block of A lie in its 1 KB
-  // (see the loads below): any 8 and any 16 consecutive lanes read all banks once
-  // (a packed A is in the operand's order already: lane l reads at 16 l)
-  const int aslot = (packed & PACKED_A) ? lane : 16 * (lane % 4) + 4 * ((lane % 16) / 4) + ((lane / 16) ^ (lane % 4));
+  // Where the 16 bytes of row lane % 16, columns 8 (lane / 16) .. of a block of A lie among its KB pieces of 1 KB (see the loads below).
+  // (A packed A is in the operand's order already: lane l reads at 16 l.)
+  int aslot[KB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const int r = lane % 16, g = lane / 16;
+    if (a_packed)
+      aslot[kb] = kb * (AB + WB) * 64 + lane;
+    else if constexpr (KB == 2)
+      aslot[kb] = (r / 8) * (AB + WB) * 64 + 8 * (r % 8) + ((4 * kb + g) ^ (r / 2));
+    else
+      aslot[kb] = kb * (AB + WB) * 64 + 16 * (lane % 4) + 4 * (r / 4) + (g ^ (lane % 4));
+  }
 
   // the tokens' slots, which the epilogue reads, are asked for before everything else: the row's, and those of the quad's four tokens
   // (8,192 rows of fused projections of 4,800 and 3,840 columns: 166 -> 160 and 115 -> 108 us)
@@ -141,22 +156,27 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
     const int q = min(wave + u * NW, PER - 1);
     const int b = q % (AB + WB), kb = q / (AB + WB);      // block b of the stage's slab kb
     if (b < AB) {
-      // 16 lanes in a row take 64 bytes from each of four rows (g, g + 4, g + 8, g + 12 of the block):
-      // four cache lines, where a lane per row would touch sixteen
-      const int g = lane / 16, h = (lane % 16) / 4, piece = (lane % 4) ^ g;
-      if (packed & PACKED_A) {      // a block of packed rows is 1 KB as it lies, like a block of W
-        src[u] = A + static_cast<size_t>(min(m0 / 16 + b, (M + 15) / 16 - 1)) * kall * 512 + lane * 8;
-        step[u] = 512;
+      if (a_packed) {      // a block of packed rows is 1 KB as it lies, like a block of W
+        src[u] = A + static_cast<size_t>(min(m0 / 16 + b, (M + 15) / 16 - 1)) * kall * 512 + kb * 512 + lane * 8;
+        step[u] = 512 * KB;
+      } else if constexpr (KB == 2) {
+        // a stage's columns are one cache line of a row: 1 KB is 8 rows x 128 bytes, rows 0 .. 7 of the block in the first slab's place and
+        // 8 .. 15 in the second's
+        const int r = 8 * kb + lane / 8, piece = (lane % 8) ^ (r / 2);
+        src[u] = A + static_cast<size_t>(min(m0 + b * 16 + r, M - 1)) * lda + piece * 8;
+        step[u] = 64;
       } else {
-        src[u] = A + static_cast<size_t>(min(m0 + b * 16 + 4 * h + g, M - 1)) * lda + piece * 8;
-        step[u] = 32;
+        // 16 lanes in a row take 64 bytes from each of four rows (g, g + 4, g + 8, g + 12 of the block):
+        // four cache lines, where a lane per row would touch sixteen
+        const int g = lane / 16, h = (lane % 16) / 4, piece = (lane % 4) ^ g;
+        src[u] = A + static_cast<size_t>(min(m0 + b * 16 + 4 * h + g, M - 1)) * lda + kb * 32 + piece * 8;
+        step[u] = 32 * KB;
       }
     } else {
-      src[u] = W + static_cast<size_t>(min(n0 / 16 + b - AB, nblocks - 1)) * kall * 512 + lane * 8;
-      step[u] = 512;
+      src[u] = W + static_cast<size_t>(min(n0 / 16 + b - AB, nblocks - 1)) * kall * 512 + kb * 512 + lane * 8;
+      step[u] = 512 * KB;
     }
-    src[u] += (static_cast<size_t>(first) * KB + kb) * step[u];
-    step[u] *= KB;
+    src[u] += static_cast<size_t>(first) * step[u];
   }
   auto issue = [&](int kt) {
     u32x4* slab = lds + (kt % STAGES) * SLAB;
@@ -194,7 +214,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
       for (int kb = 0; kb < KB; ++kb) {
         const u32x4* sl = slab + kb * (AB + WB) * 64;
 #pragma unroll
-        for (int i = 0; i < TM; ++i) af[kb][i] = __builtin_bit_cast(bf16x8, sl[(wmb + i) * 64 + aslot]);
+        for (int i = 0; i < TM; ++i) af[kb][i] = __builtin_bit_cast(bf16x8, slab[(wmb + i) * 64 + aslot[kb]]);
 #pragma unroll
         for (int j = 0; j < TN; ++j) wf[kb][j] = __builtin_bit_cast(bf16x8, sl[(AB + wnb + j) * 64 + lane]);
       }
@@ -229,7 +249,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
         const u32x4* sl = slab + kb * (AB + WB) * 64;
         bf16x8 af[TM], wf[TN];
   #pragma unroll
-        for (int i = 0; i < TM; ++i) af[i] = __builtin_bit_cast(bf16x8, sl[(wmb + i) * 64 + aslot]);
+        for (int i = 0; i < TM; ++i) af[i] = __builtin_bit_cast(bf16x8, slab[(wmb + i) * 64 + aslot[kb]]);
   #pragma unroll
         for (int j = 0; j < TN; ++j) wf[j] = __builtin_bit_cast(bf16x8, sl[(AB + wnb + j) * 64 + lane]);
   #pragma unroll
@@ -363,7 +383,7 @@ bool takes(const void* A, int lda, const void* W, const float* bias, const void*
 }
 
 
-template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false>
+template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false, int A_IN = 2>
 static int launch(const Args& a, hipStream_t stream) {
   constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
@@ -371,13 +391,13 @@ static int launch(const Args& a, hipStream_t stream) {
   if (a.K % (32 * KB) != 0) return DN_ERR_SHAPE;
   static bool raised = false;      // more than 64 KB of LDS has to be asked for once per kernel
   if (lds > 65536 && !raised) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     if (e != hipSuccess) return static_cast<int>(e);
     raised = true;
   }
   const int split_slabs = (a.K / (32 * KB) + a.splits - 1) / a.splits;
-  hipLaunchKernelGGL((gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING>), dim3(tiles_m * tiles_n, a.part ? a.splits : 1),
+  hipLaunchKernelGGL((gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN>), dim3(tiles_m * tiles_n, a.part ? a.splits : 1),
                      dim3(WM * WN * 64), lds, stream, static_cast<const bf16_t*>(a.A), a.lda,
                      static_cast<const bf16_t*>(a.W), a.bias, static_cast<TC*>(a.C), a.ldc, a.resid, a.ldr, a.M, a.N, a.K,
                      a.epi, a.packed, tiles_m, tiles_n, a.kv ? *a.kv : KVScatter{}, a.part, split_slabs);
@@ -389,6 +409,19 @@ static int launch_as(const Args& a, hipStream_t stream) {
   if (a.kv) return launch<bf16_t, WM, WN, TM, TN, STAGES, true, KB>(a, stream);
   if (a.out_dtype == DN_BF16 && !a.resid) return launch<bf16_t, WM, WN, TM, TN, STAGES, false, KB>(a, stream);
   return launch<float, WM, WN, TM, TN, STAGES, false, KB>(a, stream);
+}
+
+// (for steps of 65 to 256 rows: a kernel each for A in rows and for packed A, since the choice at run time stands in front of the first loads)
+template <int WM, int WN, int TM, int TN, int STAGES, int KB, int A_IN>
+static int launch_mid_a(const Args& a, hipStream_t stream) {
+  if (a.kv) return launch<bf16_t, WM, WN, TM, TN, STAGES, true, KB, false, A_IN>(a, stream);
+  if (a.out_dtype == DN_BF16 && !a.resid) return launch<bf16_t, WM, WN, TM, TN, STAGES, false, KB, false, A_IN>(a, stream);
+  return launch<float, WM, WN, TM, TN, STAGES, false, KB, false, A_IN>(a, stream);
+}
+
+template <int WM, int WN, int TM, int TN, int STAGES, int KB>
+static int launch_mid(const Args& a, hipStream_t stream) {
+  return (a.packed & PACKED_A) ? launch_mid_a<WM, WN, TM, TN, STAGES, KB, 1>(a, stream) : launch_mid_a<WM, WN, TM, TN, STAGES, KB, 0>(a, stream);
 }
 
 // (for tiles that never write the cache: the variant with the cache write is not built)
@@ -494,17 +527,16 @@ int run(const Args& a, hipStream_t stream) {
     // are more than the chip has CUs, tiles of 128 x 64 with two blocks a wave (at 256 rows 23.3 -> 20.2 and
     // 18.1 -> 15.2 us).  The narrow ones, whose K is shared out, take neither way faster: four waves as before.
     if (wide_mid(a.M, a.N) && !a.part)
-      return mid_tiles_64(a.M, a.N) <= CUS ? launch_as<4, 4, 1, 1, 4, 2>(a, stream) : launch_as<4, 4, 2, 1, 4, 2>(a, stream);
-    return launch_as<2, 2, 2, 2, 4, 2>(a, stream);
+      return mid_tiles_64(a.M, a.N) <= CUS ? launch_mid<4, 4, 1, 1, 4, 2>(a, stream) : launch_mid<4, 4, 2, 1, 4, 2>(a, stream);
+    return launch_mid<2, 2, 2, 2, 4, 2>(a, stream);
   }
   // Tiles of 128 and 256 rows: sixteen waves a workgroup, four a SIMD, as 8 x 2 (a wave: 32 rows x a half of the
   // tile's columns) or 4 x 4, where eight waves as 4 x 2 with twice the rows each left the SIMDs waiting (a wave
   // waits on a counter for more than half of its life and the matrix cores were busy 30 % of the time).  At 2,048
   // rows of the XL layer: 56.1 -> 41.0, 25.2 -> 21.3, 57.1 -> 46.6 and 71.8 -> 56.9 us.  Two slabs a stage where K
-  // allows it; a long K wants more stages in flight than a short one (with two, the MLP projection of 4,096 rows
-  // took 145 us for 125), and LDS decides how many fit.  The cache write's epilogue needs registers that sixteen
+  // allows it (whole cache lines of A's rows), else one in as many stages as fit in LDS.  The cache write's epilogue needs registers that sixteen
   // waves do not leave beside seven column blocks and more a wave: those keep eight waves.
-  const bool sixteen = !a.part, two = a.K % 64 == 0, short_k = a.K < 4096;
+  const bool sixteen = !a.part, two = a.K % 64 == 0;
   switch (pick(a.M, a.N, a.part ? a.K / a.splits : a.K, a.kv != nullptr)) {
     case 0:      // (the small tiles with sixteen waves too, where one round of them covers the product: several
                  // workgroups of four waves share a CU, one of sixteen has it alone)
@@ -523,15 +555,15 @@ int run(const Args& a, hipStream_t stream) {
       return launch_as<8, 2, 2, 5, 3, 2>(a, stream);
     case 4:
       if (!sixteen) return launch_as<4, 2, 4, 6, 4>(a, stream);
-      return two && short_k ? launch_as<8, 2, 2, 6, 2, 2>(a, stream) : launch_as<8, 2, 2, 6, 3>(a, stream);
+      return two ? launch_as<8, 2, 2, 6, 2, 2>(a, stream) : launch_as<8, 2, 2, 6, 3>(a, stream);
     case 5:
       if (a.kv || !sixteen) return launch_as<4, 2, 4, 7, 4>(a, stream);
-      return two && short_k ? launch_without_kv<8, 2, 2, 7, 2, 2>(a, stream) : launch_without_kv<8, 2, 2, 7, 5>(a, stream);
+      return two ? launch_without_kv<8, 2, 2, 7, 2, 2>(a, stream) : launch_without_kv<8, 2, 2, 7, 5>(a, stream);
     case 6:
       if (a.kv || !sixteen) return launch_as<4, 2, 4, 8, 4>(a, stream);
-      return two && short_k ? launch_without_kv<8, 2, 2, 8, 2, 2>(a, stream) : launch_without_kv<8, 2, 2, 8, 3>(a, stream);
+      return two ? launch_without_kv<8, 2, 2, 8, 2, 2>(a, stream) : launch_without_kv<8, 2, 2, 8, 3>(a, stream);
     case 7:
-      if (sixteen && two && tiles_of(a.M, a.N, 64, 64) <= CUS) return launch_as<4, 4, 1, 1, 4, 2>(a, stream);
+      if (sixteen && two && tiles_of(a.M, a.N, 64, 64) <= CUS) return launch_mid<4, 4, 1, 1, 4, 2>(a, stream);
       return launch_as<2, 2, 2, 2, 4>(a, stream);
     default: return launch_as<2, 2, 1, 2, 4>(a, stream);
   }

@@ -383,6 +383,23 @@ def test_the_norm_inside_products_refuses_what_it_cannot_take():
         ops().linear_norm_out(rnd(17, 64, dtype=torch.bfloat16), wp, None, rnd(17, 32), c, *ops().norm_stream_buffers(17, 32, DEV))
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 2048, 64), (70, 100, 4160), (130, 4096, 192), (257, 1280, 1280), (300, 2100, 128), (511, 3840, 1280), (1000, 640, 4160),
+                                   (2100, 1664, 4096), (3500, 1284, 5120), (2049, 6400, 320)])
+def test_many_rows_products_put_every_piece_of_a_row_in_its_place(M, N, K):
+    """Small whole numbers, whose sums 32 bits hold exactly whatever their order: rows with a gap between them, in products
+    with one and with two slabs a stage, in whole and in shares of K; a row that has no neighbour but the end of A."""
+    o = ops()
+    g = torch.Generator().manual_seed(M + K)
+    a = torch.randint(-3, 4, (M, K + 24), generator=g).to(torch.bfloat16).cuda()[:, 8:8 + K]
+    w = torch.randint(-3, 4, (N, K), generator=g).to(torch.bfloat16).cuda()
+    want = (a.double() @ w.double().t()).float()
+    pw = o.pack_matrix(w)
+    assert torch.equal(o.linear(a, pw, out=torch.empty((M, N), device="cuda")), want)
+    assert torch.equal(o.linear(a, pw, residual=torch.zeros((M, N), device="cuda")), want)
+    if o.linear_deferred_shares(M, pw):
+        assert torch.equal(o.linear_deferred(a, pw).sum(0), want)
+
+
 @pytest.mark.parametrize("M", [100, 129, 200, 256, 300, 1000, 2100, 4200])
 @pytest.mark.parametrize("rows_in", ["packed", "rows"])
 @pytest.mark.parametrize("K", [160, 192, 4160])
