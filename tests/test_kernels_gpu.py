@@ -641,6 +641,21 @@ def test_attention_mfma_kernel_for_portions(H, Hkv, dh, ps, window):
         assert T2 == 200 and torch.equal(packed.rows(), rows)
 
 
+@pytest.mark.parametrize("H,Hkv,dh,ps,extras", [(4, 2, 64, 16, {}), (2, 2, 16, 48, {}), (3, 1, 128, 32, dict(window=100)), (1, 1, 256, 16, {}),
+                                                (2, 1, 48, 16, dict(window=70, keep_first=20, sink=True)), (2, 2, 80, 64, dict(chunk=96, softcap=3.0))])
+def test_attention_of_single_rows_beside_portions(H, Hkv, dh, ps, extras):
+    """Tiles of one row in the kernel for portions, with contexts at the edges of a wave's 64 keys and of a workgroup's walk, beside a
+    portion and a tile of two rows."""
+    seq_lens = [1, 2, 63, 64, 65, 256, 257, 511, 512, 513, 1100, 130, 200]
+    new_rows = [1] * 11 + [2, 150]
+    q, k, v, bt, tiles, T = paged_case(seq_lens, new_rows, H, Hkv, dh, ps, torch.bfloat16, seed=dh)
+    out = torch.zeros(T, H * dh, dtype=torch.bfloat16, device=DEV)
+    ops().attention(q[:, :H * dh], out, k, v, bt, tiles, H, dh ** -0.5, tiles_wide=paged_case.wide, **extras)
+    want = torch.zeros(T, H * dh, dtype=torch.float32, device=DEV)      # (the plain kernel in 32-bit, on the same numbers)
+    ops().attention(q[:, :H * dh].float(), want, k.float(), v.float(), bt, tiles, H, dh ** -0.5, **extras)
+    assert torch.allclose(out.float(), want, **TOL[torch.bfloat16])
+
+
 @pytest.mark.parametrize("H,Hkv,dh,ps,window", [(8, 8, 64, 16, 0), (8, 2, 32, 32, 40), (8, 4, 64, 48, 0),
                                                 (8, 8, 96, 16, 0), (8, 2, 128, 32, 60), (8, 8, 80, 16, 0),
                                                 (8, 4, 160, 16, 30), (8, 8, 256, 16, 0)])
