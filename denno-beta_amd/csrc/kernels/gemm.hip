@@ -79,7 +79,7 @@ extern "C" int dn_gemm(const void* A, int lda, const void* W, const float* bias,
 // pools (keys [page, Hkv, page_size, dh], values [page, Hkv, dh, page_size], of C's type), written by the kernel
 // that adds the segments' sums.  Only where the product has that kernel: dn_gemm_plain_qkv_takes.
 extern "C" int dn_gemm_plain_qkv_takes(const void* A, int lda, const void* W, int M, int N, int K, int dtype) {
-  if (plain::work_floats(M, N, K) <= 0) return 0;
+  if (!plain::joins_of(M, N, K)) return 0;
   return plain::few_rows_take_of(dtype, A, lda, W, M, K);
 }
 

@@ -119,6 +119,7 @@ __device__ __forceinline__ void scatter_kv(const KVScatter& kv, int m, int nn, b
 
 namespace plain {
 long work_floats(int M, int N, int K);
+int joins_of(int M, int N, int K);      // whether a product that few_rows_take_of takes ends in a kernel that writes the cache as well
 int few_rows_take_of(int dtype, const void* A, int lda, const void* W, int M, int K);
 int run_of(int in_dtype, int out_dtype, const void* A, int lda, const void* W, const float* bias, void* C, int ldc,
            float* resid, int ldr, int M, int N, int K, int epilogue, float* work, long have, hipStream_t stream);

@@ -4,8 +4,9 @@
 // The plain product: 32-bit arithmetic for any dtype, one order of summation for every element
 // whatever M is, so that logits do not depend on how a step was cut: K goes in segments of SEG; a
 // segment's sum runs k ascending from zero, one fused multiply-add a step; the segments' sums are
-// added in ascending order, starting from zero.  Two kernels keep to it.  Many rows (M > 64): 64 x 64
-// tiles on the matrix cores, a workgroup walks all of K.  Few rows: a tile of 8 to 64 rows x 64 columns, and where the
+// added in ascending order, starting from zero.  Three kernels keep to it.  Many rows (M > 64): 64 x 64
+// tiles on the matrix cores, a workgroup walks all of K.  Up to 16 rows (`chain_takes`): 8 or 16 columns and all of K a
+// workgroup, on the matrix cores too.  Between them: a tile of 8 to 64 rows x 64 columns, and where the
 // column tiles alone do not fill the chip every segment is a workgroup of its own, which asks for its
 // whole share of W (64 x 128: 32 KB) at once and leaves its sum in a workspace; a second kernel adds
 // the segments' sums in order and ends with the epilogue.  (Few rows used to run in the many-rows
@@ -194,6 +195,132 @@ __device__ __forceinline__ void load4(const bf16_t* p, float* v) {
   v[2] = __uint_as_float(x.y << 16), v[3] = __uint_as_float(x.y & 0xffff0000u);
 }
 
+// Where the key and value columns of a fused projection of few rows go besides C (slot_map == null: nowhere):
+// as KVScatter says it, with pools of C's own type.
+template <typename TC>
+struct KVRows {
+  const int32_t* slot_map;
+  TC* k_pool;
+  TC* v_pool;
+  int q_width, kv_width, dh, page_size, Hkv;
+};
+
+// such a column's value, as `finish` stored it in C, at its token's place in the cache
+template <typename TC>
+__device__ __forceinline__ void to_cache(float tot, int m, int n, const float* bias, int epi, const KVRows<TC>& kv) {
+  if (kv.slot_map == nullptr || n < kv.q_width) return;
+  const int slot = kv.slot_map[m];
+  if (slot < 0) return;
+  int c = n - kv.q_width;
+  const bool is_value = c >= kv.kv_width;
+  if (is_value) c -= kv.kv_width;
+  const int page = slot / kv.page_size, off = slot % kv.page_size;
+  const int hh = c / kv.dh, d = c % kv.dh;
+  const size_t base = (static_cast<size_t>(page) * kv.Hkv + hh) * kv.page_size * kv.dh;
+  const TC x = from_float<TC>(apply_epilogue(bias ? tot + bias[n] : tot, epi));
+  if (is_value)
+    kv.v_pool[base + static_cast<size_t>(d) * kv.page_size + off] = x;
+  else
+    kv.k_pool[base + static_cast<size_t>(off) * kv.dh + d] = x;
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Four registers, four rows of 16 lanes: lane group g gives its register s to group s's register g (a 4 x 4 turn).  Written as assembly for
+// the reason that `other_half` gives, with the idle cycles that the swaps and the matrix instruction behind them want.
+__device__ __forceinline__ void turn4(float* v) {
+  unsigned a = __builtin_bit_cast(unsigned, v[0]), b = __builtin_bit_cast(unsigned, v[1]), c = __builtin_bit_cast(unsigned, v[2]),
+           d = __builtin_bit_cast(unsigned, v[3]);
+  asm volatile(
+      "s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1\n\t"
+      "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1"
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+  v[0] = __builtin_bit_cast(float, a), v[1] = __builtin_bit_cast(float, b), v[2] = __builtin_bit_cast(float, c), v[3] = __builtin_bit_cast(float, d);
+}
+
+// Up to 16 rows: one kernel.  A workgroup owns 16 columns, or, for up to 8 rows, 8, and all of K; a wave takes a segment at a time, every load of it at
+// once, straight into registers, and multiplies on the matrix cores: v_mfma_f32_16x16x4_f32 adds its four products to the sum
+// one after the other, k ascending, each with one rounding: the bits of the chain of fused multiply-adds.  Its operands want k = 4 s + g in lane group g, and a lane's
+// 16 bytes are k = 4 g + s: a 4 x 4 turn between lane groups (`turn4`).  With up to 8 rows the 16 x 16 result is two segments' 8 x 8 on its
+// diagonal: lanes l % 16 < 8 bring rows and columns of one segment, the others the same rows and columns of the next (the blocks off the diagonal
+// are dropped), so that twice as many workgroups ask for half as much each.  The segments' sums meet in LDS and are added in order.  It had been a kernel with a
+// workgroup a segment, whose operands went through LDS and vector multiply-adds, and a second one to add the sums: at 1 and 8 rows
+// 3,072 x 1,024 10.4 -> 6.1 and 10.8 -> 7.4 us, 1,024 x 1,024 7.0 -> 4.6 and 7.3 -> 5.2, 1,024 x 4,096 12.1 -> 8.7 and 12.3 -> 10.8, 1,600 x
+// 6,400 20.0 -> 14.2 and 20.6 -> 17.1, 50,257 x 1,024 75.5 -> 36.7 (5.6 TB/s of W) and 75.6 -> 50.5.  From 8 rows on what a workgroup reads of A is as much as it reads of W.
+template <typename TI, typename TC, int WAVES, bool PAIR, int NB>
+__global__ __launch_bounds__(WAVES * 64) void chain_kernel(const TI* __restrict__ A, int lda, const TI* __restrict__ W, const float* __restrict__ bias,
+                                                            TC* __restrict__ C, int ldc, float* __restrict__ resid, int ldr, int M, int N, int K,
+                                                            int epi, KVRows<TC> kv) {
+  constexpr int SIDE = PAIR ? 8 : 16, EACH = PAIR ? 2 : 1;      // rows and columns of a block of the result; segments at a time
+  constexpr int BLOCK = SIDE * SIDE / 4;
+  extern __shared__ f32x4 sums[];                               // [segment][NB][BLOCK]: place (row / 4) * SIDE + column of a block, its four rows
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), g = lane / 16, half = PAIR ? lane % 16 / 8 : 0;
+  const int n0 = blockIdx.x * (SIDE * NB), m0 = blockIdx.y * SIDE, nseg = (K + SEG - 1) / SEG;
+  const TI* arow = A + static_cast<size_t>(min(m0 + lane % SIDE, M - 1)) * lda;
+  const TI* wrow[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) wrow[b] = W + static_cast<size_t>(min(n0 + b * SIDE + lane % SIDE, N - 1)) * K;
+  for (int s0 = wave * EACH; s0 < nseg; s0 += WAVES * EACH) {
+    const int k0 = (s0 + half) * SEG + 4 * g;
+    float w[NB][SEG / 16][4], a[SEG / 16][4];
+    // (never a conditional load: what lies beyond K is read from the row's end and counts as zeros, the weight as well as the row)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int q = 0; q < SEG / 16; ++q) load4(wrow[b] + min(k0 + 16 * q, K - 4), w[b][q]);
+#pragma unroll
+    for (int q = 0; q < SEG / 16; ++q) load4(arow + min(k0 + 16 * q, K - 4), a[q]);
+    f32x4 acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < SEG / 16; ++q) {
+      if ((s0 + EACH) * SEG > K) {      // (the same for the whole wave)
+        const bool inside = k0 + 16 * q < K;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          a[q][i] = inside ? a[q][i] : 0.f;
+#pragma unroll
+          for (int b = 0; b < NB; ++b) w[b][q][i] = inside ? w[b][q][i] : 0.f;
+        }
+      }
+      turn4(a[q]);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        turn4(w[b][q]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][i], w[b][q][i], acc[b], 0, 0, 0);
+      }
+    }
+    // acc[b][r]: row 4 g + r, column lane % 16
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if (!PAIR)
+        sums[(s0 * NB + b) * BLOCK + lane] = acc[b];
+      else if (g / 2 == half && s0 + half < nseg)
+        sums[((s0 + half) * NB + b) * BLOCK + g % 2 * 8 + lane % 8] = acc[b];
+    }
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < NB * SIDE * SIDE; t += WAVES * 64) {
+    const int b = t / (SIDE * SIDE), row = t / SIDE % SIDE, m = m0 + row, n = n0 + b * SIDE + t % SIDE;
+    if (m >= M || n >= N) continue;
+    const float* p = reinterpret_cast<const float*>(sums) + (b * BLOCK + (row / 4) * SIDE + t % SIDE) * 4 + row % 4;
+    float tot = 0.f;
+    int s = 0;
+    for (; s + 8 <= nseg; s += 8) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = p[(s + i) * NB * BLOCK * 4];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) tot += v[i];
+    }
+    for (; s < nseg; ++s) tot += p[s * NB * BLOCK * 4];
+    finish<TC>(tot, m, n, bias, C, ldc, resid, ldr, epi);
+    to_cache<TC>(tot, m, n, bias, epi, kv);
+  }
+}
+
 // Few rows.  A workgroup: RM rows x 64 columns, the segments [seg0, seg0 + nseg) of K.  part == null:
 // it owns all segments and ends with the epilogue; else it owns one (blockIdx.z) and writes its sum to
 // part[seg][m][n].  A segment's share of W (64 rows x 128 k) and of A is asked for at once, 16 bytes a
@@ -301,16 +428,6 @@ __global__ __launch_bounds__(256) void rows_kernel(const TI* __restrict__ A, int
   }
 }
 
-// Where the key and value columns of a fused projection of few rows go besides C (slot_map == null: nowhere):
-// as KVScatter says it, with pools of C's own type.
-template <typename TC>
-struct KVRows {
-  const int32_t* slot_map;
-  TC* k_pool;
-  TC* v_pool;
-  int q_width, kv_width, dh, page_size, Hkv;
-};
-
 // the segments' sums of each element, added in ascending order from zero, then the epilogue; the keys and values
 // among the columns also go to their tokens' places in the cache, so that no kernel has to copy them there
 template <typename TC>
@@ -332,28 +449,17 @@ __global__ __launch_bounds__(256) void join_kernel(const float* __restrict__ par
   }
   for (; s < nseg; ++s) tot += p[s * step];
   finish<TC>(tot, m, n, bias, C, ldc, resid, ldr, epi);
-  if (kv.slot_map != nullptr && n >= kv.q_width) {
-    const int slot = kv.slot_map[m];
-    if (slot < 0) return;
-    int c = n - kv.q_width;
-    const bool is_value = c >= kv.kv_width;
-    if (is_value) c -= kv.kv_width;
-    const int page = slot / kv.page_size, off = slot % kv.page_size;
-    const int hh = c / kv.dh, d = c % kv.dh;
-    const size_t base = (static_cast<size_t>(page) * kv.Hkv + hh) * kv.page_size * kv.dh;
-    const TC x = from_float<TC>(apply_epilogue(bias ? tot + bias[n] : tot, epi));      // what finish stored in C
-    if (is_value)
-      kv.v_pool[base + static_cast<size_t>(d) * kv.page_size + off] = x;
-    else
-      kv.k_pool[base + static_cast<size_t>(off) * kv.dh + d] = x;
-  }
+  to_cache<TC>(tot, m, n, bias, epi, kv);
 }
 
 constexpr int FEW_ROWS = 64;
+// Whether chain_kernel takes a product that few_rows_take takes: its segments' sums fit 60 KB of LDS, and beyond 8 rows the segments are as many as its
+// waves take in two turns (16 rows x 1,600 columns from K = 6,400: 28.4 us, 22.3 in the kernel with a workgroup a segment).
+static bool chain_takes(int M, int K) { return M <= 8 ? K <= 60 * SEG : M <= 16 && K <= 32 * SEG; }
 
 // floats of workspace that a product of M rows needs (0: none)
 long work_floats(int M, int N, int K) {
-  if (M > FEW_ROWS) return 0;
+  if (M > FEW_ROWS || chain_takes(M, K)) return 0;
   const int nseg = (K + SEG - 1) / SEG;
   const long tiles = (N + BN - 1) / BN;
   if (nseg < 2 || tiles >= 384) return 0;      // the column tiles alone fill the chip
@@ -400,6 +506,35 @@ static int run(const void* A, int lda, const void* W, const float* bias, void* C
 #undef DN_MANY
     return 0;
   }
+  if (chain_takes(M, K)) {
+    const int nseg = (K + SEG - 1) / SEG;
+    // 9 to 16 rows of few columns: two workgroups of 8 rows, since 16 columns each leave most CUs without work (1,024 x 1,024 at 16 rows 6.9 us and
+    // 5.3, from K = 4,096 18.4 and 11.1; 3,072 columns 7.5 and 9.3).  5 to 8 rows of very many columns: two blocks of columns, since the rows are read again by every
+    // workgroup (50,257 x 1,024: 8 rows 55.0 and 50.5; 1 row 36.7 and 41.8).
+    const bool pair = M <= 8 || N < 2048, wide = M > 4 && M <= 8 && N >= 16384;
+    const int turns = pair ? (nseg + 1) / 2 : nseg, side = pair ? 8 : 16, cols = wide ? 2 * side : side;
+#define DN_CHAIN(WAVES, PAIR, NB)                                                                                                       \
+  hipLaunchKernelGGL((chain_kernel<TI, TC, WAVES, PAIR, NB>), dim3((N + cols - 1) / cols, (M + side - 1) / side), dim3(WAVES * 64),     \
+                     static_cast<size_t>(nseg) * NB * side * side * sizeof(float), stream, a, lda, w, bias, c, ldc, resid, ldr, M, N, K, \
+                     epi, kv)
+#define DN_CHAIN_W(PAIR, NB)   \
+  if (turns <= 4)              \
+    DN_CHAIN(4, PAIR, NB);     \
+  else if (turns <= 8)         \
+    DN_CHAIN(8, PAIR, NB);     \
+  else                         \
+    DN_CHAIN(16, PAIR, NB)
+    if (pair && wide) {
+      DN_CHAIN_W(true, 2);
+    } else if (pair) {
+      DN_CHAIN_W(true, 1);
+    } else {
+      DN_CHAIN_W(false, 1);
+    }
+#undef DN_CHAIN_W
+#undef DN_CHAIN
+    return 0;
+  }
   const long need = work_floats(M, N, K);
   if (need > 0 && (work == nullptr || have < need)) return DN_ERR_SHAPE;     // dn_gemm_work_floats says how much
   float* part = need > 0 ? work : nullptr;
@@ -422,6 +557,8 @@ static int run(const void* A, int lda, const void* W, const float* bias, void* C
 }
 
 // -- what the entry points call (one function per choice of types) ---------------------------------------
+int joins_of(int M, int N, int K) { return work_floats(M, N, K) > 0 || (chain_takes(M, K) && K > SEG); }
+
 int few_rows_take_of(int dtype, const void* A, int lda, const void* W, int M, int K) {
   return dtype == DN_F32 ? few_rows_take<float>(A, lda, W, M, K) : dtype == DN_BF16 ? few_rows_take<bf16_t>(A, lda, W, M, K) : 0;
 }

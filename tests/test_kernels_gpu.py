@@ -511,6 +511,26 @@ def test_linear_rows_do_not_depend_on_the_batch():
         assert torch.equal(sub, full[rows])
 
 
+@pytest.mark.parametrize("N,K", [(7, 4), (17, 132), (2047, 1024), (2049, 124), (16385, 260), (24, 4096), (24, 4100), (9, 7680), (9, 7684)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_plain_linear_of_up_to_16_rows_at_its_edges(N, K, dtype):
+    """Rows, columns and inner sizes on both sides of where the kernel for up to 16 rows changes its form or ends, among numbers whose products are
+    subnormal, with infinities and NaN in the last columns' weights and behind the rows: the same bits as among 100 rows."""
+    a = rnd(100, K + 8, seed=1, dtype=dtype)
+    a[:, K:] = float("nan")
+    a[3::5] *= 2.0 ** -70
+    w = rnd(N, K, seed=2, dtype=dtype)
+    w[::3] *= 2.0 ** -70
+    w[-1, -1], w[-1, 0], w[-2, 0] = float("inf"), float("-inf"), float("nan")
+    rows = a[:, :K]
+    full = ops().linear(rows, w, None, out=torch.empty(100, N, device=DEV))
+    assert (full[3, :-2].abs() < 2.0 ** -126).any() and full[:, -2].isnan().all()
+    for n in (1, 4, 5, 8, 9, 16, 17):
+        got = ops().linear(rows[3:3 + n], w, None, out=torch.empty(n, N, device=DEV))
+        assert torch.equal(got.view(torch.int32)[~full[3:3 + n].isnan()], full[3:3 + n].view(torch.int32)[~full[3:3 + n].isnan()])
+        assert torch.equal(got.isnan(), full[3:3 + n].isnan())
+
+
 @pytest.mark.parametrize("N,K", [(1600, 1600), (1600, 6400), (50257, 320), (100, 96), (333, 200), (4800, 1608)])
 def test_plain_linear_has_one_order_of_summation_whatever_the_rows(N, K):
     """The 32-bit product has two kernels (up to 64 rows, where K's segments may be workgroups of their
