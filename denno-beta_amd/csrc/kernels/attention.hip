@@ -672,6 +672,104 @@ __global__ __launch_bounds__(64) void row_tile64_kernel(
   mine[2 + lane] = a;
 }
 
+// The same for a context of up to ROW_WALK_TILES tiles, in one kernel: a workgroup is a row and a head, its waves take a tile of keys each, leave (m_T, l_T, a_T) in LDS, and the first wave joins them in ascending order, a lane per dim.  A lane brings its key's 64
+// dims straight into registers (16 bytes a load: a key's 256 bytes are two cache lines that the wave's other loads find in the vector cache), so nothing but
+// the probabilities goes through LDS.  Both kernels -> this one, 16 heads: 1 row of 50 keys 8.6 -> 4.8 us, 8 rows of 200 10.1 -> 7.6, of 500 13.7 -> 12.5, 32 rows of
+// 300 22.8 -> 20.6.  With two turns of the waves it loses where the rows are few or very many (1 row of 1,024 keys 15.7 and 19.9, 64 of 1,000 102 and 112).
+constexpr int ROW_WALK_TILES = 8;
+
+template <typename T, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void row_walk64_kernel(
+    const T* __restrict__ q, int ldq, T* __restrict__ out, int ldo, const T* __restrict__ k_pool, const T* __restrict__ v_pool,
+    const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ tile_seq,
+    const int32_t* __restrict__ tile_pos0, int n_key_tiles, int H, int Hkv, int page_size, float scale, int window, ScoreExtras ex) {
+  constexpr int DH = 64, BK = 64, QUADS = BK / 4;
+  __shared__ __attribute__((aligned(16))) float Qs[DH];
+  __shared__ __attribute__((aligned(16))) float Ps[WAVES][BK];
+  __shared__ float m_of[ROW_WALK_TILES], l_of[ROW_WALK_TILES], a_of[ROW_WALK_TILES][DH];
+  const int h = blockIdx.x, tile = blockIdx.y;
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const float qd = to_float(q[static_cast<size_t>(tile) * ldq + h * DH + lane]);
+  const int seq = tile_seq[tile];
+  if (seq < 0) return;                 // the whole workgroup
+  const int pos = tile_pos0[tile];
+  const int lo = first_key(pos, window, ex.chunk);
+  const float* bias = ex.bias ? ex.bias + static_cast<size_t>(h) * ex.span : nullptr;
+  const int hk = h / (H / Hkv);
+  const int32_t* bt = block_tables + static_cast<size_t>(seq) * max_blocks;
+  const float NEG_INF = -INFINITY;
+  if (wave == 0) Qs[lane] = qd;
+  const int ktile = wave, kt = ktile * BK, key = kt + lane;
+  const bool some = ktile < n_key_tiles && kt <= pos && !(kt + BK <= lo && kt >= ex.keep);      // the same for the whole wave
+  float kv[DH / 4][4], vv[QUADS][4];
+  int page = -1;
+  if (some) {
+    page = key <= pos ? bt[key / page_size] : -1;
+    const T* kr = k_pool + ((static_cast<size_t>(max(page, 0)) * Hkv + hk) * page_size + key % page_size) * DH;
+#pragma unroll
+    for (int i = 0; i < DH / 4; ++i) load4(kr + 4 * i, kv[i]);
+    // (four keys from a multiple of 4 lie in one page)
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) {
+      const int p = __builtin_amdgcn_readlane(page, 4 * i);
+      load4(v_pool + ((static_cast<size_t>(max(p, 0)) * Hkv + hk) * DH + lane) * page_size + (kt + 4 * i) % page_size, vv[i]);
+    }
+  }
+  __syncthreads();      // Qs is there
+  float tmax = NEG_INF;
+  if (some) {
+    // keys beyond the row's position and pages given back count as zeros, as in load_tile
+    float dot = 0.f;
+#pragma unroll
+    for (int i = 0; i < DH / 4; ++i) {
+      const float4 a = *reinterpret_cast<const float4*>(&Qs[4 * i]);
+      dot = fmaf(a.x, kv[i][0], dot);
+      dot = fmaf(a.y, kv[i][1], dot);
+      dot = fmaf(a.z, kv[i][2], dot);
+      dot = fmaf(a.w, kv[i][3], dot);
+    }
+    if (page < 0) dot = 0.f;
+    const float sc = reads_key(key, lo, pos, ex.keep) ? score_of(dot, scale, ex.cap, bias, pos - key, ex.span) : NEG_INF;
+    tmax = wave_max(sc);
+    Ps[wave][lane] = sc > NEG_INF ? expf(sc - tmax) : 0.f;
+  }
+  __syncthreads();
+  if (some) {
+    // the sum of p as 16 threads of a row make it in the kernels above
+    float psum = 0.f;
+    if (lane < 16)
+      for (int cc = 0; cc < BK / 16; ++cc) psum += Ps[wave][lane + 16 * cc];
+    psum = group_reduce<16>(psum, SumOp());
+    // a lane per dim: the tile's keys in ascending order, as dim_sum sums them
+    float a = 0.f;
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) {
+      const int p = __builtin_amdgcn_readlane(page, 4 * i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!(p >= 0 && kt + 4 * i + e <= pos)) vv[i][e] = 0.f;
+      const float4 p4 = *reinterpret_cast<const float4*>(&Ps[wave][4 * i]);
+      a = fmaf(p4.x, vv[i][0], a);
+      a = fmaf(p4.y, vv[i][1], a);
+      a = fmaf(p4.z, vv[i][2], a);
+      a = fmaf(p4.w, vv[i][3], a);
+    }
+    a_of[ktile][lane] = a;
+    if (lane == 0) l_of[ktile] = psum;
+  }
+  if (lane == 0 && ktile < n_key_tiles) m_of[ktile] = tmax;
+  __syncthreads();
+  if (wave > 0) return;
+  float m = NEG_INF, l = 0.f, acc[1] = {0.f};
+  for (int kt = 0; kt < n_key_tiles; ++kt) {
+    if (!(m_of[kt] > NEG_INF)) continue;
+    const float a_t[1] = {a_of[kt][lane]};
+    join_tile(m, l, acc, m_of[kt], l_of[kt], a_t, 1);
+  }
+  const float inv = 1.0f / (ex.sink ? l + expf(sink_score(ex, h) - m) : l);
+  out[static_cast<size_t>(tile) * ldo + h * DH + lane] = from_float<T>(acc[0] * inv);
+}
+
 template <typename T>
 __global__ void row_join_kernel(const float* __restrict__ part, T* __restrict__ out, int ldo,
                                 const int32_t* __restrict__ tile_seq, int n_key_tiles, int H, int dh, ScoreExtras ex) {
@@ -826,6 +924,22 @@ extern "C" int dn_attention_rows_extras(const void* q, int ldq, void* out, int l
   dim3 grid(n_key_tiles, H, n_tiles), block(plain::THREADS);
   const bool wave_tiles = dh == 64 && page_size % 4 == 0 && reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 &&
                           reinterpret_cast<uintptr_t>(v_pool) % 16 == 0;
+#define DN_WALK(T, WAVES)                                                                                                    \
+  hipLaunchKernelGGL((plain::row_walk64_kernel<T, WAVES>), dim3(H, n_tiles), dim3(64 * WAVES), 0, stream,                    \
+                     static_cast<const T*>(q), ldq, static_cast<T*>(out), ldo, static_cast<const T*>(k_pool),                \
+                     static_cast<const T*>(v_pool), block_tables, max_blocks, tile_seq, tile_pos0, n_key_tiles, H, Hkv,       \
+                     page_size, scale, window, ex)
+  if (wave_tiles && n_key_tiles <= plain::ROW_WALK_TILES) {
+    if (dtype == DN_F32) {
+      if (n_key_tiles <= 4) DN_WALK(float, 4); else DN_WALK(float, 8);
+    } else if (dtype == DN_BF16) {
+      if (n_key_tiles <= 4) DN_WALK(bf16_t, 4); else DN_WALK(bf16_t, 8);
+    } else {
+      return DN_ERR_DTYPE;
+    }
+    return dn_launch_status();
+  }
+#undef DN_WALK
 #define DN_ROWS(T)                                                                                                   \
   if (wave_tiles)                                                                                                    \
     hipLaunchKernelGGL(plain::row_tile64_kernel<T>, grid, dim3(64), 0, stream, static_cast<const T*>(q), ldq,        \

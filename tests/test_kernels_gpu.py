@@ -839,6 +839,21 @@ def test_attention_rows_do_not_depend_on_the_batch(dh, ps):
     assert torch.equal(two[0], win[49]) and torch.equal(two[1], win[139])
 
 
+@pytest.mark.parametrize("longest", [64, 256, 257, 511, 512, 513, 1025])
+@pytest.mark.parametrize("ps,extras", [(16, {}), (4, dict(window=100)), (64, dict(window=70, keep_first=20, sink=True)), (20, dict(chunk=96, softcap=3.0))])
+def test_single_rows_in_32_bit_are_the_same_bits_at_every_length(longest, ps, extras):
+    """Steps of single rows with heads of 64, contexts at the edges of the tiles of keys and of the lengths where the kernel changes, an absent request
+    among them: the bits of the kernel for portions."""
+    H, Hkv = 4, 2
+    lengths = [n for n in (1, 2, 63, 64, 65, 128, 255, 256, 257, 511, 513, 1000, 1024) if n < longest] + [longest]
+    q, k, v, bt, tiles, T = paged_case(lengths, [1] * len(lengths), H, Hkv, 64, ps, torch.float32, seed=longest)
+    tiles[0, 0] = -1
+    want, got = torch.zeros(T, H * 64, device=DEV), torch.zeros(T, H * 64, device=DEV)
+    ops().attention(q[:, :H * 64], want, k, v, bt, tiles, H, 0.125, **extras)
+    ops().attention(q[:, :H * 64], got, k, v, bt, tiles, H, 0.125, single_rows=True, max_context=longest, **extras)
+    assert torch.equal(got, want) and got[1:].abs().min(dim=1).values.max() > 0 and not got[0].any()
+
+
 def test_sample_greedy_and_walk():
     V = 50257
     logits = rnd(6, V, seed=3, scale=2.0)
