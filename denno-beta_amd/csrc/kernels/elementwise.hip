@@ -3,6 +3,8 @@
 // 32-bit; only what feeds a matrix product is rounded to bfloat16.
 #include "common.h"
 
+#include <type_traits>
+
 // ---------------------------------------------------------------------------------------
 // x[t,:] = wte[token_t,:] * token_scale + wpe[pos_t,:]   (crates/denno-engine/src/model/gpt2.rs:142-150,
 // where the scale is 1), as the first two entries of a list of tables that are added up.
@@ -253,12 +255,31 @@ __global__ __launch_bounds__(256) void layernorm_row_kernel(const float* __restr
       tot[i] = 0.f;
       pb[i] = pend.bias ? pend.bias[min(static_cast<int>(threadIdx.x) + i * 256, E - 1)] : 0.f;
     }
-    for (int sh = 0; sh < pend.shares; ++sh) {
-      float p[VPT];
+    // up to four shares are asked for at a time (one after the other, each was a trip to memory of its own) and added in order: 384 rows x 1,024 columns,
+    // four shares 4.3 -> 3.6 us, 320 x 1,280, two 3.9 -> 3.6
+    auto add = [&](auto batch, int sh0) {
+      constexpr int B = decltype(batch)::value;
+      float p[B][VPT];
 #pragma unroll
-      for (int i = 0; i < VPT; ++i) p[i] = pr[sh * pend.stride + min(static_cast<int>(threadIdx.x) + i * 256, E - 1)];
+      for (int u = 0; u < B; ++u)
 #pragma unroll
-      for (int i = 0; i < VPT; ++i) tot[i] += p[i];
+        for (int i = 0; i < VPT; ++i)
+          p[u][i] = pr[min(sh0 + u, pend.shares - 1) * pend.stride + min(static_cast<int>(threadIdx.x) + i * 256, E - 1)];
+#pragma unroll
+      for (int u = 0; u < B; ++u)
+        if (sh0 + u < pend.shares) {
+#pragma unroll
+          for (int i = 0; i < VPT; ++i) tot[i] += p[u][i];
+        }
+    };
+    if constexpr (VPT > 8) {      // (long rows do not leave the registers)
+      for (int sh = 0; sh < pend.shares; ++sh) add(std::integral_constant<int, 1>{}, sh);
+    } else if (pend.shares <= 2) {
+      add(std::integral_constant<int, 2>{}, 0);
+    } else if (pend.shares == 3) {
+      add(std::integral_constant<int, 3>{}, 0);
+    } else {
+      for (int sh = 0; sh < pend.shares; sh += 4) add(std::integral_constant<int, 4>{}, sh);
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
@@ -297,8 +318,13 @@ template <typename TO>
 static void launch_layernorm(const float* x, const float* gamma, const float* beta, TO* out, const int32_t* rows,
                              int R, int E, float eps, int packed, hipStream_t stream) {
   const PendingSum none{};
+  // (a row's loads are as many as its columns need: 8,192 x 1,280 15.7 -> 14.2 us with six a thread for eight, 2,048 x 1,024 5.7 -> 5.0 with four)
   if (E <= 512)
     hipLaunchKernelGGL((layernorm_row_kernel<TO, 2>), dim3(R), dim3(256), 0, stream, x, gamma, beta, out, rows, E, eps, packed, none, nullptr);
+  else if (E <= 1024)
+    hipLaunchKernelGGL((layernorm_row_kernel<TO, 4>), dim3(R), dim3(256), 0, stream, x, gamma, beta, out, rows, E, eps, packed, none, nullptr);
+  else if (E <= 1536)
+    hipLaunchKernelGGL((layernorm_row_kernel<TO, 6>), dim3(R), dim3(256), 0, stream, x, gamma, beta, out, rows, E, eps, packed, none, nullptr);
   else if (E <= 2048)
     hipLaunchKernelGGL((layernorm_row_kernel<TO, 8>), dim3(R), dim3(256), 0, stream, x, gamma, beta, out, rows, E, eps, packed, none, nullptr);
   else if (E <= 8192)
@@ -327,6 +353,10 @@ extern "C" int dn_layernorm_join(float* x, const float* part, int shares, long l
   do {                      \
     if (E <= 512)           \
       DN_LNJ(TO, 2);        \
+    else if (E <= 1024)     \
+      DN_LNJ(TO, 4);        \
+    else if (E <= 1536)     \
+      DN_LNJ(TO, 6);        \
     else if (E <= 2048)     \
       DN_LNJ(TO, 8);        \
     else                    \
