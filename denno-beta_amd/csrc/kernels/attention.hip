@@ -991,6 +991,7 @@ namespace decode {
 // that is no power of two (48, 80, 96, ...) the lanes beyond the key's last piece hold zeros.
 constexpr int lanes_per_key(int dh) { return dh <= 16 ? 2 : dh <= 32 ? 4 : dh <= 64 ? 8 : dh <= 128 ? 16 : 32; }
 
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
 // This lane's 16 bytes of a query (zeros in a lane without a piece, which add nothing to a score).
 template <int DH>
 __device__ __forceinline__ bf16x8 query_piece(const bf16_t* q) {
@@ -1008,10 +1009,10 @@ struct RowSums {
 };
 
 // One row and head, its keys shared out among the workgroup's waves 64 at a time: the whole of a workgroup of the kernel for steps of single rows, and of
-// the kernel for portions where a tile is one row.  qv: query_piece of the row's query; bt: its request's block table; mypart: where a split leaves its result (n_splits > 1).
-template <int DH, int WAVES, bool POW2, bool EXTRAS>
+// the kernel for portions where a tile is one row.  qv: query_piece of the row's query; bt: its request's block table; part: where splits leave their results (n_splits > 1).
+template <int DH, int WAVES, bool POW2, bool EXTRAS, bool EARLY = false>
 __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const int32_t* bt, bf16_t* __restrict__ out, int ldo,
-                                        const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, float* mypart, int split, int n_splits,
+                                        const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, float* part, int split, int n_splits,
                                         int chunks, int h, int H, int Hkv, int page_size, int page_shift, float scale, int window,
                                         const ScoreExtras& ex, RowSums<DH, WAVES>& sums) {
   static_assert(DH % 16 == 0 && DH >= 16 && DH <= 256, "head size");
@@ -1025,6 +1026,7 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);   // (a scalar)
   const int sub = lane % LPK, grp = lane / LPK;
   const bool holds = PIECES == LPK || sub < PIECES;     // (a lane without a piece: zeros, which add nothing to a score)
+  float* mypart = part + ((static_cast<size_t>(row) * H + h) * n_splits + split) * (DH + 2);
   const int lo = first_key(pos, window, EXTRAS ? ex.chunk : 0);
   const float* bias = EXTRAS && ex.bias ? ex.bias + static_cast<size_t>(h) * ex.span : nullptr;
   const int keep = EXTRAS ? ex.keep : 0;
@@ -1042,9 +1044,7 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
     return;
   }
   const int hk = h / (H / Hkv);
-  float qr[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) qr[i] = static_cast<float>(qv[i]) * scale;
+  const u32x4 q4 = __builtin_bit_cast(u32x4, qv);
   float m_run = NEG_INF, l_run = 0.f;
   float acc[DPL];
 #pragma unroll
@@ -1054,18 +1054,32 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
     const int tile_no = first_tile + c * WAVES + wave;
     if (tile_no >= n_tiles_read) continue;     // the same for the whole wave; no barrier in this loop
     const int kbase = 64 * (tile_no < kept_tiles ? tile_no : rest + (tile_no - kept_tiles));
-    // values: lane = dim; 16 keys of one page at a time.  They are asked for first, before the keys
-    // (whose use would otherwise stand between them and memory): keys and values then make one trip
-    bf16x8 v0[4][DPL], v1[4][DPL];
+    // The pages of the tile's four runs of 16 keys, by the scalar unit and all at once: the keys and the values of a run lie in one page, so nothing else has to be looked
+    // up.  (Looked up one by one in front of each run's values, and again by every lane for its keys, they were five trips to memory in a row.)  A run that
+    // the row does not read is replaced by the last one that it does.
+    const int last_run = (pos / 16) * 16, last_page = bt[page_index(last_run)];
+    int at[4], page[4];
     bool live[4];
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) {
       const int kb = kbase + blk * 16;
       live[blk] = kb <= pos && (kb + 16 > lo || kb < keep);
-      const int kk = live[blk] ? kb : (pos / 16) * 16;
-      const int page = bt[page_index(kk)];
-      live[blk] = live[blk] && page >= 0;
-      const bf16_t* vb = v_pool + (static_cast<size_t>(max(page, 0)) * Hkv + hk) * DH * page_size + page_offset(kk);
+      at[blk] = live[blk] ? kb : last_run;
+      page[blk] = bt[page_index(at[blk])];
+    }
+    asm volatile("" ::"s"(last_page), "s"(page[0]), "s"(page[1]), "s"(page[2]), "s"(page[3]));
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      live[blk] = live[blk] && page[blk] >= 0;
+      at[blk] = page_offset(page[blk] >= 0 ? at[blk] : last_run);
+      page[blk] = page[blk] >= 0 ? page[blk] : last_page;
+    }
+    // values: lane = dim; 16 keys of one page at a time.  They are asked for first, before the keys
+    // (whose use would otherwise stand between them and memory): keys and values then make one trip
+    bf16x8 v0[4][DPL], v1[4][DPL];
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      const bf16_t* vb = v_pool + (static_cast<size_t>(page[blk]) * Hkv + hk) * DH * page_size + at[blk];
 #pragma unroll
       for (int i = 0; i < DPL; ++i) {
         const int d = min(lane + 64 * i, DH - 1);
@@ -1075,19 +1089,27 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
     }
     // scores: lane (key group grp, part sub of the key); after the sum over the key's lanes every
     // lane of group grp holds, in sc[it], the score of key kbase + it * KPI + grp
-    float sc[LPK];
+    float sc[LPK], qr[8];
 #pragma unroll
     for (int it0 = 0; it0 < LPK; it0 += GROUP) {
       bf16x8 kv[GROUP];
 #pragma unroll
       for (int u = 0; u < GROUP; ++u) {
-        const int key = kbase + (it0 + u) * KPI + grp;
-        const int kk = reads_key(key, lo, pos, keep) ? key : pos;     // a key that surely has a page
-        const int page = bt[page_index(kk)];
+        // (a load's keys are of one run, or, 32 keys a load, of two: a key that the row does not read comes from a run that is there, and is masked)
+        constexpr int RUNS = KPI / 16;
+        const int it = it0 + u, b0 = it * KPI / 16, key16 = (it * KPI + grp) % 16;
+        const int pg = RUNS > 1 && grp >= 16 ? page[b0 + (RUNS > 1)] : page[b0], off = (RUNS > 1 && grp >= 16 ? at[b0 + (RUNS > 1)] : at[b0]) + key16;
         kv[u] = bf16x8{};
         if (holds)
           kv[u] = *reinterpret_cast<const bf16x8*>(
-              k_pool + ((static_cast<size_t>(page) * Hkv + hk) * page_size + page_offset(kk)) * DH + sub * 8);
+              k_pool + ((static_cast<size_t>(pg) * Hkv + hk) * page_size + off) * DH + sub * 8);
+      }
+      // (the query is waited for behind the keys' loads: scaled in front of the loop it was a trip to memory in front of the page table's)
+      if (it0 == 0) {
+        u32x4 here = q4;
+        asm volatile("" : "+v"(here));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) qr[i] = to_float(bf16_t{static_cast<uint16_t>(here[i / 2] >> (i % 2 * 16))}) * scale;
       }
 #pragma unroll
       for (int u = 0; u < GROUP; ++u) {
@@ -1105,7 +1127,9 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
 #pragma unroll
     for (int it = 0; it < LPK; ++it) m_c = fmaxf(m_c, sc[it]);
     m_c = wave_max(m_c);
-    if (!(m_c > NEG_INF)) continue;
+    // EARLY: no branch from here on, nor for runs that the row does not read, whose probabilities are 0: behind a branch the compiler asks for the values only
+    // when the scores are made, a second trip to memory (in half the registers, which is better where many workgroups share a CU)
+    if (!EARLY && !(m_c > NEG_INF)) continue;
     const float m_new = fmaxf(m_run, m_c);
     const float alpha = m_run > NEG_INF ? __expf(m_run - m_new) : 0.f;
     float p[LPK];
@@ -1122,7 +1146,7 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
     for (int i = 0; i < DPL; ++i) acc[i] *= alpha;
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) {
-      if (!live[blk]) continue;
+      if (!EARLY && !live[blk]) continue;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int key = blk * 16 + j;      // key = it * KPI + grp: held by lane grp * LPK in p[it]
@@ -1623,7 +1647,7 @@ extern "C" int dn_attention_flash_extras(const void* q, int ldq, void* out, int 
 // exchanges inside the loop.
 // ---------------------------------------------------------------------------------------
 namespace decode {
-template <int DH, int WAVES, bool POW2, bool EXTRAS = false>   // head size (a multiple of 16 up to 256); waves per workgroup; ScoreExtras
+template <int DH, int WAVES, bool POW2, bool EXTRAS = false, bool EARLY = false>   // head size (a multiple of 16 up to 256); waves per workgroup; ScoreExtras; see one_row
 __global__ __launch_bounds__(WAVES * 64) void partial_kernel(const bf16_t* __restrict__ q, int ldq, bf16_t* __restrict__ out,
                                                        int ldo, const bf16_t* __restrict__ k_pool,
                                                        const bf16_t* __restrict__ v_pool,
@@ -1639,10 +1663,13 @@ __global__ __launch_bounds__(WAVES * 64) void partial_kernel(const bf16_t* __res
   // are addressed by the workgroup's index, so their loads do not wait for the tile table's.
   const int split = blockIdx.x, h = blockIdx.y, tile = blockIdx.z;
   const bf16x8 qv = query_piece<DH>(q + static_cast<size_t>(tile) * ldq + h * DH);
-  if (tile_seq[tile] < 0) return;
-  one_row<DH, WAVES, POW2, EXTRAS>(qv, tile, tile_pos0[tile], block_tables + static_cast<size_t>(tile) * max_blocks, out, ldo, k_pool, v_pool,
-                                   part + ((static_cast<size_t>(tile) * H + h) * n_splits + split) * (DH + 2), split, n_splits, chunks, h, H, Hkv,
-                                   page_size, page_shift, scale, window, ex, sums);
+  // Request, position and every argument are asked for together: left to itself the compiler waits for the request, then for the arguments that the
+  // rest needs, then for the position, three trips in front of the page table's.
+  const int seq = tile_seq[tile], pos = tile_pos0[tile];
+  asm volatile("" ::"s"(seq), "s"(pos), "s"(k_pool), "s"(v_pool), "s"(page_size), "s"(window));
+  if (seq < 0) return;
+  one_row<DH, WAVES, POW2, EXTRAS, EARLY>(qv, tile, pos, block_tables + static_cast<size_t>(tile) * max_blocks, out, ldo, k_pool, v_pool, part, split, n_splits,
+                                   chunks, h, H, Hkv, page_size, page_shift, scale, window, ex, sums);
 }
 
 __global__ void join_kernel(const float* __restrict__ part, bf16_t* __restrict__ out, int ldo,
@@ -1706,6 +1733,10 @@ extern "C" int dn_attention_decode_extras(const void* q, int ldq, void* out, int
   while ((1 << page_shift) < page_size) ++page_shift;
   const bool pow2 = (1 << page_shift) == page_size;
   if (extras && !pow2) return DN_ERR_SHAPE;
+  // (with pages looked up together and the query waited for last, every other size gained too: 203 rows of 40 keys 10.9 -> 9.9, 8 rows of 1,000, 25 heads 11.2 -> 11.0)
+  // Short contexts and a workgroup a CU at most: nothing else hides a trip to memory (1 row of 50 keys, 16 heads 4.0 -> 3.7 us, 16 rows of 200 4.4 -> 4.2; 203
+  // rows of 40, 20 heads 9.9 and 13.3, so not there; with eight and sixteen waves level or slower by 2 %)
+  const bool early = waves == 4 && pow2 && !extras && dh <= 128 && static_cast<long>(n_splits) * H * n_tiles <= 256;
 #define DN_DECODE_P(L, W, P, X)                                                                                       \
   hipLaunchKernelGGL((decode::partial_kernel<L, W, P, X>), grid, block, 0, stream, static_cast<const bf16_t*>(q), ldq, \
                      static_cast<bf16_t*>(out), ldo, static_cast<const bf16_t*>(k_pool),                              \
@@ -1721,6 +1752,11 @@ extern "C" int dn_attention_decode_extras(const void* q, int ldq, void* out, int
       DN_DECODE_P(L, W, false, false); \
   } while (0)
 #define DN_DECODE(D)                  \
+  if (early) {                        \
+    hipLaunchKernelGGL((decode::partial_kernel<D, 4, true, false, true>), grid, block, 0, stream, static_cast<const bf16_t*>(q), ldq, \
+                       static_cast<bf16_t*>(out), ldo, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), block_tables, \
+                       max_blocks, tile_seq, tile_row0, tile_pos0, part, n_splits, chunks, H, Hkv, page_size, page_shift, scale, window, ex); \
+  } else                              \
   if (waves == 16) {                  \
     if constexpr (D <= 64) DN_DECODE_W(D, 16); \
   } else if (waves == 8) {            \

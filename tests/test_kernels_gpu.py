@@ -839,6 +839,23 @@ def test_attention_rows_do_not_depend_on_the_batch(dh, ps):
     assert torch.equal(two[0], win[49]) and torch.equal(two[1], win[139])
 
 
+@pytest.mark.parametrize("dh,ps", [(64, 16), (16, 32), (128, 64), (80, 16), (32, 48)])
+def test_a_single_row_is_the_same_bits_alone_and_among_many(dh, ps):
+    """Steps of single rows with contexts of up to 256 keys, where few workgroups ask for their values before the scores are made and many do not."""
+    H, Hkv = 4, 2
+    lengths = [1, 15, 16, 17, 48, 63, 64, 65, 80, 129, 200, 255, 256] * 6
+    q, k, v, bt, tiles, T = paged_case(lengths, [1] * len(lengths), H, Hkv, dh, ps, torch.bfloat16, seed=dh)
+    many = torch.zeros(T, H * dh, dtype=torch.bfloat16, device=DEV)
+    ops().attention(q[:, :H * dh], many, k, v, bt, tiles, H, dh ** -0.5, single_rows=True, max_context=256)
+    want = R.attention(q[:, :H * dh], torch.zeros(T, H * dh, device=DEV), k, v, bt, tiles, H, dh ** -0.5, 0)
+    assert torch.allclose(many.float(), want, **TOL[torch.bfloat16])
+    for r in range(13):
+        one = torch.zeros(1, H * dh, dtype=torch.bfloat16, device=DEV)
+        ops().attention(q[r:r + 1, :H * dh], one, k, v, bt[r:r + 1].contiguous(), i32([[0], [0], [1], [lengths[r] - 1]]), H, dh ** -0.5, single_rows=True,
+                        max_context=256)
+        assert torch.equal(one[0], many[r]), lengths[r]
+
+
 @pytest.mark.parametrize("longest", [64, 256, 257, 511, 512, 513, 1025])
 @pytest.mark.parametrize("ps,extras", [(16, {}), (4, dict(window=100)), (64, dict(window=70, keep_first=20, sink=True)), (20, dict(chunk=96, softcap=3.0))])
 def test_single_rows_in_32_bit_are_the_same_bits_at_every_length(longest, ps, extras):
