@@ -983,217 +983,6 @@ __device__ __forceinline__ bf16x8 to_bf16x8(const float* v) {
   return __builtin_bit_cast(bf16x8, w);
 }
 
-namespace decode {
-// POW2: page_size = 1 << page_shift; a key's page and its place in the page are then a shift and a mask (a lane
-// works out a dozen such pairs per 64 keys before it can ask for the keys and values: as divisions by a number
-// known only at run time they were some six hundred instructions in front of the loads)
-// A key's 16-byte pieces lie on LPK lanes side by side, LPK the power of two that holds them: with a head size
-// that is no power of two (48, 80, 96, ...) the lanes beyond the key's last piece hold zeros.
-constexpr int lanes_per_key(int dh) { return dh <= 16 ? 2 : dh <= 32 ? 4 : dh <= 64 ? 8 : dh <= 128 ? 16 : 32; }
-
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
-// This lane's 16 bytes of a query (zeros in a lane without a piece, which add nothing to a score).
-template <int DH>
-__device__ __forceinline__ bf16x8 query_piece(const bf16_t* q) {
-  constexpr int LPK = lanes_per_key(DH), PIECES = DH / 8;
-  const int sub = threadIdx.x % 64 % LPK;
-  bf16x8 qv = {};
-  if (PIECES == LPK || sub < PIECES) qv = *reinterpret_cast<const bf16x8*>(q + sub * 8);
-  return qv;
-}
-
-// the waves' maxima, sums and weighted values, in LDS
-template <int DH, int WAVES>
-struct RowSums {
-  float m[WAVES], l[WAVES], acc[WAVES][DH];
-};
-
-// One row and head, its keys shared out among the workgroup's waves 64 at a time: the whole of a workgroup of the kernel for steps of single rows, and of
-// the kernel for portions where a tile is one row.  qv: query_piece of the row's query; bt: its request's block table; part: where splits leave their results (n_splits > 1).
-template <int DH, int WAVES, bool POW2, bool EXTRAS, bool EARLY = false>
-__device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const int32_t* bt, bf16_t* __restrict__ out, int ldo,
-                                        const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, float* part, int split, int n_splits,
-                                        int chunks, int h, int H, int Hkv, int page_size, int page_shift, float scale, int window,
-                                        const ScoreExtras& ex, RowSums<DH, WAVES>& sums) {
-  static_assert(DH % 16 == 0 && DH >= 16 && DH <= 256, "head size");
-  constexpr int LPK = lanes_per_key(DH);
-  constexpr int PIECES = DH / 8;         // 16-byte pieces of a key: the lanes sub < PIECES of its LPK
-  auto page_index = [&](int key) { return POW2 ? key >> page_shift : key / page_size; };
-  auto page_offset = [&](int key) { return POW2 ? key & (page_size - 1) : key % page_size; };
-  constexpr int KPI = 64 / LPK;          // keys per load instruction
-  constexpr int DPL = (DH + 63) / 64;    // dims per lane in the second product
-  constexpr int GROUP = LPK < 8 ? LPK : 8;   // load instructions issued together
-  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);   // (a scalar)
-  const int sub = lane % LPK, grp = lane / LPK;
-  const bool holds = PIECES == LPK || sub < PIECES;     // (a lane without a piece: zeros, which add nothing to a score)
-  float* mypart = part + ((static_cast<size_t>(row) * H + h) * n_splits + split) * (DH + 2);
-  const int lo = first_key(pos, window, EXTRAS ? ex.chunk : 0);
-  const float* bias = EXTRAS && ex.bias ? ex.bias + static_cast<size_t>(h) * ex.span : nullptr;
-  const int keep = EXTRAS ? ex.keep : 0;
-  const float to_tanh = EXTRAS && ex.cap > 0.f ? 2.0f * 1.44269504088896340736f / ex.cap : 0.f;
-  // the tiles of 64 keys that the row reads, counted from 0: those of the kept first keys, then those from `lo` on
-  const int kept_tiles = (keep + 63) / 64, rest = max(lo / 64, kept_tiles), last_tile = pos / 64;
-  const int n_tiles_read = kept_tiles > last_tile ? last_tile + 1 : kept_tiles + (last_tile - rest + 1);
-  const int first_tile = split * chunks * WAVES;
-  const float NEG_INF = -INFINITY;
-  if (first_tile >= n_tiles_read) {
-    if (n_splits > 1 && threadIdx.x == 0) {
-      mypart[0] = NEG_INF;     // the join skips it
-      mypart[1] = 0.f;
-    }
-    return;
-  }
-  const int hk = h / (H / Hkv);
-  const u32x4 q4 = __builtin_bit_cast(u32x4, qv);
-  float m_run = NEG_INF, l_run = 0.f;
-  float acc[DPL];
-#pragma unroll
-  for (int i = 0; i < DPL; ++i) acc[i] = 0.f;
-
-  for (int c = 0; c < chunks; ++c) {
-    const int tile_no = first_tile + c * WAVES + wave;
-    if (tile_no >= n_tiles_read) continue;     // the same for the whole wave; no barrier in this loop
-    const int kbase = 64 * (tile_no < kept_tiles ? tile_no : rest + (tile_no - kept_tiles));
-    // The pages of the tile's four runs of 16 keys, by the scalar unit and all at once: the keys and the values of a run lie in one page, so nothing else has to be looked
-    // up.  (Looked up one by one in front of each run's values, and again by every lane for its keys, they were five trips to memory in a row.)  A run that
-    // the row does not read is replaced by the last one that it does.
-    const int last_run = (pos / 16) * 16, last_page = bt[page_index(last_run)];
-    int at[4], page[4];
-    bool live[4];
-#pragma unroll
-    for (int blk = 0; blk < 4; ++blk) {
-      const int kb = kbase + blk * 16;
-      live[blk] = kb <= pos && (kb + 16 > lo || kb < keep);
-      at[blk] = live[blk] ? kb : last_run;
-      page[blk] = bt[page_index(at[blk])];
-    }
-    asm volatile("" ::"s"(last_page), "s"(page[0]), "s"(page[1]), "s"(page[2]), "s"(page[3]));
-#pragma unroll
-    for (int blk = 0; blk < 4; ++blk) {
-      live[blk] = live[blk] && page[blk] >= 0;
-      at[blk] = page_offset(page[blk] >= 0 ? at[blk] : last_run);
-      page[blk] = page[blk] >= 0 ? page[blk] : last_page;
-    }
-    // values: lane = dim; 16 keys of one page at a time.  They are asked for first, before the keys
-    // (whose use would otherwise stand between them and memory): keys and values then make one trip
-    bf16x8 v0[4][DPL], v1[4][DPL];
-#pragma unroll
-    for (int blk = 0; blk < 4; ++blk) {
-      const bf16_t* vb = v_pool + (static_cast<size_t>(page[blk]) * Hkv + hk) * DH * page_size + at[blk];
-#pragma unroll
-      for (int i = 0; i < DPL; ++i) {
-        const int d = min(lane + 64 * i, DH - 1);
-        v0[blk][i] = *reinterpret_cast<const bf16x8*>(vb + static_cast<size_t>(d) * page_size);
-        v1[blk][i] = *reinterpret_cast<const bf16x8*>(vb + static_cast<size_t>(d) * page_size + 8);
-      }
-    }
-    // scores: lane (key group grp, part sub of the key); after the sum over the key's lanes every
-    // lane of group grp holds, in sc[it], the score of key kbase + it * KPI + grp
-    float sc[LPK], qr[8];
-#pragma unroll
-    for (int it0 = 0; it0 < LPK; it0 += GROUP) {
-      bf16x8 kv[GROUP];
-#pragma unroll
-      for (int u = 0; u < GROUP; ++u) {
-        // (a load's keys are of one run, or, 32 keys a load, of two: a key that the row does not read comes from a run that is there, and is masked)
-        constexpr int RUNS = KPI / 16;
-        const int it = it0 + u, b0 = it * KPI / 16, key16 = (it * KPI + grp) % 16;
-        const int pg = RUNS > 1 && grp >= 16 ? page[b0 + (RUNS > 1)] : page[b0], off = (RUNS > 1 && grp >= 16 ? at[b0 + (RUNS > 1)] : at[b0]) + key16;
-        kv[u] = bf16x8{};
-        if (holds)
-          kv[u] = *reinterpret_cast<const bf16x8*>(
-              k_pool + ((static_cast<size_t>(pg) * Hkv + hk) * page_size + off) * DH + sub * 8);
-      }
-      // (the query is waited for behind the keys' loads: scaled in front of the loop it was a trip to memory in front of the page table's)
-      if (it0 == 0) {
-        u32x4 here = q4;
-        asm volatile("" : "+v"(here));
-#pragma unroll
-        for (int i = 0; i < 8; ++i) qr[i] = to_float(bf16_t{static_cast<uint16_t>(here[i / 2] >> (i % 2 * 16))}) * scale;
-      }
-#pragma unroll
-      for (int u = 0; u < GROUP; ++u) {
-        const int key = kbase + (it0 + u) * KPI + grp;
-        float dot = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) dot = fmaf(qr[i], static_cast<float>(kv[u][i]), dot);
-        dot = group_reduce<LPK>(dot, SumOp());
-        if (EXTRAS && ex.cap > 0.f) dot = ex.cap * tanh_of_exp2(dot * to_tanh);
-        if (EXTRAS && bias) dot += bias[min(max(pos - key, 0), ex.span - 1)];
-        sc[it0 + u] = reads_key(key, lo, pos, keep) ? dot : NEG_INF;
-      }
-    }
-    float m_c = NEG_INF;
-#pragma unroll
-    for (int it = 0; it < LPK; ++it) m_c = fmaxf(m_c, sc[it]);
-    m_c = wave_max(m_c);
-    // EARLY: no branch from here on, nor for runs that the row does not read, whose probabilities are 0: behind a branch the compiler asks for the values only
-    // when the scores are made, a second trip to memory (in half the registers, which is better where many workgroups share a CU)
-    if (!EARLY && !(m_c > NEG_INF)) continue;
-    const float m_new = fmaxf(m_run, m_c);
-    const float alpha = m_run > NEG_INF ? __expf(m_run - m_new) : 0.f;
-    float p[LPK];
-    float psum = 0.f;
-#pragma unroll
-    for (int it = 0; it < LPK; ++it) {
-      p[it] = sc[it] > NEG_INF ? __expf(sc[it] - m_new) : 0.f;
-      psum += p[it];
-    }
-    // each key is held by LPK lanes: its first lane counts it
-    l_run = l_run * alpha + wave_sum(sub == 0 ? psum : 0.f);
-    m_run = m_new;
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) acc[i] *= alpha;
-#pragma unroll
-    for (int blk = 0; blk < 4; ++blk) {
-      if (!EARLY && !live[blk]) continue;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int key = blk * 16 + j;      // key = it * KPI + grp: held by lane grp * LPK in p[it]
-        const float pj = lane_value(p[key / KPI], (key % KPI) * LPK);
-#pragma unroll
-        for (int i = 0; i < DPL; ++i)
-          acc[i] = fmaf(pj, static_cast<float>(j < 8 ? v0[blk][i][j] : v1[blk][i][j - 8]), acc[i]);
-      }
-    }
-  }
-  if (lane == 0) {
-    sums.m[wave] = m_run;
-    sums.l[wave] = l_run;
-  }
-#pragma unroll
-  for (int i = 0; i < DPL; ++i)
-    if (lane + 64 * i < DH) sums.acc[wave][lane + 64 * i] = acc[i];
-  __syncthreads();
-  for (int d = threadIdx.x; d < DH; d += WAVES * 64) {
-    float M = sums.m[0];
-#pragma unroll
-    for (int w = 1; w < WAVES; ++w) M = fmaxf(M, sums.m[w]);
-    float L = 0.f, A = 0.f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      if (sums.m[w] > NEG_INF) {
-        float f = __expf(sums.m[w] - M);
-        L += sums.l[w] * f;
-        A += sums.acc[w][d] * f;
-      }
-    }
-    if (n_splits == 1) {
-      if (EXTRAS && ex.sink) L += __expf(sink_score(ex, h) - M);      // (a key without a value)
-      out[ldo > 0 ? static_cast<size_t>(row) * ldo + h * DH + d : packed_index(row, h * DH + d, H * DH / 32)] =
-          from_float<bf16_t>(A / L);
-    } else {
-      mypart[2 + d] = A;
-      if (d == 0) {
-        mypart[0] = M;
-        mypart[1] = L;
-      }
-    }
-  }
-}
-
-}  // namespace decode
-
 // ---------------------------------------------------------------------------------------
 // flash: portions of prompts.  A workgroup takes up to 128 consecutive rows of one request
 // and one head.  It has GROUPS x 4 waves: wave w owns the 32 rows 32 (w % 4), and the groups
@@ -1255,19 +1044,6 @@ __global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(DH
   const int seq = tile_seq[tile];
   if (seq < 0) return;                       // the whole workgroup
   const int row0 = tile_row0[tile], nrows = tile_nrows[tile], pos0 = tile_pos0[tile];
-  if (nrows == 1) {
-    // A tile of one row (a decoded token beside portions): in the walk below two waves of the workgroup would have a row to work for, 32 keys each a step,
-    // and the longest context among such rows would be the whole step's time.  All waves take 64 keys each at a time instead, as in a step of single rows.
-    // One row behind 1,000 keys, 20 heads of 64: 21.3 -> 7.6 us; 20 rows of up to 784 keys beside portions of 192 and 108: 19.7 -> 15.6 (now the
-    // portions' own walk); 200 rows of 300 keys beside a portion of 64: 79.4 -> 56.6; 10 heads of 128 31.9 -> 26.2.
-    using Sums = decode::RowSums<DH, 4 * GROUPS>;
-    static_assert(sizeof(Sums) <= sizeof(smem), "one row's sums lie where the tiles would");
-    decode::one_row<DH, 4 * GROUPS, POW2, EXTRAS>(decode::query_piece<DH>(q + static_cast<size_t>(row0) * ldq + h * DH), row0, pos0,
-                                                  block_tables + static_cast<size_t>(seq) * max_blocks, out, ldo, k_pool, v_pool, nullptr, 0, 1,
-                                                  (pos0 / 64 + 4 * GROUPS) / (4 * GROUPS), h, H, Hkv, page_size, page_shift, scale, window, ex,
-                                                  *reinterpret_cast<Sums*>(smem));
-    return;
-  }
   // (the wave's number through readfirstlane: what follows from it, the wave's rows and keys, which tiles it
   // carries and whether a tile touches an edge, is then worked out once per wave by the scalar unit, and its
   // page numbers come by scalar loads)
@@ -1647,7 +1423,16 @@ extern "C" int dn_attention_flash_extras(const void* q, int ldq, void* out, int 
 // exchanges inside the loop.
 // ---------------------------------------------------------------------------------------
 namespace decode {
-template <int DH, int WAVES, bool POW2, bool EXTRAS = false, bool EARLY = false>   // head size (a multiple of 16 up to 256); waves per workgroup; ScoreExtras; see one_row
+// POW2: page_size = 1 << page_shift; a key's page and its place in the page are then a shift and a mask (a lane
+// works out a dozen such pairs per 64 keys before it can ask for the keys and values: as divisions by a number
+// known only at run time they were some six hundred instructions in front of the loads)
+// A key's 16-byte pieces lie on LPK lanes side by side, LPK the power of two that holds them: with a head size
+// that is no power of two (48, 80, 96, ...) the lanes beyond the key's last piece hold zeros.
+constexpr int lanes_per_key(int dh) { return dh <= 16 ? 2 : dh <= 32 ? 4 : dh <= 64 ? 8 : dh <= 128 ? 16 : 32; }
+
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+
+template <int DH, int WAVES, bool POW2, bool EXTRAS = false, bool EARLY = false>   // head size (a multiple of 16 up to 256); waves per workgroup; ScoreExtras; see EARLY below
 __global__ __launch_bounds__(WAVES * 64) void partial_kernel(const bf16_t* __restrict__ q, int ldq, bf16_t* __restrict__ out,
                                                        int ldo, const bf16_t* __restrict__ k_pool,
                                                        const bf16_t* __restrict__ v_pool,
@@ -1658,18 +1443,195 @@ __global__ __launch_bounds__(WAVES * 64) void partial_kernel(const bf16_t* __res
                                                        float* __restrict__ part, int n_splits, int chunks, int H,
                                                        int Hkv, int page_size, int page_shift, float scale,
                                                        int window, ScoreExtras ex) {
-  __shared__ RowSums<DH, WAVES> sums;
+  static_assert(DH % 16 == 0 && DH >= 16 && DH <= 256, "head size");
+  constexpr int LPK = lanes_per_key(DH);
+  constexpr int PIECES = DH / 8;         // 16-byte pieces of a key: the lanes sub < PIECES of its LPK
+  auto page_index = [&](int key) { return POW2 ? key >> page_shift : key / page_size; };
+  auto page_offset = [&](int key) { return POW2 ? key & (page_size - 1) : key % page_size; };
+  constexpr int KPI = 64 / LPK;          // keys per load instruction
+  constexpr int DPL = (DH + 63) / 64;    // dims per lane in the second product
+  constexpr int GROUP = LPK < 8 ? LPK : 8;   // load instructions issued together
+  __shared__ float wm[WAVES], wl[WAVES];
+  __shared__ float wacc[WAVES][DH];
   // In a step of single rows request s brings row s and is tile s: the block table and the query
   // are addressed by the workgroup's index, so their loads do not wait for the tile table's.
   const int split = blockIdx.x, h = blockIdx.y, tile = blockIdx.z;
-  const bf16x8 qv = query_piece<DH>(q + static_cast<size_t>(tile) * ldq + h * DH);
-  // Request, position and every argument are asked for together: left to itself the compiler waits for the request, then for the arguments that the
-  // rest needs, then for the position, three trips in front of the page table's.
+  const int row = tile;
+  const int32_t* bt = block_tables + static_cast<size_t>(tile) * max_blocks;
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);   // (a scalar)
+  const int sub = lane % LPK, grp = lane / LPK;
+  const bool holds = PIECES == LPK || sub < PIECES;     // (a lane without a piece: zeros, which add nothing to a score)
+  bf16x8 qv = {};
+  if (holds) qv = *reinterpret_cast<const bf16x8*>(q + static_cast<size_t>(row) * ldq + h * DH + sub * 8);
+  // Request, position and every argument are asked for together: left to itself the compiler waits for the request, then
+  // for the arguments that the rest needs, then for the position, three trips in front of the page table's.
   const int seq = tile_seq[tile], pos = tile_pos0[tile];
   asm volatile("" ::"s"(seq), "s"(pos), "s"(k_pool), "s"(v_pool), "s"(page_size), "s"(window));
   if (seq < 0) return;
-  one_row<DH, WAVES, POW2, EXTRAS, EARLY>(qv, tile, pos, block_tables + static_cast<size_t>(tile) * max_blocks, out, ldo, k_pool, v_pool, part, split, n_splits,
-                                   chunks, h, H, Hkv, page_size, page_shift, scale, window, ex, sums);
+  float* mypart = part + ((static_cast<size_t>(tile) * H + h) * n_splits + split) * (DH + 2);
+  const int lo = first_key(pos, window, EXTRAS ? ex.chunk : 0);
+  const float* bias = EXTRAS && ex.bias ? ex.bias + static_cast<size_t>(h) * ex.span : nullptr;
+  const int keep = EXTRAS ? ex.keep : 0;
+  const float to_tanh = EXTRAS && ex.cap > 0.f ? 2.0f * 1.44269504088896340736f / ex.cap : 0.f;
+  // the tiles of 64 keys that the row reads, counted from 0: those of the kept first keys, then those from `lo` on
+  const int kept_tiles = (keep + 63) / 64, rest = max(lo / 64, kept_tiles), last_tile = pos / 64;
+  const int n_tiles_read = kept_tiles > last_tile ? last_tile + 1 : kept_tiles + (last_tile - rest + 1);
+  const int first_tile = split * chunks * WAVES;
+  const float NEG_INF = -INFINITY;
+  if (first_tile >= n_tiles_read) {
+    if (n_splits > 1 && threadIdx.x == 0) {
+      mypart[0] = NEG_INF;     // the join skips it
+      mypart[1] = 0.f;
+    }
+    return;
+  }
+  const int hk = h / (H / Hkv);
+  const u32x4 q4 = __builtin_bit_cast(u32x4, qv);
+  float m_run = NEG_INF, l_run = 0.f;
+  float acc[DPL];
+#pragma unroll
+  for (int i = 0; i < DPL; ++i) acc[i] = 0.f;
+
+  for (int c = 0; c < chunks; ++c) {
+    const int tile_no = first_tile + c * WAVES + wave;
+    if (tile_no >= n_tiles_read) continue;     // the same for the whole wave; no barrier in this loop
+    const int kbase = 64 * (tile_no < kept_tiles ? tile_no : rest + (tile_no - kept_tiles));
+    // The pages of the tile's four runs of 16 keys, by the scalar unit and all at once: the keys and the values of a run lie in one page, so nothing else has to be looked
+    // up.  (Looked up one by one in front of each run's values, and again by every lane for its keys, they were five trips to memory in a row.)  A run that
+    // the row does not read is replaced by the last one that it does.
+    const int last_run = (pos / 16) * 16, last_page = bt[page_index(last_run)];
+    int at[4], page[4];
+    bool live[4];
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      const int kb = kbase + blk * 16;
+      live[blk] = kb <= pos && (kb + 16 > lo || kb < keep);
+      at[blk] = live[blk] ? kb : last_run;
+      page[blk] = bt[page_index(at[blk])];
+    }
+    asm volatile("" ::"s"(last_page), "s"(page[0]), "s"(page[1]), "s"(page[2]), "s"(page[3]));
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      live[blk] = live[blk] && page[blk] >= 0;
+      at[blk] = page_offset(page[blk] >= 0 ? at[blk] : last_run);
+      page[blk] = page[blk] >= 0 ? page[blk] : last_page;
+    }
+    // values: lane = dim; 16 keys of one page at a time.  They are asked for first, before the keys
+    // (whose use would otherwise stand between them and memory): keys and values then make one trip
+    bf16x8 v0[4][DPL], v1[4][DPL];
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      const bf16_t* vb = v_pool + (static_cast<size_t>(page[blk]) * Hkv + hk) * DH * page_size + at[blk];
+#pragma unroll
+      for (int i = 0; i < DPL; ++i) {
+        const int d = min(lane + 64 * i, DH - 1);
+        v0[blk][i] = *reinterpret_cast<const bf16x8*>(vb + static_cast<size_t>(d) * page_size);
+        v1[blk][i] = *reinterpret_cast<const bf16x8*>(vb + static_cast<size_t>(d) * page_size + 8);
+      }
+    }
+    // scores: lane (key group grp, part sub of the key); after the sum over the key's lanes every
+    // lane of group grp holds, in sc[it], the score of key kbase + it * KPI + grp
+    float sc[LPK], qr[8];
+#pragma unroll
+    for (int it0 = 0; it0 < LPK; it0 += GROUP) {
+      bf16x8 kv[GROUP];
+#pragma unroll
+      for (int u = 0; u < GROUP; ++u) {
+        // (a load's keys are of one run, or, 32 keys a load, of two: a key that the row does not read comes from a run that is there, and is masked)
+        constexpr int RUNS = KPI / 16;
+        const int it = it0 + u, b0 = it * KPI / 16, key16 = (it * KPI + grp) % 16;
+        const int pg = RUNS > 1 && grp >= 16 ? page[b0 + (RUNS > 1)] : page[b0], off = (RUNS > 1 && grp >= 16 ? at[b0 + (RUNS > 1)] : at[b0]) + key16;
+        kv[u] = bf16x8{};
+        if (holds)
+          kv[u] = *reinterpret_cast<const bf16x8*>(
+              k_pool + ((static_cast<size_t>(pg) * Hkv + hk) * page_size + off) * DH + sub * 8);
+      }
+      // (the query is waited for behind the keys' loads: scaled in front of the loop it was a trip to memory in front of the page table's)
+      if (it0 == 0) {
+        u32x4 here = q4;
+        asm volatile("" : "+v"(here));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) qr[i] = to_float(bf16_t{static_cast<uint16_t>(here[i / 2] >> (i % 2 * 16))}) * scale;
+      }
+#pragma unroll
+      for (int u = 0; u < GROUP; ++u) {
+        const int key = kbase + (it0 + u) * KPI + grp;
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) dot = fmaf(qr[i], static_cast<float>(kv[u][i]), dot);
+        dot = group_reduce<LPK>(dot, SumOp());
+        if (EXTRAS && ex.cap > 0.f) dot = ex.cap * tanh_of_exp2(dot * to_tanh);
+        if (EXTRAS && bias) dot += bias[min(max(pos - key, 0), ex.span - 1)];
+        sc[it0 + u] = reads_key(key, lo, pos, keep) ? dot : NEG_INF;
+      }
+    }
+    float m_c = NEG_INF;
+#pragma unroll
+    for (int it = 0; it < LPK; ++it) m_c = fmaxf(m_c, sc[it]);
+    m_c = wave_max(m_c);
+    // EARLY: no branch from here on, nor for runs that the row does not read, whose probabilities are 0: behind a branch the compiler asks for the values only
+    // when the scores are made, a second trip to memory (in half the registers, which is better where many workgroups share a CU)
+    if (!EARLY && !(m_c > NEG_INF)) continue;
+    const float m_new = fmaxf(m_run, m_c);
+    const float alpha = m_run > NEG_INF ? __expf(m_run - m_new) : 0.f;
+    float p[LPK];
+    float psum = 0.f;
+#pragma unroll
+    for (int it = 0; it < LPK; ++it) {
+      p[it] = sc[it] > NEG_INF ? __expf(sc[it] - m_new) : 0.f;
+      psum += p[it];
+    }
+    // each key is held by LPK lanes: its first lane counts it
+    l_run = l_run * alpha + wave_sum(sub == 0 ? psum : 0.f);
+    m_run = m_new;
+#pragma unroll
+    for (int i = 0; i < DPL; ++i) acc[i] *= alpha;
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      if (!EARLY && !live[blk]) continue;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int key = blk * 16 + j;      // key = it * KPI + grp: held by lane grp * LPK in p[it]
+        const float pj = lane_value(p[key / KPI], (key % KPI) * LPK);
+#pragma unroll
+        for (int i = 0; i < DPL; ++i)
+          acc[i] = fmaf(pj, static_cast<float>(j < 8 ? v0[blk][i][j] : v1[blk][i][j - 8]), acc[i]);
+      }
+    }
+  }
+  if (lane == 0) {
+    wm[wave] = m_run;
+    wl[wave] = l_run;
+  }
+#pragma unroll
+  for (int i = 0; i < DPL; ++i)
+    if (lane + 64 * i < DH) wacc[wave][lane + 64 * i] = acc[i];
+  __syncthreads();
+  for (int d = threadIdx.x; d < DH; d += WAVES * 64) {
+    float M = wm[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) M = fmaxf(M, wm[w]);
+    float L = 0.f, A = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      if (wm[w] > NEG_INF) {
+        float f = __expf(wm[w] - M);
+        L += wl[w] * f;
+        A += wacc[w][d] * f;
+      }
+    }
+    if (n_splits == 1) {
+      if (EXTRAS && ex.sink) L += __expf(sink_score(ex, h) - M);      // (a key without a value)
+      out[ldo > 0 ? static_cast<size_t>(row) * ldo + h * DH + d : packed_index(row, h * DH + d, H * DH / 32)] =
+          from_float<bf16_t>(A / L);
+    } else {
+      mypart[2 + d] = A;
+      if (d == 0) {
+        mypart[0] = M;
+        mypart[1] = L;
+      }
+    }
+  }
 }
 
 __global__ void join_kernel(const float* __restrict__ part, bf16_t* __restrict__ out, int ldo,

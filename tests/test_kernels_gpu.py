@@ -676,6 +676,28 @@ def test_attention_of_single_rows_beside_portions(H, Hkv, dh, ps, extras):
     assert torch.allclose(out.float(), want, **TOL[torch.bfloat16])
 
 
+@pytest.mark.parametrize("H,Hkv,dh,ps,extras", [(4, 2, 64, 16, {}), (2, 2, 16, 48, {}), (3, 1, 128, 32, dict(window=100)), (2, 2, 80, 64, {}),
+                                                (2, 1, 48, 16, dict(window=70, keep_first=20, sink=True)), (2, 2, 96, 64, dict(chunk=96, softcap=3.0))])
+def test_rows_of_portions_in_bfloat16_do_not_depend_on_the_cut(H, Hkv, dh, ps, extras):
+    """The last 129 rows of a context, whose last row has a tile to itself, and the same rows in portions of other lengths, single rows among
+    them, alone and beside another request's rows: the same bits."""
+    q, k, v, bt, _, T = paged_case([700, 300], [129, 1], H, Hkv, dh, ps, torch.bfloat16, seed=dh)
+
+    def run(cuts, beside):
+        out, first = torch.zeros(T, H * dh, dtype=torch.bfloat16, device=DEV), 0
+        for n in cuts:
+            table = [(0, first + i, min(128, n - i), 571 + first + i) for i in range(0, n, 128)] + ([(1, 129, 1, 299)] if beside else [])
+            tiles = i32(table).t().contiguous()
+            ops().attention(q[:, :H * dh], out, k, v, bt, tiles, H, dh ** -0.5, tiles_wide=tiles, **extras)
+            first += n
+        assert first == 129
+        return out[:129]
+
+    whole = run([129], False)
+    for cuts in ([128, 1], [1, 128], [100, 29], [64, 1, 63, 1], [1] * 3 + [126]):
+        assert torch.equal(run(cuts, False), whole) and torch.equal(run(cuts, True), whole), cuts
+
+
 @pytest.mark.parametrize("H,Hkv,dh,ps,window", [(8, 8, 64, 16, 0), (8, 2, 32, 32, 40), (8, 4, 64, 48, 0),
                                                 (8, 8, 96, 16, 0), (8, 2, 128, 32, 60), (8, 8, 80, 16, 0),
                                                 (8, 4, 160, 16, 30), (8, 8, 256, 16, 0)])
