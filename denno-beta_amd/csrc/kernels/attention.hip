@@ -1431,18 +1431,31 @@ namespace decode {
 constexpr int lanes_per_key(int dh) { return dh <= 16 ? 2 : dh <= 32 ? 4 : dh <= 64 ? 8 : dh <= 128 ? 16 : 32; }
 
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+// This lane's 16 bytes of a query (zeros in a lane without a piece, which add nothing to a score).
+template <int DH>
+__device__ __forceinline__ bf16x8 query_piece(const bf16_t* q) {
+  constexpr int LPK = lanes_per_key(DH), PIECES = DH / 8;
+  const int sub = threadIdx.x % 64 % LPK;
+  bf16x8 qv = {};
+  if (PIECES == LPK || sub < PIECES) qv = *reinterpret_cast<const bf16x8*>(q + sub * 8);
+  return qv;
+}
 
-template <int DH, int WAVES, bool POW2, bool EXTRAS = false, bool EARLY = false>   // head size (a multiple of 16 up to 256); waves per workgroup; ScoreExtras; see EARLY below
-__global__ __launch_bounds__(WAVES * 64) void partial_kernel(const bf16_t* __restrict__ q, int ldq, bf16_t* __restrict__ out,
-                                                       int ldo, const bf16_t* __restrict__ k_pool,
-                                                       const bf16_t* __restrict__ v_pool,
-                                                       const int32_t* __restrict__ block_tables, int max_blocks,
-                                                       const int32_t* __restrict__ tile_seq,
-                                                       const int32_t* __restrict__ tile_row0,
-                                                       const int32_t* __restrict__ tile_pos0,
-                                                       float* __restrict__ part, int n_splits, int chunks, int H,
-                                                       int Hkv, int page_size, int page_shift, float scale,
-                                                       int window, ScoreExtras ex) {
+// the waves' maxima, sums and weighted values, in LDS
+template <int DH, int WAVES>
+struct RowSums {
+  float m[WAVES], l[WAVES], acc[WAVES][DH];
+};
+
+// One row and head, its keys shared out among the workgroup's waves 64 at a time: the whole of a workgroup.  qv: query_piece of
+// the row's query; bt: its request's block table; part: where splits leave their results (n_splits > 1).
+// (A function of its own for what the compiler makes of it: written out in the kernel, the values are asked for early whatever
+// EARLY says, in 116 registers where 63 do: 200 rows of 50 keys, 16 heads of 64 9.1 -> 11.4 us.)
+template <int DH, int WAVES, bool POW2, bool EXTRAS, bool EARLY = false>
+__device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const int32_t* bt, bf16_t* __restrict__ out, int ldo,
+                                        const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, float* part, int split, int n_splits,
+                                        int chunks, int h, int H, int Hkv, int page_size, int page_shift, float scale, int window,
+                                        const ScoreExtras& ex, RowSums<DH, WAVES>& sums) {
   static_assert(DH % 16 == 0 && DH >= 16 && DH <= 256, "head size");
   constexpr int LPK = lanes_per_key(DH);
   constexpr int PIECES = DH / 8;         // 16-byte pieces of a key: the lanes sub < PIECES of its LPK
@@ -1451,24 +1464,10 @@ __global__ __launch_bounds__(WAVES * 64) void partial_kernel(const bf16_t* __res
   constexpr int KPI = 64 / LPK;          // keys per load instruction
   constexpr int DPL = (DH + 63) / 64;    // dims per lane in the second product
   constexpr int GROUP = LPK < 8 ? LPK : 8;   // load instructions issued together
-  __shared__ float wm[WAVES], wl[WAVES];
-  __shared__ float wacc[WAVES][DH];
-  // In a step of single rows request s brings row s and is tile s: the block table and the query
-  // are addressed by the workgroup's index, so their loads do not wait for the tile table's.
-  const int split = blockIdx.x, h = blockIdx.y, tile = blockIdx.z;
-  const int row = tile;
-  const int32_t* bt = block_tables + static_cast<size_t>(tile) * max_blocks;
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);   // (a scalar)
   const int sub = lane % LPK, grp = lane / LPK;
   const bool holds = PIECES == LPK || sub < PIECES;     // (a lane without a piece: zeros, which add nothing to a score)
-  bf16x8 qv = {};
-  if (holds) qv = *reinterpret_cast<const bf16x8*>(q + static_cast<size_t>(row) * ldq + h * DH + sub * 8);
-  // Request, position and every argument are asked for together: left to itself the compiler waits for the request, then
-  // for the arguments that the rest needs, then for the position, three trips in front of the page table's.
-  const int seq = tile_seq[tile], pos = tile_pos0[tile];
-  asm volatile("" ::"s"(seq), "s"(pos), "s"(k_pool), "s"(v_pool), "s"(page_size), "s"(window));
-  if (seq < 0) return;
-  float* mypart = part + ((static_cast<size_t>(tile) * H + h) * n_splits + split) * (DH + 2);
+  float* mypart = part + ((static_cast<size_t>(row) * H + h) * n_splits + split) * (DH + 2);
   const int lo = first_key(pos, window, EXTRAS ? ex.chunk : 0);
   const float* bias = EXTRAS && ex.bias ? ex.bias + static_cast<size_t>(h) * ex.span : nullptr;
   const int keep = EXTRAS ? ex.keep : 0;
@@ -1600,24 +1599,24 @@ __global__ __launch_bounds__(WAVES * 64) void partial_kernel(const bf16_t* __res
     }
   }
   if (lane == 0) {
-    wm[wave] = m_run;
-    wl[wave] = l_run;
+    sums.m[wave] = m_run;
+    sums.l[wave] = l_run;
   }
 #pragma unroll
   for (int i = 0; i < DPL; ++i)
-    if (lane + 64 * i < DH) wacc[wave][lane + 64 * i] = acc[i];
+    if (lane + 64 * i < DH) sums.acc[wave][lane + 64 * i] = acc[i];
   __syncthreads();
   for (int d = threadIdx.x; d < DH; d += WAVES * 64) {
-    float M = wm[0];
+    float M = sums.m[0];
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) M = fmaxf(M, wm[w]);
+    for (int w = 1; w < WAVES; ++w) M = fmaxf(M, sums.m[w]);
     float L = 0.f, A = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      if (wm[w] > NEG_INF) {
-        float f = __expf(wm[w] - M);
-        L += wl[w] * f;
-        A += wacc[w][d] * f;
+      if (sums.m[w] > NEG_INF) {
+        float f = __expf(sums.m[w] - M);
+        L += sums.l[w] * f;
+        A += sums.acc[w][d] * f;
       }
     }
     if (n_splits == 1) {
@@ -1632,6 +1631,31 @@ __global__ __launch_bounds__(WAVES * 64) void partial_kernel(const bf16_t* __res
       }
     }
   }
+}
+
+template <int DH, int WAVES, bool POW2, bool EXTRAS = false, bool EARLY = false>   // head size (a multiple of 16 up to 256); waves per workgroup; ScoreExtras; see one_row
+__global__ __launch_bounds__(WAVES * 64) void partial_kernel(const bf16_t* __restrict__ q, int ldq, bf16_t* __restrict__ out,
+                                                       int ldo, const bf16_t* __restrict__ k_pool,
+                                                       const bf16_t* __restrict__ v_pool,
+                                                       const int32_t* __restrict__ block_tables, int max_blocks,
+                                                       const int32_t* __restrict__ tile_seq,
+                                                       const int32_t* __restrict__ tile_row0,
+                                                       const int32_t* __restrict__ tile_pos0,
+                                                       float* __restrict__ part, int n_splits, int chunks, int H,
+                                                       int Hkv, int page_size, int page_shift, float scale,
+                                                       int window, ScoreExtras ex) {
+  __shared__ RowSums<DH, WAVES> sums;
+  // In a step of single rows request s brings row s and is tile s: the block table and the query
+  // are addressed by the workgroup's index, so their loads do not wait for the tile table's.
+  const int split = blockIdx.x, h = blockIdx.y, tile = blockIdx.z;
+  const bf16x8 qv = query_piece<DH>(q + static_cast<size_t>(tile) * ldq + h * DH);
+  // Request, position and every argument are asked for together: left to itself the compiler waits for the request, then for the arguments that the
+  // rest needs, then for the position, three trips in front of the page table's.
+  const int seq = tile_seq[tile], pos = tile_pos0[tile];
+  asm volatile("" ::"s"(seq), "s"(pos), "s"(k_pool), "s"(v_pool), "s"(page_size), "s"(window));
+  if (seq < 0) return;
+  one_row<DH, WAVES, POW2, EXTRAS, EARLY>(qv, tile, pos, block_tables + static_cast<size_t>(tile) * max_blocks, out, ldo, k_pool, v_pool, part, split, n_splits,
+                                   chunks, h, H, Hkv, page_size, page_shift, scale, window, ex, sums);
 }
 
 __global__ void join_kernel(const float* __restrict__ part, bf16_t* __restrict__ out, int ldo,
