@@ -1568,8 +1568,10 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
 #pragma unroll
     for (int it = 0; it < LPK; ++it) m_c = fmaxf(m_c, sc[it]);
     m_c = wave_max(m_c);
-    // EARLY: no branch from here on, nor for runs that the row does not read, whose probabilities are 0: behind a branch the compiler asks for the values only
-    // when the scores are made, a second trip to memory (in half the registers, which is better where many workgroups share a CU)
+    // EARLY: no branch from here on, nor for runs that the row does not read: behind a branch the compiler asks for the values
+    // only when the scores are made, a second trip to memory (in half the registers, which is better where many workgroups
+    // share a CU).  What a branch would have stepped over is made zeros instead: its probabilities are 0, but the values that
+    // stand in for it need not be finite, and 0 times infinity is not 0.
     if (!EARLY && !(m_c > NEG_INF)) continue;
     const float m_new = fmaxf(m_run, m_c);
     const float alpha = m_run > NEG_INF ? __expf(m_run - m_new) : 0.f;
@@ -1588,6 +1590,14 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) {
       if (!EARLY && !live[blk]) continue;
+      if constexpr (EARLY) {
+        const uint32_t there = live[blk] && m_c > NEG_INF ? 0xffffffffu : 0u;      // the same for the whole wave
+#pragma unroll
+        for (int i = 0; i < DPL; ++i) {
+          v0[blk][i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v0[blk][i]) & there);
+          v1[blk][i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v1[blk][i]) & there);
+        }
+      }
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int key = blk * 16 + j;      // key = it * KPI + grp: held by lane grp * LPK in p[it]

@@ -878,6 +878,33 @@ def test_a_single_row_is_the_same_bits_alone_and_among_many(dh, ps):
         assert torch.equal(one[0], many[r]), lengths[r]
 
 
+@pytest.mark.parametrize("dh,ps", [(64, 16), (16, 32), (128, 64), (80, 16)])
+def test_a_single_row_meets_infinite_values_alone_as_among_many(dh, ps):
+    """Infinite values at a row's last key, and at 64 keys whose scores are all minus infinity: what a row does not read, or weighs with
+    nothing, adds nothing, also in steps of few workgroups."""
+    H, Hkv = 4, 2
+    lengths = [1, 6, 16, 17, 40, 64, 70, 129, 200, 256] * 8
+    q, k, v, bt, tiles, T = paged_case(lengths, [1] * len(lengths), H, Hkv, dh, ps, torch.bfloat16, seed=dh + 1)
+    q[:, 0:H * dh:dh] = 1.0
+    for r, n in enumerate(lengths):
+        v[bt[r, (n - 1) // ps], :, 0, (n - 1) % ps] = float("inf")
+        v[bt[r, (n - 1) // ps], :, 1, (n - 1) % ps] = float("-inf")
+        if r % 2 and n > 128:
+            for key in range(64, 128):
+                k[bt[r, key // ps], :, key % ps, 0] = float("-inf")
+                v[bt[r, key // ps], :, 2, key % ps] = float("inf")
+    many = torch.zeros(T, H * dh, dtype=torch.bfloat16, device=DEV)
+    ops().attention(q[:, :H * dh], many, k, v, bt, tiles, H, dh ** -0.5, single_rows=True, max_context=256)
+    assert not many.isnan().any()
+    heads = many.view(T, H, dh)
+    assert (heads[:, :, 0] == float("inf")).all() and (heads[:, :, 1] == float("-inf")).all() and heads[:, :, 2:].isfinite().all()
+    for r in range(10):
+        one = torch.zeros(1, H * dh, dtype=torch.bfloat16, device=DEV)
+        ops().attention(q[r:r + 1, :H * dh], one, k, v, bt[r:r + 1].contiguous(), i32([[0], [0], [1], [lengths[r] - 1]]), H, dh ** -0.5,
+                        single_rows=True, max_context=256)
+        assert torch.equal(one[0], many[r]), lengths[r]
+
+
 @pytest.mark.parametrize("longest", [64, 256, 257, 511, 512, 513, 1025])
 @pytest.mark.parametrize("ps,extras", [(16, {}), (4, dict(window=100)), (64, dict(window=70, keep_first=20, sink=True)), (20, dict(chunk=96, softcap=3.0))])
 def test_single_rows_in_32_bit_are_the_same_bits_at_every_length(longest, ps, extras):
