@@ -1733,27 +1733,24 @@ extern "C" int dn_attention_decode_extras(const void* q, int ldq, void* out, int
   // Short contexts and a workgroup a CU at most: nothing else hides a trip to memory (1 row of 50 keys, 16 heads 4.0 -> 3.7 us, 16 rows of 200 4.4 -> 4.2; 203
   // rows of 40, 20 heads 9.9 and 13.3, so not there; with eight and sixteen waves level or slower by 2 %)
   const bool early = waves == 4 && pow2 && !extras && dh <= 128 && static_cast<long>(n_splits) * H * n_tiles <= 256;
-#define DN_DECODE_P(L, W, P, X)                                                                                       \
-  hipLaunchKernelGGL((decode::partial_kernel<L, W, P, X>), grid, block, 0, stream, static_cast<const bf16_t*>(q), ldq, \
+#define DN_DECODE_P(L, W, P, X, E)                                                                                       \
+  hipLaunchKernelGGL((decode::partial_kernel<L, W, P, X, E>), grid, block, 0, stream, static_cast<const bf16_t*>(q), ldq, \
                      static_cast<bf16_t*>(out), ldo, static_cast<const bf16_t*>(k_pool),                              \
                      static_cast<const bf16_t*>(v_pool), block_tables, max_blocks, tile_seq, tile_row0, tile_pos0,    \
                      part, n_splits, chunks, H, Hkv, page_size, page_shift, scale, window, ex)
 #define DN_DECODE_W(L, W)    \
   do {                       \
     if (extras)              \
-      DN_DECODE_P(L, W, true, true);   \
+      DN_DECODE_P(L, W, true, true, false);   \
     else if (pow2)           \
-      DN_DECODE_P(L, W, true, false);  \
+      DN_DECODE_P(L, W, true, false, false);  \
     else                     \
-      DN_DECODE_P(L, W, false, false); \
+      DN_DECODE_P(L, W, false, false, false); \
   } while (0)
 #define DN_DECODE(D)                  \
   if (early) {                        \
-    hipLaunchKernelGGL((decode::partial_kernel<D, 4, true, false, true>), grid, block, 0, stream, static_cast<const bf16_t*>(q), ldq, \
-                       static_cast<bf16_t*>(out), ldo, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), block_tables, \
-                       max_blocks, tile_seq, tile_row0, tile_pos0, part, n_splits, chunks, H, Hkv, page_size, page_shift, scale, window, ex); \
-  } else                              \
-  if (waves == 16) {                  \
+    if constexpr (D <= 128) DN_DECODE_P(D, 4, true, false, true); \
+  } else if (waves == 16) {           \
     if constexpr (D <= 64) DN_DECODE_W(D, 16); \
   } else if (waves == 8) {            \
     if constexpr (D <= 128) DN_DECODE_W(D, 8);  \
