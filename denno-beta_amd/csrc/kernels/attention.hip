@@ -894,10 +894,29 @@ extern "C" int dn_attention_portions(const void* q, int ldq, void* out, int ldo,
   return dn_launch_status();
 }
 
-// A step of single rows with the plain kernels, every tile of keys a workgroup of its own: the same bits as
-// dn_attention gives (one order of summation).  max_context: the longest context of the step; part:
-// n_tiles * H * ceil(max_context / tile) * (dh + 2) floats, the tile being dn_attention_rows_tile(dh) keys.
+// A step of single rows with the plain kernels: the same bits as dn_attention gives (one order of summation).  Every tile of
+// keys, dn_attention_rows_tile(dh) of them, is a wave of its row's workgroup (one_workgroup_takes), or a workgroup of its own whose
+// result a second kernel joins.  max_context: the longest context of the step; part: dn_attention_rows_part_floats() floats,
+// n_tiles * H * ceil(max_context / tile) * (dh + 2) where there is a second kernel, else 0 (part is not read then and may be null).
 extern "C" int dn_attention_rows_tile(int dh) { return plain::tile_keys(dh); }
+
+namespace {
+// whether the kernels for heads of 64 take these pools
+bool wave_tiles_take(const void* k_pool, const void* v_pool, int dh, int page_size) {
+  return dh == 64 && page_size % 4 == 0 && reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 && reinterpret_cast<uintptr_t>(v_pool) % 16 == 0;
+}
+
+bool one_workgroup_takes(const void* k_pool, const void* v_pool, int dh, int page_size, int n_key_tiles) {
+  return wave_tiles_take(k_pool, v_pool, dh, page_size) && n_key_tiles <= plain::ROW_WALK_TILES;
+}
+}  // namespace
+
+extern "C" long dn_attention_rows_part_floats(const void* k_pool, const void* v_pool, int n_tiles, int max_context, int H, int dh,
+                                              int page_size) {
+  const int BK = plain::tile_keys(dh), n_key_tiles = (max_context + BK - 1) / BK;
+  if (one_workgroup_takes(k_pool, v_pool, dh, page_size, n_key_tiles)) return 0;
+  return static_cast<long>(n_tiles) * H * n_key_tiles * (dh + 2);
+}
 
 extern "C" int dn_attention_rows(const void* q, int ldq, void* out, int ldo, const void* k_pool, const void* v_pool,
                                  const int32_t* block_tables, int max_blocks, const int32_t* tile_seq,
@@ -916,20 +935,21 @@ extern "C" int dn_attention_rows_extras(const void* q, int ldq, void* out, int l
   if (chunk < 0 || !(cap >= 0.f) || (bias && span < 1) || !keep_ok(keep, window, chunk)) return DN_ERR_SHAPE;
   const ScoreExtras ex{chunk, bias, span, sink, sink_at, keep, cap};
   if (dh < 16 || dh > 256 || dh % 16 != 0 || Hkv < 1 || H % Hkv != 0 || page_size < 1 || max_blocks < 1 ||
-      max_context < 1 || !part || n_tiles > 65535 || H > 65535)
+      max_context < 1 || n_tiles > 65535 || H > 65535)
     return DN_ERR_SHAPE;
   const int BK = plain::tile_keys(dh);
   const int n_key_tiles = (max_context + BK - 1) / BK;
+  const bool one_workgroup = one_workgroup_takes(k_pool, v_pool, dh, page_size, n_key_tiles);
+  if (!one_workgroup && !part) return DN_ERR_SHAPE;
   const size_t lds = sizeof(float) * (static_cast<size_t>(dh) + 2 * static_cast<size_t>(BK) * (dh + 1) + 5 * BK);
   dim3 grid(n_key_tiles, H, n_tiles), block(plain::THREADS);
-  const bool wave_tiles = dh == 64 && page_size % 4 == 0 && reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 &&
-                          reinterpret_cast<uintptr_t>(v_pool) % 16 == 0;
+  const bool wave_tiles = wave_tiles_take(k_pool, v_pool, dh, page_size);
 #define DN_WALK(T, WAVES)                                                                                                    \
   hipLaunchKernelGGL((plain::row_walk64_kernel<T, WAVES>), dim3(H, n_tiles), dim3(64 * WAVES), 0, stream,                    \
                      static_cast<const T*>(q), ldq, static_cast<T*>(out), ldo, static_cast<const T*>(k_pool),                \
                      static_cast<const T*>(v_pool), block_tables, max_blocks, tile_seq, tile_pos0, n_key_tiles, H, Hkv,       \
                      page_size, scale, window, ex)
-  if (wave_tiles && n_key_tiles <= plain::ROW_WALK_TILES) {
+  if (one_workgroup) {
     if (dtype == DN_F32) {
       if (n_key_tiles <= 4) DN_WALK(float, 4); else DN_WALK(float, 8);
     } else if (dtype == DN_BF16) {

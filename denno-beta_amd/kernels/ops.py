@@ -187,6 +187,9 @@ def _declare(name, lib):
     if name == "sequence":
         lib.dn_delta_chunks_floats.argtypes = [I, I, I, I, I]
         lib.dn_delta_chunks_floats.restype = c_longlong
+    if name == "attention":
+        lib.dn_attention_rows_part_floats.argtypes = [P, P, I, I, I, I, I]
+        lib.dn_attention_rows_part_floats.restype = c_longlong
     if name == "gemm":
         lib.dn_gemm_work_floats.argtypes = [I, I, I, I]
         lib.dn_gemm_work_floats.restype = c_longlong
@@ -752,15 +755,15 @@ def attention(q, out, k_pool, v_pool, block_tables, tiles, n_heads, scale, windo
     n_tiles = tiles.shape[1]
     base = tiles.data_ptr()
     if single_rows and max_context > 0 and dh % 16 == 0:
-        # a step of single rows in the plain kernels: every tile of keys a workgroup of its own, the
-        # tiles' results joined in order by a second kernel; the same bits as the kernel below gives
+        # a step of single rows in the plain kernels: every tile of keys a wave of its row's workgroup, or a workgroup of
+        # its own whose result a second kernel joins, in order; the same bits as the kernel below gives
         _need(max_context <= block_tables.shape[1] * ps, "attention: max_context exceeds the block tables")
         _need(n_tiles == T, "attention: a step of single rows has a tile for every row")
-        key_tiles = -(-max_context // lib.dn_attention_rows_tile(dh))
-        part = torch.empty(n_tiles * n_heads * key_tiles * (dh + 2), dtype=torch.float32, device=q.device)
+        part_floats = lib.dn_attention_rows_part_floats(k_pool.data_ptr(), v_pool.data_ptr(), n_tiles, int(max_context), n_heads, dh, ps)
+        part = torch.empty(part_floats, dtype=torch.float32, device=q.device) if part_floats else None
         _ok(lib.dn_attention_rows_extras(
             q.data_ptr(), ldq, out.data_ptr(), ldo, k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),
-            block_tables.shape[1], base, base + 12 * n_tiles, n_tiles, part.data_ptr(), int(max_context), n_heads, Hkv,
+            block_tables.shape[1], base, base + 12 * n_tiles, n_tiles, _ptr(part), int(max_context), n_heads, Hkv,
             dh, ps, float(scale), int(window), int(chunk), _ptr(bias), span, int(sink), _ptr(sink_at), keep_first, float(softcap),
             _CODE[q.dtype], _stream()), "attention (single rows)")
         return out

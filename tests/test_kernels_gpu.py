@@ -920,6 +920,20 @@ def test_single_rows_in_32_bit_are_the_same_bits_at_every_length(longest, ps, ex
     assert torch.equal(got, want) and got[1:].abs().min(dim=1).values.max() > 0 and not got[0].any()
 
 
+@pytest.mark.parametrize("dtype,ps", [(torch.float32, 16), (torch.bfloat16, 20)])
+@pytest.mark.parametrize("longest,taken", [(512, 0), (513, 1)])
+def test_single_rows_take_a_workspace_where_a_second_kernel_reads_it(dtype, ps, longest, taken):
+    q, k, v, bt, tiles, T = paged_case([longest, 3], [1, 1], 4, 2, 64, ps, dtype)
+    out = torch.zeros(T, 256, dtype=dtype, device=DEV)
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    ops().attention(q[:, :256], out, k, v, bt, tiles, 4, 0.125, single_rows=True, max_context=longest)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == taken
+    lib, base = ops()._lib("attention"), tiles.data_ptr()
+    if taken:      # (refused without one, on the host)
+        assert lib.dn_attention_rows(q.data_ptr(), q.stride(0), out.data_ptr(), 256, k.data_ptr(), v.data_ptr(), bt.data_ptr(), bt.shape[1], base,
+                                     base + 24, T, None, longest, 4, 2, 64, ps, 0.125, 0, ops()._CODE[dtype], ops()._stream()) == -2
+
+
 def test_sample_greedy_and_walk():
     V = 50257
     logits = rnd(6, V, seed=3, scale=2.0)
