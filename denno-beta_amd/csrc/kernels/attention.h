@@ -61,8 +61,8 @@ int dn_attention_portions(const void* q, int ldq, void* out, int ldo, const void
 // dn_attention_rows_tile(dh) keys a wave or a workgroup of its own; part: dn_attention_rows_part_floats() floats (0: not read,
 // may be null), never more than n_tiles * H * ceil(max_context / dn_attention_rows_tile(dh)) * (dh + 2)
 int dn_attention_rows_tile(int dh);
-long dn_attention_rows_part_floats(const void* k_pool, const void* v_pool, int n_tiles, int max_context, int H, int dh,
-                                   int page_size);
+long dn_attention_rows_part_floats(const void* k_pool, const void* v_pool, int n_tiles, int max_context, int H, int Hkv,
+                                   int dh, int page_size, int dtype);
 int dn_attention_rows(const void* q, int ldq, void* out, int ldo, const void* k_pool, const void* v_pool,
                       const int32_t* block_tables, int max_blocks, const int32_t* tile_seq, const int32_t* tile_pos0,
                       int n_tiles, float* part, int max_context, int H, int Hkv, int dh, int page_size, float scale,

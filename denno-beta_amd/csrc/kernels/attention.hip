@@ -672,10 +672,13 @@ __global__ __launch_bounds__(64) void row_tile64_kernel(
   mine[2 + lane] = a;
 }
 
-// The same for a context of up to ROW_WALK_TILES tiles, in one kernel: a workgroup is a row and a head, its waves take a tile of keys each, leave (m_T, l_T, a_T) in LDS, and the first wave joins them in ascending order, a lane per dim.  A lane brings its key's 64
-// dims straight into registers (16 bytes a load: a key's 256 bytes are two cache lines that the wave's other loads find in the vector cache), so nothing but
-// the probabilities goes through LDS.  Both kernels -> this one, 16 heads: 1 row of 50 keys 8.6 -> 4.8 us, 8 rows of 200 10.1 -> 7.6, of 500 13.7 -> 12.5, 32 rows of
-// 300 22.8 -> 20.6.  With two turns of the waves it loses where the rows are few or very many (1 row of 1,024 keys 15.7 and 19.9, 64 of 1,000 102 and 112).
+// The same for a context of up to ROW_WALK_TILES tiles, in one kernel: a workgroup is a row and a head, its waves take a tile
+// of keys each, leave (m_T, l_T, a_T) in LDS, and the first wave joins them in ascending order, a lane per dim.  A lane brings its
+// key's 64 dims straight into registers (16 bytes a load: a key's 256 bytes are two cache lines that the wave's other loads
+// find in the vector cache), so nothing but the probabilities goes through LDS.  It is bound by its chain of trips to memory
+// (request, pages, keys and values).  Both kernels -> this one, 16 heads: 1 row of 50 keys 8.6 -> 4.8 us, 8 rows of 200 10.1 -> 7.6,
+// of 500 13.7 -> 12.5.  Which steps take it: one_workgroup_takes.  With two turns of the waves it loses where the rows are
+// few or very many (1 row of 1,024 keys 15.7 and 19.9, 64 of 1,000 102 and 112).
 constexpr int ROW_WALK_TILES = 8;
 
 template <typename T, int WAVES>
@@ -906,15 +909,31 @@ bool wave_tiles_take(const void* k_pool, const void* v_pool, int dh, int page_si
   return dh == 64 && page_size % 4 == 0 && reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 && reinterpret_cast<uintptr_t>(v_pool) % 16 == 0;
 }
 
-bool one_workgroup_takes(const void* k_pool, const void* v_pool, int dh, int page_size, int n_key_tiles) {
-  return wave_tiles_take(k_pool, v_pool, dh, page_size) && n_key_tiles <= plain::ROW_WALK_TILES;
+// Whether a row's tiles of keys are the waves of one workgroup.  A wave holds 153 registers, so a CU has room for three workgroups
+// of four waves or one of eight: up to 768 or 256 of them nothing waits for room and the one kernel is ahead (32-bit, 16 heads:
+// 48 rows of 64 keys 1.4 times as fast as the two kernels, 48 of 256 1.2, 16 of 512 1.26).  Beyond, what counts is how
+// many of the waves have keys.  One or two tiles leave two or three waves of four without (64 rows of 60 keys 0.93,
+// 512 rows 0.67, of 128 keys 0.93), five to eight an eighth to three and a CU only eight waves (24 rows of 320 keys 1.05, 36 of 12 heads 0.99, 64 0.87, 512 0.78);
+// three or four tiles are level (512 rows of 256 keys 1.00, of 190 0.99) and ahead where contexts are shorter than the longest that a
+// captured step allows (512 rows of 100 keys, longest 256: 1.34).  Where heads share keys the two kernels find them in the
+// caches, and half as many workgroups are the line (16 heads over 4: 24 rows of 256 keys 1.02, 64 0.95; 8 of 512 1.06, 16 0.95).
+// 16-bit keys are half the bytes to wait for: 768 for five to eight tiles (48 rows of 512 keys 1.19, 128 0.98), no line
+// for two to four (512 rows of 128 keys 0.95, of 256 1.17).
+bool one_workgroup_takes(const void* k_pool, const void* v_pool, int n_tiles, int H, int Hkv, int dh, int page_size, int n_key_tiles,
+                         int dtype) {
+  if (!wave_tiles_take(k_pool, v_pool, dh, page_size) || n_key_tiles > plain::ROW_WALK_TILES) return false;
+  const long groups = static_cast<long>(n_tiles) * H;
+  if (dtype == DN_BF16) return groups <= 768 || (n_key_tiles >= 2 && n_key_tiles <= 4);
+  const int shared = H > Hkv ? 2 : 1;
+  if (n_key_tiles > 4) return groups <= 256 / shared;
+  return groups <= 768 / shared || (shared == 1 && n_key_tiles >= 3);
 }
 }  // namespace
 
-extern "C" long dn_attention_rows_part_floats(const void* k_pool, const void* v_pool, int n_tiles, int max_context, int H, int dh,
-                                              int page_size) {
+extern "C" long dn_attention_rows_part_floats(const void* k_pool, const void* v_pool, int n_tiles, int max_context, int H, int Hkv, int dh,
+                                              int page_size, int dtype) {
   const int BK = plain::tile_keys(dh), n_key_tiles = (max_context + BK - 1) / BK;
-  if (one_workgroup_takes(k_pool, v_pool, dh, page_size, n_key_tiles)) return 0;
+  if (one_workgroup_takes(k_pool, v_pool, n_tiles, H, Hkv, dh, page_size, n_key_tiles, dtype)) return 0;
   return static_cast<long>(n_tiles) * H * n_key_tiles * (dh + 2);
 }
 
@@ -939,7 +958,7 @@ extern "C" int dn_attention_rows_extras(const void* q, int ldq, void* out, int l
     return DN_ERR_SHAPE;
   const int BK = plain::tile_keys(dh);
   const int n_key_tiles = (max_context + BK - 1) / BK;
-  const bool one_workgroup = one_workgroup_takes(k_pool, v_pool, dh, page_size, n_key_tiles);
+  const bool one_workgroup = one_workgroup_takes(k_pool, v_pool, n_tiles, H, Hkv, dh, page_size, n_key_tiles, dtype);
   if (!one_workgroup && !part) return DN_ERR_SHAPE;
   const size_t lds = sizeof(float) * (static_cast<size_t>(dh) + 2 * static_cast<size_t>(BK) * (dh + 1) + 5 * BK);
   dim3 grid(n_key_tiles, H, n_tiles), block(plain::THREADS);

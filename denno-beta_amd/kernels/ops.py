@@ -188,7 +188,7 @@ def _declare(name, lib):
         lib.dn_delta_chunks_floats.argtypes = [I, I, I, I, I]
         lib.dn_delta_chunks_floats.restype = c_longlong
     if name == "attention":
-        lib.dn_attention_rows_part_floats.argtypes = [P, P, I, I, I, I, I]
+        lib.dn_attention_rows_part_floats.argtypes = [P, P, I, I, I, I, I, I, I]
         lib.dn_attention_rows_part_floats.restype = c_longlong
     if name == "gemm":
         lib.dn_gemm_work_floats.argtypes = [I, I, I, I]
@@ -759,7 +759,8 @@ def attention(q, out, k_pool, v_pool, block_tables, tiles, n_heads, scale, windo
         # its own whose result a second kernel joins, in order; the same bits as the kernel below gives
         _need(max_context <= block_tables.shape[1] * ps, "attention: max_context exceeds the block tables")
         _need(n_tiles == T, "attention: a step of single rows has a tile for every row")
-        part_floats = lib.dn_attention_rows_part_floats(k_pool.data_ptr(), v_pool.data_ptr(), n_tiles, int(max_context), n_heads, dh, ps)
+        part_floats = lib.dn_attention_rows_part_floats(k_pool.data_ptr(), v_pool.data_ptr(), n_tiles, int(max_context), n_heads, Hkv, dh,
+                                                        ps, _CODE[q.dtype])
         part = torch.empty(part_floats, dtype=torch.float32, device=q.device) if part_floats else None
         _ok(lib.dn_attention_rows_extras(
             q.data_ptr(), ldq, out.data_ptr(), ldo, k_pool.data_ptr(), v_pool.data_ptr(), block_tables.data_ptr(),

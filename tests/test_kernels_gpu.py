@@ -920,6 +920,20 @@ def test_single_rows_in_32_bit_are_the_same_bits_at_every_length(longest, ps, ex
     assert torch.equal(got, want) and got[1:].abs().min(dim=1).values.max() > 0 and not got[0].any()
 
 
+@pytest.mark.parametrize("dtype,H,Hkv,ps,longest,rows", [(torch.float32, 16, 16, 16, 64, 48), (torch.float32, 16, 16, 16, 257, 16), (torch.float32, 16, 4, 16, 256, 24),
+                                                         (torch.float32, 16, 4, 16, 300, 8), (torch.bfloat16, 16, 4, 20, 64, 48), (torch.bfloat16, 16, 4, 4, 300, 48)])
+def test_as_many_single_rows_as_one_kernel_takes_and_one_more(dtype, H, Hkv, ps, longest, rows):
+    """The bits of the plain kernel for portions on both sides of the rule."""
+    lengths = ([longest, 1, 63, 64, longest - 1] * rows)[:rows + 1]
+    q, k, v, bt, tiles, T = paged_case(lengths, [1] * (rows + 1), H, Hkv, 64, ps, dtype, seed=rows)
+    want = torch.zeros(T, H * 64, dtype=dtype, device=DEV)
+    ops().attention(q[:, :H * 64], want, k, v, bt, tiles, H, 0.125)
+    for n in (rows, rows + 1):
+        some, got = tiles[:, :n].contiguous(), torch.zeros(n, H * 64, dtype=dtype, device=DEV)
+        ops().attention(q[:n, :H * 64], got, k, v, bt, some, H, 0.125, single_rows=True, max_context=longest)
+        assert torch.equal(got, want[:n]) and (got != 0).any(dim=1).all()
+
+
 @pytest.mark.parametrize("dtype,ps", [(torch.float32, 16), (torch.bfloat16, 20)])
 @pytest.mark.parametrize("longest,taken", [(512, 0), (513, 1)])
 def test_single_rows_take_a_workspace_where_a_second_kernel_reads_it(dtype, ps, longest, taken):
