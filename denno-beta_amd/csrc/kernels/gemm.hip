@@ -77,7 +77,7 @@ extern "C" int dn_gemm(const void* A, int lda, const void* W, const float* bias,
 // The fused projection of few rows in the plain kernels (32-bit, or bfloat16 weights in rows): C [M, N] = A . W^T +
 // bias, and the key columns (q_width ..) and the value columns behind them also go to the slots slot_map[m] of the
 // pools (keys [page, Hkv, page_size, dh], values [page, Hkv, dh, page_size], of C's type), written by the kernel
-// that adds the segments' sums.  Only where the product has that kernel: dn_gemm_plain_qkv_takes.
+// that adds the segments' sums, the product's own or a second one.  Only where that is so: dn_gemm_plain_qkv_takes.
 extern "C" int dn_gemm_plain_qkv_takes(const void* A, int lda, const void* W, int M, int N, int K, int dtype) {
   if (!plain::joins_of(M, N, K)) return 0;
   return plain::few_rows_take_of(dtype, A, lda, W, M, K);

@@ -5,8 +5,8 @@
 // whatever M is, so that logits do not depend on how a step was cut: K goes in segments of SEG; a
 // segment's sum runs k ascending from zero, one fused multiply-add a step; the segments' sums are
 // added in ascending order, starting from zero.  Three kernels keep to it.  Many rows (M > 64): 64 x 64
-// tiles on the matrix cores, a workgroup walks all of K.  Up to 16 rows (`chain_takes`): 8 or 16 columns and all of K a
-// workgroup, on the matrix cores too.  Between them: a tile of 8 to 64 rows x 64 columns, and where the
+// tiles on the matrix cores, a workgroup walks all of K.  Up to 16 rows (`chain_takes`): 8 or 16 columns
+// and all of K a workgroup, on the matrix cores too.  Else: a tile of 8 to 64 rows x 64 columns, and where the
 // column tiles alone do not fill the chip every segment is a workgroup of its own, which asks for its
 // whole share of W (64 x 128: 32 KB) at once and leaves its sum in a workspace; a second kernel adds
 // the segments' sums in order and ends with the epilogue.  (Few rows used to run in the many-rows
@@ -238,15 +238,18 @@ __device__ __forceinline__ void turn4(float* v) {
   v[0] = __builtin_bit_cast(float, a), v[1] = __builtin_bit_cast(float, b), v[2] = __builtin_bit_cast(float, c), v[3] = __builtin_bit_cast(float, d);
 }
 
-// Up to 16 rows: one kernel.  A workgroup owns 16 columns, or, for up to 8 rows, 8, and all of K; a wave takes a segment at a time, every load of it at
-// once, straight into registers, and multiplies on the matrix cores: v_mfma_f32_16x16x4_f32 adds its four products to the sum
-// one after the other, k ascending, each with one rounding: the bits of the chain of fused multiply-adds.  Its operands want k = 4 s + g in lane group g, and a lane's
-// 16 bytes are k = 4 g + s: a 4 x 4 turn between lane groups (`turn4`).  With up to 8 rows the 16 x 16 result is two segments' 8 x 8 on its
-// diagonal: lanes l % 16 < 8 bring rows and columns of one segment, the others the same rows and columns of the next (the blocks off the diagonal
-// are dropped), so that twice as many workgroups ask for half as much each.  The segments' sums meet in LDS and are added in order.  It had been a kernel with a
-// workgroup a segment, whose operands went through LDS and vector multiply-adds, and a second one to add the sums: at 1 and 8 rows
-// 3,072 x 1,024 10.4 -> 6.1 and 10.8 -> 7.4 us, 1,024 x 1,024 7.0 -> 4.6 and 7.3 -> 5.2, 1,024 x 4,096 12.1 -> 8.7 and 12.3 -> 10.8, 1,600 x
-// 6,400 20.0 -> 14.2 and 20.6 -> 17.1, 50,257 x 1,024 75.5 -> 36.7 (5.6 TB/s of W) and 75.6 -> 50.5.  From 8 rows on what a workgroup reads of A is as much as it reads of W.
+// Up to 16 rows: one kernel (where: chain_takes).  A workgroup owns 16 columns, or, for up to 8 rows, 8, and all of K; a wave
+// takes a segment at a time, every load of it at once, straight into registers, and multiplies on the matrix cores:
+// v_mfma_f32_16x16x4_f32 adds its four products to the sum one after the other, k ascending, each with one rounding: the
+// bits of the chain of fused multiply-adds.  Its operands want k = 4 s + g in lane group g, and a lane's 16 bytes are
+// k = 4 g + s: a 4 x 4 turn between lane groups (`turn4`).  With up to 8 rows the 16 x 16 result is two segments' 8 x 8 on its
+// diagonal: lanes l % 16 < 8 bring rows and columns of one segment, the others the same rows and columns of the next (the
+// blocks off the diagonal are dropped), so that twice as many workgroups ask for half as much each.  The segments' sums meet in
+// LDS and are added in order.  A kernel with a workgroup a segment, whose operands go through LDS and vector
+// multiply-adds, and a second one that adds the sums, against this one at 1 and 8 rows: 3,072 x 1,024 10.4 -> 6.1 and
+// 10.8 -> 7.4 us, 1,024 x 1,024 7.0 -> 4.6 and 7.3 -> 5.2, 1,024 x 4,096 12.1 -> 8.7 and 12.3 -> 10.8, 1,600 x 6,400 20.0 -> 14.2
+// and 20.6 -> 17.1, 50,257 x 1,024 75.5 -> 36.7 (5.6 TB/s of W) and 75.6 -> 50.5.  At one row it is bound by W's bytes and its
+// chain of trips to memory; from 8 rows on what a workgroup reads of A is as much as it reads of W.
 template <typename TI, typename TC, int WAVES, bool PAIR, int NB>
 __global__ __launch_bounds__(WAVES * 64) void chain_kernel(const TI* __restrict__ A, int lda, const TI* __restrict__ W, const float* __restrict__ bias,
                                                             TC* __restrict__ C, int ldc, float* __restrict__ resid, int ldr, int M, int N, int K,
@@ -453,13 +456,35 @@ __global__ __launch_bounds__(256) void join_kernel(const float* __restrict__ par
 }
 
 constexpr int FEW_ROWS = 64;
-// Whether chain_kernel takes a product that few_rows_take takes: its segments' sums fit 60 KB of LDS, and beyond 8 rows the segments are as many as its
-// waves take in two turns (16 rows x 1,600 columns from K = 6,400: 28.4 us, 22.3 in the kernel with a workgroup a segment).
-static bool chain_takes(int M, int K) { return M <= 8 ? K <= 60 * SEG : M <= 16 && K <= 32 * SEG; }
+// Whether chain_kernel takes a product that few_rows_take takes.  Times of a kernel with a workgroup a segment and its join
+// over those of chain_kernel, 32-bit, weights from memory:
+// * A workgroup's 16 waves take 32 segments a turn (16 where it has 16 rows), and one of 8 columns has all of K to itself,
+//   where a workgroup a segment spreads few columns over the chip: the fewer the columns and the more rows of A are read
+//   beside W's, the earlier a long K is better off there (256 columns: 1 row at K = 3,072 1.13 and 4,096 0.99, 8 rows at 2,048 1.12 and 3,072 0.95;
+//   512: 4 rows at 4,096 0.99, 8 at 3,072 1.01 and 4,096 0.90; 768: 8 at 6,400 1.00 and 7,680 0.88; 1,024: 8 at 7,680 0.99 and 12,288
+//   0.88; 1,600: 8 at 16,384 1.07, 16 at 3,072 1.00 and 4,096 0.95; 3,072, one and a half workgroups a CU: 8 at 7,680 0.95 and
+//   16,384 0.89, 16 at 7,680 1.03; 8,192: 8 at 6,400 0.96, 8,192 1.18, 16,384 1.01).  The sums take 256 bytes of LDS a
+//   segment (512 with two blocks of columns, 1 KB with 16 rows): 64 KB at most.
+// * A workgroup costs the same however short K is, and there are eight times as many of 8 columns (8,192 columns: K = 64 0.90, 128 1.14;
+//   16,384: 128 0.75, 256 1.28; 50,257, whose tiles of 64 fill the chip without shares of K: 128 0.67, 256 1.08; with 16 columns and 16 rows
+//   16,384: 32 0.85, 64 1.02; 50,257: 96 0.86, 128 1.03).
+static bool chain_takes(int M, int N, int K) {
+  if (M > 16) return false;
+  const bool sixteen = M > 8 && N >= 2048;      // (workgroups of 16 rows and columns: see `run`)
+  if (N > 2048 && K < (sixteen ? min(N / 256, 128) : min(N / 64, 256))) return false;
+  int longest;
+  if (M <= 5)
+    longest = N < 512 ? 3072 : N < 768 ? 4096 : N < 1024 ? 7680 : N < 1536 ? 12288 : 16384;
+  else if (M <= 8)
+    longest = N < 512 ? 2048 : N < 768 ? 3072 : N < 1024 ? 6400 : N < 1536 || (N > 2048 && N < 4096) ? 7680 : 16384;
+  else
+    longest = N < 512 ? 3072 : N < 768 ? 4096 : N < 1024 ? 6400 : N < 1536 ? 7680 : N < 3072 ? 4096 : 7680;
+  return K <= longest;
+}
 
 // floats of workspace that a product of M rows needs (0: none)
 long work_floats(int M, int N, int K) {
-  if (M > FEW_ROWS || chain_takes(M, K)) return 0;
+  if (M > FEW_ROWS || chain_takes(M, N, K)) return 0;
   const int nseg = (K + SEG - 1) / SEG;
   const long tiles = (N + BN - 1) / BN;
   if (nseg < 2 || tiles >= 384) return 0;      // the column tiles alone fill the chip
@@ -475,8 +500,8 @@ static bool few_rows_take(const void* A, int lda, const void* W, int M, int K) {
          lda % 4 == 0 && K % 4 == 0;
 }
 
-// kv: a fused projection's cache write, done by the kernel that joins the segments (so only where there is one:
-// few_rows_take and work_floats > 0)
+// kv: a fused projection's cache write, done by chain_kernel or by the kernel that joins the segments (so only where one of
+// them runs: few_rows_take and joins_of)
 template <typename TI, typename TC>
 static int run(const void* A, int lda, const void* W, const float* bias, void* C, int ldc, float* resid, int ldr, int M,
                int N, int K, int epi, float* work, long have, hipStream_t stream, KVRows<TC> kv = KVRows<TC>{}) {
@@ -506,11 +531,12 @@ static int run(const void* A, int lda, const void* W, const float* bias, void* C
 #undef DN_MANY
     return 0;
   }
-  if (chain_takes(M, K)) {
+  if (chain_takes(M, N, K)) {
     const int nseg = (K + SEG - 1) / SEG;
-    // 9 to 16 rows of few columns: two workgroups of 8 rows, since 16 columns each leave most CUs without work (1,024 x 1,024 at 16 rows 6.9 us and
-    // 5.3, from K = 4,096 18.4 and 11.1; 3,072 columns 7.5 and 9.3).  5 to 8 rows of very many columns: two blocks of columns, since the rows are read again by every
-    // workgroup (50,257 x 1,024: 8 rows 55.0 and 50.5; 1 row 36.7 and 41.8).
+    // 9 to 16 rows of few columns: two workgroups of 8 rows, since 16 columns each leave most CUs without work (1,024 x 1,024
+    // at 16 rows 6.9 us and 5.3, from K = 4,096 18.4 and 11.1; 3,072 columns 7.5 and 9.3).  5 to 8 rows of very many
+    // columns: two blocks of columns, since the rows are read again by every workgroup (50,257 x 1,024: 8 rows 55.0 and 50.5;
+    // 1 row 36.7 and 41.8).
     const bool pair = M <= 8 || N < 2048, wide = M > 4 && M <= 8 && N >= 16384;
     const int turns = pair ? (nseg + 1) / 2 : nseg, side = pair ? 8 : 16, cols = wide ? 2 * side : side;
 #define DN_CHAIN(WAVES, PAIR, NB)                                                                                                       \
@@ -557,7 +583,8 @@ static int run(const void* A, int lda, const void* W, const float* bias, void* C
 }
 
 // -- what the entry points call (one function per choice of types) ---------------------------------------
-int joins_of(int M, int N, int K) { return work_floats(M, N, K) > 0 || (chain_takes(M, K) && K > SEG); }
+// (a product of one segment keeps the cache's own kernel behind it, whichever kernel makes it)
+int joins_of(int M, int N, int K) { return work_floats(M, N, K) > 0 || (chain_takes(M, N, K) && K > SEG); }
 
 int few_rows_take_of(int dtype, const void* A, int lda, const void* W, int M, int K) {
   return dtype == DN_F32 ? few_rows_take<float>(A, lda, W, M, K) : dtype == DN_BF16 ? few_rows_take<bf16_t>(A, lda, W, M, K) : 0;

@@ -511,7 +511,9 @@ def test_linear_rows_do_not_depend_on_the_batch():
         assert torch.equal(sub, full[rows])
 
 
-@pytest.mark.parametrize("N,K", [(7, 4), (17, 132), (2047, 1024), (2049, 124), (16385, 260), (24, 4096), (24, 4100), (9, 7680), (9, 7684)])
+@pytest.mark.parametrize("N,K", [(7, 4), (17, 132), (2047, 1024), (2049, 124), (16385, 260), (24, 4096), (24, 4100), (9, 7680), (9, 7684), (511, 2048), (511, 2052),
+                                 (511, 3072), (511, 3076), (767, 4100), (1023, 6400), (1023, 6404), (1023, 7684), (1535, 7684), (1535, 12288), (1535, 12292),
+                                 (1536, 16384), (1536, 16388), (3072, 7680), (3072, 7684), (8192, 124), (8192, 128), (16400, 60), (16400, 252), (16400, 256)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_plain_linear_of_up_to_16_rows_at_its_edges(N, K, dtype):
     """Rows, columns and inner sizes on both sides of where the kernel for up to 16 rows changes its form or ends, among numbers whose products are
