@@ -255,31 +255,31 @@ __global__ __launch_bounds__(256) void layernorm_row_kernel(const float* __restr
       tot[i] = 0.f;
       pb[i] = pend.bias ? pend.bias[min(static_cast<int>(threadIdx.x) + i * 256, E - 1)] : 0.f;
     }
-    // up to four shares are asked for at a time (one after the other, each was a trip to memory of its own) and added in order: 384 rows x 1,024 columns,
-    // four shares 4.3 -> 3.6 us, 320 x 1,280, two 3.9 -> 3.6
+    // up to four shares are asked for at a time (one after the other, each was a trip to memory of its own) and added in
+    // order: 384 rows x 1,024 columns, four shares 4.3 -> 3.6 us, 320 x 1,280, two 3.9 -> 3.6
     auto add = [&](auto batch, int sh0) {
       constexpr int B = decltype(batch)::value;
       float p[B][VPT];
 #pragma unroll
       for (int u = 0; u < B; ++u)
 #pragma unroll
-        for (int i = 0; i < VPT; ++i)
-          p[u][i] = pr[min(sh0 + u, pend.shares - 1) * pend.stride + min(static_cast<int>(threadIdx.x) + i * 256, E - 1)];
+        for (int i = 0; i < VPT; ++i) p[u][i] = pr[(sh0 + u) * pend.stride + min(static_cast<int>(threadIdx.x) + i * 256, E - 1)];
 #pragma unroll
       for (int u = 0; u < B; ++u)
-        if (sh0 + u < pend.shares) {
 #pragma unroll
-          for (int i = 0; i < VPT; ++i) tot[i] += p[u][i];
-        }
+        for (int i = 0; i < VPT; ++i) tot[i] += p[u][i];
     };
-    if constexpr (VPT > 8) {      // (long rows do not leave the registers)
-      for (int sh = 0; sh < pend.shares; ++sh) add(std::integral_constant<int, 1>{}, sh);
-    } else if (pend.shares <= 2) {
-      add(std::integral_constant<int, 2>{}, 0);
-    } else if (pend.shares == 3) {
-      add(std::integral_constant<int, 3>{}, 0);
-    } else {
-      for (int sh = 0; sh < pend.shares; sh += 4) add(std::integral_constant<int, 4>{}, sh);
+    constexpr int AT_ONCE = VPT > 8 ? 1 : 4;      // (long rows do not leave the registers)
+    int sh = 0;
+    for (; sh + AT_ONCE <= pend.shares; sh += AT_ONCE) add(std::integral_constant<int, AT_ONCE>{}, sh);
+    if constexpr (AT_ONCE > 1) {
+      const int rest = pend.shares - sh;
+      if (rest == 3)
+        add(std::integral_constant<int, 3>{}, sh);
+      else if (rest == 2)
+        add(std::integral_constant<int, 2>{}, sh);
+      else if (rest == 1)
+        add(std::integral_constant<int, 1>{}, sh);
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {

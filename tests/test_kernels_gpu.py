@@ -1204,6 +1204,20 @@ def test_a_product_whose_sum_the_next_norm_adds(M, N, K, rows_in):
     assert o.linear_deferred_shares(M, o.pack_matrix(rnd(4800, K, seed=7, dtype=torch.bfloat16))) == 0
 
 
+@pytest.mark.parametrize("shares", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("E", [40, 513, 1024, 1280, 1537, 2049])
+def test_a_norm_adds_any_number_of_shares_in_order(E, shares):
+    """The bits of the kernel that only adds, whose order of sums is the shares', and the norm against the plain one."""
+    o, x0, part, bias = ops(), rnd(5, E, seed=1), torch.stack([rnd(5, E, seed=9 + s, scale=4.0 ** -s) for s in range(shares)]), rnd(E, seed=2)
+    gamma, beta, x, out = 1 + rnd(E, seed=3, scale=0.1), rnd(E, seed=4, scale=0.1), x0.clone(), torch.empty(5, E, device=DEV)
+    o.layernorm_join(x, part, bias, gamma, beta, 1e-5, out)
+    want = torch.zeros_like(x0)
+    for p in part:
+        want = want + p
+    assert torch.equal(x, x0 + (want + bias)) and torch.equal(x, o.join(part, bias, x0.clone()))
+    assert torch.allclose(out, R.layernorm(x, gamma, beta, 1e-5, torch.empty_like(out), None), **TOL[torch.float32])
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 40, 100])
 @pytest.mark.parametrize("K", [8, 16, 24, 32, 40, 56])
 def test_few_rows_product_with_an_inner_size_below_64(M, K):
