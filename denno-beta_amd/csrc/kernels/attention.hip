@@ -1499,7 +1499,7 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
   constexpr int LPK = lanes_per_key(DH);
   constexpr int PIECES = DH / 8;         // 16-byte pieces of a key: the lanes sub < PIECES of its LPK
   auto page_index = [&](int key) { return POW2 ? key >> page_shift : key / page_size; };
-  auto page_offset = [&](int key) { return POW2 ? key & (page_size - 1) : key % page_size; };
+  auto place_in = [&](int key, int index) { return POW2 ? key & (page_size - 1) : key - index * page_size; };      // (page index)
   constexpr int KPI = 64 / LPK;          // keys per load instruction
   constexpr int DPL = (DH + 63) / 64;    // dims per lane in the second product
   constexpr int GROUP = LPK < 8 ? LPK : 8;   // load instructions issued together
@@ -1534,24 +1534,31 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
     const int tile_no = first_tile + c * WAVES + wave;
     if (tile_no >= n_tiles_read) continue;     // the same for the whole wave; no barrier in this loop
     const int kbase = 64 * (tile_no < kept_tiles ? tile_no : rest + (tile_no - kept_tiles));
-    // The pages of the tile's four runs of 16 keys, by the scalar unit and all at once: the keys and the values of a run lie in one page, so nothing else has to be looked
-    // up.  (Looked up one by one in front of each run's values, and again by every lane for its keys, they were five trips to memory in a row.)  A run that
-    // the row does not read is replaced by the last one that it does.
-    const int last_run = (pos / 16) * 16, last_page = bt[page_index(last_run)];
+    // The pages of the tile's four runs of 16 keys, by the scalar unit and all at once: the keys and the values of a run lie in
+    // one page, so nothing else has to be looked up.  (Looked up one by one in front of each run's values, and again by every
+    // lane for its keys, they were five trips to memory in a row.)  A run that the row does not read is replaced by the last one
+    // that it does.  Places in pages are worked out while the pages are on their way (behind them, where a page is no power
+    // of two keys, the divisions cost heads of 16 on pages of 48 3 to 6 %).
+    // Against the lookups one by one: 203 rows of 40 keys, 20 heads of 64 10.9 -> 9.9 us, 8 rows of 1,000, 25 heads 11.2 ->
+    // 11.0; heads of 48 to 224 that are no power of two 1.1 to 2 times as fast, of 16 to 128 level to 1.2; heads of 256 -3 % (200 rows of
+    // 200 keys, 16 heads 115.8 -> 119.7) or -5 % (8 rows of 4,000 108.4 -> 114.7) where many of them read many keys, since
+    // keys and values are now asked for at once, and up to 1.2 elsewhere.
+    const int last_run = (pos / 16) * 16, last_index = page_index(last_run), last_at = place_in(last_run, last_index), last_page = bt[last_index];
     int at[4], page[4];
     bool live[4];
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) {
       const int kb = kbase + blk * 16;
       live[blk] = kb <= pos && (kb + 16 > lo || kb < keep);
-      at[blk] = live[blk] ? kb : last_run;
-      page[blk] = bt[page_index(at[blk])];
+      const int run = live[blk] ? kb : last_run, index = page_index(run);
+      at[blk] = place_in(run, index);
+      page[blk] = bt[index];
     }
     asm volatile("" ::"s"(last_page), "s"(page[0]), "s"(page[1]), "s"(page[2]), "s"(page[3]));
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) {
       live[blk] = live[blk] && page[blk] >= 0;
-      at[blk] = page_offset(page[blk] >= 0 ? at[blk] : last_run);
+      at[blk] = page[blk] >= 0 ? at[blk] : last_at;
       page[blk] = page[blk] >= 0 ? page[blk] : last_page;
     }
     // values: lane = dim; 16 keys of one page at a time.  They are asked for first, before the keys
@@ -1768,9 +1775,9 @@ extern "C" int dn_attention_decode_extras(const void* q, int ldq, void* out, int
   while ((1 << page_shift) < page_size) ++page_shift;
   const bool pow2 = (1 << page_shift) == page_size;
   if (extras && !pow2) return DN_ERR_SHAPE;
-  // (with pages looked up together and the query waited for last, every other size gained too: 203 rows of 40 keys 10.9 -> 9.9, 8 rows of 1,000, 25 heads 11.2 -> 11.0)
-  // Short contexts and a workgroup a CU at most: nothing else hides a trip to memory (1 row of 50 keys, 16 heads 4.0 -> 3.7 us, 16 rows of 200 4.4 -> 4.2; 203
-  // rows of 40, 20 heads 9.9 and 13.3, so not there; with eight and sixteen waves level or slower by 2 %)
+  // Short contexts and a workgroup a CU at most: nothing else hides a trip to memory (1 row of 50 keys, 16 heads 4.0 -> 3.7
+  // us, 16 rows of 200 4.4 -> 4.2; 203 rows of 40, 20 heads 9.9 and 13.3, so not there; with eight and sixteen waves level or
+  // slower by 2 %)
   const bool early = waves == 4 && pow2 && !extras && dh <= 128 && static_cast<long>(n_splits) * H * n_tiles <= 256;
 #define DN_DECODE_P(L, W, P, X, E)                                                                                       \
   hipLaunchKernelGGL((decode::partial_kernel<L, W, P, X, E>), grid, block, 0, stream, static_cast<const bf16_t*>(q), ldq, \
