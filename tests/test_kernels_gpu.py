@@ -42,7 +42,7 @@ def test_embed(dtype, E):
     assert torch.equal(out, wte[tok.long()].float())
 
 
-@pytest.mark.parametrize("E", [40, 100, 1600, 3000, 9000])
+@pytest.mark.parametrize("E", [40, 100, 513, 700, 1024, 1025, 1280, 1536, 1600, 3000, 9000])
 def test_layernorm(E):
     x = rnd(9, E, seed=3, scale=3.0) + 1.5
     g, b = rnd(E, seed=4), rnd(E, seed=5)
@@ -213,6 +213,30 @@ def test_linear_qkv_in_the_plain_kernels(dtype, M, K, ps):
     R.kv_write(want, H * dh, (H + Hkv) * dh, slots, want_pools[0], want_pools[1])
     assert torch.equal(out, want) and torch.equal(queries, want[:, :H * dh])
     assert torch.equal(pools[0], want_pools[0]) and torch.equal(pools[1], want_pools[1])
+    assert pools[0].abs().sum() > 0 and pools[1].abs().sum() > 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [9, 12, 16])
+@pytest.mark.parametrize("H,Hkv,K", [(5, 3, 260), (111, 8, 260), (112, 8, 264), (114, 8, 512)])
+def test_linear_qkv_of_9_to_16_rows_in_the_plain_kernels(dtype, M, H, Hkv, K):
+    """On both sides of 2,048 columns, where workgroups of 8 rows give way to workgroups of 16: the cache as the product followed by the
+    reference's write leaves it, bit for bit, rows without a slot in both halves of the rows."""
+    dh, ps, n_pages = 16, 12, 8
+    N = (H + 2 * Hkv) * dh
+    a, w, bias = rnd(M, K, seed=1, dtype=dtype), rnd(N, K, seed=2, dtype=dtype, scale=0.2), rnd(N, seed=3)
+    slots = torch.randperm(n_pages * ps, generator=torch.Generator().manual_seed(M))[:M].to(torch.int32)
+    slots[2] = slots[8] = -1
+    slots = slots.to(DEV)
+    pools = [torch.zeros(n_pages, Hkv, ps, dh, dtype=dtype, device=DEV), torch.zeros(n_pages, Hkv, dh, ps, dtype=dtype, device=DEV)]
+    want_pools = [torch.zeros_like(p) for p in pools]
+    out, want = torch.full((M, N), 7.0, dtype=dtype, device=DEV), torch.empty(M, N, dtype=dtype, device=DEV)
+    before = ops().launches
+    ops().linear_qkv(a, w, bias, out, slots, pools[0], pools[1], H * dh)
+    assert ops().launches - before == 1
+    ops().linear(a, w, bias, out=want)
+    R.kv_write(want, H * dh, (H + Hkv) * dh, slots, want_pools[0], want_pools[1])
+    assert torch.equal(out, want) and torch.equal(pools[0], want_pools[0]) and torch.equal(pools[1], want_pools[1])
     assert pools[0].abs().sum() > 0 and pools[1].abs().sum() > 0
 
 
@@ -920,6 +944,19 @@ def test_single_rows_in_32_bit_are_the_same_bits_at_every_length(longest, ps, ex
     ops().attention(q[:, :H * 64], want, k, v, bt, tiles, H, 0.125, **extras)
     ops().attention(q[:, :H * 64], got, k, v, bt, tiles, H, 0.125, single_rows=True, max_context=longest, **extras)
     assert torch.equal(got, want) and got[1:].abs().min(dim=1).values.max() > 0 and not got[0].any()
+
+
+@pytest.mark.parametrize("longest", [1, 64, 256, 257, 512, 513])
+@pytest.mark.parametrize("ps,extras", [(4, {}), (20, dict(window=100)), (48, dict(window=70, keep_first=20, sink=True)), (20, dict(chunk=96, softcap=3.0))])
+def test_single_rows_in_bfloat16_on_pages_that_the_split_kernel_does_not_take(longest, ps, extras):
+    """Heads of 64 in the plain kernels for single rows: the bits of the plain kernel for portions."""
+    H, Hkv = 4, 2
+    lengths = [n for n in (1, 2, 63, 64, 65, 128, 255, 256, 257, 511) if n < longest] + [longest]
+    q, k, v, bt, tiles, T = paged_case(lengths, [1] * len(lengths), H, Hkv, 64, ps, torch.bfloat16, seed=longest)
+    want, got = torch.zeros(T, H * 64, dtype=torch.bfloat16, device=DEV), torch.zeros(T, H * 64, dtype=torch.bfloat16, device=DEV)
+    ops().attention(q[:, :H * 64], want, k, v, bt, tiles, H, 0.125, **extras)
+    ops().attention(q[:, :H * 64], got, k, v, bt, tiles, H, 0.125, single_rows=True, max_context=longest, **extras)
+    assert torch.equal(got, want) and (got != 0).any(dim=1).all()
 
 
 @pytest.mark.parametrize("dtype,H,Hkv,ps,longest,rows", [(torch.float32, 16, 16, 16, 64, 48), (torch.float32, 16, 16, 16, 257, 16), (torch.float32, 16, 4, 16, 256, 24),
