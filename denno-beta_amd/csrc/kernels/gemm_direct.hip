@@ -4,18 +4,21 @@
 // Many rows, bfloat16, slabs carried from memory straight into LDS (global_load_lds_dwordx4: 16
 // bytes per lane, lane l's at the wave's LDS address + 16 l, no register and no LDS store between).
 // A slab of 32 along K is a list of 1 KB blocks in the packed layout, 16 rows x 32 columns each:
-// a block of W is 1 KB of memory as it lies and is read back at 16 l by lane l; rows of A are put in place
-// by the load itself, in an order of its own.  Where a stage has two slabs (K a multiple of 64), 1 KB of A is 8 rows x 128
-// bytes: whole cache lines.  From the L2 into LDS a CU takes 110 GB/s in pieces of 1 KB, 105 so, and 68 where a load takes 64
-// bytes from each of 16 rows, which is what a stage of one slab leaves (16 lanes then take 64 bytes from each of four rows: with a lane per row the lookups, 52 per
-// load on average, kept the vector cache busy for three quarters of the kernel's time).  With 64 bytes a row everywhere: 320 x 3,840
-// x 1,280 15.9 us, now 13.7; 3,500 x 1,280 x 5,120 88.6 -> 70.0; 8,192 x 3,840 x 1,280 110.4 -> 98.4; 8,192 x 6,400 x 1,600 201.5 -> 194; 2,048 x 4,800 x 1,600
-// 44.4 -> 42.8; two slabs a stage for tiles of 192 and more columns with a long K too (it had been one slab in more stages):
-// 8,192 x 1,600 x 6,400 169.5 -> 161.  The 16-byte pieces of a row are exchanged by the row's number so that the operand read (lane l wants
-// row l % 16, piece l / 16) meets every bank once: LDS serves lanes 0-3, 12-15 and 20-27 together, 4-11, 16-19 and 28-31, and
-// the same 32 lanes on (an order that is free of conflicts for 16 lanes in a row only was slower by 0.3 us a product of 512 rows).  STAGES
-// stages of KB slabs are in flight (vmcnt counts a wave's own loads; one barrier per stage publishes them and
-// frees the stage read before).
+// a block of W is 1 KB of memory as it lies and is read back at 16 l by lane l; rows of A are put in place by the load
+// itself, in an order of its own.  Where a stage has two slabs (K a multiple of 64), 1 KB of A is 8 rows x 128 bytes: whole cache
+// lines.  From the L2 into LDS a CU takes 110 GB/s in pieces of 1 KB, 105 so, and 68 where a load takes 64 bytes from each of 16
+// rows, which is what a stage of one slab leaves (16 lanes then take 64 bytes from each of four rows: with a lane per row the
+// lookups, 52 per load on average, kept the vector cache busy for three quarters of the kernel's time).  64 bytes a row
+// everywhere -> whole lines: 320 x 3,840 x 1,280 15.9 -> 13.7 us; 3,500 x 1,280 x 5,120 88.6 -> 70.0; 8,192 x 3,840 x 1,280
+// 110.4 -> 98.4; 8,192 x 6,400 x 1,600 201.5 -> 194; 2,048 x 4,800 x 1,600 44.4 -> 42.8.  Tiles whose last rows are missing had
+// their loads nearly free before (a missing row reads the last one again) and lose 1 to 8 % where K is a power of two
+// (65 x 2,048 x 8,192 34.3 -> 36.7, 400 x 3,072 x 1,024 10.7 -> 11.1); whole tiles of the same widths gain 4 to 10 %.  Two slabs a
+// stage for tiles of 192 and more columns with a long K too, against one slab in more stages: 8,192 x 1,600 x 6,400
+// 169.5 -> 161.  The 16-byte pieces of a row are exchanged by the row's number so that the operand read (lane l wants row
+// l % 16, piece l / 16) meets every bank once: LDS serves lanes 0-3, 12-15 and 20-27 together, 4-11, 16-19 and 28-31, and the
+// same 32 lanes on (an order that is free of conflicts for 16 lanes in a row only was slower by 0.3 us a product of 512 rows).
+// STAGES stages of KB slabs are in flight (vmcnt counts a wave's own loads; one barrier per stage publishes them and frees the
+// stage read before).
 //
 // The MFMA takes W as its first operand and A as its second: a lane then holds four consecutive
 // columns of one row of C, which it stores as 8 bytes (bfloat16) or adds as 16 (the 32-bit
@@ -26,6 +29,7 @@
 // but a wave's chain of loads, waits and barriers, and the rounding of tiles to 256 CUs.  Measured per tile and
 // slab with eight waves: time = 2.26e-7 us x BM x BN (matrix cores at nine tenths of their peak) + 3.07e-5 us x
 // (BM + BN) (loads), the two adding up rather than overlapping, + 1.9e-4 us x BM x BN for the stores at the end.
+// (Measured with 64 bytes of a row of A a load; whole lines shorten the loads' share, by more for narrow tiles.)
 // The tile is chosen per product from a list, by that model: the largest that still fills the chip in whole
 // rounds (a tile count just above a multiple of 256 costs a whole further round); and the waves of a workgroup
 // are as many as give every SIMD four (see `run`), so that one of them can issue while the others wait.
@@ -160,8 +164,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
         src[u] = A + static_cast<size_t>(min(m0 / 16 + b, (M + 15) / 16 - 1)) * kall * 512 + kb * 512 + lane * 8;
         step[u] = 512 * KB;
       } else if constexpr (KB == 2) {
-        // a stage's columns are one cache line of a row: 1 KB is 8 rows x 128 bytes, rows 0 .. 7 of the block in the first slab's place and
-        // 8 .. 15 in the second's
+        // a stage's columns are one cache line of a row: 1 KB is 8 rows x 128 bytes, rows 0 .. 7 of the block in the first
+        // slab's place and 8 .. 15 in the second's
         const int r = 8 * kb + lane / 8, piece = (lane % 8) ^ (r / 2);
         src[u] = A + static_cast<size_t>(min(m0 + b * 16 + r, M - 1)) * lda + piece * 8;
         step[u] = 64;
@@ -411,7 +415,8 @@ static int launch_as(const Args& a, hipStream_t stream) {
   return launch<float, WM, WN, TM, TN, STAGES, false, KB>(a, stream);
 }
 
-// (for steps of 65 to 256 rows: a kernel each for A in rows and for packed A, since the choice at run time stands in front of the first loads)
+// (for steps of 65 to 256 rows: a kernel each for A in rows and for packed A, since the choice at run time stands in front of
+// the first loads)
 template <int WM, int WN, int TM, int TN, int STAGES, int KB, int A_IN>
 static int launch_mid_a(const Args& a, hipStream_t stream) {
   if (a.kv) return launch<bf16_t, WM, WN, TM, TN, STAGES, true, KB, false, A_IN>(a, stream);
