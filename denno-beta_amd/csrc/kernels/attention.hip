@@ -897,10 +897,11 @@ extern "C" int dn_attention_portions(const void* q, int ldq, void* out, int ldo,
   return dn_launch_status();
 }
 
-// A step of single rows with the plain kernels: the same bits as dn_attention gives (one order of summation).  Every tile of
-// keys, dn_attention_rows_tile(dh) of them, is a wave of its row's workgroup (one_workgroup_takes), or a workgroup of its own whose
-// result a second kernel joins.  max_context: the longest context of the step; part: dn_attention_rows_part_floats() floats,
-// n_tiles * H * ceil(max_context / tile) * (dh + 2) where there is a second kernel, else 0 (part is not read then and may be null).
+// A step of single rows with the plain kernels: the same bits as dn_attention gives (one order of summation).  Every tile
+// of keys, dn_attention_rows_tile(dh) of them, is a wave of its row's workgroup (one_workgroup_takes), or a workgroup of its
+// own whose result a second kernel joins.  max_context: the longest context of the step; part:
+// dn_attention_rows_part_floats() floats, n_tiles * H * ceil(max_context / tile) * (dh + 2) where there is a second kernel,
+// else 0 (part is not read then and may be null).
 extern "C" int dn_attention_rows_tile(int dh) { return plain::tile_keys(dh); }
 
 namespace {
@@ -909,16 +910,18 @@ bool wave_tiles_take(const void* k_pool, const void* v_pool, int dh, int page_si
   return dh == 64 && page_size % 4 == 0 && reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 && reinterpret_cast<uintptr_t>(v_pool) % 16 == 0;
 }
 
-// Whether a row's tiles of keys are the waves of one workgroup.  A wave holds 153 registers, so a CU has room for three workgroups
-// of four waves or one of eight: up to 768 or 256 of them nothing waits for room and the one kernel is ahead (32-bit, 16 heads:
-// 48 rows of 64 keys 1.4 times as fast as the two kernels, 48 of 256 1.2, 16 of 512 1.26).  Beyond, what counts is how
-// many of the waves have keys.  One or two tiles leave two or three waves of four without (64 rows of 60 keys 0.93,
-// 512 rows 0.67, of 128 keys 0.93), five to eight an eighth to three and a CU only eight waves (24 rows of 320 keys 1.05, 36 of 12 heads 0.99, 64 0.87, 512 0.78);
-// three or four tiles are level (512 rows of 256 keys 1.00, of 190 0.99) and ahead where contexts are shorter than the longest that a
-// captured step allows (512 rows of 100 keys, longest 256: 1.34).  Where heads share keys the two kernels find them in the
-// caches, and half as many workgroups are the line (16 heads over 4: 24 rows of 256 keys 1.02, 64 0.95; 8 of 512 1.06, 16 0.95).
-// 16-bit keys are half the bytes to wait for: 768 for five to eight tiles (48 rows of 512 keys 1.19, 128 0.98), no line
-// for two to four (512 rows of 128 keys 0.95, of 256 1.17).
+// Whether a row's tiles of keys are the waves of one workgroup.  Behind each size: the two kernels' time over this one's.
+// * A wave holds 153 registers, so a CU has room for three workgroups of four waves or one of eight: up to 768 or 256 of
+//   them nothing waits for room (32-bit, 16 heads: 48 rows of 64 keys 1.41, 48 of 256 1.24, 16 of 512 1.26).
+// * Beyond, what counts is how many of the waves have keys.  One or two tiles leave three or two of four without (64 rows of
+//   60 keys 0.93, 512 of 60 0.67, 512 of 128 0.93).  Five to eight tiles leave up to three of eight without, and a CU
+//   holds no more than the eight (24 rows of 320 keys 1.05, with 12 heads 0.99; 64 rows 0.87, 512 0.78).  Three or four
+//   are level (512 rows of 256 keys 1.00, of 190 0.99), and ahead where contexts are shorter than the longest that a
+//   captured step allows (512 rows of 100 keys, longest 256: 1.34).
+// * Where heads share keys the two kernels find them in the caches, and half as many workgroups are the line (16 heads over
+//   4: 24 rows of 256 keys 1.02, 64 0.95; 8 of 512 1.06, 16 0.95).
+// * 16-bit keys are half the bytes to wait for: 768 for five to eight tiles too (48 rows of 512 keys 1.19, 128 0.98), and no
+//   line for two to four (512 rows of 128 keys 0.95, of 256 1.17).
 bool one_workgroup_takes(const void* k_pool, const void* v_pool, int n_tiles, int H, int Hkv, int dh, int page_size, int n_key_tiles,
                          int dtype) {
   if (!wave_tiles_take(k_pool, v_pool, dh, page_size) || n_key_tiles > plain::ROW_WALK_TILES) return false;
@@ -1539,11 +1542,12 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
     // lane for its keys, they were five trips to memory in a row.)  A run that the row does not read is replaced by the last one
     // that it does.  Places in pages are worked out while the pages are on their way (behind them, where a page is no power
     // of two keys, the divisions cost heads of 16 on pages of 48 3 to 6 %).
-    // Against the lookups one by one: 203 rows of 40 keys, 20 heads of 64 10.9 -> 9.9 us, 8 rows of 1,000, 25 heads 11.2 ->
-    // 11.0; heads of 48 to 224 that are no power of two 1.1 to 2 times as fast, of 16 to 128 level to 1.2; heads of 256 -3 % (200 rows of
-    // 200 keys, 16 heads 115.8 -> 119.7) or -5 % (8 rows of 4,000 108.4 -> 114.7) where many of them read many keys, since
-    // keys and values are now asked for at once, and up to 1.2 elsewhere.
-    const int last_run = (pos / 16) * 16, last_index = page_index(last_run), last_at = place_in(last_run, last_index), last_page = bt[last_index];
+    // Against the lookups one by one: 203 rows of 40 keys, 20 heads of 64 10.9 -> 9.9 us, 8 rows of 1,000, 25 heads 11.2
+    // -> 11.0; heads of 48 to 224 that are no power of two 1.1 to 2 times as fast, of 16 to 128 level to 1.2; heads of 256
+    // up to 1.2, but 3 to 5 % slower where many of them read many keys, since keys and values are now asked for at once (200 rows
+    // of 200 keys, 16 heads 115.8 -> 119.7, 8 rows of 4,000 108.4 -> 114.7).
+    const int last_run = (pos / 16) * 16, last_index = page_index(last_run);
+    const int last_at = place_in(last_run, last_index), last_page = bt[last_index];
     int at[4], page[4];
     bool live[4];
 #pragma unroll
@@ -1582,7 +1586,8 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
       bf16x8 kv[GROUP];
 #pragma unroll
       for (int u = 0; u < GROUP; ++u) {
-        // (a load's keys are of one run, or, 32 keys a load, of two: a key that the row does not read comes from a run that is there, and is masked)
+        // (a load's keys are of one run, or, 32 keys a load, of two: a key that the row does not read comes from a run
+        // that is there, and is masked)
         constexpr int RUNS = KPI / 16;
         const int it = it0 + u, b0 = it * KPI / 16, key16 = (it * KPI + grp) % 16;
         const int pg = RUNS > 1 && grp >= 16 ? page[b0 + (RUNS > 1)] : page[b0], off = (RUNS > 1 && grp >= 16 ? at[b0 + (RUNS > 1)] : at[b0]) + key16;
@@ -1591,7 +1596,8 @@ __device__ __forceinline__ void one_row(const bf16x8 qv, int row, int pos, const
           kv[u] = *reinterpret_cast<const bf16x8*>(
               k_pool + ((static_cast<size_t>(pg) * Hkv + hk) * page_size + off) * DH + sub * 8);
       }
-      // (the query is waited for behind the keys' loads: scaled in front of the loop it was a trip to memory in front of the page table's)
+      // (the query is waited for behind the keys' loads: scaled in front of the loop it was a trip to memory in front of the
+      // page table's)
       if (it0 == 0) {
         u32x4 here = q4;
         asm volatile("" : "+v"(here));

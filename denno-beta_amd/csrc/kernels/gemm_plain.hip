@@ -456,18 +456,21 @@ __global__ __launch_bounds__(256) void join_kernel(const float* __restrict__ par
 }
 
 constexpr int FEW_ROWS = 64;
-// Whether chain_kernel takes a product that few_rows_take takes.  Times of a kernel with a workgroup a segment and its join
-// over those of chain_kernel, 32-bit, weights from memory:
+// Whether chain_kernel takes a product that few_rows_take takes.  Behind each size: the time of the kernel with a workgroup a
+// segment and its join over chain_kernel's, 32-bit, weights from memory.
 // * A workgroup's 16 waves take 32 segments a turn (16 where it has 16 rows), and one of 8 columns has all of K to itself,
 //   where a workgroup a segment spreads few columns over the chip: the fewer the columns and the more rows of A are read
-//   beside W's, the earlier a long K is better off there (256 columns: 1 row at K = 3,072 1.13 and 4,096 0.99, 8 rows at 2,048 1.12 and 3,072 0.95;
-//   512: 4 rows at 4,096 0.99, 8 at 3,072 1.01 and 4,096 0.90; 768: 8 at 6,400 1.00 and 7,680 0.88; 1,024: 8 at 7,680 0.99 and 12,288
-//   0.88; 1,600: 8 at 16,384 1.07, 16 at 3,072 1.00 and 4,096 0.95; 3,072, one and a half workgroups a CU: 8 at 7,680 0.95 and
-//   16,384 0.89, 16 at 7,680 1.03; 8,192: 8 at 6,400 0.96, 8,192 1.18, 16,384 1.01).  The sums take 256 bytes of LDS a
-//   segment (512 with two blocks of columns, 1 KB with 16 rows): 64 KB at most.
-// * A workgroup costs the same however short K is, and there are eight times as many of 8 columns (8,192 columns: K = 64 0.90, 128 1.14;
-//   16,384: 128 0.75, 256 1.28; 50,257, whose tiles of 64 fill the chip without shares of K: 128 0.67, 256 1.08; with 16 columns and 16 rows
-//   16,384: 32 0.85, 64 1.02; 50,257: 96 0.86, 128 1.03).
+//   beside W's, the earlier a long K is better off there.
+//     256 columns: 1 row at K = 3,072 1.13, 4,096 0.99; 8 rows at 2,048 1.12, 3,072 0.95
+//     512: 4 rows at 4,096 0.99; 8 at 3,072 1.01, 4,096 0.90            768: 8 rows at 6,400 1.00, 7,680 0.88
+//     1,024: 8 rows at 7,680 0.99, 12,288 0.88                          1,600: 8 rows at 16,384 1.07; 16 at 3,072 1.00, 4,096 0.95
+//     3,072 (one and a half workgroups a CU): 8 rows at 7,680 0.95, 16,384 0.89; 16 at 7,680 1.03
+//     8,192: 8 rows at 6,400 0.96, 8,192 1.18, 16,384 1.01
+//   The sums take 256 bytes of LDS a segment (512 with two blocks of columns, 1 KB with 16 rows): 64 KB at most.
+// * A workgroup costs the same however short K is, and there are eight times as many of 8 columns.
+//     8,192 columns: K = 64 0.90, 128 1.14                              16,384: 128 0.75, 256 1.28
+//     50,257 (whose tiles of 64 fill the chip without shares of K): 128 0.67, 256 1.08
+//     with 16 rows and columns: 16,384: 32 0.85, 64 1.02                50,257: 96 0.86, 128 1.03
 static bool chain_takes(int M, int N, int K) {
   if (M > 16) return false;
   const bool sixteen = M > 8 && N >= 2048;      // (workgroups of 16 rows and columns: see `run`)
@@ -583,7 +586,8 @@ static int run(const void* A, int lda, const void* W, const float* bias, void* C
 }
 
 // -- what the entry points call (one function per choice of types) ---------------------------------------
-// (a product of one segment keeps the cache's own kernel behind it, whichever kernel makes it)
+// (not a product of one segment, though chain_kernel could: inner sizes of up to 128 are no model's that waits for a launch, and
+// the cache's own kernel stays behind them as it stands behind more than 64 rows)
 int joins_of(int M, int N, int K) { return work_floats(M, N, K) > 0 || (chain_takes(M, N, K) && K > SEG); }
 
 int few_rows_take_of(int dtype, const void* A, int lda, const void* W, int M, int K) {
