@@ -214,6 +214,75 @@ __global__ __launch_bounds__(256) void depth_mix_kernel(const float* hist, size_
   }
 }
 
+// What stands behind the last sublayer of a layer whose stream is an average over depth, in one kernel: the sublayer's result y goes
+// into the layer's plane as rmsnorm_add_kernel takes it (x = hist[n - 1], changed in place), out = sum_j w[j] hist[j] as
+// depth_mix_kernel makes it, and (next_out) the norm that reads out next, as rmsnorm_kernel makes it: the same sums in the same
+// order, the same bits.  A workgroup a row of up to 256 N columns, held in registers.  Bound by launches where the rows are few (three kernels of
+// 2 to 3 us each were their trips to memory and little else) and by its bytes where they are many (the row is read back by none of the three):
+// 8 rows of 1,024 behind the third layer 6.7 -> 3.7 us, 2,136 rows 18.4 -> 11.4, 48 rows of 2,048 behind the eighth 8.5 -> 5.4.  The planes, which wait for nothing, are asked for
+// some at a time, before the row's own norm is summed up.
+template <int N>
+__global__ __launch_bounds__(256) void close_mix_kernel(const void* y, int y_dt, size_t ldy, const float* weight, const float* scale, float mult,
+                                                        float eps, float* hist, size_t plane, int n, const float* w, float* out, int width,
+                                                        const float* next_w, float next_eps, void* next_out, int next_dt, size_t ldn) {
+  constexpr int PL = N <= 4 ? 4 : N <= 8 ? 2 : 1;      // planes at a time
+  __shared__ float sh[4];
+  const size_t row = static_cast<size_t>(blockIdx.x) * width;
+  float* x = hist + static_cast<size_t>(n - 1) * plane + row;
+  float v[N] = {}, lw[N] = {}, sc[N] = {}, xs[N] = {}, nw[N] = {}, acc[N] = {};
+  if (N > 1 || static_cast<int>(threadIdx.x) < width) {
+    hold_row<N>(y, static_cast<size_t>(blockIdx.x) * ldy, y_dt, width, v);
+    hold_row<N>(x, 0, DN_F32, width, xs);
+    if (weight) hold_row<N>(weight, 0, DN_F32, width, lw);
+    if (scale) hold_row<N>(scale, 0, DN_F32, width, sc);
+    if (next_out && next_w) hold_row<N>(next_w, 0, DN_F32, width, nw);
+    for (int j0 = 0; j0 < n - 1; j0 += PL) {
+      float h[PL][N], wj[PL];
+#pragma unroll
+      for (int q = 0; q < PL; ++q) {
+        const int j = min(j0 + q, n - 2);      // (a plane beyond the last is read again, and not added)
+        wj[q] = w[j];
+        hold_row<N>(hist, static_cast<size_t>(j) * plane + row, DN_F32, width, h[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < PL; ++q)
+        if (j0 + q < n - 1)
+#pragma unroll
+          for (int i = 0; i < N; ++i) acc[i] = fmaf(wj[q], h[q][i], acc[i]);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (static_cast<int>(threadIdx.x) + 256 * i < width) ss = fmaf(v[i], v[i], ss);
+  ss = block_sum_256(ss, sh);
+  const float inv = 1.0f / sqrtf(ss / static_cast<float>(width) + eps), wl = w[n - 1];
+  float after = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    v[i] *= inv;
+    if (weight) v[i] *= lw[i];
+    if (scale) v[i] *= sc[i];
+    xs[i] = fmaf(mult, v[i], xs[i]);
+    acc[i] = fmaf(wl, xs[i], acc[i]);
+    if (c < width) {
+      x[c] = xs[i];
+      out[row + c] = acc[i];
+      after = fmaf(acc[i], acc[i], after);
+    }
+  }
+  if (!next_out) return;
+  after = block_sum_256(after, sh);
+  const float inv2 = 1.0f / sqrtf(after / static_cast<float>(width) + next_eps);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = threadIdx.x + 256 * i;
+    const float z = acc[i] * inv2;
+    if (c < width) store_as(next_out, static_cast<size_t>(blockIdx.x) * ldn + c, next_dt, next_w ? z * nw[i] : z);
+  }
+}
+
 // out[t, :] = [a[t, :wa] | b[t, :wb]]
 __global__ __launch_bounds__(256) void concat_kernel(const float* a, size_t lda, int wa, const float* b, size_t ldb, int wb,
                                                      void* out, int out_dt) {
@@ -2303,6 +2372,31 @@ int dn_depth_mix(const float* hist, long long plane, int n, const float* w, floa
   const long long groups = (total + 3) / 4;
   hipLaunchKernelGGL(depth_mix_kernel, dim3(static_cast<unsigned>((groups + 255) / 256)), dim3(256), 0, stream, hist,
                      static_cast<size_t>(plane), n, w, out, static_cast<size_t>(total), vec);
+  return dn_launch_status();
+}
+
+// (one workgroup a row, up to 4,096 columns: wider rows take dn_rmsnorm_add, dn_depth_mix and dn_rmsnorm)
+int dn_close_mix(const void* y, int y_dt, long long ldy, const float* weight, const float* scale, float mult, float eps, float* hist,
+                 long long plane, int n, const float* w, float* out, int T, int width, const float* next_w, float next_eps, void* next_out,
+                 int next_dt, long long ldn, hipStream_t stream) {
+  if (!float_kind(y_dt) || (next_out && !float_kind(next_dt))) return DN_ERR_DTYPE;
+  if (T < 0 || width < 1 || width > 4096 || n < 1 || ldy < width || plane < static_cast<long long>(T) * width || (next_out && ldn < width))
+    return DN_ERR_SHAPE;
+  if (T == 0) return 0;
+#define DN_CLOSE_MIX(N)                                                                                                          \
+  hipLaunchKernelGGL(close_mix_kernel<N>, dim3(T), dim3(256), 0, stream, y, y_dt, static_cast<size_t>(ldy), weight, scale, mult,  \
+                     eps, hist, static_cast<size_t>(plane), n, w, out, width, next_w, next_eps, next_out, next_dt, static_cast<size_t>(ldn))
+  if (width <= 256)
+    DN_CLOSE_MIX(1);
+  else if (width <= 512)
+    DN_CLOSE_MIX(2);
+  else if (width <= 1024)
+    DN_CLOSE_MIX(4);
+  else if (width <= 2048)
+    DN_CLOSE_MIX(8);
+  else
+    DN_CLOSE_MIX(16);
+#undef DN_CLOSE_MIX
   return dn_launch_status();
 }
 

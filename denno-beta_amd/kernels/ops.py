@@ -133,6 +133,7 @@ def _declare(name, lib):
             "dn_concat_cast": [P, c_longlong, I, P, c_longlong, I, P, I, I, P],
             "dn_rmsnorm_add": [P, I, c_longlong, P, P, F, P, c_longlong, I, I, F, P, c_longlong, P, F, P, I, c_longlong, P],
             "dn_depth_mix": [P, c_longlong, I, P, P, c_longlong, P],
+            "dn_close_mix": [P, I, c_longlong, P, P, F, F, P, c_longlong, I, P, P, I, I, P, F, P, I, c_longlong, P],
             "dn_unit_heads": [P, c_longlong, P, c_longlong, I, I, I, F, F, P],
             "dn_conv_rows": [P, c_longlong, P, P, P, P, P, I, I, I, I, I, I, P, I, c_longlong, c_longlong, P],
             "dn_history_update": [P, I, c_longlong, P, P, P, I, I, I, c_longlong, P],
@@ -1083,16 +1084,51 @@ def rmsnorm_add(y, weight, scale, mult, eps, x, gate=None, then=None):
     return x
 
 
+class OpenPlanes:
+    """The planes that an average over depth reads where the last of them has not yet taken the sublayer's result that goes into it:
+    rmsnorm_add(y, weight, scale, mult, eps, hist[last]) is still to come.  `depth_mix` does that, the average and the norm that
+    reads the average next in one kernel (then = (weight or None, eps, out); `normed` is `out` once its rows are there, else None);
+    whoever reads a plane (`planes[j]`) has the result put in first."""
+
+    def __init__(self, hist, last, y, weight, scale, mult, eps, then=None):
+        self.hist, self.last, self.add, self.then = hist, last, (y, weight, scale, mult, eps), then
+        self.normed = None
+
+    def close(self):
+        if self.add is not None:
+            rmsnorm_add(*self.add, self.hist[self.last])
+            self.add = None
+        return self.hist
+
+    def __getitem__(self, j):
+        return self.close()[j]
+
+
 def depth_mix(hist, n, weights, out):
-    """out = sum over j < n of weights[j] * hist[j], j ascending; hist: 32-bit [planes, rows, width], contiguous; weights:
-    at least n 32-bit numbers; out: 32-bit [rows, width], contiguous; it may be a plane of hist from n on."""
+    """out = sum over j < n of weights[j] * hist[j], j ascending; hist: 32-bit [planes, rows, width], contiguous, or OpenPlanes
+    of such; weights: at least n 32-bit numbers; out: 32-bit [rows, width], contiguous; it may be a plane of hist from n on."""
+    planes = hist if isinstance(hist, OpenPlanes) else None
+    if planes is not None:
+        # (rows that a workgroup of the one kernel does not hold, and a result that is not the last plane's: one after the other)
+        hist = planes.hist if planes.hist.shape[2] <= 4096 and planes.last == n - 1 else planes.close()
     _dev(hist, "hist", (torch.float32,), 3), _dev(out, "out", (torch.float32,), 2)
     _f32vec(weights, "weights")
-    planes, T, width = hist.shape
-    _need(hist.is_contiguous() and out.is_contiguous() and tuple(out.shape) == (T, width) and 1 <= n <= planes
+    count, T, width = hist.shape
+    _need(hist.is_contiguous() and out.is_contiguous() and tuple(out.shape) == (T, width) and 1 <= n <= count
           and weights.numel() >= n, "depth_mix: shapes")
-    _ok(_lib("sequence").dn_depth_mix(hist.data_ptr(), T * width, n, weights.data_ptr(), out.data_ptr(), T * width, _stream()),
-        "depth_mix")
+    if planes is None or planes.add is None:
+        _ok(_lib("sequence").dn_depth_mix(hist.data_ptr(), T * width, n, weights.data_ptr(), out.data_ptr(), T * width, _stream()),
+            "depth_mix")
+        return out
+    y, weight, scale, mult, eps = planes.add
+    _dev(y, "y", _FLOATS, 2)
+    _need(tuple(y.shape) == (T, width), "depth_mix: the sublayer's result")
+    _f32vec(weight, "weight", width), _f32vec(scale, "scale", width)
+    _ok(_lib("sequence").dn_close_mix(y.data_ptr(), _CODE[y.dtype], _rows(y, "y"), _ptr(weight), _ptr(scale), float(mult), float(eps),
+                                      hist.data_ptr(), T * width, n, weights.data_ptr(), out.data_ptr(), T, width,
+                                      *_then(planes.then, T, width, "depth_mix"), _stream()), "depth_mix")
+    planes.add = None
+    planes.normed = planes.then[2] if planes.then is not None else None
     return out
 
 

@@ -191,6 +191,7 @@ class SandwichBlock:
     the model and a vector of the layer ride along).  A block whose feed-forward is "none" ends after the mixer."""
 
     SLOTS = {"norm1": "norm", "mixer": "mixer", "post1": "norm", "norm2": "norm", "ffn": "feed_forward", "post2": "norm"}
+    opens_planes = True       # leaves its last result to an average over depth behind it (Runtime.average)
 
     def __init__(self, norm1, mixer, post1, norm2, ffn, post2):
         self.norm1, self.mixer, self.post1, self.norm2, self.ffn, self.post2 = norm1, mixer, post1, norm2, ffn, post2
@@ -215,13 +216,30 @@ class SandwichBlock:
         part.forward(*args, accumulate_into=y)
         return y
 
+    def first_norm(self):
+        """The norm that reads the residual stream first in this block."""
+        return self.norm1
+
     def forward(self, x, ctx, caches, runtime):
+        # The norm in front of a sublayer is made by the kernel that takes the sublayer before into the stream, where that norm is a
+        # plain one; across blocks the rows travel in runtime.normed_rows.  Where an average over depth stands behind the
+        # block, its kernel takes the last sublayer's result into the block's plane as well (runtime.average).
+        act = runtime.act_dtype
         runtime.stream_stats = None
-        h = self.norm1.forward(x, runtime.act_dtype)
-        self.post1.add_into(self._result(self.mixer, x, h, ctx, caches[0]), x)
+        came, runtime.normed_rows = runtime.normed_rows, None
+        h = came[1] if came is not None and came[0] is self.norm1 else self.norm1.forward(x, act)
+        y, post, nxt = self._result(self.mixer, x, h, ctx, caches[0]), self.post1, runtime.next_norm
         if self.has_ffn:
-            h = self.norm2.forward(x, runtime.act_dtype)
-            self.post2.add_into(self._result(self.ffn, x, h, ctx), x)
+            h = post.add_into(y, x, then=self.norm2, out_dtype=act)
+            if h is None:
+                h = self.norm2.forward(x, act)
+            y, post = self._result(self.ffn, x, h, ctx), self.post2
+        if runtime.average is not None:
+            runtime.average = post.open_planes(y, *runtime.average, then=nxt, out_dtype=act)
+            return
+        h = post.add_into(y, x, then=nxt, out_dtype=act)
+        if h is not None and nxt is not None:
+            runtime.normed_rows = (nxt, h)
 
 
 @ARRANGEMENTS.register("gated_sandwich")
@@ -234,6 +252,7 @@ class GatedSandwichBlock(SandwichBlock):
 
     SLOTS = {"norm1": "norm", "mixer": "mixer", "gate1": "gate", "post1": "norm", "norm2": "norm", "ffn": "feed_forward",
              "gate2": "gate", "post2": "norm", "side": "token_input"}
+    opens_planes = False
 
     def __init__(self, norm1, mixer, gate1, post1, norm2, ffn, gate2, post2, side):
         super().__init__(norm1, mixer, post1, norm2, ffn, post2)

@@ -322,15 +322,25 @@ class DecoderModel:
                 rt.stream_deferred = None
             if not getattr(block, "keeps_cast", False):
                 rt.stream_cast = None
+            own = kept is not None and x.data_ptr() == kept[i + 1].data_ptr()      # (an injection makes new rows)
+            rt.average = (kept, i + 1) if own and getattr(block, "opens_planes", False) else None
             block.forward(x, ctx, [cache.view(c, call.writes_cache) for c in call.caches()], rt)
             if kept is not None:
                 if rt.stream_deferred is not None:
                     rt.stream_deferred.flush(x)
                 rt.stream_stats = rt.stream_deferred = rt.normed_rows = rt.stream_cast = None
-                if x.data_ptr() != kept[i + 1].data_ptr():      # (an injection made new rows)
+                if not own:
                     kept[i + 1].copy_(x)
+                planes, rt.average = rt.average, None
                 w = self.averages.get(i)
-                x = ops.depth_mix(kept, i + 2, w, kept[i + 2]) if w is not None else ops.depth_mix(kept[i + 1:], 1, self._one, kept[i + 2])
+                if w is None and planes is not None:
+                    planes.close()
+                if w is None:
+                    x = ops.depth_mix(kept[i + 1:], 1, self._one, kept[i + 2])
+                else:
+                    x = ops.depth_mix(kept if planes is None else planes, i + 2, w, kept[i + 2])
+                    if planes is not None and planes.normed is not None:
+                        rt.normed_rows = (rt.next_norm, planes.normed)
         if rt.stream_deferred is not None:
             rt.stream_deferred.flush(x)
         rt.stream_stats = rt.next_norm = rt.stream_deferred = rt.normed_rows = rt.stream_cast = None

@@ -104,6 +104,10 @@ class StreamRMSNorm(RMSNorm):
         ops.rmsnorm_add(y, self.weight, self.scale, self.mult, self.eps, x, gate=gate, then=nxt)
         return nxt[2] if nxt is not None else None
 
+    def open_planes(self, y, hist, last, then=None, out_dtype=None):
+        """The same with the stream being plane `last` of hist, left to the average over depth behind it (ops.OpenPlanes)."""
+        return ops.OpenPlanes(hist, last, y, self.weight, self.scale, self.mult, self.eps, then=following_norm(then, hist[last], out_dtype))
+
 
 def following_norm(norm, x, out_dtype):
     """(weight, eps, rows to fill) for a kernel that, having changed the stream's rows x, norms them for `norm` as well; None
