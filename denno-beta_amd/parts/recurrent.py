@@ -240,9 +240,10 @@ class ChannelDelta(Part):
         z = self.proj(h, out_dtype=F32)
         x = torch.empty((T, C), dtype=F32, device=dev)
         # the three convolutions, silu, and queries and keys made unit vectors (the queries times dim^(-1/2)): one kernel
+        single = ctx.single_rows and cache.writes
         ops.conv_heads(z[:, :C], self.conv, past, ctx.row_start, ctx.state_slots, x, 2 * self.n_qk_heads, self.head_dim,
-                       self.n_qk_heads, self.query_scale, 1.0, self.unit_eps, H, self.value_dim)
-        if self.taps > 1 and cache.writes:
+                       self.n_qk_heads, self.query_scale, 1.0, self.unit_eps, H, self.value_dim, move_on=single)
+        if self.taps > 1 and cache.writes and not single:
             ops.history_update(z[:, :C], past, ctx.row_start, ctx.state_slots)
         q, k, v = x[:, :qk], x[:, qk:2 * qk], x[:, 2 * qk:]
         low = self.low(h, out_dtype=self.a2.weight.dtype)
