@@ -90,6 +90,11 @@ __device__ __forceinline__ float other_half(float v) {
   return __builtin_bit_cast(float, (threadIdx.x & 32) ? a : b);
 }
 
+__device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
+
+// log(1 + e^z), without overflow
+__device__ __forceinline__ float softplus_f(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
+
 static inline int dn_launch_status() { return static_cast<int>(hipGetLastError()); }
 
 // A packed matrix: blocks of 16 rows x 32 columns, 1 KB each and contiguous, block (r / 16, k / 32)

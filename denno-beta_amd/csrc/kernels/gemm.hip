@@ -74,6 +74,43 @@ extern "C" int dn_gemm(const void* A, int lda, const void* W, const float* bias,
   return rc != 0 ? rc : dn_launch_status();
 }
 
+// C [M, N] = act(A . W^T + bias) for an activation with numbers of its own (EPI_XIELU and on, see gemm_common.h), packed W: in the
+// epilogue of the kernel that dn_gemm would run, where it has that activation: the few-rows kernels with up to 64 rows have all
+// three, the many-rows kernel EPI_XIELU.  A kernel between the products is a launch (2 to 3 us of a decode step), and with many rows
+// a pass over the product's 32-bit result (2,136 rows of 4,096 columns 12 us).
+static int act_route(const void* A, int lda, const void* W, const float* bias, const void* C, int ldc, int M, int N, int K, int out_dtype,
+                     int kind, int packed) {
+  if (M < 1 || N < 1 || K < 1 || !(packed & PACKED_W) || (packed & PACKED_C) || K % 8 != 0 || ldc < N) return 0;
+  if ((packed & PACKED_A) ? M > 256 : lda < K) return 0;
+  if (kind < EPI_XIELU || kind > EPI_EXP_NEG_SOFTPLUS || out_dtype != (kind == EPI_XIELU ? DN_BF16 : DN_F32)) return 0;
+  const bool few = skinny::takes(A, lda, W, M, K, packed);
+  const bool many = direct::takes(A, lda, W, bias, C, ldc, nullptr, 0, N, K, out_dtype, packed);
+  if (many && (!few || direct::beats_few_rows(M, N, K))) return kind == EPI_XIELU ? 2 : 0;
+  return few && M <= 64 ? 1 : 0;
+}
+
+extern "C" int dn_gemm_act_takes(const void* A, int lda, const void* W, const float* bias, const void* C, int ldc, int M, int N, int K,
+                                 int out_dtype, int kind, int packed) {
+  return act_route(A, lda, W, bias, C, ldc, M, N, K, out_dtype, kind, packed) != 0;
+}
+
+extern "C" int dn_gemm_act(const void* A, int lda, const void* W, const float* bias, void* C, int ldc, int M, int N, int K, int out_dtype,
+                           int kind, const float* numbers, int cols, int packed, hipStream_t stream) {
+  const int route = act_route(A, lda, W, bias, C, ldc, M, N, K, out_dtype, kind, packed);
+  if (route == 0 || (kind != EPI_SILU && !numbers)) return DN_ERR_SHAPE;
+  const ActNumbers act{numbers, cols};
+  if (route == 2) {
+    direct::Args a{A, lda, W, bias, C, ldc, nullptr, 0, M, N, K, out_dtype, kind, packed, nullptr};
+    a.act = act;
+    const int rc = direct::run(a, stream);
+    return rc != 0 ? rc : dn_launch_status();
+  }
+  skinny::Call c{A, lda, W, bias, C, ldc, nullptr, 0, M, N, K, out_dtype, kind, packed, nullptr};
+  c.act = act;
+  skinny::run(c, stream);
+  return dn_launch_status();
+}
+
 // The fused projection of few rows in the plain kernels (32-bit, or bfloat16 weights in rows): C [M, N] = A . W^T +
 // bias, and the key columns (q_width ..) and the value columns behind them also go to the slots slot_map[m] of the
 // pools (keys [page, Hkv, page_size, dh], values [page, Hkv, dh, page_size], of C's type), written by the kernel

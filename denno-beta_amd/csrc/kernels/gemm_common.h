@@ -33,6 +33,43 @@ __device__ __forceinline__ float apply_epilogue_fast(float v, int epi) {
   return v;
 }
 
+// Activations with numbers of their own (dn_gemm_act), in place of a kernel between two products:
+//   EPI_XIELU             v > 0: p[0] v^2 + v / 2; else p[1] (e^v - 1 - v) + v / 2     (bfloat16 results)
+//   EPI_SILU              v sigmoid(v) in the first `cols` columns, v in the others
+//   EPI_EXP_NEG_SOFTPLUS  exp(-p[column] log(1 + e^v))
+#define EPI_XIELU 4
+#define EPI_SILU 5
+#define EPI_EXP_NEG_SOFTPLUS 6
+struct ActNumbers {
+  const float* p;
+  int cols;
+};
+
+// e^v - 1 - v for v <= 0 without its cancellation near 0: the series there (2e-7 of the result at most), the hardware's exponential
+// beyond.  Some fifteen instructions where expm1f takes several dozen, which shows in the epilogue of a product with many columns.
+__device__ __forceinline__ float xielu_fast(float v, float a, float b) {
+  float s = fmaf(v, 1.0f / 40320.0f, 1.0f / 5040.0f);
+  s = fmaf(s, v, 1.0f / 720.0f);
+  s = fmaf(s, v, 1.0f / 120.0f);
+  s = fmaf(s, v, 1.0f / 24.0f);
+  s = fmaf(s, v, 1.0f / 6.0f);
+  s = fmaf(s, v, 0.5f);
+  const float near = s * v * v, far = __builtin_amdgcn_exp2f(1.4426950408889634f * v) - 1.0f - v;
+  return v > 0.f ? fmaf(a * v, v, 0.5f * v) : fmaf(b, v > -0.5f ? near : far, 0.5f * v);
+}
+
+// p, q: what act_numbers gives for the column
+__device__ __forceinline__ float apply_activation(float v, int epi, float p, float q) {
+  if (epi == EPI_XIELU) return xielu_fast(v, p, q);
+  if (epi == EPI_SILU) return p != 0.f ? v * sigmoid_f(v) : v;
+  if (epi == EPI_EXP_NEG_SOFTPLUS) return expf(-p * softplus_f(v));
+  return apply_epilogue_fast(v, epi);
+}
+__device__ __forceinline__ float act_first(const ActNumbers& a, int epi, int column) {
+  return epi == EPI_SILU ? (column < a.cols ? 1.f : 0.f) : epi >= EPI_XIELU ? a.p[epi == EPI_EXP_NEG_SOFTPLUS ? column : 0] : 0.f;
+}
+__device__ __forceinline__ float act_second(const ActNumbers& a, int epi) { return epi == EPI_XIELU ? a.p[1] : 0.f; }
+
 // Where a fused projection's key and value columns go besides C: columns q_width .. of row m are
 // the keys, then the values, of the token whose slot is slot_map[m] (page * page_size + offset,
 // < 0: none).  Pools as in the cache: keys [page, Hkv, page_size, dh], values [page, Hkv, dh, page_size].
@@ -146,6 +183,7 @@ struct Call {
   const void* A; int lda; const void* W; const float* bias; void* C; int ldc; float* resid; int ldr;
   int M, N, K, out_dtype, epi, packed;
   const KVScatter* kv;
+  ActNumbers act{nullptr, 0};
 };
 bool takes(const void* A, int lda, const void* W, int M, int K, int packed);
 void run(const Call& c, hipStream_t stream);
@@ -163,6 +201,7 @@ namespace direct {
 struct Args {
   const void* A; int lda; const void* W; const float* bias; void* C; int ldc; float* resid; int ldr;
   int M, N, K, out_dtype, epi, packed; const KVScatter* kv;
+  ActNumbers act{nullptr, 0};                  // EPI_XIELU's numbers
   float* part = nullptr; int splits = 1;       // part: K in `splits` shares, their sums in part[share][m][n]
 };
 struct Shape { int bm, bn, stages; };

@@ -90,14 +90,15 @@ __device__ __forceinline__ void tile_at(int pid, int tiles_m, int tiles_n, int b
 // other tiles of 256 rows do not take turns: with bfloat16 results and K up to 3,200 they are level to 15 % slower so (256 x 128: 2,048 x 4,096 x 1,024
 // 26.0 -> 28.7 us; 256 x 224: 2,048 x 6,400 x 1,600 46.8 -> 52.6; 256 x 256: 8,192 x 4,096 x 1,024 79.6 -> 91.4; 192 and more columns with
 // slabs of 32 a stage, since three stages of 64 do not fit in LDS).  Left open: from K = 5,120 on they would gain 3 to 12 % (8,192 x 2,048 x 8,192 225.6 -> 199.3).
-// A_IN: A comes in rows (0), packed (1), or as `packed` says (2).
-template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false, int A_IN = 2>
+// A_IN: A comes in rows (0), packed (1), or as `packed` says (2).  XIELU: the epilogue is that activation (a kernel of its own: its
+// instructions beside the others' cost every product registers).
+template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false, int A_IN = 2, bool XIELU = false>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __restrict__ A, int lda,
                                                            const bf16_t* __restrict__ W, const float* __restrict__ bias,
                                                            TC* __restrict__ C, int ldc, float* __restrict__ resid, int ldr,
                                                            int M, int N, int K, int epi, int packed, int tiles_m,
                                                            int tiles_n, KVScatter kv, float* __restrict__ part,
-                                                           int split_slabs) {
+                                                           int split_slabs, const float* __restrict__ act) {
   constexpr int NW = WM * WN;
   const bool a_packed = A_IN == 2 ? (packed & PACKED_A) != 0 : A_IN == 1;
   constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
@@ -297,6 +298,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
     }
     return;
   }
+  float act_a = 0.f, act_b = 0.f;
+  if constexpr (XIELU) act_a = act[0], act_b = act[1];
   // every load of the epilogue before its first store: a wait for a load is a wait for the stores
   // issued before it as well (one counter), and a load per column block made the blocks take turns
   floatx4 bvs[TN];
@@ -334,8 +337,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
         for (int r = 0; r < 4; ++r) o[r] = apply_epilogue_fast(v[r], epi);
         *reinterpret_cast<floatx4*>(C + static_cast<size_t>(m) * ldc + n) = o;
       } else {
-        const uint2 cv = pack4(apply_epilogue_fast(v[0], epi), apply_epilogue_fast(v[1], epi), apply_epilogue_fast(v[2], epi),
-                               apply_epilogue_fast(v[3], epi));
+        auto finish = [&](float e) { return XIELU ? xielu_fast(e, act_a, act_b) : apply_epilogue_fast(e, epi); };
+        const uint2 cv = pack4(finish(v[0]), finish(v[1]), finish(v[2]), finish(v[3]));
         // (in packed rows, four columns from a multiple of 4 are 8 bytes side by side too)
         if (!KV || n < kv.c_cols)
           *reinterpret_cast<uint2*>(C + ((packed & PACKED_C) ? packed_index(m, n, N / 32) : static_cast<size_t>(m) * ldc + n)) = cv;
@@ -387,25 +390,33 @@ bool takes(const void* A, int lda, const void* W, const float* bias, const void*
 }
 
 
-template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false, int A_IN = 2>
-static int launch(const Args& a, hipStream_t stream) {
+template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false, int A_IN = 2, bool XIELU = false>
+static int launch_kernel(const Args& a, hipStream_t stream) {
   constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
   constexpr size_t lds = static_cast<size_t>(STAGES) * KB * (BM + BN) / 16 * 1024;
   if (a.K % (32 * KB) != 0) return DN_ERR_SHAPE;
   static bool raised = false;      // more than 64 KB of LDS has to be asked for once per kernel
   if (lds > 65536 && !raised) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN, XIELU>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     if (e != hipSuccess) return static_cast<int>(e);
     raised = true;
   }
   const int split_slabs = (a.K / (32 * KB) + a.splits - 1) / a.splits;
-  hipLaunchKernelGGL((gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN>), dim3(tiles_m * tiles_n, a.part ? a.splits : 1),
+  hipLaunchKernelGGL((gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN, XIELU>), dim3(tiles_m * tiles_n, a.part ? a.splits : 1),
                      dim3(WM * WN * 64), lds, stream, static_cast<const bf16_t*>(a.A), a.lda,
                      static_cast<const bf16_t*>(a.W), a.bias, static_cast<TC*>(a.C), a.ldc, a.resid, a.ldr, a.M, a.N, a.K,
-                     a.epi, a.packed, tiles_m, tiles_n, a.kv ? *a.kv : KVScatter{}, a.part, split_slabs);
+                     a.epi, a.packed, tiles_m, tiles_n, a.kv ? *a.kv : KVScatter{}, a.part, split_slabs, a.act.p);
   return 0;
+}
+
+template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false, int A_IN = 2>
+static int launch(const Args& a, hipStream_t stream) {
+  if constexpr (!KV && sizeof(TC) == 2) {
+    if (a.epi == EPI_XIELU) return launch_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN, true>(a, stream);
+  }
+  return launch_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN>(a, stream);
 }
 
 template <int WM, int WN, int TM, int TN, int STAGES, int KB = 1>

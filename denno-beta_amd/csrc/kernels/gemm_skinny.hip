@@ -35,7 +35,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
                                                            const bf16_t* __restrict__ W,
                                                            const float* __restrict__ bias, TC* __restrict__ C,
                                                            int ldc, float* __restrict__ resid, int ldr, int M, int N,
-                                                           int K, int epi, int packed, KVScatter kv, NormIO nio) {
+                                                           int K, int epi, int packed, KVScatter kv, NormIO nio, ActNumbers act) {
   constexpr int BLOCKS = MB * NB;                          // 16 x 16 blocks of C in this workgroup
   constexpr int PASSES = (BLOCKS + WAVES - 1) / WAVES;     // wave w finishes blocks w, w + WAVES, ...
   __shared__ floatx4 red[WAVES][BLOCKS][64];
@@ -57,11 +57,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   float epi_bias[PASSES];
   float epi_x[PASSES][4];
   int epi_slot[KV ? PASSES : 1][4];
+  constexpr bool ACT = !KV && NORM == NORM_NONE && MB <= 4;      // (dn_gemm_act comes here with up to 64 rows)
+  float epi_act[ACT ? PASSES : 1];
+  const float epi_act2 = ACT ? act_second(act, epi) : 0.f;
   float epi_norm[NORM != NORM_NONE ? PASSES : 1];          // NORM_IN: c1 of the lane's column; NORM_OUT: the next norm's gamma
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) {
     const int blk = wave + p * WAVES;
     epi_bias[p] = 0.f;
+    if constexpr (ACT) epi_act[p] = 0.f;
     if constexpr (NORM != NORM_NONE) {
       const int nn = min(n0 + (blk < BLOCKS ? blk % NB : 0) * 16 + col, N - 1);
       epi_norm[p] = NORM == NORM_IN ? nio.c1[nn] : nio.gamma_out[nn];
@@ -76,6 +80,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
       const int mb = blk / NB, nb = blk % NB;
       const int nn = min(n0 + nb * 16 + col, N - 1);
       if (bias) epi_bias[p] = bias[nn];
+      if constexpr (ACT) epi_act[p] = act_first(act, epi, nn);
       if constexpr (KV) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -244,7 +249,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
           nio.copy_out[nio.ldcopy > 0 ? static_cast<size_t>(m) * nio.ldcopy + nn : packed_index(m, nn, N / 32)] =
               from_float<bf16_t>((epi_x[p][r] + v) * epi_norm[p]);
       } else {
-        TC cv = from_float<TC>(apply_epilogue_fast(v, epi));
+        TC cv = from_float<TC>(ACT ? apply_activation(v, epi, epi_act[ACT ? p : 0], epi_act2) : apply_epilogue_fast(v, epi));
         if (!KV || nn < kv.c_cols)
           C[(packed & PACKED_C) ? packed_index(m, nn, N / 32) : static_cast<size_t>(m) * ldc + nn] = cv;
         if constexpr (KV) scatter_kv_at(kv, epi_slot[p][r], nn, cv);
@@ -266,7 +271,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
                                                              const bf16_t* __restrict__ W,
                                                              const float* __restrict__ bias, TC* __restrict__ C,
                                                              int ldc, float* __restrict__ resid, int ldr, int M,
-                                                             int N, int K, int epi, KVScatter kv, NormIO nio) {
+                                                             int N, int K, int epi, KVScatter kv, NormIO nio, ActNumbers act) {
   typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
   constexpr int U = 4;                                     // pairs of steps in flight per wave
   constexpr int ROW = 9 * 8;                               // elements per row of a wave's piece: 8 chunks and one of padding
@@ -288,9 +293,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   float epi_bias = 0.f;
   float epi_x[4] = {0.f, 0.f, 0.f, 0.f};
   int epi_slot[4] = {-1, -1, -1, -1};
+  constexpr bool ACT = !KV && NORM == NORM_NONE;
+  float epi_act = 0.f, epi_act2 = 0.f;
   if (wave == 0) {
     const int nn = min(n0 + col, N - 1);
     if (bias) epi_bias = bias[nn];
+    if constexpr (ACT) epi_act = act_first(act, epi, nn), epi_act2 = act_second(act, epi);
     if constexpr (KV) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) epi_slot[r] = g * 4 + r < M ? kv.slot_map[g * 4 + r] : -1;
@@ -421,7 +429,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
         if constexpr (NORM == NORM_OUT)
           nio.copy_out[static_cast<size_t>(m) * nio.ldcopy + nn] = from_float<bf16_t>((epi_x[r] + v) * epi_gamma);
       } else {
-        const TC cv = from_float<TC>(apply_epilogue_fast(v, epi));
+        const TC cv = from_float<TC>(ACT ? apply_activation(v, epi, epi_act, epi_act2) : apply_epilogue_fast(v, epi));
         if (!KV || nn < kv.c_cols) C[static_cast<size_t>(m) * ldc + nn] = cv;
         if constexpr (KV) scatter_kv_at(kv, epi_slot[r], nn, cv);
       }
@@ -450,7 +458,7 @@ static void launch_one(const Call& c, hipStream_t stream) {
   KVScatter kv = c.kv ? *c.kv : KVScatter{};
   hipLaunchKernelGGL((gemm_kernel<MB, NB, WAVES, U, TC, KV>), grid, block, 0, stream,
                      static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,
-                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, NormIO{});
+                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, NormIO{}, c.act);
 }
 
 // the same with the norm before the product (NORM_IN: bfloat16 out) or after it (NORM_OUT: into the
@@ -462,7 +470,7 @@ static void launch_norm(const Call& c, const NormIO& nio, int norm, hipStream_t 
 #define DN_LN(TC, KV, NORM)                                                                                        \
   hipLaunchKernelGGL((gemm_kernel<MB, NB, WAVES, U, TC, KV, NORM>), grid, block, 0, stream,                       \
                      static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,             \
-                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, nio)
+                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, nio, c.act)
   if (norm == NORM_OUT)
     DN_LN(float, false, NORM_OUT);
   else if (c.kv)
@@ -501,11 +509,11 @@ static void launch16_one(const Call& c, hipStream_t stream) {
   if (c.M > 8)
     hipLaunchKernelGGL((gemm16_kernel<WAVES, TC, KV, NORM_NONE, true>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0, stream,
                        static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,
-                       static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, NormIO{});
+                       static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, NormIO{}, c.act);
   else
     hipLaunchKernelGGL((gemm16_kernel<WAVES, TC, KV, NORM_NONE, false>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0, stream,
                        static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,
-                       static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, NormIO{});
+                       static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, NormIO{}, c.act);
 }
 
 // the same with the norm before the product (NORM_IN: bfloat16 out) or after it (NORM_OUT: into the residual stream)
@@ -516,7 +524,7 @@ static void launch16_norm(const Call& c, const NormIO& nio, int norm, hipStream_
 #define DN_L16_ROWS(TC, KV, NORM, TWO)                                                                                   \
   hipLaunchKernelGGL((gemm16_kernel<WAVES, TC, KV, NORM, TWO>), grid, block, 0, stream, static_cast<const bf16_t*>(c.A), \
                      c.lda, static_cast<const bf16_t*>(c.W), c.bias, static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr,       \
-                     c.M, c.N, c.K, c.epi, kv, nio)
+                     c.M, c.N, c.K, c.epi, kv, nio, c.act)
 #define DN_L16(TC, KV, NORM)                 \
   do {                                       \
     if (c.M > 8)                             \

@@ -678,11 +678,6 @@ __global__ __launch_bounds__(1024) void token_input_kernel(float* x, size_t ldx,
 enum { ACT_SILU = 0, ACT_SIGMOID = 1, ACT_TANH = 2, ACT_EXP_NEG_EXP = 3, ACT_BOUNDED_SIGMOID = 4, ACT_EXP_NEG_SOFTPLUS = 5, ACT_XIELU = 6,
        ACT_RELU2 = 7 };
 
-__device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
-
-// log(1 + e^z), without overflow
-__device__ __forceinline__ float softplus_f(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
-
 __device__ __forceinline__ float activation(int kind, float z, float lower) {
   switch (kind) {
     case ACT_EXP_NEG_SOFTPLUS: return expf(-lower * softplus_f(z));      // (lower: the rate of the column)

@@ -106,6 +106,8 @@ def _declare(name, lib):
         },
         "gemm": {
             "dn_gemm": [P, I, P, P, P, I, P, I, I, I, I, I, I, I, I, P, c_longlong, P],
+            "dn_gemm_act_takes": [P, I, P, P, P, I, I, I, I, I, I, I],
+            "dn_gemm_act": [P, I, P, P, P, I, I, I, I, I, I, P, I, I, P],
             "dn_gemm_plain_qkv_takes": [P, I, P, I, I, I, I],
             "dn_gemm_plain_qkv": [P, I, P, P, P, I, I, I, I, I, P, P, P, I, I, I, I, P, c_longlong, P],
             "dn_pack_matrix": [P, P, I, I, P],
@@ -530,6 +532,36 @@ def linear(a, w, bias=None, out=None, epilogue="none", residual=None):
                              _CODE[a.dtype], _CODE[out.dtype], epi, packed, _ptr(work), work_floats, _stream()),
         "linear" if _timed is None else f"linear {K} -> {N}" + (f", {epilogue}" if epi else ""))
     return out
+
+
+ACT_EPILOGUES = {"xielu": 4, "silu": 5, "exp_neg_softplus": 6}
+
+
+def linear_act(a, w, kind, out, bias=None, numbers=None, cols=None):
+    """out = act(a @ w.T + bias) in one kernel, for the activations of `activate` that have numbers of their own: "xielu" (numbers:
+    (a, b); bfloat16 out), "silu" of the first `cols` columns, the others as they are (32-bit out), "exp_neg_softplus" (numbers: the rates,
+    one a column; 32-bit out).  -> whether it did: False, and nothing written, where no kernel takes these operands (the caller then
+    runs `linear` and `activate`)."""
+    if not isinstance(w, PackedMatrix):
+        return False
+    M, K = a.shape
+    lda, N, packed = _operands(a, w, "linear_act")
+    _dev(out, "out", (torch.bfloat16,) if kind == "xielu" else (torch.float32,), 2)
+    _need(tuple(out.shape) == (M, N), "linear_act: out shape")
+    if bias is not None:
+        _f32vec(bias, "bias", N)
+    if kind != "silu":
+        _f32vec(numbers, "numbers", 2 if kind == "xielu" else N)
+    _need((cols is not None and 0 <= cols <= N) if kind == "silu" else numbers is not None, "linear_act: the activation's numbers")
+    if M == 0:
+        return True
+    lib, ldc, code = _lib_quiet("gemm"), _rows(out, "out"), ACT_EPILOGUES[kind]
+    if not lib.dn_gemm_act_takes(a.data_ptr(), lda, w.data_ptr(), _ptr(bias), out.data_ptr(), ldc, M, N, K, _CODE[out.dtype], code, packed):
+        return False
+    _ok(_lib("gemm").dn_gemm_act(a.data_ptr(), lda, w.data_ptr(), _ptr(bias), out.data_ptr(), ldc, M, N, K, _CODE[out.dtype], code,
+                                 _ptr(numbers) if kind != "silu" else 0, cols or 0, packed, _stream()),
+        "linear_act" if _timed is None else f"linear {K} -> {N}, {kind}")
+    return True
 
 
 def linear_deferred_shares(n_rows, w):

@@ -21,7 +21,8 @@ class DenseMLP(Part):
     product's epilogue, in 32-bit, before the rounding to the activation dtype.
 
     activation "xielu": z > 0: softplus(p) z^2 + z / 2; else (1/2 + softplus(q)) (e^z - 1 - z) + z / 2, with (p, q) the two
-    numbers of the tensor `activation_params`; it runs as a kernel of its own on the first product's 32-bit result.
+    numbers of the tensor `activation_params`; it runs in the first product's epilogue where a kernel has both, else as one of its own
+    on the product's 32-bit result.
     activation "poly_norm": s_1 n(z) + s_2 n(z^2) + s_3 n(z^3) + s_0 over the row of `inner` values, with s_1, s_2, s_3, s_0 the tensor's four
     numbers in this order, entrywise powers and n(v) = v / sqrt(mean(v^2) + eps); likewise a kernel of its own."""
     graph_safe = True
@@ -75,12 +76,16 @@ class DenseMLP(Part):
     def forward(self, h, ctx, accumulate_into, stats=None, deferred=None):
         n = h.shape[0]
         if self.activation in ACTIVATION_KERNELS:
-            z = self.up(h, out_dtype=F32)
-            f = torch.empty(z.shape, dtype=self.runtime.act_dtype, device=z.device)
-            if self.activation == "poly_norm":
-                ops.poly_norm(z, self.act_numbers, self.eps, f)
-            else:
-                ops.activate(z, self.activation, f, lower=self.act_numbers)
+            act, f = self.runtime.act_dtype, None
+            if self.activation == "xielu" and act == torch.bfloat16:
+                f = self.up.activated(h, "xielu", act, numbers=self.act_numbers)
+            if f is None:
+                z = self.up(h, out_dtype=F32)
+                f = torch.empty(z.shape, dtype=act, device=z.device)
+                if self.activation == "poly_norm":
+                    ops.poly_norm(z, self.act_numbers, self.eps, f)
+                else:
+                    ops.activate(z, self.activation, f, lower=self.act_numbers)
         else:
             f = self.up(h, out_dtype=self.runtime.act_dtype, epilogue=ACTIVATION_EPILOGUES[self.activation],
                         packed_out=self.up.few_rows(n) and self.down.packed_input(n) and accumulate_into is not None)

@@ -127,6 +127,14 @@ class Linear:
             out = torch.empty((a.shape[0], self.out_features), dtype=out_dtype or a.dtype, device=a.device)
         return ops.linear(a, self.weight, self.bias, out=out, epilogue=epilogue)
 
+    def activated(self, a, kind, out_dtype, bias=None, numbers=None, cols=None):
+        """ops.linear_act of the rows `a` with this weight and its bias (or the one given) as a new tensor of out_dtype, or None where
+        no kernel does both."""
+        if not isinstance(self.weight, ops.PackedMatrix) or a.dtype != self.weight.dtype:
+            return None
+        out = torch.empty((a.shape[0], self.out_features), dtype=out_dtype, device=a.device)
+        return out if ops.linear_act(a, self.weight, kind, out, bias=self.bias if bias is None else bias, numbers=numbers, cols=cols) else None
+
     def project_qkv(self, a, out_dtype, slot_map, k_pool, v_pool, q_width):
         """The fused projection: the key and value columns go to the cache's pages, the queries
         [M, q_width] come back (where one kernel does both, the other columns are stored nowhere else)."""

@@ -151,9 +151,10 @@ class Lightning(Part):
 
     def forward(self, h, ctx, cache, accumulate_into):
         act, T, qk, vw = self.runtime.act_dtype, h.shape[0], self.qk, self.vw
-        z = self.proj(h, out_dtype=F32)
-        qkv = z[:, :2 * qk + vw]
-        ops.activate(qkv, "silu", qkv)
+        z = self.proj.activated(h, "silu", F32, cols=2 * qk + vw)      # (q, k and v; the gate's columns as they are)
+        if z is None:
+            z = self.proj(h, out_dtype=F32)
+            ops.activate(z[:, :2 * qk + vw], "silu", z[:, :2 * qk + vw])
         o = torch.empty((T, vw), dtype=F32, device=h.device)
         ops.state_scan(z[:, :qk], z[:, qk:2 * qk], z[:, 2 * qk:2 * qk + vw], None, None, cache.state, ctx.row_start, ctx.state_slots,
                        self.n_heads, self.head_dim, self.value_dim, o, read_after=True, w_head=self.decay_t)
@@ -250,8 +251,10 @@ class ChannelDelta(Part):
         a_in, g_in = low[:, :self.decay_rank], low[:, self.decay_rank:]
         if not self._views_fit:      # (rows that the products cannot read where they lie)
             a_in, g_in = a_in.contiguous(), g_in.contiguous()
-        g = self.a2(a_in, out_dtype=F32)
-        ops.activate(g, "exp_neg_softplus", g, bias=self.dt_bias, lower=self.rate)
+        g = self.a2.activated(a_in, "exp_neg_softplus", F32, bias=self.dt_bias, numbers=self.rate)
+        if g is None:
+            g = self.a2(a_in, out_dtype=F32)
+            ops.activate(g, "exp_neg_softplus", g, bias=self.dt_bias, lower=self.rate)
         gate = self.g2(g_in, out_dtype=F32)
         o = torch.empty((T, vw), dtype=F32, device=dev)
         # (beta = sigmoid of the projection's columns behind the channels, taken inside the scan)
