@@ -31,6 +31,13 @@ __device__ __forceinline__ int first_key(int pos, int window, int chunk) {
   return lo;
 }
 
+// log2(page_size) where that is a power of two, else -1
+static int page_shift_of(int page_size) {
+  int shift = 0;
+  while ((1 << shift) < page_size) ++shift;
+  return (1 << shift) == page_size ? shift : -1;
+}
+
 // whether the row at `pos`, whose window begins at `lo`, reads `key`
 __device__ __forceinline__ bool reads_key(int key, int lo, int pos, int keep) { return key <= pos && (key >= lo || key < keep); }
 
@@ -296,6 +303,7 @@ __global__ __launch_bounds__(THREADS) void attention_kernel(
   }
 }
 
+constexpr int CUS = 256;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // The value of the lane 16 away inside each half of the wave (an exchange through the LDS crossbar, no memory).
@@ -306,30 +314,40 @@ __device__ __forceinline__ float other_row(float v) {
 // Portions, 32-bit, on the matrix cores: the sums of attention_kernel in the same order, so the same bits.
 // v_mfma_f32_16x16x4_f32 adds its four products one after the other, k ascending, each with one rounding and subnormals
 // kept: exactly key_dot's chain over the dims and dim_sum's over the keys.  attention_kernel reads two numbers from LDS a
-// multiply-add, which bounds it: two portions of 1,024 rows with 16 heads of 64 take it 778 us a layer and this one 129.
+// multiply-add, which bounds it: two portions of 1,024 rows with 16 heads of 64 take it 778 us a layer and this one 83: 133 with branches
+// around every score and its exponential and with the tiles of a head side by side (105 in the order below, which is of use with two
+// workgroups a CU and more: four such portions 209 -> 137, two with 25 heads 241 -> 129, three of 1,000 with 20 heads of 48 165 -> 115; the
+// branches: one portion 96 -> 75, eight of 16 to 160 rows 20.9 -> 17.4, three at positions 300 to 1,023 94 -> 78).
 // A workgroup is 64 rows of a wide tile (half = which 64), a wave 16 of them.  K . Q^T puts a row's scores on the four lanes
 // row, row + 16, row + 32, row + 48; the keys of a run of 16 go to the product's rows in the order 0 4 8 12 1 5 9 13 ..., so
 // that lane row + 16 q holds the keys 4 r + q in its register r: just what V^T . P^T wants as its second operand in step r.
 // Both operands wait in LDS with every 16 numbers that a product walks through turned 4 x 4, so that a lane reads its four
 // steps in one 16-byte load.  The next tile's keys and values wait in registers, the pages of the one after it too.
 // NDIM: head size / 16 (up to 8); the keys of a tile: tile_keys(head size).
-template <int NDIM>
+// EXTRAS: scores have a soft cap or a bias by distance (their branches per score, and one per exponential, were most of a tile's instructions:
+// a tile of 64 keys took a wave alone 14,000 cycles, 4,100 of them matrix instructions).
+template <int NDIM, bool EXTRAS>
 __global__ __launch_bounds__(256, 2) void portion_kernel(
     const float* __restrict__ q, int ldq, float* __restrict__ out, int ldo, const float* __restrict__ k_pool,
     const float* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_blocks,
     const int32_t* __restrict__ tile_seq, const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ tile_nrows,
-    const int32_t* __restrict__ tile_pos0, int H, int Hkv, int page_size, float scale, int window, ScoreExtras ex) {
+    const int32_t* __restrict__ tile_pos0, int H, int Hkv, int page_size, int page_shift, float scale, int window, ScoreExtras ex) {
   constexpr int DH = 16 * NDIM, BK = NDIM <= 4 ? 64 : 32, NC = BK / 16, KLD = DH + 4, VLD = BK + 4;
   __shared__ __attribute__((aligned(16))) float Ks[BK * KLD];
   __shared__ __attribute__((aligned(16))) float Vs[DH * VLD];
-  const int tile = blockIdx.x / 2, half = 1 - blockIdx.x % 2, h = blockIdx.y;     // (the half with more keys first)
+  // The tile table lists the longest contexts first; workgroups go through it tile by tile, all heads of a half together (the half with
+  // more keys first).  Where a CU gets two of them at once and no third, the second ones go through it backwards, a short one beside every
+  // long one.
+  const int all = gridDim.x, id = blockIdx.x, place = id >= CUS && all <= 2 * CUS ? all - 1 - (id - CUS) : id;
+  const int h = place % H, tile = place / H / 2, half = 1 - place / H % 2;
   const int seq = tile_seq[tile];
   const int nrows = min(64, tile_nrows[tile] - 64 * half);
   if (seq < 0 || nrows <= 0) return;
   const int row0 = tile_row0[tile] + 64 * half, pos0 = tile_pos0[tile] + 64 * half;
   const int hk = h / (H / Hkv);
   const int32_t* bt = block_tables + static_cast<size_t>(seq) * max_blocks;
-  const int t = threadIdx.x, lane = t % 64, w0 = t / 64 * 16;
+  // (the wave's number as a scalar: what follows from it is the scalar unit's work)
+  const int t = threadIdx.x, lane = t % 64, w0 = __builtin_amdgcn_readfirstlane(t / 64) * 16;
   const int i16 = lane % 16, quarter = lane / 16;
   const bool row_ok = w0 + i16 < nrows;
   const int pos = pos0 + w0 + i16;
@@ -337,7 +355,12 @@ __global__ __launch_bounds__(256, 2) void portion_kernel(
   const int last_pos = pos0 + nrows - 1;
   const int wave_last = pos0 + min(w0 + 16, nrows) - 1;      // (a wave without rows: below its own first)
   const bool wave_ok = w0 < nrows;
-  const float* bias = ex.bias ? ex.bias + static_cast<size_t>(h) * ex.span : nullptr;
+  const int wave_first = pos0 + w0, wave_lo = first_key(wave_last, window, ex.chunk);      // (no row of the wave begins later)
+  const float* bias = EXTRAS && ex.bias ? ex.bias + static_cast<size_t>(h) * ex.span : nullptr;
+  const float cap = EXTRAS ? ex.cap : 0.f;
+  // (a division by a number known only at run time is some twenty-five instructions)
+  auto page_index = [&](int key) { return page_shift >= 0 ? key >> page_shift : key / page_size; };
+  auto page_offset = [&](int key) { return page_shift >= 0 ? key & (page_size - 1) : key % page_size; };
   const float NEG_INF = -INFINITY;
 
   // the wave's queries: step s of the product over the dims reads dim 4 s + quarter
@@ -349,22 +372,22 @@ __global__ __launch_bounds__(256, 2) void portion_kernel(
   }
 
   // loader: 16 dims of a key, and 16 keys of a dim (one page: pages hold a multiple of 16 keys)
-  const bool loads = t < BK * NDIM;
+  const bool loads = BK * NDIM >= 256 || t < BK * NDIM;
   const int k_key = t / NDIM, k_a = t % NDIM, v_dim = t / NC, v_c = t % NC;
   const TileWalk walk(BK, first_key(pos0, window, ex.chunk), ex.keep);
-  auto page_of = [&](int key) { return loads && key <= last_pos ? bt[key / page_size] : -1; };
+  auto page_of = [&](int key) { return loads && key <= last_pos ? bt[page_index(key)] : -1; };
   float4 kr[4], vr[4];
   auto ask = [&](int kt, int k_page, int v_page) {
     const int kkey = kt + k_key, vkey = kt + 16 * v_c;
 #pragma unroll
     for (int b = 0; b < 4; ++b) kr[b] = vr[b] = float4{0.f, 0.f, 0.f, 0.f};
     if (k_page >= 0) {
-      const float* p = k_pool + ((static_cast<size_t>(k_page) * Hkv + hk) * page_size + kkey % page_size) * DH + 16 * k_a;
+      const float* p = k_pool + ((static_cast<size_t>(k_page) * Hkv + hk) * page_size + page_offset(kkey)) * DH + 16 * k_a;
 #pragma unroll
       for (int b = 0; b < 4; ++b) kr[b] = *reinterpret_cast<const float4*>(p + 4 * b);
     }
     if (v_page >= 0) {
-      const float* p = v_pool + ((static_cast<size_t>(v_page) * Hkv + hk) * DH + v_dim) * page_size + vkey % page_size;
+      const float* p = v_pool + ((static_cast<size_t>(v_page) * Hkv + hk) * DH + v_dim) * page_size + page_offset(vkey);
 #pragma unroll
       for (int b = 0; b < 4; ++b) vr[b] = *reinterpret_cast<const float4*>(p + 4 * b);
     }
@@ -421,15 +444,26 @@ __global__ __launch_bounds__(256, 2) void portion_kernel(
           s[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.w, qv[4 * a + 3], s[c], 0, 0, 0);
         }
       float m_t = NEG_INF;
+      if (kt + BK - 1 <= wave_first && kt >= wave_lo && w0 + 16 <= nrows) {      // every row reads every key of the tile
 #pragma unroll
-      for (int c = 0; c < NC; ++c)
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = kt + 16 * c + 4 * r + quarter;
-          const bool ok = row_ok && reads_key(key, lo, pos, ex.keep);
-          s[c][r] = ok ? score_of(s[c][r], scale, ex.cap, bias, pos - key, ex.span) : NEG_INF;
-          m_t = fmaxf(m_t, s[c][r]);
-        }
+          for (int r = 0; r < 4; ++r) {
+            s[c][r] = score_of(s[c][r], scale, cap, bias, pos - (kt + 16 * c + 4 * r + quarter), ex.span);
+            m_t = fmaxf(m_t, s[c][r]);
+          }
+      } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int key = kt + 16 * c + 4 * r + quarter;
+            // (worked out and not taken: a distance below 0 is no place in the bias)
+            const float score = score_of(s[c][r], scale, cap, bias, max(pos - key, 0), ex.span);
+            s[c][r] = row_ok & (key <= pos) & ((key >= lo) | (key < ex.keep)) ? score : NEG_INF;
+            m_t = fmaxf(m_t, s[c][r]);
+          }
+      }
       m_t = fmaxf(m_t, other_row(m_t));
       m_t = fmaxf(m_t, other_half(m_t));
       // the sum of p over the keys g, g + 16, ... for each g = 4 r + quarter, then the sixteen sums as group_reduce<16> joins them
@@ -439,7 +473,8 @@ __global__ __launch_bounds__(256, 2) void portion_kernel(
         float psum = 0.f;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-          s[c][r] = s[c][r] > NEG_INF ? expf(s[c][r] - m_t) : 0.f;
+          const float e = expf(s[c][r] - m_t);      // (not a number where the tile has no key for the row: not taken)
+          s[c][r] = s[c][r] > NEG_INF ? e : 0.f;
           psum += s[c][r];
         }
         psum += other_row(psum);
@@ -459,10 +494,7 @@ __global__ __launch_bounds__(256, 2) void portion_kernel(
           float4 v4 = *reinterpret_cast<const float4*>(vf + 16 * d * VLD + 16 * c);
           if (edge) {
             const int over = wave_last - (kt + 16 * c + quarter);
-            if (over < 0) v4.x = 0.f;
-            if (over < 4) v4.y = 0.f;
-            if (over < 8) v4.z = 0.f;
-            if (over < 12) v4.w = 0.f;
+            v4.x = over < 0 ? 0.f : v4.x, v4.y = over < 4 ? 0.f : v4.y, v4.z = over < 8 ? 0.f : v4.z, v4.w = over < 12 ? 0.f : v4.w;
           }
           a_t[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.x, s[c][0], a_t[d], 0, 0, 0);
           a_t[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4.y, s[c][1], a_t[d], 0, 0, 0);
@@ -876,12 +908,17 @@ extern "C" int dn_attention_portions(const void* q, int ldq, void* out, int ldo,
       reinterpret_cast<uintptr_t>(v_pool) % 16 != 0)
     return DN_ERR_SHAPE;
   const ScoreExtras ex{chunk, bias, span, sink, sink_at, keep, cap};
+#define DN_PORTION_KERNEL(ND, EXTRAS)                                                                                 \
+  hipLaunchKernelGGL((plain::portion_kernel<ND, EXTRAS>), dim3(2 * n_tiles * H), dim3(256), 0, stream,                \
+                     static_cast<const float*>(q), ldq, static_cast<float*>(out), ldo,                                \
+                     static_cast<const float*>(k_pool), static_cast<const float*>(v_pool), block_tables, max_blocks,   \
+                     tile_seq, tile_row0, tile_nrows, tile_pos0, H, Hkv, page_size, page_shift_of(page_size), scale, window, ex)
 #define DN_PORTION(ND)                                                                                                \
   case ND:                                                                                                            \
-    hipLaunchKernelGGL((plain::portion_kernel<ND>), dim3(2 * n_tiles, H), dim3(256), 0, stream,                       \
-                       static_cast<const float*>(q), ldq, static_cast<float*>(out), ldo,                              \
-                       static_cast<const float*>(k_pool), static_cast<const float*>(v_pool), block_tables, max_blocks, \
-                       tile_seq, tile_row0, tile_nrows, tile_pos0, H, Hkv, page_size, scale, window, ex);             \
+    if (bias || cap > 0.f)                                                                                            \
+      DN_PORTION_KERNEL(ND, true);                                                                                    \
+    else                                                                                                              \
+      DN_PORTION_KERNEL(ND, false);                                                                                   \
     break
   switch (dh / 16) {
     DN_PORTION(1);
@@ -894,6 +931,7 @@ extern "C" int dn_attention_portions(const void* q, int ldq, void* out, int ldo,
     DN_PORTION(8);
   }
 #undef DN_PORTION
+#undef DN_PORTION_KERNEL
   return dn_launch_status();
 }
 
