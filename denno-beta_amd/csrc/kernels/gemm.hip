@@ -98,15 +98,38 @@ extern "C" int dn_gemm_act(const void* A, int lda, const void* W, const float* b
                            int kind, const float* numbers, int cols, int packed, hipStream_t stream) {
   const int route = act_route(A, lda, W, bias, C, ldc, M, N, K, out_dtype, kind, packed);
   if (route == 0 || (kind != EPI_SILU && !numbers)) return DN_ERR_SHAPE;
-  const ActNumbers act{numbers, cols};
   if (route == 2) {
     direct::Args a{A, lda, W, bias, C, ldc, nullptr, 0, M, N, K, out_dtype, kind, packed, nullptr};
-    a.act = act;
+    a.act = numbers;
     const int rc = direct::run(a, stream);
     return rc != 0 ? rc : dn_launch_status();
   }
   skinny::Call c{A, lda, W, bias, C, ldc, nullptr, 0, M, N, K, out_dtype, kind, packed, nullptr};
-  c.act = act;
+  c.ends.p = numbers, c.ends.cols = kind == EPI_SILU ? cols : N;
+  skinny::run(c, stream);
+  return dn_launch_status();
+}
+
+// Two products of the same rows in one launch (up to 64 rows): C2 [M, n2] bfloat16 = A . W[:n2]^T, C [M, N - n2] 32-bit =
+// A . W[n2:]^T.  A launch of a decode step less (2 to 3 us; a product of 128 columns is little else).
+extern "C" int dn_gemm_two(const void* A, int lda, const void* W, void* C2, int ldc2, int n2, void* C, int ldc, int M, int N, int K,
+                           hipStream_t stream) {
+  if (M < 1 || M > 64 || n2 < 1 || n2 >= N || K < 8 || lda < K || ldc2 < n2 || ldc < N - n2 || !C2 || !C) return DN_ERR_SHAPE;
+  if (!skinny::takes(A, lda, W, M, K, PACKED_W)) return DN_ERR_SHAPE;
+  skinny::Call c{A, lda, W, nullptr, C, ldc, nullptr, 0, M, N, K, DN_F32, EPI_NONE, PACKED_W, nullptr};
+  c.ends.n2 = n2, c.ends.C2 = static_cast<bf16_t*>(C2), c.ends.ldc2 = ldc2;
+  skinny::run(c, stream);
+  return dn_launch_status();
+}
+
+// Two products of neighbouring columns of the same rows in one launch (up to 64 rows): C [M, N] 32-bit = [exp(-rate log(1 + e^z)) | A[:, K:2K] .
+// W[n1:]^T + bias[n1:]], z = A[:, :K] . W[:n1]^T + bias[:n1] (bias: N numbers, rate: n1; n1 a multiple of 64, K of 8).
+extern "C" int dn_gemm_pair(const void* A, int lda, const void* W, const float* bias, const float* rate, void* C, int ldc, int M, int N, int n1,
+                            int K, hipStream_t stream) {
+  if (M < 1 || M > 64 || n1 < 64 || n1 % 64 != 0 || n1 >= N || K < 8 || lda < 2 * K || ldc < N || !bias || !rate || !C) return DN_ERR_SHAPE;
+  if (!skinny::takes(A, lda, W, M, K, PACKED_W)) return DN_ERR_SHAPE;
+  skinny::Call c{A, lda, W, bias, C, ldc, nullptr, 0, M, N, K, DN_F32, EPI_EXP_NEG_SOFTPLUS, PACKED_W, nullptr};
+  c.ends.p = rate, c.ends.cols = n1, c.ends.a_from = n1, c.ends.a_shift = K;
   skinny::run(c, stream);
   return dn_launch_status();
 }

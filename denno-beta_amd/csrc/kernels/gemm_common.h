@@ -33,16 +33,22 @@ __device__ __forceinline__ float apply_epilogue_fast(float v, int epi) {
   return v;
 }
 
-// Activations with numbers of their own (dn_gemm_act), in place of a kernel between two products:
+// Activations with numbers of their own (dn_gemm_act), in place of a kernel between two products; columns from `cols` on have none:
 //   EPI_XIELU             v > 0: p[0] v^2 + v / 2; else p[1] (e^v - 1 - v) + v / 2     (bfloat16 results)
-//   EPI_SILU              v sigmoid(v) in the first `cols` columns, v in the others
+//   EPI_SILU              v sigmoid(v)
 //   EPI_EXP_NEG_SOFTPLUS  exp(-p[column] log(1 + e^v))
 #define EPI_XIELU 4
 #define EPI_SILU 5
 #define EPI_EXP_NEG_SOFTPLUS 6
-struct ActNumbers {
+// What else a product of few rows with 32-bit results may do: its first n2 columns go to C2 in bfloat16 and the others to C from
+// its first column on (dn_gemm_two); its columns from a_from on read A's columns from a_shift on (dn_gemm_pair).
+struct Ends {
   const float* p;
   int cols;
+  int n2;
+  bf16_t* C2;
+  int ldc2;
+  int a_from, a_shift;
 };
 
 // e^v - 1 - v for v <= 0 without its cancellation near 0: the series there (2e-7 of the result at most), the hardware's exponential
@@ -58,17 +64,18 @@ __device__ __forceinline__ float xielu_fast(float v, float a, float b) {
   return v > 0.f ? fmaf(a * v, v, 0.5f * v) : fmaf(b, v > -0.5f ? near : far, 0.5f * v);
 }
 
-// p, q: what act_numbers gives for the column
-__device__ __forceinline__ float apply_activation(float v, int epi, float p, float q) {
+// p, q: what act_first and act_second give for the column
+__device__ __forceinline__ float apply_activation(float v, int epi, int column, const Ends& ends, float p, float q) {
+  if (epi < EPI_XIELU) return apply_epilogue_fast(v, epi);
+  if (column >= ends.cols) return v;
   if (epi == EPI_XIELU) return xielu_fast(v, p, q);
-  if (epi == EPI_SILU) return p != 0.f ? v * sigmoid_f(v) : v;
-  if (epi == EPI_EXP_NEG_SOFTPLUS) return expf(-p * softplus_f(v));
-  return apply_epilogue_fast(v, epi);
+  if (epi == EPI_SILU) return v * sigmoid_f(v);
+  return expf(-p * softplus_f(v));
 }
-__device__ __forceinline__ float act_first(const ActNumbers& a, int epi, int column) {
-  return epi == EPI_SILU ? (column < a.cols ? 1.f : 0.f) : epi >= EPI_XIELU ? a.p[epi == EPI_EXP_NEG_SOFTPLUS ? column : 0] : 0.f;
+__device__ __forceinline__ float act_first(const Ends& ends, int epi, int column) {
+  return epi == EPI_XIELU ? ends.p[0] : epi == EPI_EXP_NEG_SOFTPLUS ? ends.p[min(column, ends.cols - 1)] : 0.f;
 }
-__device__ __forceinline__ float act_second(const ActNumbers& a, int epi) { return epi == EPI_XIELU ? a.p[1] : 0.f; }
+__device__ __forceinline__ float act_second(const Ends& ends, int epi) { return epi == EPI_XIELU ? ends.p[1] : 0.f; }
 
 // Where a fused projection's key and value columns go besides C: columns q_width .. of row m are
 // the keys, then the values, of the token whose slot is slot_map[m] (page * page_size + offset,
@@ -183,7 +190,7 @@ struct Call {
   const void* A; int lda; const void* W; const float* bias; void* C; int ldc; float* resid; int ldr;
   int M, N, K, out_dtype, epi, packed;
   const KVScatter* kv;
-  ActNumbers act{nullptr, 0};
+  Ends ends{};
 };
 bool takes(const void* A, int lda, const void* W, int M, int K, int packed);
 void run(const Call& c, hipStream_t stream);
@@ -201,7 +208,7 @@ namespace direct {
 struct Args {
   const void* A; int lda; const void* W; const float* bias; void* C; int ldc; float* resid; int ldr;
   int M, N, K, out_dtype, epi, packed; const KVScatter* kv;
-  ActNumbers act{nullptr, 0};                  // EPI_XIELU's numbers
+  const float* act = nullptr;                  // EPI_XIELU's numbers
   float* part = nullptr; int splits = 1;       // part: K in `splits` shares, their sums in part[share][m][n]
 };
 struct Shape { int bm, bn, stages; };

@@ -407,7 +407,7 @@ static int launch_kernel(const Args& a, hipStream_t stream) {
   hipLaunchKernelGGL((gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN, XIELU>), dim3(tiles_m * tiles_n, a.part ? a.splits : 1),
                      dim3(WM * WN * 64), lds, stream, static_cast<const bf16_t*>(a.A), a.lda,
                      static_cast<const bf16_t*>(a.W), a.bias, static_cast<TC*>(a.C), a.ldc, a.resid, a.ldr, a.M, a.N, a.K,
-                     a.epi, a.packed, tiles_m, tiles_n, a.kv ? *a.kv : KVScatter{}, a.part, split_slabs, a.act.p);
+                     a.epi, a.packed, tiles_m, tiles_n, a.kv ? *a.kv : KVScatter{}, a.part, split_slabs, a.act);
   return 0;
 }
 

@@ -108,6 +108,8 @@ def _declare(name, lib):
             "dn_gemm": [P, I, P, P, P, I, P, I, I, I, I, I, I, I, I, P, c_longlong, P],
             "dn_gemm_act_takes": [P, I, P, P, P, I, I, I, I, I, I, I],
             "dn_gemm_act": [P, I, P, P, P, I, I, I, I, I, I, P, I, I, P],
+            "dn_gemm_two": [P, I, P, P, I, I, P, I, I, I, I, P],
+            "dn_gemm_pair": [P, I, P, P, P, P, I, I, I, I, I, P],
             "dn_gemm_plain_qkv_takes": [P, I, P, I, I, I, I],
             "dn_gemm_plain_qkv": [P, I, P, P, P, I, I, I, I, I, P, P, P, I, I, I, I, P, c_longlong, P],
             "dn_pack_matrix": [P, P, I, I, P],
@@ -562,6 +564,50 @@ def linear_act(a, w, kind, out, bias=None, numbers=None, cols=None):
                                  _ptr(numbers) if kind != "silu" else 0, cols or 0, packed, _stream()),
         "linear_act" if _timed is None else f"linear {K} -> {N}, {kind}")
     return True
+
+
+def stacked(first, second):
+    """(both, first, second): two packed matrices with as many columns as each other, the second's rows behind the first's, and each again as
+    a view of that; None where they are not such (the first's rows are whole blocks of 16)."""
+    if not (isinstance(first, PackedMatrix) and isinstance(second, PackedMatrix)):
+        return None
+    if first.shape[1] != second.shape[1] or first.shape[0] % 16 != 0:
+        return None
+    data, n = torch.cat([first.data, second.data]), first.data.numel()
+    return (PackedMatrix(data, (first.shape[0] + second.shape[0], first.shape[1])), PackedMatrix(data[:n], first.shape),
+            PackedMatrix(data[n:], second.shape))
+
+
+FEW_ROWS_MAX = 64      # the rows up to which linear_two and linear_pair run
+
+
+def linear_two(a, w, n_first):
+    """(a @ w[:n_first].T in bfloat16, a @ w[n_first:].T in 32-bit), two products of the same up to 64 rows in one launch; w packed."""
+    M, K = a.shape
+    lda, N, packed = _operands(a, w, "linear_two")
+    _need(packed == PACKED_W and 1 <= M <= FEW_ROWS_MAX and 0 < n_first < N, lambda: f"linear_two: {M} rows x {tuple(w.shape)}, {n_first} first")
+    first = torch.empty((M, n_first), dtype=torch.bfloat16, device=a.device)
+    rest = torch.empty((M, N - n_first), dtype=torch.float32, device=a.device)
+    _ok(_lib("gemm").dn_gemm_two(a.data_ptr(), lda, w.data_ptr(), first.data_ptr(), n_first, n_first, rest.data_ptr(), N - n_first, M, N, K,
+                                 _stream()), "linear_two" if _timed is None else f"linear {K} -> {n_first} + {N - n_first}")
+    return first, rest
+
+
+def linear_pair(a, w, n_first, bias, rate):
+    """(exp(-rate * log(1 + e^z)), a[:, K:] @ w[n_first:].T + bias[n_first:]) with z = a[:, :K] @ w[:n_first].T + bias[:n_first], both
+    32-bit columns of one tensor, in one launch; a: up to 64 bfloat16 rows of 2K, w packed [N, K]; bias: N numbers, rate: n_first;
+    n_first a multiple of 64, K of 8."""
+    N, K = w.shape
+    M = a.shape[0]
+    _need(tuple(a.shape) == (M, 2 * K) and 1 <= M <= FEW_ROWS_MAX and 0 < n_first < N and n_first % 64 == 0 and K % 8 == 0,
+          lambda: f"linear_pair: rows {tuple(a.shape)} x {tuple(w.shape)}, {n_first} first")
+    lda, _, packed = _operands(a[:, :K], w, "linear_pair")
+    _need(packed == PACKED_W, "linear_pair: w must be packed")
+    _f32vec(bias, "bias", N), _f32vec(rate, "rate", n_first)
+    out = torch.empty((M, N), dtype=torch.float32, device=a.device)
+    _ok(_lib("gemm").dn_gemm_pair(a.data_ptr(), lda, w.data_ptr(), bias.data_ptr(), rate.data_ptr(), out.data_ptr(), N, M, N, n_first, K,
+                                  _stream()), "linear_pair" if _timed is None else f"linear 2 x {K} -> {n_first} + {N - n_first}")
+    return out[:, :n_first], out[:, n_first:]
 
 
 def linear_deferred_shares(n_rows, w):

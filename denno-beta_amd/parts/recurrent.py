@@ -232,13 +232,26 @@ class ChannelDelta(Part):
         # the second halves of the small products read columns of the first halves' rows where those start at 16 bytes
         per = 16 // (2 if self.a2.weight.dtype == torch.bfloat16 else 4)
         self._views_fit = self.decay_rank % per == 0 and (self.decay_rank + self.gate_rank) % per == 0
+        # steps of few rows run the two products that read h in one launch, and the two second halves where they are of one rank
+        self.both, self.halves = ops.stacked(self.low.weight, self.proj.weight), None
+        if self.both is not None:
+            self.both, self.low.weight, self.proj.weight = self.both
+        if self.decay_rank == self.gate_rank and self.decay_rank % 8 == 0 and self.gw % 64 == 0:
+            self.halves = ops.stacked(self.a2.weight, self.g2.weight)
+        if self.halves is not None:
+            self.halves, self.a2.weight, self.g2.weight = self.halves
+            self.halves_bias = torch.cat([self.dt_bias.reshape(-1), self.dt_bias.new_zeros(self.vw)])      # (the gate has none)
 
     def forward(self, h, ctx, cache, accumulate_into):
         act, T, dev = self.runtime.act_dtype, h.shape[0], h.device
         qk, vw, C, H = self.qk, self.vw, self.channels, self.n_heads
         n_state = self.gw * self.value_dim
         state, past = cache.state[:, :n_state], cache.state[:, n_state:]
-        z = self.proj(h, out_dtype=F32)
+        low, few = None, 0 < T <= ops.FEW_ROWS_MAX
+        if few and self.both is not None and h.dtype == torch.bfloat16:
+            low, z = ops.linear_two(h, self.both, self.low.out_features)
+        else:
+            z = self.proj(h, out_dtype=F32)
         x = torch.empty((T, C), dtype=F32, device=dev)
         # the three convolutions, silu, and queries and keys made unit vectors (the queries times dim^(-1/2)): one kernel
         single = ctx.single_rows and cache.writes
@@ -247,15 +260,19 @@ class ChannelDelta(Part):
         if self.taps > 1 and cache.writes and not single:
             ops.history_update(z[:, :C], past, ctx.row_start, ctx.state_slots)
         q, k, v = x[:, :qk], x[:, qk:2 * qk], x[:, 2 * qk:]
-        low = self.low(h, out_dtype=self.a2.weight.dtype)
-        a_in, g_in = low[:, :self.decay_rank], low[:, self.decay_rank:]
-        if not self._views_fit:      # (rows that the products cannot read where they lie)
-            a_in, g_in = a_in.contiguous(), g_in.contiguous()
-        g = self.a2.activated(a_in, "exp_neg_softplus", F32, bias=self.dt_bias, numbers=self.rate)
-        if g is None:
-            g = self.a2(a_in, out_dtype=F32)
-            ops.activate(g, "exp_neg_softplus", g, bias=self.dt_bias, lower=self.rate)
-        gate = self.g2(g_in, out_dtype=F32)
+        if low is None:
+            low = self.low(h, out_dtype=self.a2.weight.dtype)
+        if few and self.halves is not None and low.dtype == torch.bfloat16:
+            g, gate = ops.linear_pair(low, self.halves, self.gw, self.halves_bias, self.rate)
+        else:
+            a_in, g_in = low[:, :self.decay_rank], low[:, self.decay_rank:]
+            if not self._views_fit:      # (rows that the products cannot read where they lie)
+                a_in, g_in = a_in.contiguous(), g_in.contiguous()
+            g = self.a2.activated(a_in, "exp_neg_softplus", F32, bias=self.dt_bias, numbers=self.rate)
+            if g is None:
+                g = self.a2(a_in, out_dtype=F32)
+                ops.activate(g, "exp_neg_softplus", g, bias=self.dt_bias, lower=self.rate)
+            gate = self.g2(g_in, out_dtype=F32)
         o = torch.empty((T, vw), dtype=F32, device=dev)
         # (beta = sigmoid of the projection's columns behind the channels, taken inside the scan)
         ops.state_scan(q, k, v, g, None, state, ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, beta=z[:, C:C + H],

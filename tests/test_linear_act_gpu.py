@@ -70,3 +70,40 @@ def test_silu_and_decays_have_the_bits_of_two_kernels(M, N, K):
     assert did == (M <= 64)
     if did:
         assert torch.equal(out, ops.activate(z, "exp_neg_softplus", torch.empty_like(z), bias=bias, lower=rates))
+
+
+@pytest.mark.parametrize("M", [1, 2, 8, 9, 16, 17, 33, 64])
+@pytest.mark.parametrize("first,rest,K", [(128, 1544, 1024), (16, 3, 8), (64, 3000, 512), (80, 40000, 40)])
+def test_two_products_of_the_same_rows(M, first, rest, K):
+    from denno_beta_amd.kernels import ops
+    a, w1, _, make = _operands(M, first, K)
+    w2 = ops.pack_matrix((make(rest, K) * K ** -0.5).bfloat16())
+    both, v1, v2 = ops.stacked(w1, w2)
+    assert torch.equal(v1.rows(), w1.rows()) and torch.equal(v2.rows(), w2.rows()) and both.shape == (first + rest, K)
+    low, z = ops.linear_two(a, both, first)
+    # (the same kernel for both lays a sum out in another order only where K is cut among more waves)
+    one = ops.linear(a, both, out=torch.empty(M, first + rest, device="cuda"))
+    assert torch.equal(z, one[:, first:]) and torch.equal(low, one[:, :first].bfloat16())
+    assert torch.allclose(z, ops.linear(a, w2, out=torch.empty(M, rest, device="cuda")), rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("M", [1, 2, 8, 9, 16, 17, 33, 64])
+@pytest.mark.parametrize("n1,n2,K", [(512, 1024, 64), (64, 8, 8), (256, 2560, 72), (2560, 5120, 16)])
+def test_two_products_of_neighbouring_columns(M, n1, n2, K):
+    from denno_beta_amd.kernels import ops
+    _, w1, _, make = _operands(M, n1, K)
+    w2, low, rate, bias = ops.pack_matrix((make(n2, K) * K ** -0.5).bfloat16()), make(M, 2 * K).bfloat16(), make(n1).exp(), make(n1 + n2)
+    both = ops.stacked(w1, w2)[0]
+    g, gate = ops.linear_pair(low, both, n1, bias, rate)
+    z = ops.linear(low[:, :K], w1, out=torch.empty(M, n1, device="cuda"))
+    assert torch.allclose(g, ops.activate(z, "exp_neg_softplus", torch.empty_like(z), bias=bias[:n1], lower=rate), rtol=1e-5, atol=1e-6)
+    assert torch.allclose(gate, ops.linear(low[:, K:], w2, bias[n1:].contiguous(), out=torch.empty(M, n2, device="cuda")), rtol=1e-5, atol=1e-6)
+    with pytest.raises(Exception):      # (a bias for the first columns only: the kernel would read beyond it)
+        ops.linear_pair(low, both, n1, bias[:n1], rate)
+
+
+def test_matrices_that_do_not_stack():
+    from denno_beta_amd.kernels import ops
+    _, w1, _, make = _operands(1, 24, 64)      # (24 rows are one and a half blocks)
+    _, w2, _, _ = _operands(1, 16, 72)
+    assert ops.stacked(w1, w1) is None and ops.stacked(w2, w1) is None and ops.stacked(make(16, 64).bfloat16(), w1) is None
