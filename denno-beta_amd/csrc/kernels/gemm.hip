@@ -104,7 +104,8 @@ extern "C" int dn_gemm_act(const void* A, int lda, const void* W, const float* b
     const int rc = direct::run(a, stream);
     return rc != 0 ? rc : dn_launch_status();
   }
-  skinny::Call c{A, lda, W, bias, C, ldc, nullptr, 0, M, N, K, out_dtype, kind, packed, nullptr};
+  skinny::Call c{A, lda, W, bias, C, ldc, nullptr, 0, M, N, K, out_dtype, EPI_NONE, packed, nullptr};
+  c.end = kind == EPI_EXP_NEG_SOFTPLUS ? END_PAIR : END_ACT;
   c.ends.p = numbers, c.ends.cols = kind == EPI_SILU ? cols : N;
   skinny::run(c, stream);
   return dn_launch_status();
@@ -117,7 +118,8 @@ extern "C" int dn_gemm_two(const void* A, int lda, const void* W, void* C2, int 
   if (M < 1 || M > 64 || n2 < 1 || n2 >= N || K < 8 || lda < K || ldc2 < n2 || ldc < N - n2 || !C2 || !C) return DN_ERR_SHAPE;
   if (!skinny::takes(A, lda, W, M, K, PACKED_W)) return DN_ERR_SHAPE;
   skinny::Call c{A, lda, W, nullptr, C, ldc, nullptr, 0, M, N, K, DN_F32, EPI_NONE, PACKED_W, nullptr};
-  c.ends.n2 = n2, c.ends.C2 = static_cast<bf16_t*>(C2), c.ends.ldc2 = ldc2;
+  c.end = END_TWO;
+  c.ends.cols = n2, c.ends.C2 = static_cast<bf16_t*>(C2), c.ends.ldc2 = ldc2;
   skinny::run(c, stream);
   return dn_launch_status();
 }
@@ -128,8 +130,9 @@ extern "C" int dn_gemm_pair(const void* A, int lda, const void* W, const float* 
                             int K, hipStream_t stream) {
   if (M < 1 || M > 64 || n1 < 64 || n1 % 64 != 0 || n1 >= N || K < 8 || lda < 2 * K || ldc < N || !bias || !rate || !C) return DN_ERR_SHAPE;
   if (!skinny::takes(A, lda, W, M, K, PACKED_W)) return DN_ERR_SHAPE;
-  skinny::Call c{A, lda, W, bias, C, ldc, nullptr, 0, M, N, K, DN_F32, EPI_EXP_NEG_SOFTPLUS, PACKED_W, nullptr};
-  c.ends.p = rate, c.ends.cols = n1, c.ends.a_from = n1, c.ends.a_shift = K;
+  skinny::Call c{A, lda, W, bias, C, ldc, nullptr, 0, M, N, K, DN_F32, EPI_NONE, PACKED_W, nullptr};
+  c.end = END_PAIR;
+  c.ends.p = rate, c.ends.cols = n1, c.ends.a_shift = K;
   skinny::run(c, stream);
   return dn_launch_status();
 }

@@ -40,15 +40,17 @@ __device__ __forceinline__ float apply_epilogue_fast(float v, int epi) {
 #define EPI_XIELU 4
 #define EPI_SILU 5
 #define EPI_EXP_NEG_SOFTPLUS 6
-// What else a product of few rows with 32-bit results may do: its first n2 columns go to C2 in bfloat16 and the others to C from
-// its first column on (dn_gemm_two); its columns from a_from on read A's columns from a_shift on (dn_gemm_pair).
+// How a product of few rows ends beside the plain way; a kernel of its own each (the arguments and branches of these in the plain kernels cost
+// every product of few rows 0.15 to 0.4 us: 8 x 1,024 x 1,024 3.66 -> 3.86, 64 x 512 x 512 2.99 -> 3.45):
+//   END_ACT   bfloat16 results: EPI_XIELU; 32-bit results: EPI_SILU in the first `cols` columns
+//   END_TWO   32-bit results: the first `cols` columns go to C2 in bfloat16, the others to C from its first column on (dn_gemm_two)
+//   END_PAIR  32-bit results: EPI_EXP_NEG_SOFTPLUS in the first `cols` columns; those behind them read A's columns from a_shift on (dn_gemm_pair)
+constexpr int END_PLAIN = 0, END_ACT = 1, END_TWO = 2, END_PAIR = 3;
 struct Ends {
-  const float* p;
   int cols;
-  int n2;
+  const float* p;
   bf16_t* C2;
-  int ldc2;
-  int a_from, a_shift;
+  int ldc2, a_shift;
 };
 
 // e^v - 1 - v for v <= 0 without its cancellation near 0: the series there (2e-7 of the result at most), the hardware's exponential
@@ -64,18 +66,20 @@ __device__ __forceinline__ float xielu_fast(float v, float a, float b) {
   return v > 0.f ? fmaf(a * v, v, 0.5f * v) : fmaf(b, v > -0.5f ? near : far, 0.5f * v);
 }
 
-// p, q: what act_first and act_second give for the column
-__device__ __forceinline__ float apply_activation(float v, int epi, int column, const Ends& ends, float p, float q) {
-  if (epi < EPI_XIELU) return apply_epilogue_fast(v, epi);
-  if (column >= ends.cols) return v;
-  if (epi == EPI_XIELU) return xielu_fast(v, p, q);
-  if (epi == EPI_SILU) return v * sigmoid_f(v);
-  return expf(-p * softplus_f(v));
+// the numbers that an element's activation wants, asked for before the product, and the activation
+template <typename TC, int END, typename E>
+__device__ __forceinline__ float2 end_numbers(const E& ends, int column) {
+  if constexpr (END == END_ACT && sizeof(TC) == 2) return float2{ends.p[0], ends.p[1]};
+  if constexpr (END == END_PAIR) return float2{ends.p[min(column, ends.cols - 1)], 0.f};
+  return float2{0.f, 0.f};
 }
-__device__ __forceinline__ float act_first(const Ends& ends, int epi, int column) {
-  return epi == EPI_XIELU ? ends.p[0] : epi == EPI_EXP_NEG_SOFTPLUS ? ends.p[min(column, ends.cols - 1)] : 0.f;
+template <typename TC, int END, typename E>
+__device__ __forceinline__ float end_value(float v, int epi, int column, const E& ends, const float2& n) {
+  if constexpr (END == END_ACT && sizeof(TC) == 2) return xielu_fast(v, n.x, n.y);
+  if constexpr (END == END_ACT && sizeof(TC) == 4) return column < ends.cols ? v * sigmoid_f(v) : v;
+  if constexpr (END == END_PAIR) return column < ends.cols ? expf(-n.x * softplus_f(v)) : v;
+  return END == END_PLAIN ? apply_epilogue_fast(v, epi) : v;
 }
-__device__ __forceinline__ float act_second(const Ends& ends, int epi) { return epi == EPI_XIELU ? ends.p[1] : 0.f; }
 
 // Where a fused projection's key and value columns go besides C: columns q_width .. of row m are
 // the keys, then the values, of the token whose slot is slot_map[m] (page * page_size + offset,
@@ -190,6 +194,7 @@ struct Call {
   const void* A; int lda; const void* W; const float* bias; void* C; int ldc; float* resid; int ldr;
   int M, N, K, out_dtype, epi, packed;
   const KVScatter* kv;
+  int end = END_PLAIN;
   Ends ends{};
 };
 bool takes(const void* A, int lda, const void* W, int M, int K, int packed);

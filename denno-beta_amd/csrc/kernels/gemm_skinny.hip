@@ -29,21 +29,36 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 // taken off, not after: right where a row's mean is not large beside its spread.
 
 
+// what a kernel's last argument is (the plain kernels read none of it)
+template <int END>
+struct EndsFor {
+  typedef Ends type;
+};
+template <>
+struct EndsFor<END_PLAIN> {
+  struct type {
+    int none;
+    __host__ explicit type(const Ends&) : none(0) {}
+  };
+};
+template <int END>
+using EndsOf = typename EndsFor<END>::type;
+
 // MB row blocks and NB column blocks of 16 per workgroup; U steps of K in flight per wave.
-template <int MB, int NB, int WAVES, int U, typename TC, bool KV, int NORM = NORM_NONE>
+template <int MB, int NB, int WAVES, int U, typename TC, bool KV, int NORM = NORM_NONE, int END = END_PLAIN>
 __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restrict__ A, int lda,
                                                            const bf16_t* __restrict__ W,
                                                            const float* __restrict__ bias, TC* __restrict__ C,
                                                            int ldc, float* __restrict__ resid, int ldr, int M, int N,
-                                                           int K, int epi, int packed, KVScatter kv, NormIO nio, Ends ends) {
+                                                           int K, int epi, int packed, KVScatter kv, NormIO nio, EndsOf<END> ends) {
   constexpr int BLOCKS = MB * NB;                          // 16 x 16 blocks of C in this workgroup
   constexpr int PASSES = (BLOCKS + WAVES - 1) / WAVES;     // wave w finishes blocks w, w + WAVES, ...
   __shared__ floatx4 red[WAVES][BLOCKS][64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;   // (a scalar: what follows from it is the scalar unit's work)
   const int col = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * (16 * NB);
-  constexpr bool ACT = !KV && NORM == NORM_NONE && MB <= 4;      // (what has `ends` comes here with up to 64 rows)
-  if (ACT && n0 >= ends.a_from) A += ends.a_shift;
+  if constexpr (END == END_PAIR)
+    if (n0 >= ends.cols) A += ends.a_shift;
   const int row0 = blockIdx.y * (MB * 16);     // the rows may be shared out among workgroups too (blockIdx.y)
   const int ksteps = (K + 31) / 32, nblocks = (N + 15) / 16;
   const bf16_t* wblk[NB];
@@ -59,14 +74,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   float epi_bias[PASSES];
   float epi_x[PASSES][4];
   int epi_slot[KV ? PASSES : 1][4];
-  float epi_act[ACT ? PASSES : 1];
-  const float epi_act2 = ACT ? act_second(ends, epi) : 0.f;
+  float2 epi_act[END != END_PLAIN ? PASSES : 1];
   float epi_norm[NORM != NORM_NONE ? PASSES : 1];          // NORM_IN: c1 of the lane's column; NORM_OUT: the next norm's gamma
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) {
     const int blk = wave + p * WAVES;
     epi_bias[p] = 0.f;
-    if constexpr (ACT) epi_act[p] = 0.f;
+    if constexpr (END != END_PLAIN) epi_act[p] = float2{0.f, 0.f};
     if constexpr (NORM != NORM_NONE) {
       const int nn = min(n0 + (blk < BLOCKS ? blk % NB : 0) * 16 + col, N - 1);
       epi_norm[p] = NORM == NORM_IN ? nio.c1[nn] : nio.gamma_out[nn];
@@ -81,7 +95,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
       const int mb = blk / NB, nb = blk % NB;
       const int nn = min(n0 + nb * 16 + col, N - 1);
       if (bias) epi_bias[p] = bias[nn];
-      if constexpr (ACT) epi_act[p] = act_first(ends, epi, nn);
+      if constexpr (END != END_PLAIN) epi_act[p] = end_numbers<TC, END>(ends, nn);
       if constexpr (KV) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -250,15 +264,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
           nio.copy_out[nio.ldcopy > 0 ? static_cast<size_t>(m) * nio.ldcopy + nn : packed_index(m, nn, N / 32)] =
               from_float<bf16_t>((epi_x[p][r] + v) * epi_norm[p]);
       } else {
-        TC cv = from_float<TC>(ACT ? apply_activation(v, epi, nn, ends, epi_act[ACT ? p : 0], epi_act2) : apply_epilogue_fast(v, epi));
-        if constexpr (ACT && sizeof(TC) == 4) {
-          if (ends.n2 > 0) {
-            if (nn < ends.n2)
-              ends.C2[static_cast<size_t>(m) * ends.ldc2 + nn] = from_float<bf16_t>(v);
-            else
-              C[static_cast<size_t>(m) * ldc + nn - ends.n2] = cv;
-            continue;
-          }
+        TC cv = from_float<TC>(end_value<TC, END>(v, epi, nn, ends, epi_act[END != END_PLAIN ? p : 0]));
+        if constexpr (END == END_TWO) {
+          if (nn < ends.cols)
+            ends.C2[static_cast<size_t>(m) * ends.ldc2 + nn] = from_float<bf16_t>(v);
+          else
+            C[static_cast<size_t>(m) * ldc + nn - ends.cols] = cv;
+          continue;
         }
         if (!KV || nn < kv.c_cols)
           C[(packed & PACKED_C) ? packed_index(m, nn, N / 32) : static_cast<size_t>(m) * ldc + nn] = cv;
@@ -276,12 +288,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
 // of its own (no barrier: a wave's LDS operations keep their order) and reads the operands from
 // there, two pairs at a time through two such pieces, so that the way into LDS and out of it is
 // waited for once per two pairs.  16 columns per workgroup, sums joined through LDS in wave order, as in gemm_kernel.
-template <int WAVES, typename TC, bool KV, int NORM, bool TWO>
+template <int WAVES, typename TC, bool KV, int NORM, bool TWO, int END = END_PLAIN>
 __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __restrict__ A, int lda,
                                                              const bf16_t* __restrict__ W,
                                                              const float* __restrict__ bias, TC* __restrict__ C,
                                                              int ldc, float* __restrict__ resid, int ldr, int M,
-                                                             int N, int K, int epi, KVScatter kv, NormIO nio, Ends ends) {
+                                                             int N, int K, int epi, KVScatter kv, NormIO nio, EndsOf<END> ends) {
   typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
   constexpr int U = 4;                                     // pairs of steps in flight per wave
   constexpr int ROW = 9 * 8;                               // elements per row of a wave's piece: 8 chunks and one of padding
@@ -292,8 +304,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int col = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * 16;
-  constexpr bool ACT = !KV && NORM == NORM_NONE;
-  if (ACT && n0 >= ends.a_from) A += ends.a_shift;
+  if constexpr (END == END_PAIR)
+    if (n0 >= ends.cols) A += ends.a_shift;
   const int ksteps = (K + 31) / 32, npairs = (ksteps + 1) / 2, nblocks = (N + 15) / 16;
   const bf16_t* wblk = W + (static_cast<size_t>(min(static_cast<int>(blockIdx.x), nblocks - 1)) * ksteps * 64 + lane) * 8;
   // (TWO: rows 8 .. 15 need a second load per pair)
@@ -305,11 +317,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   float epi_bias = 0.f;
   float epi_x[4] = {0.f, 0.f, 0.f, 0.f};
   int epi_slot[4] = {-1, -1, -1, -1};
-  float epi_act = 0.f, epi_act2 = 0.f;
+  float2 epi_act{0.f, 0.f};
   if (wave == 0) {
     const int nn = min(n0 + col, N - 1);
     if (bias) epi_bias = bias[nn];
-    if constexpr (ACT) epi_act = act_first(ends, epi, nn), epi_act2 = act_second(ends, epi);
+    if constexpr (END != END_PLAIN) epi_act = end_numbers<TC, END>(ends, nn);
     if constexpr (KV) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) epi_slot[r] = g * 4 + r < M ? kv.slot_map[g * 4 + r] : -1;
@@ -440,15 +452,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
         if constexpr (NORM == NORM_OUT)
           nio.copy_out[static_cast<size_t>(m) * nio.ldcopy + nn] = from_float<bf16_t>((epi_x[r] + v) * epi_gamma);
       } else {
-        const TC cv = from_float<TC>(ACT ? apply_activation(v, epi, nn, ends, epi_act, epi_act2) : apply_epilogue_fast(v, epi));
-        if constexpr (ACT && sizeof(TC) == 4) {
-          if (ends.n2 > 0) {
-            if (nn < ends.n2)
-              ends.C2[static_cast<size_t>(m) * ends.ldc2 + nn] = from_float<bf16_t>(v);
-            else
-              C[static_cast<size_t>(m) * ldc + nn - ends.n2] = cv;
-            continue;
-          }
+        const TC cv = from_float<TC>(end_value<TC, END>(v, epi, nn, ends, epi_act));
+        if constexpr (END == END_TWO) {
+          if (nn < ends.cols)
+            ends.C2[static_cast<size_t>(m) * ends.ldc2 + nn] = from_float<bf16_t>(v);
+          else
+            C[static_cast<size_t>(m) * ldc + nn - ends.cols] = cv;
+          continue;
         }
         if (!KV || nn < kv.c_cols) C[static_cast<size_t>(m) * ldc + nn] = cv;
         if constexpr (KV) scatter_kv_at(kv, epi_slot[r], nn, cv);
@@ -471,14 +481,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
 }
 
 
-template <int MB, int NB, int WAVES, int U, typename TC, bool KV>
+template <int MB, int NB, int WAVES, int U, typename TC, bool KV, int END = END_PLAIN>
 static void launch_one(const Call& c, hipStream_t stream) {
   // (MB row blocks per workgroup: where the rows need more, the second grid dimension shares them out)
   dim3 grid((c.N + 16 * NB - 1) / (16 * NB), ((c.M + 15) / 16 + MB - 1) / MB), block(WAVES * 64);
   KVScatter kv = c.kv ? *c.kv : KVScatter{};
-  hipLaunchKernelGGL((gemm_kernel<MB, NB, WAVES, U, TC, KV>), grid, block, 0, stream,
+  hipLaunchKernelGGL((gemm_kernel<MB, NB, WAVES, U, TC, KV, NORM_NONE, END>), grid, block, 0, stream,
                      static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,
-                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, NormIO{}, c.ends);
+                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, NormIO{}, EndsOf<END>(c.ends));
 }
 
 // the same with the norm before the product (NORM_IN: bfloat16 out) or after it (NORM_OUT: into the
@@ -490,7 +500,7 @@ static void launch_norm(const Call& c, const NormIO& nio, int norm, hipStream_t 
 #define DN_LN(TC, KV, NORM)                                                                                        \
   hipLaunchKernelGGL((gemm_kernel<MB, NB, WAVES, U, TC, KV, NORM>), grid, block, 0, stream,                       \
                      static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,             \
-                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, nio, c.ends)
+                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, nio, EndsOf<END_PLAIN>(c.ends))
   if (norm == NORM_OUT)
     DN_LN(float, false, NORM_OUT);
   else if (c.kv)
@@ -518,22 +528,29 @@ void launch_mb_norm(const Call& c, const NormIO& nio, int norm, hipStream_t stre
 
 template <int MB, int NB, int WAVES, int U>
 static void launch(const Call& c, hipStream_t stream) {
+  if constexpr (MB <= 4) {      // (up to 64 rows: what the entry points take)
+    if (c.end == END_ACT && c.out_dtype == DN_BF16) return launch_one<MB, NB, WAVES, U, bf16_t, false, END_ACT>(c, stream);
+    if (c.end == END_ACT) return launch_one<MB, NB, WAVES, U, float, false, END_ACT>(c, stream);
+    if (c.end == END_TWO) return launch_one<MB, NB, WAVES, U, float, false, END_TWO>(c, stream);
+    if (c.end == END_PAIR) return launch_one<MB, NB, WAVES, U, float, false, END_PAIR>(c, stream);
+  }
   if (c.kv) return launch_one<MB, NB, WAVES, U, bf16_t, true>(c, stream);
   if (c.out_dtype == DN_BF16) return launch_one<MB, NB, WAVES, U, bf16_t, false>(c, stream);
   return launch_one<MB, NB, WAVES, U, float, false>(c, stream);
 }
 
-template <int WAVES, typename TC, bool KV>
+template <int WAVES, typename TC, bool KV, int END = END_PLAIN>
 static void launch16_one(const Call& c, hipStream_t stream) {
   KVScatter kv = c.kv ? *c.kv : KVScatter{};
+#define DN_L16_ONE(TWO)                                                                                                 \
+  hipLaunchKernelGGL((gemm16_kernel<WAVES, TC, KV, NORM_NONE, TWO, END>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0,   \
+                     stream, static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,           \
+                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, NormIO{}, EndsOf<END>(c.ends))
   if (c.M > 8)
-    hipLaunchKernelGGL((gemm16_kernel<WAVES, TC, KV, NORM_NONE, true>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0, stream,
-                       static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,
-                       static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, NormIO{}, c.ends);
+    DN_L16_ONE(true);
   else
-    hipLaunchKernelGGL((gemm16_kernel<WAVES, TC, KV, NORM_NONE, false>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0, stream,
-                       static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,
-                       static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, NormIO{}, c.ends);
+    DN_L16_ONE(false);
+#undef DN_L16_ONE
 }
 
 // the same with the norm before the product (NORM_IN: bfloat16 out) or after it (NORM_OUT: into the residual stream)
@@ -544,7 +561,7 @@ static void launch16_norm(const Call& c, const NormIO& nio, int norm, hipStream_
 #define DN_L16_ROWS(TC, KV, NORM, TWO)                                                                                   \
   hipLaunchKernelGGL((gemm16_kernel<WAVES, TC, KV, NORM, TWO>), grid, block, 0, stream, static_cast<const bf16_t*>(c.A), \
                      c.lda, static_cast<const bf16_t*>(c.W), c.bias, static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr,       \
-                     c.M, c.N, c.K, c.epi, kv, nio, c.ends)
+                     c.M, c.N, c.K, c.epi, kv, nio, EndsOf<END_PLAIN>(c.ends))
 #define DN_L16(TC, KV, NORM)                 \
   do {                                       \
     if (c.M > 8)                             \
@@ -564,6 +581,10 @@ static void launch16_norm(const Call& c, const NormIO& nio, int norm, hipStream_
 
 template <int WAVES>
 static void launch16(const Call& c, hipStream_t stream) {
+  if (c.end == END_ACT && c.out_dtype == DN_BF16) return launch16_one<WAVES, bf16_t, false, END_ACT>(c, stream);
+  if (c.end == END_ACT) return launch16_one<WAVES, float, false, END_ACT>(c, stream);
+  if (c.end == END_TWO) return launch16_one<WAVES, float, false, END_TWO>(c, stream);
+  if (c.end == END_PAIR) return launch16_one<WAVES, float, false, END_PAIR>(c, stream);
   if (c.kv) return launch16_one<WAVES, bf16_t, true>(c, stream);
   if (c.out_dtype == DN_BF16) return launch16_one<WAVES, bf16_t, false>(c, stream);
   return launch16_one<WAVES, float, false>(c, stream);
