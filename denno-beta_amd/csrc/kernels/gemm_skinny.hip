@@ -174,9 +174,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
       for (int i = 0; i < SP; ++i)
         if (lane + 64 * i < nio.blocks_in) {
           const float d = st[t][i].x - mean;
-          sq += st[t][i].y + 16.f * d * d;
+          sq += st[t][i].y + nio.block * d * d;
         }
-      const float var = wave_sum(sq) / (16.f * blocks);
+      const float var = wave_sum(sq) / (nio.block * blocks);
       if (lane == 0) {
         rowstat[row][0] = row0 + row < M ? mean : 0.f;
         rowstat[row][1] = row0 + row < M ? 1.0f / sqrtf(var + nio.eps) : 0.f;
@@ -420,9 +420,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
       for (int i = 0; i < SP; ++i)
         if (lane + 64 * i < nio.blocks_in) {
           const float d = st[t][i].x - mean;
-          sq += st[t][i].y + 16.f * d * d;
+          sq += st[t][i].y + nio.block * d * d;
         }
-      const float var = wave_sum(sq) / (16.f * blocks);
+      const float var = wave_sum(sq) / (nio.block * blocks);
       if (lane == 0) {
         rowstat[row][0] = row < M ? mean : 0.f;
         rowstat[row][1] = row < M ? 1.0f / sqrtf(var + nio.eps) : 0.f;
@@ -477,6 +477,109 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
           *reinterpret_cast<float2*>(nio.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x) * 2) = float2{mean, sq};
       }
     }
+  }
+}
+
+
+// Up to 8 rows of a product with few columns: gemm16_kernel with 8 columns a workgroup.  A CU takes 50 to 60 GB/s of what its XCD's L2 does not
+// hold, whatever it asks for ahead, so a workgroup of 16 columns waits for its own share of W (205 KB at K = 6,400) while half of the
+// CUs have none.  A pair of steps is one load of W: lanes l % 16 < 8 bring 8 columns of the first step, the others the same
+// columns of the second.  The product of the second step takes them with the halves of every 16 lanes exchanged; what columns 8 .. 15 of the
+// results add up to is nothing and is dropped.  A column's sums are gemm16_kernel's, in its order: the same bits.  A lane ends one element.
+constexpr int ROW_ROTATE_8 = 0x128;      // (DPP: lane i of each 16 takes from lane i - 8 of the same 16)
+template <int WAVES, int U, typename TC, int NORM>
+__global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
+                                                            const float* __restrict__ bias, TC* __restrict__ C, int ldc,
+                                                            float* __restrict__ resid, int ldr, int M, int N, int K, int epi,
+                                                            NormIO nio) {
+  typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+  constexpr int ROW = 9 * 8;                               // elements per row of a wave's piece: 8 chunks and one of padding
+  constexpr int PIECES = U < 2 ? 1 : 2;                    // pairs turned round at a time
+  __shared__ floatx4 red[WAVES][64];
+  __shared__ __attribute__((aligned(16))) bf16_t turn[WAVES][PIECES][8 * ROW];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const int col = lane % 16, g = lane / 16, second = col / 8;
+  const int n0 = blockIdx.x * 8, nn = n0 + lane % 8, mm = lane / 8;      // (the element that a lane of the first wave ends)
+  const int ksteps = (K + 31) / 32, npairs = (ksteps + 1) / 2;
+  const bf16_t* wblk = W + (static_cast<size_t>(blockIdx.x / 2) * ksteps * 64 + g * 16 + (blockIdx.x % 2) * 8 + col % 8) * 8;
+  // what the epilogue will read is asked for first of all
+  float epi_bias = 0.f, epi_x = 0.f, epi_gamma = 1.f;
+  if (wave == 0) {
+    const int c = min(nn, N - 1);
+    if (bias) epi_bias = bias[c];
+    if (resid) epi_x = resid[static_cast<size_t>(min(mm, M - 1)) * ldr + c];
+    if constexpr (NORM == NORM_OUT) epi_gamma = nio.gamma_out[c];
+  }
+  // never a conditional load; a step beyond K reads W's first block and meets zeros of A, whose chunks beyond K come from the row's start
+  const int lrow = lane / 8, lch = lane % 8;               // as loader: row and 16-byte chunk of the pair's 128 bytes
+  const bf16_t* asafe = A + static_cast<size_t>(min(lrow, M - 1)) * lda;
+  const bf16_t* a0 = asafe + lch * 8;
+  bf16_t* mine = turn[wave][0];
+  const u32x4 zero4 = {0u, 0u, 0u, 0u};
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int p0 = wave; p0 < npairs; p0 += WAVES * U) {
+    u32x4 b[U], al[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int step = 2 * (p0 + u * WAVES) + second;
+      b[u] = *reinterpret_cast<const u32x4*>(step < ksteps ? wblk + static_cast<size_t>(step) * 512 : W + lane * 8);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + u * WAVES;
+      al[u] = *reinterpret_cast<const u32x4*>(p * 64 + lch * 8 < K ? a0 + p * 64 : asafe);
+    }
+#pragma unroll
+    for (int u0 = 0; u0 < U; u0 += PIECES) {
+#pragma unroll
+      for (int i = 0; i < PIECES && u0 + i < U; ++i) {
+        const int p = p0 + (u0 + i) * WAVES;
+        *reinterpret_cast<u32x4*>(mine + i * 8 * ROW + lrow * ROW + lch * 8) = p < npairs && p * 64 + lch * 8 < K ? al[u0 + i] : zero4;
+      }
+      // as operand: lane (row col, chunk g) of each of a pair's two steps; rows 8 .. 15 are the others again, their results nothing's
+      bf16x8 f[PIECES][2];
+#pragma unroll
+      for (int i = 0; i < PIECES && u0 + i < U; ++i) {
+        const bf16_t* piece = mine + i * 8 * ROW + (col % 8) * ROW;
+        f[i][0] = *reinterpret_cast<const bf16x8*>(piece + g * 8);
+        f[i][1] = *reinterpret_cast<const bf16x8*>(piece + (4 + g) * 8);
+      }
+#pragma unroll
+      for (int i = 0; i < PIECES && u0 + i < U; ++i) {
+        u32x4 other;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          other[e] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b[u0 + i][e]), ROW_ROTATE_8, 0xf, 0xf, true));
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i][0], __builtin_bit_cast(bf16x8, b[u0 + i]), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i][1], __builtin_bit_cast(bf16x8, other), acc, 0, 0, 0);
+      }
+    }
+  }
+  red[wave][lane] = acc;
+  __syncthreads();
+  // acc[r] of lane (col, g) is row g*4 + r, column n0 + col
+  if (wave > 0) return;
+  const float* at = reinterpret_cast<const float*>(&red[0][(mm / 4) * 16 + lane % 8]) + mm % 4;
+  float sum = at[0];
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) sum += at[w * 64 * 4];
+  const float v = sum + epi_bias;
+  if constexpr (NORM == NORM_OUT) {
+    // a row's 8 columns lie in 8 lanes side by side (N is a multiple of 16)
+    const float x = epi_x + v;
+    const float mean = group_reduce<8>(x, SumOp()) * (1.0f / 8.0f);
+    const float d = x - mean;
+    const float sq = group_reduce<8>(d * d, SumOp());
+    if (lane % 8 == 0 && mm < M)
+      *reinterpret_cast<float2*>(nio.stats_out + (static_cast<size_t>(mm) * gridDim.x + blockIdx.x) * 2) = float2{mean, sq};
+  }
+  if (mm >= M || nn >= N) return;
+  if (resid) {
+    resid[static_cast<size_t>(mm) * ldr + nn] = epi_x + v;
+    if constexpr (NORM == NORM_OUT)
+      nio.copy_out[static_cast<size_t>(mm) * nio.ldcopy + nn] = from_float<bf16_t>((epi_x + v) * epi_gamma);
+  } else {
+    C[static_cast<size_t>(mm) * ldc + nn] = from_float<TC>(apply_epilogue_fast(v, epi));
   }
 }
 
@@ -553,6 +656,37 @@ static void launch16_one(const Call& c, hipStream_t stream) {
 #undef DN_L16_ONE
 }
 
+// Where gemm8_kernel runs: up to 8 rows of at most 2,048 columns, whose 256 workgroups the chip has CUs for (beyond, 16 columns a workgroup
+// give every CU its own too, and read A half as often: 2,304 columns from K = 9,216 at 8 rows 13.6 us so, 16 to 17 in eights).
+bool eight_columns(int M, int N) { return M <= 8 && N <= 2048; }
+
+// The pairs in flight per wave are as many as make its share of K whole rounds: loads of what is not there cost as much as the others
+// (1,024 x 1,024 at 8 rows 3.1 us with 2, 3.5 with 4, 4.2 with 8; 1,024 x 4,096 5.1, 4.8, 4.8; 1,600 x 6,400 9.3, 9.2, 8.3 and 8.1 with 6).
+// gemm16_kernel -> this, with the next norm's statistics, 1 and 8 rows: 1,024 x 1,024 3.7 -> 3.0 and 4.2 -> 3.1 us, 1,600 x 1,600 3.9 -> 3.7 and 4.3 -> 3.8,
+// 1,024 x 4,096 5.0 -> 4.5 and 5.6 -> 4.8, 1,600 x 6,400 8.8 -> 7.6 and 10.1 -> 8.1, 2,048 x 8,192 10.2 -> 8.8 and 11.9 -> 9.6.
+template <int WAVES, typename TC, int NORM>
+static void launch8(const Call& c, const NormIO& nio, hipStream_t stream) {
+  constexpr int MOST = 8;
+  const int share = ((c.K + 63) / 64 + WAVES - 1) / WAVES, rounds = (share + MOST - 1) / MOST;
+#define DN_L8(U)                                                                                                                          \
+  case U:                                                                                                                                 \
+    hipLaunchKernelGGL((gemm8_kernel<WAVES, U, TC, NORM>), dim3((c.N + 7) / 8), dim3(WAVES * 64), 0, stream, static_cast<const bf16_t*>(c.A), \
+                       c.lda, static_cast<const bf16_t*>(c.W), c.bias, static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K,       \
+                       c.epi, nio);                                                                                                       \
+    break
+  switch ((share + rounds - 1) / rounds) {
+    DN_L8(1);
+    DN_L8(2);
+    DN_L8(3);
+    DN_L8(4);
+    DN_L8(5);
+    DN_L8(6);
+    DN_L8(7);
+    DN_L8(8);
+  }
+#undef DN_L8
+}
+
 // the same with the norm before the product (NORM_IN: bfloat16 out) or after it (NORM_OUT: into the residual stream)
 template <int WAVES>
 static void launch16_norm(const Call& c, const NormIO& nio, int norm, hipStream_t stream) {
@@ -569,7 +703,9 @@ static void launch16_norm(const Call& c, const NormIO& nio, int norm, hipStream_
     else                                     \
       DN_L16_ROWS(TC, KV, NORM, false);      \
   } while (0)
-  if (norm == NORM_OUT)
+  if (norm == NORM_OUT && nio.block == 8.f)
+    launch8<WAVES, float, NORM_OUT>(c, nio, stream);
+  else if (norm == NORM_OUT)
     DN_L16(float, false, NORM_OUT);
   else if (c.kv)
     DN_L16(bf16_t, true, NORM_IN);
@@ -601,6 +737,10 @@ static void launch_mb(const Call& c, hipStream_t stream) {
   // column blocks per workgroup, the rows shared out among workgroups (at 1,600 x 1,600: 6.7 us at 128 rows and 8.0
   // at 256, where sixteen row blocks x one column block took 7.7 and 12.6: every workgroup read all rows)
   if (mb > 4 && c.N < 2048 && c.K < 4096) return launch<4, 2, WAVES, 4>(c, stream);
+  if (mb == 1 && !(c.packed & (PACKED_A | PACKED_C)) && eight_columns(c.M, c.N) && !c.kv && c.end == END_PLAIN) {
+    if (c.out_dtype == DN_BF16 && !c.resid) return launch8<WAVES, bf16_t, NORM_NONE>(c, NormIO{}, stream);
+    return launch8<WAVES, float, NORM_NONE>(c, NormIO{}, stream);
+  }
   if (mb == 1 && !(c.packed & (PACKED_A | PACKED_C)) && c.M > 1) return launch16<WAVES>(c, stream);
   if (mb == 1) return launch<1, 1, WAVES, 8>(c, stream);
   if (mb > 4) {
