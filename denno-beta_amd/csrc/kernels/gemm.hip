@@ -215,7 +215,7 @@ extern "C" int dn_gemm_norm_out(const void* A, int lda, const void* W, const flo
   const int packed = PACKED_W | (lda == 0 ? PACKED_A : 0);
   if (!skinny::takes(A, lda, W, M, K, packed)) return DN_ERR_SHAPE;
   skinny::Call c{A, lda, W, bias, nullptr, 0, resid, ldr, M, N, K, DN_F32, EPI_NONE, packed, nullptr};
-  skinny::NormIO nio{nullptr, 0, nullptr, 0.f, 0, gamma, static_cast<bf16_t*>(copy), ldcopy, stats, static_cast<float>(block)};
+  skinny::NormIO nio{nullptr, block, nullptr, 0.f, 0, gamma, static_cast<bf16_t*>(copy), ldcopy, stats};
   if (M > 16)
     skinny::launch_mb_norm(c, nio, NORM_OUT, stream);
   else
@@ -253,7 +253,7 @@ extern "C" int dn_gemm_norm_in(const void* A, int lda, const float* stats, const
   }
   skinny::Call c{A, lda, W, c2, C, ldc, nullptr, 0, M, N, K, DN_BF16, epilogue, packed | (ldc == 0 ? PACKED_C : 0),
                  slot_map ? &kv : nullptr};
-  skinny::NormIO nio{stats, K / block, c1, eps, no_mean ? 1 : 0, nullptr, nullptr, 0, nullptr, static_cast<float>(block)};
+  skinny::NormIO nio{stats, K / block, c1, eps, no_mean ? 1 : 0, nullptr, nullptr, 0, nullptr};
   if (M > 16)
     skinny::launch_mb_norm(c, nio, NORM_IN, stream);
   else

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   // wave does it in its first turn of the loop below, which every wave has: K >= 1024); the finishing
   // waves meet them behind the barrier further down
   auto join_stats = [&]() {
-    const float blocks = static_cast<float>(nio.blocks_in);
+    const float blocks = static_cast<float>(nio.blocks_in), wide = nio.blocks_in * 16 == K ? 16.f : 8.f;      // pairs of statistics a row, columns a pair
 #pragma unroll
     for (int t = 0; t < SR; ++t) {
       const int row = wave + t * WAVES;
@@ -174,9 +174,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
       for (int i = 0; i < SP; ++i)
         if (lane + 64 * i < nio.blocks_in) {
           const float d = st[t][i].x - mean;
-          sq += st[t][i].y + nio.block * d * d;
+          sq += st[t][i].y + wide * d * d;
         }
-      const float var = wave_sum(sq) / (nio.block * blocks);
+      const float var = wave_sum(sq) / (wide * blocks);
       if (lane == 0) {
         rowstat[row][0] = row0 + row < M ? mean : 0.f;
         rowstat[row][1] = row0 + row < M ? 1.0f / sqrtf(var + nio.eps) : 0.f;
@@ -288,18 +288,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
 // of its own (no barrier: a wave's LDS operations keep their order) and reads the operands from
 // there, two pairs at a time through two such pieces, so that the way into LDS and out of it is
 // waited for once per two pairs.  16 columns per workgroup, sums joined through LDS in wave order, as in gemm_kernel.
-template <int WAVES, typename TC, bool KV, int NORM, bool TWO, int END = END_PLAIN>
+template <int WAVES, int U, typename TC, bool KV, int NORM, bool TWO, int END = END_PLAIN>
 __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __restrict__ A, int lda,
                                                              const bf16_t* __restrict__ W,
                                                              const float* __restrict__ bias, TC* __restrict__ C,
                                                              int ldc, float* __restrict__ resid, int ldr, int M,
                                                              int N, int K, int epi, KVScatter kv, NormIO nio, EndsOf<END> ends) {
   typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
-  constexpr int U = 4;                                     // pairs of steps in flight per wave
   constexpr int ROW = 9 * 8;                               // elements per row of a wave's piece: 8 chunks and one of padding
   __shared__ floatx4 red[WAVES][64];
-  constexpr int PIECES = 2;                                // pairs turned round at a time
-  static_assert(U % PIECES == 0, "pairs in flight come in whole groups");
+  constexpr int PIECES = U < 2 ? 1 : 2;                    // pairs turned round at a time
   __shared__ __attribute__((aligned(16))) bf16_t turn[WAVES][PIECES][16 * ROW];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int col = lane % 16, g = lane / 16;
@@ -376,7 +374,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
 #pragma unroll
     for (int u0 = 0; u0 < U; u0 += PIECES) {
 #pragma unroll
-      for (int i = 0; i < PIECES; ++i) {
+      for (int i = 0; i < PIECES && u0 + i < U; ++i) {
         const int p = p0 + (u0 + i) * WAVES;
         const bool ok = p < npairs && p * 64 + lch * 8 < K;
         bf16_t* piece = mine + i * 16 * ROW;
@@ -386,13 +384,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
       // as operand: lane (row col, chunk g) of each of a pair's two steps
       bf16x8 f[PIECES][2];
 #pragma unroll
-      for (int i = 0; i < PIECES; ++i) {
+      for (int i = 0; i < PIECES && u0 + i < U; ++i) {
         const bf16_t* piece = mine + i * 16 * ROW;
         f[i][0] = *reinterpret_cast<const bf16x8*>(piece + col * ROW + g * 8);
         f[i][1] = *reinterpret_cast<const bf16x8*>(piece + col * ROW + (4 + g) * 8);
       }
 #pragma unroll
-      for (int i = 0; i < PIECES; ++i) {
+      for (int i = 0; i < PIECES && u0 + i < U; ++i) {
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i][0], b[u0 + i][0], acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i][1], b[u0 + i][1], acc, 0, 0, 0);
       }
@@ -406,7 +404,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   if (NORM == NORM_IN || wave < npairs) ask(wave, b0, al0);
   if constexpr (NORM == NORM_IN) {
     // the rows' means and 1 / sqrt(var + eps) for wave 0, which meets them behind the barrier further down
-    const float blocks = static_cast<float>(nio.blocks_in);
+    const float blocks = static_cast<float>(nio.blocks_in), wide = nio.blocks_in * 16 == K ? 16.f : 8.f;      // pairs of statistics a row, columns a pair
 #pragma unroll
     for (int t = 0; t < SR; ++t) {
       const int row = wave + t * WAVES;
@@ -420,9 +418,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
       for (int i = 0; i < SP; ++i)
         if (lane + 64 * i < nio.blocks_in) {
           const float d = st[t][i].x - mean;
-          sq += st[t][i].y + nio.block * d * d;
+          sq += st[t][i].y + wide * d * d;
         }
-      const float var = wave_sum(sq) / (nio.block * blocks);
+      const float var = wave_sum(sq) / (wide * blocks);
       if (lane == 0) {
         rowstat[row][0] = row < M ? mean : 0.f;
         rowstat[row][1] = row < M ? 1.0f / sqrtf(var + nio.eps) : 0.f;
@@ -526,15 +524,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int p = p0 + u * WAVES;
-      al[u] = *reinterpret_cast<const u32x4*>(p * 64 + lch * 8 < K ? a0 + p * 64 : asafe);
+      const int at = p0 + u * WAVES;
+      al[u] = *reinterpret_cast<const u32x4*>(at * 64 + lch * 8 < K ? a0 + at * 64 : asafe);
     }
 #pragma unroll
     for (int u0 = 0; u0 < U; u0 += PIECES) {
 #pragma unroll
       for (int i = 0; i < PIECES && u0 + i < U; ++i) {
-        const int p = p0 + (u0 + i) * WAVES;
-        *reinterpret_cast<u32x4*>(mine + i * 8 * ROW + lrow * ROW + lch * 8) = p < npairs && p * 64 + lch * 8 < K ? al[u0 + i] : zero4;
+        const int pair = p0 + (u0 + i) * WAVES;
+        *reinterpret_cast<u32x4*>(mine + i * 8 * ROW + lrow * ROW + lch * 8) = pair < npairs && pair * 64 + lch * 8 < K ? al[u0 + i] : zero4;
       }
       // as operand: lane (row col, chunk g) of each of a pair's two steps; rows 8 .. 15 are the others again, their results nothing's
       bf16x8 f[PIECES][2];
@@ -642,18 +640,38 @@ static void launch(const Call& c, hipStream_t stream) {
   return launch_one<MB, NB, WAVES, U, float, false>(c, stream);
 }
 
-template <int WAVES, typename TC, bool KV, int END = END_PLAIN>
-static void launch16_one(const Call& c, hipStream_t stream) {
+// the pairs in flight per wave that make its share of K whole rounds of at most `most` (loads of what is not there cost as much as the
+// others)
+template <int WAVES>
+static int pairs_ahead(int K, int most) {
+  const int share = ((K + 63) / 64 + WAVES - 1) / WAVES, rounds = (share + most - 1) / most;
+  return (share + rounds - 1) / rounds;
+}
+
+// Four pairs ahead at most.  (Always four before -> as many as the share wants, 8 rows: 4,096 x 1,024 4.3 -> 4.0 us, 50,257 x 1,024 27.5 -> 23.8,
+// x 1,280 31.8 -> 28.7, 32,000 x 1,024 18.7 -> 16.0; with the norm before, 3,072 x 1,024 4.6 -> 4.3, 5,120 x 1,280 6.9 -> 6.6; K = 1,600 and 2,048 level.)
+template <int WAVES, int U, typename TC, bool KV, int NORM, int END>
+static void launch16_ahead(const Call& c, const NormIO& nio, hipStream_t stream) {
   KVScatter kv = c.kv ? *c.kv : KVScatter{};
-#define DN_L16_ONE(TWO)                                                                                                 \
-  hipLaunchKernelGGL((gemm16_kernel<WAVES, TC, KV, NORM_NONE, TWO, END>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0,   \
-                     stream, static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,           \
-                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, NormIO{}, EndsOf<END>(c.ends))
+#define DN_L16(TWO)                                                                                                       \
+  hipLaunchKernelGGL((gemm16_kernel<WAVES, U, TC, KV, NORM, TWO, END>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0,       \
+                     stream, static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,             \
+                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, nio, EndsOf<END>(c.ends))
   if (c.M > 8)
-    DN_L16_ONE(true);
+    DN_L16(true);
   else
-    DN_L16_ONE(false);
-#undef DN_L16_ONE
+    DN_L16(false);
+#undef DN_L16
+}
+
+template <int WAVES, typename TC, bool KV, int NORM = NORM_NONE, int END = END_PLAIN>
+static void launch16_one(const Call& c, const NormIO& nio, hipStream_t stream) {
+  switch (pairs_ahead<WAVES>(c.K, 4)) {
+    case 1: return launch16_ahead<WAVES, 1, TC, KV, NORM, END>(c, nio, stream);
+    case 2: return launch16_ahead<WAVES, 2, TC, KV, NORM, END>(c, nio, stream);
+    case 3: return launch16_ahead<WAVES, 3, TC, KV, NORM, END>(c, nio, stream);
+    default: return launch16_ahead<WAVES, 4, TC, KV, NORM, END>(c, nio, stream);
+  }
 }
 
 // Where gemm8_kernel runs: up to 8 rows of at most 2,048 columns, whose 256 workgroups the chip has CUs for (beyond, 16 columns a workgroup
@@ -666,15 +684,13 @@ bool eight_columns(int M, int N) { return M <= 8 && N <= 2048; }
 // 1,024 x 4,096 5.0 -> 4.5 and 5.6 -> 4.8, 1,600 x 6,400 8.8 -> 7.6 and 10.1 -> 8.1, 2,048 x 8,192 10.2 -> 8.8 and 11.9 -> 9.6.
 template <int WAVES, typename TC, int NORM>
 static void launch8(const Call& c, const NormIO& nio, hipStream_t stream) {
-  constexpr int MOST = 8;
-  const int share = ((c.K + 63) / 64 + WAVES - 1) / WAVES, rounds = (share + MOST - 1) / MOST;
-#define DN_L8(U)                                                                                                                          \
-  case U:                                                                                                                                 \
-    hipLaunchKernelGGL((gemm8_kernel<WAVES, U, TC, NORM>), dim3((c.N + 7) / 8), dim3(WAVES * 64), 0, stream, static_cast<const bf16_t*>(c.A), \
-                       c.lda, static_cast<const bf16_t*>(c.W), c.bias, static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K,       \
-                       c.epi, nio);                                                                                                       \
+#define DN_L8(U)                                                                                                          \
+  case U:                                                                                                                 \
+    hipLaunchKernelGGL((gemm8_kernel<WAVES, U, TC, NORM>), dim3((c.N + 7) / 8), dim3(WAVES * 64), 0, stream,              \
+                       static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,                   \
+                       static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, nio);                          \
     break
-  switch ((share + rounds - 1) / rounds) {
+  switch (pairs_ahead<WAVES>(c.K, 8)) {
     DN_L8(1);
     DN_L8(2);
     DN_L8(3);
@@ -690,40 +706,22 @@ static void launch8(const Call& c, const NormIO& nio, hipStream_t stream) {
 // the same with the norm before the product (NORM_IN: bfloat16 out) or after it (NORM_OUT: into the residual stream)
 template <int WAVES>
 static void launch16_norm(const Call& c, const NormIO& nio, int norm, hipStream_t stream) {
-  KVScatter kv = c.kv ? *c.kv : KVScatter{};
-  const dim3 grid((c.N + 15) / 16), block(WAVES * 64);
-#define DN_L16_ROWS(TC, KV, NORM, TWO)                                                                                   \
-  hipLaunchKernelGGL((gemm16_kernel<WAVES, TC, KV, NORM, TWO>), grid, block, 0, stream, static_cast<const bf16_t*>(c.A), \
-                     c.lda, static_cast<const bf16_t*>(c.W), c.bias, static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr,       \
-                     c.M, c.N, c.K, c.epi, kv, nio, EndsOf<END_PLAIN>(c.ends))
-#define DN_L16(TC, KV, NORM)                 \
-  do {                                       \
-    if (c.M > 8)                             \
-      DN_L16_ROWS(TC, KV, NORM, true);       \
-    else                                     \
-      DN_L16_ROWS(TC, KV, NORM, false);      \
-  } while (0)
-  if (norm == NORM_OUT && nio.block == 8.f)
-    launch8<WAVES, float, NORM_OUT>(c, nio, stream);
-  else if (norm == NORM_OUT)
-    DN_L16(float, false, NORM_OUT);
-  else if (c.kv)
-    DN_L16(bf16_t, true, NORM_IN);
-  else
-    DN_L16(bf16_t, false, NORM_IN);
-#undef DN_L16
-#undef DN_L16_ROWS
+  if (norm == NORM_OUT && nio.blocks_in == 8) return launch8<WAVES, float, NORM_OUT>(c, nio, stream);
+  if (norm == NORM_OUT) return launch16_one<WAVES, float, false, NORM_OUT>(c, nio, stream);
+  if (c.kv) return launch16_one<WAVES, bf16_t, true, NORM_IN>(c, nio, stream);
+  return launch16_one<WAVES, bf16_t, false, NORM_IN>(c, nio, stream);
 }
 
 template <int WAVES>
 static void launch16(const Call& c, hipStream_t stream) {
-  if (c.end == END_ACT && c.out_dtype == DN_BF16) return launch16_one<WAVES, bf16_t, false, END_ACT>(c, stream);
-  if (c.end == END_ACT) return launch16_one<WAVES, float, false, END_ACT>(c, stream);
-  if (c.end == END_TWO) return launch16_one<WAVES, float, false, END_TWO>(c, stream);
-  if (c.end == END_PAIR) return launch16_one<WAVES, float, false, END_PAIR>(c, stream);
-  if (c.kv) return launch16_one<WAVES, bf16_t, true>(c, stream);
-  if (c.out_dtype == DN_BF16) return launch16_one<WAVES, bf16_t, false>(c, stream);
-  return launch16_one<WAVES, float, false>(c, stream);
+  const NormIO none{};
+  if (c.end == END_ACT && c.out_dtype == DN_BF16) return launch16_one<WAVES, bf16_t, false, NORM_NONE, END_ACT>(c, none, stream);
+  if (c.end == END_ACT) return launch16_one<WAVES, float, false, NORM_NONE, END_ACT>(c, none, stream);
+  if (c.end == END_TWO) return launch16_one<WAVES, float, false, NORM_NONE, END_TWO>(c, none, stream);
+  if (c.end == END_PAIR) return launch16_one<WAVES, float, false, NORM_NONE, END_PAIR>(c, none, stream);
+  if (c.kv) return launch16_one<WAVES, bf16_t, true>(c, none, stream);
+  if (c.out_dtype == DN_BF16) return launch16_one<WAVES, bf16_t, false>(c, none, stream);
+  return launch16_one<WAVES, float, false>(c, none, stream);
 }
 
 // With more than 16 rows every workgroup reads all of A (16 cache lines per load and 16 lanes,
