@@ -280,6 +280,57 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   }
 }
 
+// The arguments of the two kernels below.  The first 14 words come in scalar registers with the launch, the others by a trip to memory that
+// every wave makes before it can ask for anything they name (two cache lines of arguments more made a product 0.4 us slower): so what the first
+// loads want stands in front, packed: `rows` is the rows and three flags; p is the statistics (NORM_IN), else what the results go to
+// or are added to; q is the slot map (NORM_IN), else the leading dimension of p (a pointer in any case: through a pointer made from a number the
+// compiler loads by instructions that are waited for one by one, 0.5 us more).
+// In this order the operands' loads leave 0.2 to 0.5 us sooner, 8 rows: with the norm before, 3,072 x 1,024 4.3 -> 4.0 us, 5,120 x 1,280 6.6 -> 6.1,
+// 6,400 x 1,600 7.6 -> 7.2; with the norm after, 1,024 x 1,024 3.1 -> 3.0, 1,280 x 5,120 6.4 -> 6.0, 1,600 x 6,400 8.1 -> 7.6; 50,257 x 1,024 23.8 -> 23.0.
+constexpr int FIRST_ROWS = 255, FIRST_ADDS = 256, FIRST_EIGHTS = 512;      // (NORM_IN: statistics by blocks of 8 columns)
+template <int END>
+struct Late {
+  void* C;      // NORM_IN
+  int ldc, epi;
+  const float* c1;
+  float eps;
+  int no_mean;
+  const float* gamma_out;
+  bf16_t* copy_out;
+  float* stats_out;
+  int ldcopy;
+  KVScatter kv;
+  EndsOf<END> ends;
+};
+
+// Brings what the epilogue takes from `late` into scalar registers here, behind the first loads of the operands (left to the compiler these
+// arguments were fetched where they are used, at the kernel's end, and the trip to memory came on top: a q | k | v of 4,800 columns 7.8 us for 7.2).
+template <int NORM, bool KV, int END>
+__device__ __forceinline__ void late_at_hand(const Late<END>& late) {
+  if constexpr (NORM == NORM_IN) asm volatile("" ::"s"(late.C), "s"(late.ldc), "s"(late.eps), "s"(late.no_mean));
+  if constexpr (NORM == NORM_OUT) asm volatile("" ::"s"(late.copy_out), "s"(late.stats_out), "s"(late.ldcopy));
+  if constexpr (NORM != NORM_OUT) asm volatile("" ::"s"(late.epi));
+  if constexpr (KV)
+    asm volatile("" ::"s"(late.kv.k_pool), "s"(late.kv.v_pool), "s"(late.kv.q_width), "s"(late.kv.page_size), "s"(late.kv.c_cols));
+  if constexpr (END == END_TWO) asm volatile("" ::"s"(late.ends.C2), "s"(late.ends.ldc2), "s"(late.ends.cols));
+}
+
+struct First {
+  int rows;
+  const void* p;
+  const void* q;
+};
+static First first_of(const Call& c, const NormIO& nio, int norm) {
+  if (norm == NORM_IN)
+    return First{c.M | (nio.blocks_in * 16 == c.K ? 0 : FIRST_EIGHTS), nio.stats_in, c.kv ? c.kv->slot_map : nullptr};
+  return First{c.M | (c.resid ? FIRST_ADDS : 0), c.resid ? static_cast<const void*>(c.resid) : c.C, reinterpret_cast<const void*>(static_cast<uintptr_t>(c.resid ? c.ldr : c.ldc))};
+}
+template <int END>
+static Late<END> late_of(const Call& c, const NormIO& nio) {
+  return Late<END>{c.C, c.ldc, c.epi, nio.c1, nio.eps, nio.no_mean, nio.gamma_out, nio.copy_out, nio.stats_out, nio.ldcopy,
+                   c.kv ? *c.kv : KVScatter{}, EndsOf<END>(c.ends)};
+}
+
 // Up to 16 rows of A in rows.  In the operands' layout 16 lanes are 16 rows, and a load of A from
 // memory touches as many cache lines (four times as many lookups as the packed W costs, and they
 // were what this product of 8 rows waited for).  Here a wave takes the steps of K in pairs
@@ -289,12 +340,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
 // there, two pairs at a time through two such pieces, so that the way into LDS and out of it is
 // waited for once per two pairs.  16 columns per workgroup, sums joined through LDS in wave order, as in gemm_kernel.
 template <int WAVES, int U, typename TC, bool KV, int NORM, bool TWO, int END = END_PLAIN>
-__global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __restrict__ A, int lda,
-                                                             const bf16_t* __restrict__ W,
-                                                             const float* __restrict__ bias, TC* __restrict__ C,
-                                                             int ldc, float* __restrict__ resid, int ldr, int M,
-                                                             int N, int K, int epi, KVScatter kv, NormIO nio, EndsOf<END> ends) {
+__global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int rows, int N,
+                                                             int K, const void* __restrict__ p, const float* __restrict__ bias, const void* __restrict__ q,
+                                                             Late<END> late) {
   typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+  const int M = rows & FIRST_ROWS;
+  TC* C = static_cast<TC*>(NORM == NORM_IN ? late.C : const_cast<void*>(p));
+  float* resid = NORM != NORM_IN && (rows & FIRST_ADDS) ? static_cast<float*>(const_cast<void*>(p)) : nullptr;
+  const int ldc = NORM == NORM_IN ? late.ldc : static_cast<int>(reinterpret_cast<uintptr_t>(q)), ldr = ldc;
+  const float* stats_in = static_cast<const float*>(p);
+  const int32_t* slot_map = NORM == NORM_IN ? static_cast<const int32_t*>(q) : late.kv.slot_map;
   constexpr int ROW = 9 * 8;                               // elements per row of a wave's piece: 8 chunks and one of padding
   __shared__ floatx4 red[WAVES][64];
   constexpr int PIECES = U < 2 ? 1 : 2;                    // pairs turned round at a time
@@ -303,7 +358,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   const int col = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * 16;
   if constexpr (END == END_PAIR)
-    if (n0 >= ends.cols) A += ends.a_shift;
+    if (n0 >= late.ends.cols) A += late.ends.a_shift;
   const int ksteps = (K + 31) / 32, npairs = (ksteps + 1) / 2, nblocks = (N + 15) / 16;
   const bf16_t* wblk = W + (static_cast<size_t>(min(static_cast<int>(blockIdx.x), nblocks - 1)) * ksteps * 64 + lane) * 8;
   // (TWO: rows 8 .. 15 need a second load per pair)
@@ -316,13 +371,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   float epi_x[4] = {0.f, 0.f, 0.f, 0.f};
   int epi_slot[4] = {-1, -1, -1, -1};
   float2 epi_act{0.f, 0.f};
+  const int blocks_in = rows & FIRST_EIGHTS ? K / 8 : K / 16;      // (NORM_IN)
   if (wave == 0) {
     const int nn = min(n0 + col, N - 1);
     if (bias) epi_bias = bias[nn];
-    if constexpr (END != END_PLAIN) epi_act = end_numbers<TC, END>(ends, nn);
     if constexpr (KV) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) epi_slot[r] = g * 4 + r < M ? kv.slot_map[g * 4 + r] : -1;
+      for (int r = 0; r < 4; ++r) epi_slot[r] = g * 4 + r < M ? slot_map[g * 4 + r] : -1;
     }
     if (resid) {
 #pragma unroll
@@ -338,11 +393,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
       const int row = min(wave + t * WAVES, M - 1);
 #pragma unroll
       for (int i = 0; i < SP; ++i)
-        st[t][i] = *reinterpret_cast<const float2*>(nio.stats_in + (static_cast<size_t>(row) * nio.blocks_in + min(lane + 64 * i, nio.blocks_in - 1)) * 2);
+        st[t][i] = *reinterpret_cast<const float2*>(stats_in + (static_cast<size_t>(row) * blocks_in + min(lane + 64 * i, blocks_in - 1)) * 2);
     }
-    epi_c1 = nio.c1[min(n0 + col, N - 1)];
   }
-  if constexpr (NORM == NORM_OUT) epi_gamma = nio.gamma_out[min(n0 + col, N - 1)];
   // never a conditional load; a step beyond K reads W's first block and meets zeros of A
   const int lrow = lane / 8, lch = lane % 8;               // as loader: row and 16-byte chunk of the pair's 128 bytes
   const bf16_t* a0 = A + static_cast<size_t>(min(lrow, M - 1)) * lda + lch * 8;
@@ -402,28 +455,34 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   // wait for the statistics, which were asked for before, counts these loads exactly and depends on
   // no branch), and the rows' statistics are joined while it travels
   if (NORM == NORM_IN || wave < npairs) ask(wave, b0, al0);
+  // what the epilogue reads by arguments that do not come with the launch (`Late`): behind the operands, which do not wait for those
+  const int late_column = min(n0 + col, N - 1);
+  if constexpr (NORM == NORM_IN) epi_c1 = late.c1[late_column];
+  if constexpr (NORM == NORM_OUT) epi_gamma = late.gamma_out[late_column];
+  if constexpr (END != END_PLAIN) epi_act = end_numbers<TC, END>(late.ends, late_column);
+  late_at_hand<NORM, KV>(late);
   if constexpr (NORM == NORM_IN) {
     // the rows' means and 1 / sqrt(var + eps) for wave 0, which meets them behind the barrier further down
-    const float blocks = static_cast<float>(nio.blocks_in), wide = nio.blocks_in * 16 == K ? 16.f : 8.f;      // pairs of statistics a row, columns a pair
+    const float blocks = static_cast<float>(blocks_in), wide = rows & FIRST_EIGHTS ? 8.f : 16.f;      // pairs of statistics a row, columns a pair
 #pragma unroll
     for (int t = 0; t < SR; ++t) {
       const int row = wave + t * WAVES;
       float sm = 0.f;
 #pragma unroll
       for (int i = 0; i < SP; ++i)
-        if (lane + 64 * i < nio.blocks_in) sm += st[t][i].x;
-      const float mean = nio.no_mean ? 0.f : wave_sum(sm) / blocks;      // (without it the squares are taken about 0)
+        if (lane + 64 * i < blocks_in) sm += st[t][i].x;
+      const float mean = late.no_mean ? 0.f : wave_sum(sm) / blocks;      // (without it the squares are taken about 0)
       float sq = 0.f;
 #pragma unroll
       for (int i = 0; i < SP; ++i)
-        if (lane + 64 * i < nio.blocks_in) {
+        if (lane + 64 * i < blocks_in) {
           const float d = st[t][i].x - mean;
           sq += st[t][i].y + wide * d * d;
         }
       const float var = wave_sum(sq) / (wide * blocks);
       if (lane == 0) {
         rowstat[row][0] = row < M ? mean : 0.f;
-        rowstat[row][1] = row < M ? 1.0f / sqrtf(var + nio.eps) : 0.f;
+        rowstat[row][1] = row < M ? 1.0f / sqrtf(var + late.eps) : 0.f;
       }
     }
   }
@@ -448,18 +507,18 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
       if (resid) {
         resid[static_cast<size_t>(m) * ldr + nn] = epi_x[r] + v;
         if constexpr (NORM == NORM_OUT)
-          nio.copy_out[static_cast<size_t>(m) * nio.ldcopy + nn] = from_float<bf16_t>((epi_x[r] + v) * epi_gamma);
+          late.copy_out[static_cast<size_t>(m) * late.ldcopy + nn] = from_float<bf16_t>((epi_x[r] + v) * epi_gamma);
       } else {
-        const TC cv = from_float<TC>(end_value<TC, END>(v, epi, nn, ends, epi_act));
+        const TC cv = from_float<TC>(end_value<TC, END>(v, late.epi, nn, late.ends, epi_act));
         if constexpr (END == END_TWO) {
-          if (nn < ends.cols)
-            ends.C2[static_cast<size_t>(m) * ends.ldc2 + nn] = from_float<bf16_t>(v);
+          if (nn < late.ends.cols)
+            late.ends.C2[static_cast<size_t>(m) * late.ends.ldc2 + nn] = from_float<bf16_t>(v);
           else
-            C[static_cast<size_t>(m) * ldc + nn - ends.cols] = cv;
+            C[static_cast<size_t>(m) * ldc + nn - late.ends.cols] = cv;
           continue;
         }
-        if (!KV || nn < kv.c_cols) C[static_cast<size_t>(m) * ldc + nn] = cv;
-        if constexpr (KV) scatter_kv_at(kv, epi_slot[r], nn, cv);
+        if (!KV || nn < late.kv.c_cols) C[static_cast<size_t>(m) * ldc + nn] = cv;
+        if constexpr (KV) scatter_kv_at(late.kv, epi_slot[r], nn, cv);
       }
     }
     if constexpr (NORM == NORM_OUT) {
@@ -472,7 +531,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
         const float sq = group_reduce<16>(d * d, SumOp());
         const int m = g * 4 + r;
         if (col == 0 && m < M)
-          *reinterpret_cast<float2*>(nio.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x) * 2) = float2{mean, sq};
+          *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x) * 2) = float2{mean, sq};
       }
     }
   }
@@ -486,16 +545,19 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
 // results add up to is nothing and is dropped.  A column's sums are gemm16_kernel's, in its order: the same bits.  A lane ends one element.
 constexpr int ROW_ROTATE_8 = 0x128;      // (DPP: lane i of each 16 takes from lane i - 8 of the same 16)
 template <int WAVES, int U, typename TC, int NORM>
-__global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
-                                                            const float* __restrict__ bias, TC* __restrict__ C, int ldc,
-                                                            float* __restrict__ resid, int ldr, int M, int N, int K, int epi,
-                                                            NormIO nio) {
+__global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int rows, int N, int K,
+                                                            const void* __restrict__ p, const float* __restrict__ bias, const void* __restrict__ q,
+                                                            Late<END_PLAIN> late) {
   typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+  const int M = rows & FIRST_ROWS, ldc = static_cast<int>(reinterpret_cast<uintptr_t>(q)), ldr = ldc;
+  TC* C = static_cast<TC*>(const_cast<void*>(p));
+  float* resid = rows & FIRST_ADDS ? static_cast<float*>(const_cast<void*>(p)) : nullptr;
   constexpr int ROW = 9 * 8;                               // elements per row of a wave's piece: 8 chunks and one of padding
   constexpr int PIECES = U < 2 ? 1 : 2;                    // pairs turned round at a time
   __shared__ floatx4 red[WAVES][64];
   __shared__ __attribute__((aligned(16))) bf16_t turn[WAVES][PIECES][8 * ROW];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  // (the wave's number not as a scalar: the compiler then puts a pair's loads behind a branch, and each is waited for by itself)
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int col = lane % 16, g = lane / 16, second = col / 8;
   const int n0 = blockIdx.x * 8, nn = n0 + lane % 8, mm = lane / 8;      // (the element that a lane of the first wave ends)
   const int ksteps = (K + 31) / 32, npairs = (ksteps + 1) / 2;
@@ -506,7 +568,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
     const int c = min(nn, N - 1);
     if (bias) epi_bias = bias[c];
     if (resid) epi_x = resid[static_cast<size_t>(min(mm, M - 1)) * ldr + c];
-    if constexpr (NORM == NORM_OUT) epi_gamma = nio.gamma_out[c];
   }
   // never a conditional load; a step beyond K reads W's first block and meets zeros of A, whose chunks beyond K come from the row's start
   const int lrow = lane / 8, lch = lane % 8;               // as loader: row and 16-byte chunk of the pair's 128 bytes
@@ -515,8 +576,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
   bf16_t* mine = turn[wave][0];
   const u32x4 zero4 = {0u, 0u, 0u, 0u};
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int p0 = wave; p0 < npairs; p0 += WAVES * U) {
-    u32x4 b[U], al[U];
+  u32x4 b[U], al[U];
+  auto ask = [&](int p0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int step = 2 * (p0 + u * WAVES) + second;
@@ -527,6 +588,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
       const int at = p0 + u * WAVES;
       al[u] = *reinterpret_cast<const u32x4*>(at * 64 + lch * 8 < K ? a0 + at * 64 : asafe);
     }
+  };
+  if (wave < npairs) ask(wave);
+  // behind the operands, as in gemm16_kernel
+  if constexpr (NORM == NORM_OUT) epi_gamma = late.gamma_out[min(nn, N - 1)];
+  late_at_hand<NORM, false>(late);
+  for (int p0 = wave; p0 < npairs; p0 += WAVES * U) {
+    if (p0 != wave) ask(p0);
 #pragma unroll
     for (int u0 = 0; u0 < U; u0 += PIECES) {
 #pragma unroll
@@ -569,15 +637,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
     const float d = x - mean;
     const float sq = group_reduce<8>(d * d, SumOp());
     if (lane % 8 == 0 && mm < M)
-      *reinterpret_cast<float2*>(nio.stats_out + (static_cast<size_t>(mm) * gridDim.x + blockIdx.x) * 2) = float2{mean, sq};
+      *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(mm) * gridDim.x + blockIdx.x) * 2) = float2{mean, sq};
   }
   if (mm >= M || nn >= N) return;
   if (resid) {
     resid[static_cast<size_t>(mm) * ldr + nn] = epi_x + v;
     if constexpr (NORM == NORM_OUT)
-      nio.copy_out[static_cast<size_t>(mm) * nio.ldcopy + nn] = from_float<bf16_t>((epi_x + v) * epi_gamma);
+      late.copy_out[static_cast<size_t>(mm) * late.ldcopy + nn] = from_float<bf16_t>((epi_x + v) * epi_gamma);
   } else {
-    C[static_cast<size_t>(mm) * ldc + nn] = from_float<TC>(apply_epilogue_fast(v, epi));
+    C[static_cast<size_t>(mm) * ldc + nn] = from_float<TC>(apply_epilogue_fast(v, late.epi));
   }
 }
 
@@ -652,11 +720,11 @@ static int pairs_ahead(int K, int most) {
 // x 1,280 31.8 -> 28.7, 32,000 x 1,024 18.7 -> 16.0; with the norm before, 3,072 x 1,024 4.6 -> 4.3, 5,120 x 1,280 6.9 -> 6.6; K = 1,600 and 2,048 level.)
 template <int WAVES, int U, typename TC, bool KV, int NORM, int END>
 static void launch16_ahead(const Call& c, const NormIO& nio, hipStream_t stream) {
-  KVScatter kv = c.kv ? *c.kv : KVScatter{};
+  const First f = first_of(c, nio, NORM);
 #define DN_L16(TWO)                                                                                                       \
   hipLaunchKernelGGL((gemm16_kernel<WAVES, U, TC, KV, NORM, TWO, END>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0,       \
-                     stream, static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,             \
-                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, kv, nio, EndsOf<END>(c.ends))
+                     stream, static_cast<const bf16_t*>(c.A), static_cast<const bf16_t*>(c.W), c.lda, f.rows, c.N, c.K,   \
+                     f.p, c.bias, f.q, late_of<END>(c, nio))
   if (c.M > 8)
     DN_L16(true);
   else
@@ -684,11 +752,12 @@ bool eight_columns(int M, int N) { return M <= 8 && N <= 2048; }
 // 1,024 x 4,096 5.0 -> 4.5 and 5.6 -> 4.8, 1,600 x 6,400 8.8 -> 7.6 and 10.1 -> 8.1, 2,048 x 8,192 10.2 -> 8.8 and 11.9 -> 9.6.
 template <int WAVES, typename TC, int NORM>
 static void launch8(const Call& c, const NormIO& nio, hipStream_t stream) {
+  const First f = first_of(c, nio, NORM);
 #define DN_L8(U)                                                                                                          \
   case U:                                                                                                                 \
     hipLaunchKernelGGL((gemm8_kernel<WAVES, U, TC, NORM>), dim3((c.N + 7) / 8), dim3(WAVES * 64), 0, stream,              \
-                       static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,                   \
-                       static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, nio);                          \
+                       static_cast<const bf16_t*>(c.A), static_cast<const bf16_t*>(c.W), c.lda, f.rows, c.N, c.K, f.p,    \
+                       c.bias, f.q, late_of<END_PLAIN>(c, nio));                                                          \
     break
   switch (pairs_ahead<WAVES>(c.K, 8)) {
     DN_L8(1);
@@ -739,7 +808,8 @@ static void launch_mb(const Call& c, hipStream_t stream) {
     if (c.out_dtype == DN_BF16 && !c.resid) return launch8<WAVES, bf16_t, NORM_NONE>(c, NormIO{}, stream);
     return launch8<WAVES, float, NORM_NONE>(c, NormIO{}, stream);
   }
-  if (mb == 1 && !(c.packed & (PACKED_A | PACKED_C)) && c.M > 1) return launch16<WAVES>(c, stream);
+  // (one row too, since this kernel asks for whole rounds only: 50,257 x 1,024 27.3 -> 22.1 us, 32,000 x 1,024 18.4 -> 15.1, 4,096 x 1,024 4.0 -> 3.9)
+  if (mb == 1 && !(c.packed & (PACKED_A | PACKED_C))) return launch16<WAVES>(c, stream);
   if (mb == 1) return launch<1, 1, WAVES, 8>(c, stream);
   if (mb > 4) {
     // 65 to 256 rows: 16 columns per workgroup, the waves' sums for all row blocks through LDS
