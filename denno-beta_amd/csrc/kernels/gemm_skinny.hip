@@ -44,13 +44,51 @@ struct EndsFor<END_PLAIN> {
 template <int END>
 using EndsOf = typename EndsFor<END>::type;
 
+// The arguments of this file's kernels.  The first 14 words come in scalar registers with the launch, the others by a trip to memory that
+// every wave makes before it can ask for anything they name (two cache lines of arguments more made a product 0.4 us slower): so what the first
+// loads want stands in front, packed: `rows` is the rows and three flags; p is the statistics (NORM_IN), else what the results go to
+// or are added to; q is the slot map (NORM_IN), else the leading dimension of p (a pointer in any case: through a pointer made from a number the
+// compiler loads by instructions that are waited for one by one, 0.5 us more).
+// In this order the operands' loads leave 0.2 to 0.5 us sooner, 8 rows: with the norm before, 3,072 x 1,024 4.3 -> 4.0 us, 5,120 x 1,280 6.6 -> 6.1,
+// 6,400 x 1,600 7.6 -> 7.2; with the norm after, 1,024 x 1,024 3.1 -> 3.0, 1,280 x 5,120 6.4 -> 6.0, 1,600 x 6,400 8.1 -> 7.6; 50,257 x 1,024 23.8 -> 23.0.
+constexpr int FIRST_ROWS = 255, FIRST_ADDS = 256, FIRST_EIGHTS = 512;      // (NORM_IN: statistics by blocks of 8 columns)
+template <int END>
+struct Late {
+  void* C;      // NORM_IN
+  int ldc, epi;
+  const float* c1;
+  float eps;
+  int no_mean;
+  const float* gamma_out;
+  bf16_t* copy_out;
+  float* stats_out;
+  int ldcopy;
+  KVScatter kv;
+  EndsOf<END> ends;
+};
+
+// Brings what the epilogue takes from `late` into scalar registers here, behind the first loads of the operands (left to the compiler these
+// arguments were fetched where they are used, at the kernel's end, and the trip to memory came on top: a q | k | v of 4,800 columns 7.8 us for 7.2).
+template <int NORM, bool KV, int END>
+__device__ __forceinline__ void late_at_hand(const Late<END>& late) {
+  if constexpr (NORM == NORM_IN) asm volatile("" ::"s"(late.C), "s"(late.ldc), "s"(late.eps), "s"(late.no_mean));
+  if constexpr (NORM == NORM_OUT) asm volatile("" ::"s"(late.copy_out), "s"(late.stats_out), "s"(late.ldcopy));
+  if constexpr (NORM != NORM_OUT) asm volatile("" ::"s"(late.epi));
+  if constexpr (KV)
+    asm volatile("" ::"s"(late.kv.k_pool), "s"(late.kv.v_pool), "s"(late.kv.q_width), "s"(late.kv.page_size), "s"(late.kv.c_cols));
+  if constexpr (END == END_TWO) asm volatile("" ::"s"(late.ends.C2), "s"(late.ends.ldc2), "s"(late.ends.cols));
+}
+
 // MB row blocks and NB column blocks of 16 per workgroup; U steps of K in flight per wave.
 template <int MB, int NB, int WAVES, int U, typename TC, bool KV, int NORM = NORM_NONE, int END = END_PLAIN>
-__global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restrict__ A, int lda,
-                                                           const bf16_t* __restrict__ W,
-                                                           const float* __restrict__ bias, TC* __restrict__ C,
-                                                           int ldc, float* __restrict__ resid, int ldr, int M, int N,
-                                                           int K, int epi, int packed, KVScatter kv, NormIO nio, EndsOf<END> ends) {
+__global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int M, int N, int K, int packed,
+                                                           int ldr, const void* __restrict__ first, const float* __restrict__ bias,
+                                                           Late<END> late) {
+  // (first: the statistics (NORM_IN), else the stream, or nullptr)
+  float* resid = NORM == NORM_IN ? nullptr : static_cast<float*>(const_cast<void*>(first));
+  const float* stats_in = static_cast<const float*>(first);
+  const int blocks_in = K / 16;
+  TC* C = static_cast<TC*>(late.C);
   constexpr int BLOCKS = MB * NB;                          // 16 x 16 blocks of C in this workgroup
   constexpr int PASSES = (BLOCKS + WAVES - 1) / WAVES;     // wave w finishes blocks w, w + WAVES, ...
   __shared__ floatx4 red[WAVES][BLOCKS][64];
@@ -58,7 +96,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   const int col = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * (16 * NB);
   if constexpr (END == END_PAIR)
-    if (n0 >= ends.cols) A += ends.a_shift;
+    if (n0 >= late.ends.cols) A += late.ends.a_shift;
   const int row0 = blockIdx.y * (MB * 16);     // the rows may be shared out among workgroups too (blockIdx.y)
   const int ksteps = (K + 31) / 32, nblocks = (N + 15) / 16;
   const bf16_t* wblk[NB];
@@ -81,10 +119,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
     const int blk = wave + p * WAVES;
     epi_bias[p] = 0.f;
     if constexpr (END != END_PLAIN) epi_act[p] = float2{0.f, 0.f};
-    if constexpr (NORM != NORM_NONE) {
-      const int nn = min(n0 + (blk < BLOCKS ? blk % NB : 0) * 16 + col, N - 1);
-      epi_norm[p] = NORM == NORM_IN ? nio.c1[nn] : nio.gamma_out[nn];
-    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) epi_x[p][r] = 0.f;
     if constexpr (KV) {
@@ -95,14 +129,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
       const int mb = blk / NB, nb = blk % NB;
       const int nn = min(n0 + nb * 16 + col, N - 1);
       if (bias) epi_bias[p] = bias[nn];
-      if constexpr (END != END_PLAIN) epi_act[p] = end_numbers<TC, END>(ends, nn);
-      if constexpr (KV) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = row0 + mb * 16 + g * 4 + r;
-          epi_slot[p][r] = m < M ? kv.slot_map[m] : -1;
-        }
-      }
       if (resid) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -123,7 +149,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
       const int row = min(row0 + wave + t * WAVES, M - 1);
 #pragma unroll
       for (int i = 0; i < SP; ++i)
-        st[t][i] = *reinterpret_cast<const float2*>(nio.stats_in + (static_cast<size_t>(row) * nio.blocks_in + min(lane + 64 * i, nio.blocks_in - 1)) * 2);
+        st[t][i] = *reinterpret_cast<const float2*>(stats_in + (static_cast<size_t>(row) * blocks_in + min(lane + 64 * i, blocks_in - 1)) * 2);
     }
   }
   // Loads are never conditional and nothing uses a loaded value before all loads of a round are
@@ -138,6 +164,19 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
     for (int nb = 0; nb < NB; ++nb)
       b[u][nb] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk[nb] + ks * 512 : W + lane * 8);
   }
+  // what the epilogue reads by arguments that do not come with the launch: behind the first round of W
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const int blk = min(wave + p * WAVES, BLOCKS - 1);
+    const int nn = min(n0 + blk % NB * 16 + col, N - 1);
+    if constexpr (NORM != NORM_NONE) epi_norm[p] = NORM == NORM_IN ? late.c1[nn] : late.gamma_out[nn];
+    if constexpr (END != END_PLAIN) epi_act[p] = end_numbers<TC, END>(late.ends, nn);
+    if constexpr (KV) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) epi_slot[p][r] = late.kv.slot_map[min(row0 + blk / NB * 16 + g * 4 + r, M - 1)];
+    }
+  }
+  late_at_hand<NORM, KV>(late);
 
   // A in rows, or packed like W (PACKED_A): then a wave reads 1 KB in one piece per block
   const bf16_t* arow[MB];
@@ -160,26 +199,26 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   // wave does it in its first turn of the loop below, which every wave has: K >= 1024); the finishing
   // waves meet them behind the barrier further down
   auto join_stats = [&]() {
-    const float blocks = static_cast<float>(nio.blocks_in), wide = nio.blocks_in * 16 == K ? 16.f : 8.f;      // pairs of statistics a row, columns a pair
+    const float blocks = static_cast<float>(blocks_in);      // pairs of statistics a row, 16 columns a pair
 #pragma unroll
     for (int t = 0; t < SR; ++t) {
       const int row = wave + t * WAVES;
       float sm = 0.f;
 #pragma unroll
       for (int i = 0; i < SP; ++i)
-        if (lane + 64 * i < nio.blocks_in) sm += st[t][i].x;
-      const float mean = nio.no_mean ? 0.f : wave_sum(sm) / blocks;      // (without it the squares are taken about 0)
+        if (lane + 64 * i < blocks_in) sm += st[t][i].x;
+      const float mean = late.no_mean ? 0.f : wave_sum(sm) / blocks;      // (without it the squares are taken about 0)
       float sq = 0.f;
 #pragma unroll
       for (int i = 0; i < SP; ++i)
-        if (lane + 64 * i < nio.blocks_in) {
+        if (lane + 64 * i < blocks_in) {
           const float d = st[t][i].x - mean;
-          sq += st[t][i].y + wide * d * d;
+          sq += st[t][i].y + 16.f * d * d;
         }
-      const float var = wave_sum(sq) / (wide * blocks);
+      const float var = wave_sum(sq) / (16.f * blocks);
       if (lane == 0) {
         rowstat[row][0] = row0 + row < M ? mean : 0.f;
-        rowstat[row][1] = row0 + row < M ? 1.0f / sqrtf(var + nio.eps) : 0.f;
+        rowstat[row][1] = row0 + row < M ? 1.0f / sqrtf(var + late.eps) : 0.f;
       }
     }
   };
@@ -249,7 +288,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
         const float sq = group_reduce<16>(d * d, SumOp());
         const int m = row0 + mb * 16 + g * 4 + r;
         if (col == 0 && m < M)
-          *reinterpret_cast<float2*>(nio.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x * NB + nb) * 2) = float2{mean, sq};
+          *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x * NB + nb) * 2) = float2{mean, sq};
       }
     }
 #pragma unroll
@@ -261,58 +300,23 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
       if (resid) {
         resid[static_cast<size_t>(m) * ldr + nn] = epi_x[p][r] + v;
         if constexpr (NORM == NORM_OUT)
-          nio.copy_out[nio.ldcopy > 0 ? static_cast<size_t>(m) * nio.ldcopy + nn : packed_index(m, nn, N / 32)] =
+          late.copy_out[late.ldcopy > 0 ? static_cast<size_t>(m) * late.ldcopy + nn : packed_index(m, nn, N / 32)] =
               from_float<bf16_t>((epi_x[p][r] + v) * epi_norm[p]);
       } else {
-        TC cv = from_float<TC>(end_value<TC, END>(v, epi, nn, ends, epi_act[END != END_PLAIN ? p : 0]));
+        TC cv = from_float<TC>(end_value<TC, END>(v, late.epi, nn, late.ends, epi_act[END != END_PLAIN ? p : 0]));
         if constexpr (END == END_TWO) {
-          if (nn < ends.cols)
-            ends.C2[static_cast<size_t>(m) * ends.ldc2 + nn] = from_float<bf16_t>(v);
+          if (nn < late.ends.cols)
+            late.ends.C2[static_cast<size_t>(m) * late.ends.ldc2 + nn] = from_float<bf16_t>(v);
           else
-            C[static_cast<size_t>(m) * ldc + nn - ends.cols] = cv;
+            C[static_cast<size_t>(m) * late.ldc + nn - late.ends.cols] = cv;
           continue;
         }
-        if (!KV || nn < kv.c_cols)
-          C[(packed & PACKED_C) ? packed_index(m, nn, N / 32) : static_cast<size_t>(m) * ldc + nn] = cv;
-        if constexpr (KV) scatter_kv_at(kv, epi_slot[p][r], nn, cv);
+        if (!KV || nn < late.kv.c_cols)
+          C[(packed & PACKED_C) ? packed_index(m, nn, N / 32) : static_cast<size_t>(m) * late.ldc + nn] = cv;
+        if constexpr (KV) scatter_kv_at(late.kv, epi_slot[p][r], nn, cv);
       }
     }
   }
-}
-
-// The arguments of the two kernels below.  The first 14 words come in scalar registers with the launch, the others by a trip to memory that
-// every wave makes before it can ask for anything they name (two cache lines of arguments more made a product 0.4 us slower): so what the first
-// loads want stands in front, packed: `rows` is the rows and three flags; p is the statistics (NORM_IN), else what the results go to
-// or are added to; q is the slot map (NORM_IN), else the leading dimension of p (a pointer in any case: through a pointer made from a number the
-// compiler loads by instructions that are waited for one by one, 0.5 us more).
-// In this order the operands' loads leave 0.2 to 0.5 us sooner, 8 rows: with the norm before, 3,072 x 1,024 4.3 -> 4.0 us, 5,120 x 1,280 6.6 -> 6.1,
-// 6,400 x 1,600 7.6 -> 7.2; with the norm after, 1,024 x 1,024 3.1 -> 3.0, 1,280 x 5,120 6.4 -> 6.0, 1,600 x 6,400 8.1 -> 7.6; 50,257 x 1,024 23.8 -> 23.0.
-constexpr int FIRST_ROWS = 255, FIRST_ADDS = 256, FIRST_EIGHTS = 512;      // (NORM_IN: statistics by blocks of 8 columns)
-template <int END>
-struct Late {
-  void* C;      // NORM_IN
-  int ldc, epi;
-  const float* c1;
-  float eps;
-  int no_mean;
-  const float* gamma_out;
-  bf16_t* copy_out;
-  float* stats_out;
-  int ldcopy;
-  KVScatter kv;
-  EndsOf<END> ends;
-};
-
-// Brings what the epilogue takes from `late` into scalar registers here, behind the first loads of the operands (left to the compiler these
-// arguments were fetched where they are used, at the kernel's end, and the trip to memory came on top: a q | k | v of 4,800 columns 7.8 us for 7.2).
-template <int NORM, bool KV, int END>
-__device__ __forceinline__ void late_at_hand(const Late<END>& late) {
-  if constexpr (NORM == NORM_IN) asm volatile("" ::"s"(late.C), "s"(late.ldc), "s"(late.eps), "s"(late.no_mean));
-  if constexpr (NORM == NORM_OUT) asm volatile("" ::"s"(late.copy_out), "s"(late.stats_out), "s"(late.ldcopy));
-  if constexpr (NORM != NORM_OUT) asm volatile("" ::"s"(late.epi));
-  if constexpr (KV)
-    asm volatile("" ::"s"(late.kv.k_pool), "s"(late.kv.v_pool), "s"(late.kv.q_width), "s"(late.kv.page_size), "s"(late.kv.c_cols));
-  if constexpr (END == END_TWO) asm volatile("" ::"s"(late.ends.C2), "s"(late.ends.ldc2), "s"(late.ends.cols));
 }
 
 struct First {
@@ -654,10 +658,9 @@ template <int MB, int NB, int WAVES, int U, typename TC, bool KV, int END = END_
 static void launch_one(const Call& c, hipStream_t stream) {
   // (MB row blocks per workgroup: where the rows need more, the second grid dimension shares them out)
   dim3 grid((c.N + 16 * NB - 1) / (16 * NB), ((c.M + 15) / 16 + MB - 1) / MB), block(WAVES * 64);
-  KVScatter kv = c.kv ? *c.kv : KVScatter{};
   hipLaunchKernelGGL((gemm_kernel<MB, NB, WAVES, U, TC, KV, NORM_NONE, END>), grid, block, 0, stream,
-                     static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,
-                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, NormIO{}, EndsOf<END>(c.ends));
+                     static_cast<const bf16_t*>(c.A), static_cast<const bf16_t*>(c.W), c.lda, c.M, c.N, c.K, c.packed, c.ldr, c.resid, c.bias,
+                     late_of<END>(c, NormIO{}));
 }
 
 // the same with the norm before the product (NORM_IN: bfloat16 out) or after it (NORM_OUT: into the
@@ -665,11 +668,10 @@ static void launch_one(const Call& c, hipStream_t stream) {
 template <int MB, int NB, int WAVES, int U>
 static void launch_norm(const Call& c, const NormIO& nio, int norm, hipStream_t stream) {
   dim3 grid((c.N + 16 * NB - 1) / (16 * NB), ((c.M + 15) / 16 + MB - 1) / MB), block(WAVES * 64);
-  KVScatter kv = c.kv ? *c.kv : KVScatter{};
 #define DN_LN(TC, KV, NORM)                                                                                        \
   hipLaunchKernelGGL((gemm_kernel<MB, NB, WAVES, U, TC, KV, NORM>), grid, block, 0, stream,                       \
-                     static_cast<const bf16_t*>(c.A), c.lda, static_cast<const bf16_t*>(c.W), c.bias,             \
-                     static_cast<TC*>(c.C), c.ldc, c.resid, c.ldr, c.M, c.N, c.K, c.epi, c.packed, kv, nio, EndsOf<END_PLAIN>(c.ends))
+                     static_cast<const bf16_t*>(c.A), static_cast<const bf16_t*>(c.W), c.lda, c.M, c.N, c.K, c.packed, c.ldr, \
+                     NORM == NORM_IN ? static_cast<const void*>(nio.stats_in) : c.resid, c.bias, late_of<END_PLAIN>(c, nio))
   if (norm == NORM_OUT)
     DN_LN(float, false, NORM_OUT);
   else if (c.kv)
