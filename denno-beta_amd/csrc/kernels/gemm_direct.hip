@@ -93,12 +93,11 @@ __device__ __forceinline__ void tile_at(int pid, int tiles_m, int tiles_n, int b
 // A_IN: A comes in rows (0), packed (1), or as `packed` says (2).  XIELU: the epilogue is that activation (a kernel of its own: its
 // instructions beside the others' cost every product registers).
 template <typename TC, int WM, int WN, int TM, int TN, int STAGES, bool KV, int KB = 1, bool PING = false, int A_IN = 2, bool XIELU = false>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __restrict__ A, int lda,
-                                                           const bf16_t* __restrict__ W, const float* __restrict__ bias,
-                                                           TC* __restrict__ C, int ldc, float* __restrict__ resid, int ldr,
-                                                           int M, int N, int K, int epi, int packed, int tiles_m,
-                                                           int tiles_n, KVScatter kv, float* __restrict__ part,
-                                                           int split_slabs, const float* __restrict__ act) {
+__global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int M, int N, int K, int packed,
+                                                           int tiles_m, int tiles_n, int split_slabs, const int32_t* __restrict__ slot_map,
+                                                           const float* __restrict__ bias, TC* __restrict__ C, int ldc,
+                                                           float* __restrict__ resid, int ldr, int epi, KVScatter kv,
+                                                           float* __restrict__ part, const float* __restrict__ act) {
   constexpr int NW = WM * WN;
   const bool a_packed = A_IN == 2 ? (packed & PACKED_A) != 0 : A_IN == 1;
   constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
@@ -118,8 +117,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   // its sums in part[blockIdx.y][m][n] and a second kernel adds them in order and ends with the epilogue
   // (stages of KB slabs: the host launches KB > 1 only where K is a multiple of 32 KB; split_slabs counts stages)
   const int kall = K / 32, nblocks = (N + 15) / 16;
-  const int first = part ? blockIdx.y * split_slabs : 0;
-  const int ksteps = part ? min(split_slabs, kall / KB - first) : kall / KB;
+  // (the first 14 words of the arguments come in registers with the launch: all that the first loads need.  With the bias asked for in
+  // front, us: 203 x 4,800 x 1,600 14.2 -> 13.6, 203 x 5,120 x 1,280 12.3 -> 11.7, 203 x 1,600 x 6,400 into the stream 19.9 -> 19.4, 1,024 x 1,600 x 1,600
+  // 16.4 -> 15.9, 1,024 x 3,840 x 1,280 17.0 -> 16.5)
+  const int first = blockIdx.y * split_slabs;
+  const int ksteps = min(split_slabs, kall / KB - first);
   // Where the 16 bytes of row lane % 16, columns 8 (lane / 16) .. of a block of A lie among its KB pieces of 1 KB (see the loads below).
   // (A packed A is in the operand's order already: lane l reads at 16 l.)
   int aslot[KB];
@@ -141,11 +143,23 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + (wmb + i) * 16 + lane % 16, mq = m - lane % 4;
-      kslot[i] = m < M ? kv.slot_map[m] : -1;
+      kslot[i] = m < M ? slot_map[m] : -1;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) vslot[i][e] = mq + e < M ? kv.slot_map[mq + e] : -1;
+      for (int e = 0; e < 4; ++e) vslot[i][e] = mq + e < M ? slot_map[mq + e] : -1;
     }
   }
+  // the bias, for the epilogue, in front of the operands' loads, where a tile leaves the registers for it
+  constexpr bool BIAS_FIRST = TN <= 4;
+  floatx4 bvs[TN];
+  auto ask_bias = [&]() {
+#pragma clang loop unroll(full)
+    for (int j = 0; j < TN; ++j) bvs[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (bias) {
+#pragma clang loop unroll(full)
+      for (int j = 0; j < TN; ++j) bvs[j] = *reinterpret_cast<const floatx4*>(bias + min(n0 + (wnb + j) * 16 + (lane / 16) * 4, N - 4));
+    }
+  };
+  if constexpr (BIAS_FIRST) ask_bias();
   floatx4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -194,6 +208,9 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < ksteps) issue(s);
+  // the epilogue's arguments, which do not come with the launch: here, not at the kernel's end
+  asm volatile("" ::"s"(C), "s"(ldc), "s"(resid), "s"(ldr), "s"(epi), "s"(part));
+  if constexpr (KV) asm volatile("" ::"s"(kv.k_pool), "s"(kv.v_pool), "s"(kv.q_width), "s"(kv.kv_width), "s"(kv.dh), "s"(kv.page_size), "s"(kv.c_cols));
   // this wave's share of a stage has landed when only its loads of the STAGES - 2 stages after it are out
   auto landed = [&](bool more) {
     if (!more)
@@ -302,12 +319,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   if constexpr (XIELU) act_a = act[0], act_b = act[1];
   // every load of the epilogue before its first store: a wait for a load is a wait for the stores
   // issued before it as well (one counter), and a load per column block made the blocks take turns
-  floatx4 bvs[TN];
-#pragma clang loop unroll(full)
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + (wnb + j) * 16 + (lane / 16) * 4;
-    bvs[j] = bias && n < N ? *reinterpret_cast<const floatx4*>(bias + n) : floatx4{0.f, 0.f, 0.f, 0.f};
-  }
+  if constexpr (!BIAS_FIRST) ask_bias();
 #pragma clang loop unroll(full)
   for (int j = 0; j < TN; ++j) {
     const int n = n0 + (wnb + j) * 16 + (lane / 16) * 4;
@@ -403,11 +415,11 @@ static int launch_kernel(const Args& a, hipStream_t stream) {
     if (e != hipSuccess) return static_cast<int>(e);
     raised = true;
   }
-  const int split_slabs = (a.K / (32 * KB) + a.splits - 1) / a.splits;
-  hipLaunchKernelGGL((gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN, XIELU>), dim3(tiles_m * tiles_n, a.part ? a.splits : 1),
-                     dim3(WM * WN * 64), lds, stream, static_cast<const bf16_t*>(a.A), a.lda,
-                     static_cast<const bf16_t*>(a.W), a.bias, static_cast<TC*>(a.C), a.ldc, a.resid, a.ldr, a.M, a.N, a.K,
-                     a.epi, a.packed, tiles_m, tiles_n, a.kv ? *a.kv : KVScatter{}, a.part, split_slabs, a.act);
+  const int shares = a.part ? a.splits : 1, split_slabs = (a.K / (32 * KB) + shares - 1) / shares;
+  hipLaunchKernelGGL((gemm_kernel<TC, WM, WN, TM, TN, STAGES, KV, KB, PING, A_IN, XIELU>), dim3(tiles_m * tiles_n, shares),
+                     dim3(WM * WN * 64), lds, stream, static_cast<const bf16_t*>(a.A), static_cast<const bf16_t*>(a.W),
+                     a.lda, a.M, a.N, a.K, a.packed, tiles_m, tiles_n, split_slabs, a.kv ? a.kv->slot_map : nullptr, a.part ? nullptr : a.bias,
+                     static_cast<TC*>(a.C), a.ldc, a.resid, a.ldr, a.epi, a.kv ? *a.kv : KVScatter{}, a.part, a.act);
   return 0;
 }
 
