@@ -2,7 +2,7 @@
 
 // ---------------------------------------------------------------------------------------
 // Few rows (M <= 256), bfloat16: the decode step's products, bound by reading W once.
-// A workgroup owns 16, 32 or 64 output columns; its waves split K in steps of 32 (wave w takes
+// A workgroup owns 8, 16, 32 or 64 output columns; its waves split K in steps of 32 (wave w takes
 // steps w, w + WAVES, ...), each feeding v_mfma_f32_16x16x32_bf16 with one packed block of W per
 // 16 columns straight from memory (16 bytes per lane) and the matching 16 bytes of up to four
 // 16-row blocks of A (lane = row + 16 * (k / 8)).  The waves' sums meet in LDS and are added in
@@ -22,7 +22,7 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 // so the product itself runs on rows that are not normalised, and the norm is two numbers per row in
 // the epilogue.  NORM_OUT: a product that adds into the residual stream also stores the updated rows
 // times gamma (the next norm's), rounded to bfloat16, and, for each row, the mean and the sum of
-// squared distances from it of its 16 columns.  NORM_IN: A is such a copy; each wave joins two rows'
+// squared distances from it of its 16 (gemm8_kernel: 8) columns.  NORM_IN: A is such a copy; each wave joins two rows'
 // N / 16 pairs (means are averaged; the squares add up with 16 times the squared distance of each
 // block's mean from the row's: exact, and as stable as two passes over the row) while the operands
 // travel, and wave 0 applies them at the end.  The rows are rounded to bfloat16 before the mean is
@@ -46,7 +46,7 @@ using EndsOf = typename EndsFor<END>::type;
 
 // The arguments of this file's kernels.  The first 14 words come in scalar registers with the launch, the others by a trip to memory that
 // every wave makes before it can ask for anything they name (two cache lines of arguments more made a product 0.4 us slower): so what the first
-// loads want stands in front, packed: `rows` is the rows and three flags; p is the statistics (NORM_IN), else what the results go to
+// loads want stands in front; in gemm8_kernel and gemm16_kernel packed: `rows` is the rows and two flags; p is the statistics (NORM_IN), else what the results go to
 // or are added to; q is the slot map (NORM_IN), else the leading dimension of p (a pointer in any case: through a pointer made from a number the
 // compiler loads by instructions that are waited for one by one, 0.5 us more).
 // In this order the operands' loads leave 0.2 to 0.5 us sooner, 8 rows: with the norm before, 3,072 x 1,024 4.3 -> 4.0 us, 5,120 x 1,280 6.6 -> 6.1,
