@@ -240,7 +240,7 @@ extern "C" int dn_gemm_norm_in(const void* A, int lda, const float* stats, const
   if (block != 16 && (block != 8 || M > 16 || K > 2048)) return DN_ERR_SHAPE;      // (a lane joins up to four pairs)
   if (epilogue < EPI_NONE || epilogue > EPI_RELU2) return DN_ERR_SHAPE;
   const int packed = PACKED_W | (lda == 0 ? PACKED_A : 0);
-  if (!skinny::takes(A, lda, W, M, K, packed) || reinterpret_cast<uintptr_t>(stats) % 8 != 0) return DN_ERR_SHAPE;
+  if (!skinny::takes(A, lda, W, M, K, packed) || reinterpret_cast<uintptr_t>(stats) % (block == 8 ? 16 : 8) != 0) return DN_ERR_SHAPE;
   KVScatter kv{};
   if (slot_map) {
     if (q_width < 0 || q_width + 2 * Hkv * dh != N || page_size < 1 || !k_pool || !v_pool || epilogue != EPI_NONE)

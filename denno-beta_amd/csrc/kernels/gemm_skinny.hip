@@ -29,6 +29,29 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 // taken off, not after: right where a row's mean is not large beside its spread.
 
 
+// Mean and sum of squared distances of the 8 columns that lie in 8 lanes side by side, and of 16 columns from those of their halves.  Every
+// kernel makes a row's statistics of these, so that the next norm is the same bits whatever number of columns the product before took a workgroup.
+__device__ __forceinline__ float2 eight_columns_stats(float x) {
+#pragma clang fp contract(off)
+  const float mean = group_reduce<8>(x, SumOp()) * (1.0f / 8.0f);
+  const float d = x - mean;
+  const float sq = d * d;
+  return float2{mean, group_reduce<8>(sq, SumOp())};
+}
+__device__ __forceinline__ float2 join_eights(float2 a, float2 b) {
+  const float mean = 0.5f * (a.x + b.x), d = a.x - mean, e = b.x - mean;
+  return float2{mean, fmaf(8.0f, fmaf(d, d, e * e), a.y + b.y)};
+}
+constexpr int ROW_ROTATE_8 = 0x128;      // (DPP: lane i of each 16 takes from lane i - 8 of the same 16)
+__device__ __forceinline__ float other_eight(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ROW_ROTATE_8, 0xf, 0xf, true));
+}
+// of the 16 columns in 16 lanes; right in the first 8 lanes
+__device__ __forceinline__ float2 sixteen_columns_stats(float x) {
+  const float2 own = eight_columns_stats(x);
+  return join_eights(own, float2{other_eight(own.x), other_eight(own.y)});
+}
+
 // what a kernel's last argument is (the plain kernels read none of it)
 template <int END>
 struct EndsFor {
@@ -283,12 +306,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float x = epi_x[p][r] + (s[r] + epi_bias[p]);
-        const float mean = group_reduce<16>(x, SumOp()) * (1.0f / 16.0f);
-        const float d = x - mean;
-        const float sq = group_reduce<16>(d * d, SumOp());
+        const float2 stats = sixteen_columns_stats(x);
         const int m = row0 + mb * 16 + g * 4 + r;
         if (col == 0 && m < M)
-          *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x * NB + nb) * 2) = float2{mean, sq};
+          *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x * NB + nb) * 2) = stats;
       }
     }
 #pragma unroll
@@ -375,7 +396,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   float epi_x[4] = {0.f, 0.f, 0.f, 0.f};
   int epi_slot[4] = {-1, -1, -1, -1};
   float2 epi_act{0.f, 0.f};
-  const int blocks_in = rows & FIRST_EIGHTS ? K / 8 : K / 16;      // (NORM_IN)
+  const int blocks_in = K / 16;      // (NORM_IN)
   if (wave == 0) {
     const int nn = min(n0 + col, N - 1);
     if (bias) epi_bias = bias[nn];
@@ -389,15 +410,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
     }
   }
   // (after the epilogue's loads and before the operands': they are back before the operands are)
-  float2 st[SR][SP];
+  float4 st[SR][SP];      // (of 16 columns, or of each half of them)
   float epi_c1 = 0.f, epi_gamma = 1.f;
   if constexpr (NORM == NORM_IN) {
 #pragma unroll
     for (int t = 0; t < SR; ++t) {
-      const int row = min(wave + t * WAVES, M - 1);
+      const size_t row = static_cast<size_t>(min(wave + t * WAVES, M - 1)) * blocks_in;
+      if (rows & FIRST_EIGHTS) {
 #pragma unroll
-      for (int i = 0; i < SP; ++i)
-        st[t][i] = *reinterpret_cast<const float2*>(stats_in + (static_cast<size_t>(row) * blocks_in + min(lane + 64 * i, blocks_in - 1)) * 2);
+        for (int i = 0; i < SP; ++i) st[t][i] = *reinterpret_cast<const float4*>(stats_in + (row + min(lane + 64 * i, blocks_in - 1)) * 4);
+      } else {
+#pragma unroll
+        for (int i = 0; i < SP; ++i) {
+          const float2 two = *reinterpret_cast<const float2*>(stats_in + (row + min(lane + 64 * i, blocks_in - 1)) * 2);
+          st[t][i].x = two.x, st[t][i].y = two.y;
+        }
+      }
     }
   }
   // never a conditional load; a step beyond K reads W's first block and meets zeros of A
@@ -467,7 +495,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   late_at_hand<NORM, KV>(late);
   if constexpr (NORM == NORM_IN) {
     // the rows' means and 1 / sqrt(var + eps) for wave 0, which meets them behind the barrier further down
-    const float blocks = static_cast<float>(blocks_in), wide = rows & FIRST_EIGHTS ? 8.f : 16.f;      // pairs of statistics a row, columns a pair
+    const float blocks = static_cast<float>(blocks_in);      // of 16 columns
+    if (rows & FIRST_EIGHTS) {
+#pragma unroll
+      for (int t = 0; t < SR; ++t)
+#pragma unroll
+        for (int i = 0; i < SP; ++i) {
+          const float2 both = join_eights(float2{st[t][i].x, st[t][i].y}, float2{st[t][i].z, st[t][i].w});
+          st[t][i].x = both.x, st[t][i].y = both.y;
+        }
+    }
 #pragma unroll
     for (int t = 0; t < SR; ++t) {
       const int row = wave + t * WAVES;
@@ -481,9 +518,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
       for (int i = 0; i < SP; ++i)
         if (lane + 64 * i < blocks_in) {
           const float d = st[t][i].x - mean;
-          sq += st[t][i].y + wide * d * d;
+          sq += st[t][i].y + 16.f * d * d;
         }
-      const float var = wave_sum(sq) / (wide * blocks);
+      const float var = wave_sum(sq) / (16.f * blocks);
       if (lane == 0) {
         rowstat[row][0] = row < M ? mean : 0.f;
         rowstat[row][1] = row < M ? 1.0f / sqrtf(var + late.eps) : 0.f;
@@ -530,12 +567,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float x = epi_x[r] + (sm[r] + epi_bias);
-        const float mean = group_reduce<16>(x, SumOp()) * (1.0f / 16.0f);
-        const float d = x - mean;
-        const float sq = group_reduce<16>(d * d, SumOp());
+        const float2 stats = sixteen_columns_stats(x);
         const int m = g * 4 + r;
         if (col == 0 && m < M)
-          *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x) * 2) = float2{mean, sq};
+          *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x) * 2) = stats;
       }
     }
   }
@@ -547,7 +582,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
 // CUs have none.  A pair of steps is one load of W: lanes l % 16 < 8 bring 8 columns of the first step, the others the same
 // columns of the second.  The product of the second step takes them with the halves of every 16 lanes exchanged; what columns 8 .. 15 of the
 // results add up to is nothing and is dropped.  A column's sums are gemm16_kernel's, in its order: the same bits.  A lane ends one element.
-constexpr int ROW_ROTATE_8 = 0x128;      // (DPP: lane i of each 16 takes from lane i - 8 of the same 16)
 template <int WAVES, int U, typename TC, int NORM>
 __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int rows, int N, int K,
                                                             const void* __restrict__ p, const float* __restrict__ bias, const void* __restrict__ q,
@@ -637,11 +671,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
   if constexpr (NORM == NORM_OUT) {
     // a row's 8 columns lie in 8 lanes side by side (N is a multiple of 16)
     const float x = epi_x + v;
-    const float mean = group_reduce<8>(x, SumOp()) * (1.0f / 8.0f);
-    const float d = x - mean;
-    const float sq = group_reduce<8>(d * d, SumOp());
+    const float2 stats = eight_columns_stats(x);
     if (lane % 8 == 0 && mm < M)
-      *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(mm) * gridDim.x + blockIdx.x) * 2) = float2{mean, sq};
+      *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(mm) * gridDim.x + blockIdx.x) * 2) = stats;
   }
   if (mm >= M || nn >= N) return;
   if (resid) {

@@ -51,8 +51,7 @@ def test_the_next_norms_statistics_by_eights(N, K):
             copies.append((y, copy, ops.linear_norm_in(copy, stats, c1, c2, 1e-5, next_w, torch.empty(M, 96, dtype=torch.bfloat16, device="cuda"))))
         (y16, c16, o16), (y8, c8, o8) = copies
         assert torch.equal(y16, y8) and torch.equal(c16, c8)
-        # (mean and variance to some 1e-6 from either: a rounding to bfloat16 apart at most)
-        assert torch.allclose(o16.float(), o8.float(), rtol=2.0 ** -7, atol=2.0 ** -9)
+        assert torch.equal(o16, o8)
 
 
 def test_rows_beyond_eight_take_no_statistics_by_eights():
