@@ -237,7 +237,7 @@ extern "C" int dn_gemm_norm_in(const void* A, int lda, const float* stats, const
   if (M < 1 || M > 64 || N < 1 || K < 16 || K % 16 != 0 || K > 4096 || (lda != 0 && lda < K) || !stats || !c1 || !c2 || !C)
     return DN_ERR_SHAPE;
   if (M <= 16 ? lda == 0 : (K < 1024 || K > 2048)) return DN_ERR_SHAPE;
-  if (block != 16 && (block != 8 || M > 16 || K > 2048)) return DN_ERR_SHAPE;      // (a lane joins up to four pairs)
+  if (block != 16 && (block != 8 || M > 8 || K > 2048)) return DN_ERR_SHAPE;      // (only products of up to 8 rows and 2,048 columns leave them)
   if (epilogue < EPI_NONE || epilogue > EPI_RELU2) return DN_ERR_SHAPE;
   const int packed = PACKED_W | (lda == 0 ? PACKED_A : 0);
   if (!skinny::takes(A, lda, W, M, K, packed) || reinterpret_cast<uintptr_t>(stats) % (block == 8 ? 16 : 8) != 0) return DN_ERR_SHAPE;

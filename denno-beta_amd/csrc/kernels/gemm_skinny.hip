@@ -69,12 +69,12 @@ using EndsOf = typename EndsFor<END>::type;
 
 // The arguments of this file's kernels.  The first 14 words come in scalar registers with the launch, the others by a trip to memory that
 // every wave makes before it can ask for anything they name (two cache lines of arguments more made a product 0.4 us slower): so what the first
-// loads want stands in front; in gemm8_kernel and gemm16_kernel packed: `rows` is the rows and two flags; p is the statistics (NORM_IN), else what the results go to
+// loads want stands in front; in gemm8_kernel and gemm16_kernel packed: `rows` is the rows and a flag; p is the statistics (NORM_IN), else what the results go to
 // or are added to; q is the slot map (NORM_IN), else the leading dimension of p (a pointer in any case: through a pointer made from a number the
 // compiler loads by instructions that are waited for one by one, 0.5 us more).
 // In this order the operands' loads leave 0.2 to 0.5 us sooner, 8 rows: with the norm before, 3,072 x 1,024 4.3 -> 4.0 us, 5,120 x 1,280 6.6 -> 6.1,
 // 6,400 x 1,600 7.6 -> 7.2; with the norm after, 1,024 x 1,024 3.1 -> 3.0, 1,280 x 5,120 6.4 -> 6.0, 1,600 x 6,400 8.1 -> 7.6; 50,257 x 1,024 23.8 -> 23.0.
-constexpr int FIRST_ROWS = 255, FIRST_ADDS = 256, FIRST_EIGHTS = 512;      // (NORM_IN: statistics by blocks of 8 columns)
+constexpr int FIRST_ROWS = 255, FIRST_ADDS = 256;
 template <int END>
 struct Late {
   void* C;      // NORM_IN
@@ -347,7 +347,7 @@ struct First {
 };
 static First first_of(const Call& c, const NormIO& nio, int norm) {
   if (norm == NORM_IN)
-    return First{c.M | (nio.blocks_in * 16 == c.K ? 0 : FIRST_EIGHTS), nio.stats_in, c.kv ? c.kv->slot_map : nullptr};
+    return First{c.M, nio.stats_in, c.kv ? c.kv->slot_map : nullptr};
   return First{c.M | (c.resid ? FIRST_ADDS : 0), c.resid ? static_cast<const void*>(c.resid) : c.C, reinterpret_cast<const void*>(static_cast<uintptr_t>(c.resid ? c.ldr : c.ldc))};
 }
 template <int END>
@@ -364,7 +364,7 @@ static Late<END> late_of(const Call& c, const NormIO& nio) {
 // of its own (no barrier: a wave's LDS operations keep their order) and reads the operands from
 // there, two pairs at a time through two such pieces, so that the way into LDS and out of it is
 // waited for once per two pairs.  16 columns per workgroup, sums joined through LDS in wave order, as in gemm_kernel.
-template <int WAVES, int U, typename TC, bool KV, int NORM, bool TWO, int END = END_PLAIN>
+template <int WAVES, int U, typename TC, bool KV, int NORM, bool TWO, int END = END_PLAIN, bool EIGHTS = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int rows, int N,
                                                              int K, const void* __restrict__ p, const float* __restrict__ bias, const void* __restrict__ q,
                                                              Late<END> late) {
@@ -389,7 +389,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   // (TWO: rows 8 .. 15 need a second load per pair)
   // NORM_IN: the rows' pairs of statistics are asked for before the operands (loads come back in the
   // order asked): wave w joins rows w, w + WAVES, ...; a lane holds up to SP pairs of a row
-  constexpr int SP = 4, SR = 16 / WAVES;
+  // (EIGHTS: statistics by blocks of 8 columns, 8 rows and K = 2,048 at most, so no load of a row or place that cannot be there)
+  constexpr int SP = EIGHTS ? 2 : 4, SR = (TWO ? 16 : 8) / WAVES;
   __shared__ float rowstat[16][2];
   // what the epilogue will read is asked for first of all (wave 0 finishes the block)
   float epi_bias = 0.f;
@@ -416,7 +417,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
 #pragma unroll
     for (int t = 0; t < SR; ++t) {
       const size_t row = static_cast<size_t>(min(wave + t * WAVES, M - 1)) * blocks_in;
-      if (rows & FIRST_EIGHTS) {
+      if constexpr (EIGHTS) {
 #pragma unroll
         for (int i = 0; i < SP; ++i) st[t][i] = *reinterpret_cast<const float4*>(stats_in + (row + min(lane + 64 * i, blocks_in - 1)) * 4);
       } else {
@@ -496,7 +497,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   if constexpr (NORM == NORM_IN) {
     // the rows' means and 1 / sqrt(var + eps) for wave 0, which meets them behind the barrier further down
     const float blocks = static_cast<float>(blocks_in);      // of 16 columns
-    if (rows & FIRST_EIGHTS) {
+    if constexpr (EIGHTS) {
 #pragma unroll
       for (int t = 0; t < SR; ++t)
 #pragma unroll
@@ -755,14 +756,16 @@ static int pairs_ahead(int K, int most) {
 template <int WAVES, int U, typename TC, bool KV, int NORM, int END>
 static void launch16_ahead(const Call& c, const NormIO& nio, hipStream_t stream) {
   const First f = first_of(c, nio, NORM);
-#define DN_L16(TWO)                                                                                                       \
-  hipLaunchKernelGGL((gemm16_kernel<WAVES, U, TC, KV, NORM, TWO, END>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0,       \
+#define DN_L16(TWO, EIGHTS)                                                                                               \
+  hipLaunchKernelGGL((gemm16_kernel<WAVES, U, TC, KV, NORM, TWO, END, EIGHTS>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0,       \
                      stream, static_cast<const bf16_t*>(c.A), static_cast<const bf16_t*>(c.W), c.lda, f.rows, c.N, c.K,   \
                      f.p, c.bias, f.q, late_of<END>(c, nio))
   if (c.M > 8)
-    DN_L16(true);
+    DN_L16(true, false);
+  else if (NORM == NORM_IN && nio.blocks_in * 16 != c.K)
+    DN_L16(false, NORM == NORM_IN);
   else
-    DN_L16(false);
+    DN_L16(false, false);
 #undef DN_L16
 }
 
