@@ -195,27 +195,22 @@ extern "C" int dn_join(const float* part, int shares, const float* bias, float* 
   return dn_launch_status();
 }
 
-// the columns that a pair of statistics of dn_gemm_norm_out's is best about: 8, where a workgroup has so many, or 16
-extern "C" int dn_gemm_norm_block(int M, int N) { return skinny::eight_columns(M, N) ? 8 : 16; }
-
 // A product of few rows that adds into the residual stream and leaves what the norm after it needs:
 // resid [M, N] += A . W^T + bias; copy = the updated rows times gamma [N] (that norm's weight) in
 // bfloat16, in rows of ldcopy elements or (ldcopy == 0, N a multiple of 32) as packed rows; stats
-// [M][N / block][2] = mean and sum of squared distances from it of each row's blocks of 16 columns, or of 8 where
-// dn_gemm_norm_block(M, N) says so.
+// [M][N / 16][2] = mean and sum of squared distances from it of each row's blocks of 16 columns.
 // A [M, K] bfloat16 in rows or (lda == 0) packed, W packed, N a multiple of 16.  Up to 16 rows (A in
 // rows), or 17 to 64 rows with K >= 1024.
 extern "C" int dn_gemm_norm_out(const void* A, int lda, const void* W, const float* bias, float* resid, int ldr, int M,
-                                int N, int K, const float* gamma, void* copy, int ldcopy, float* stats, int block,
+                                int N, int K, const float* gamma, void* copy, int ldcopy, float* stats,
                                 hipStream_t stream) {
   if (M < 1 || M > 64 || N < 16 || N % 16 != 0 || K < 8 || ldr < N || !resid || !copy || !stats || !gamma) return DN_ERR_SHAPE;
   if ((lda != 0 && lda < K) || (ldcopy != 0 && ldcopy < N) || (ldcopy == 0 && N % 32 != 0)) return DN_ERR_SHAPE;
   if (M <= 16 ? lda == 0 : K < 1024) return DN_ERR_SHAPE;
-  if (block != 16 && (block != 8 || M > 8)) return DN_ERR_SHAPE;
   const int packed = PACKED_W | (lda == 0 ? PACKED_A : 0);
   if (!skinny::takes(A, lda, W, M, K, packed)) return DN_ERR_SHAPE;
   skinny::Call c{A, lda, W, bias, nullptr, 0, resid, ldr, M, N, K, DN_F32, EPI_NONE, packed, nullptr};
-  skinny::NormIO nio{nullptr, block, nullptr, 0.f, 0, gamma, static_cast<bf16_t*>(copy), ldcopy, stats};
+  skinny::NormIO nio{nullptr, nullptr, 0.f, 0, gamma, static_cast<bf16_t*>(copy), ldcopy, stats};
   if (M > 16)
     skinny::launch_mb_norm(c, nio, NORM_OUT, stream);
   else
@@ -224,7 +219,7 @@ extern "C" int dn_gemm_norm_out(const void* A, int lda, const void* W, const flo
 }
 
 // The product after such a norm: C [M, N] bfloat16 = act(LayerNorm(x) . W^T + b), where A is the
-// copy of x times gamma [M, K] (in rows, or lda == 0: packed rows) and stats [M][K / block][2] what
+// copy of x times gamma [M, K] (in rows, or lda == 0: packed rows) and stats [M][K / 16][2] what
 // dn_gemm_norm_out left, c1[n] = sum_k gamma[k] W[n,k] and c2[n] = sum_k beta[k] W[n,k] + b[n].
 // no_mean: the norm is x / sqrt(mean(x^2) + eps) * gamma (no mean taken off, no beta: c1 is not used).
 // Up to 16 rows (A in rows, K a multiple of 16 up to 4,096), or 17 to 64 rows (K from 1,024 to 2,048).
@@ -233,14 +228,13 @@ extern "C" int dn_gemm_norm_out(const void* A, int lda, const void* W, const flo
 extern "C" int dn_gemm_norm_in(const void* A, int lda, const float* stats, const float* c1, const float* c2,
                                float eps, const void* W, void* C, int ldc, int M, int N, int K,
                                int epilogue, const int32_t* slot_map, void* k_pool, void* v_pool, int q_width,
-                               int Hkv, int dh, int page_size, int c_cols, int no_mean, int block, hipStream_t stream) {
+                               int Hkv, int dh, int page_size, int c_cols, int no_mean, hipStream_t stream) {
   if (M < 1 || M > 64 || N < 1 || K < 16 || K % 16 != 0 || K > 4096 || (lda != 0 && lda < K) || !stats || !c1 || !c2 || !C)
     return DN_ERR_SHAPE;
   if (M <= 16 ? lda == 0 : (K < 1024 || K > 2048)) return DN_ERR_SHAPE;
-  if (block != 16 && (block != 8 || M > 8 || K > 2048)) return DN_ERR_SHAPE;      // (only products of up to 8 rows and 2,048 columns leave them)
   if (epilogue < EPI_NONE || epilogue > EPI_RELU2) return DN_ERR_SHAPE;
   const int packed = PACKED_W | (lda == 0 ? PACKED_A : 0);
-  if (!skinny::takes(A, lda, W, M, K, packed) || reinterpret_cast<uintptr_t>(stats) % (block == 8 ? 16 : 8) != 0) return DN_ERR_SHAPE;
+  if (!skinny::takes(A, lda, W, M, K, packed) || reinterpret_cast<uintptr_t>(stats) % 8 != 0) return DN_ERR_SHAPE;
   KVScatter kv{};
   if (slot_map) {
     if (q_width < 0 || q_width + 2 * Hkv * dh != N || page_size < 1 || !k_pool || !v_pool || epilogue != EPI_NONE)
@@ -253,7 +247,7 @@ extern "C" int dn_gemm_norm_in(const void* A, int lda, const float* stats, const
   }
   skinny::Call c{A, lda, W, c2, C, ldc, nullptr, 0, M, N, K, DN_BF16, epilogue, packed | (ldc == 0 ? PACKED_C : 0),
                  slot_map ? &kv : nullptr};
-  skinny::NormIO nio{stats, K / block, c1, eps, no_mean ? 1 : 0, nullptr, nullptr, 0, nullptr};
+  skinny::NormIO nio{stats, c1, eps, no_mean ? 1 : 0, nullptr, nullptr, 0, nullptr};
   if (M > 16)
     skinny::launch_mb_norm(c, nio, NORM_IN, stream);
   else

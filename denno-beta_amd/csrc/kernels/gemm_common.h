@@ -179,17 +179,14 @@ void join_shares(const float* part, int shares, const float* bias, float* resid,
 
 namespace skinny {
 struct NormIO {
-  const float* stats_in;     // NORM_IN: [M][blocks_in][2]
-  int blocks_in;             // NORM_IN: K / block; NORM_OUT: block (the host's to know)
+  const float* stats_in;     // NORM_IN: [M][K / 16][2]
   const float* c1;           // NORM_IN: [N]  (c2 comes as the bias)
   float eps;
   int no_mean;               // NORM_IN: the norm takes no mean off (x / sqrt(mean(x^2) + eps) * gamma): the row's mean counts as 0
   const float* gamma_out;    // NORM_OUT: [N] the next norm's weight
   bf16_t* copy_out;          // NORM_OUT: [M, ldcopy] the updated rows times gamma_out in bfloat16
   int ldcopy;
-  float* stats_out;          // NORM_OUT: [M][N / block][2]
-  // (the columns that a pair of statistics is about, 16 or 8, have no field of their own: one more and the arguments reach into another cache
-  // line, whose trip every product waited for: 4,800 and 6,400 columns from K = 1,600 6.8 -> 7.25 and 7.4 -> 7.8 us)
+  float* stats_out;          // NORM_OUT: [M][N / 16][2]
 };
 
 struct Call {
@@ -200,7 +197,6 @@ struct Call {
   Ends ends{};
 };
 bool takes(const void* A, int lda, const void* W, int M, int K, int packed);
-bool eight_columns(int M, int N);      // whether a workgroup has 8 columns of the product
 void run(const Call& c, hipStream_t stream);
 void launch_mb_norm(const Call& c, const NormIO& nio, int norm, hipStream_t stream);
 void launch16_norm_of(int waves, const Call& c, const NormIO& nio, int norm, hipStream_t stream);

@@ -22,34 +22,25 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 // so the product itself runs on rows that are not normalised, and the norm is two numbers per row in
 // the epilogue.  NORM_OUT: a product that adds into the residual stream also stores the updated rows
 // times gamma (the next norm's), rounded to bfloat16, and, for each row, the mean and the sum of
-// squared distances from it of its 16 (gemm8_kernel: 8) columns.  NORM_IN: A is such a copy; each wave joins two rows'
+// squared distances from it of its 16 columns.  NORM_IN: A is such a copy; each wave joins two rows'
 // N / 16 pairs (means are averaged; the squares add up with 16 times the squared distance of each
 // block's mean from the row's: exact, and as stable as two passes over the row) while the operands
 // travel, and wave 0 applies them at the end.  The rows are rounded to bfloat16 before the mean is
 // taken off, not after: right where a row's mean is not large beside its spread.
 
 
-// Mean and sum of squared distances of the 8 columns that lie in 8 lanes side by side, and of 16 columns from those of their halves.  Every
-// kernel makes a row's statistics of these, so that the next norm is the same bits whatever number of columns the product before took a workgroup.
-__device__ __forceinline__ float2 eight_columns_stats(float x) {
+// Mean and sum of squared distances of the 16 columns that lie in 16 lanes side by side, right in the first of them: the same sums in
+// every kernel, so that the next norm is the same bits whichever kernel the product before it ran in.  (Eight columns a workgroup, 16 joined from
+// two pairs of eights, rounds otherwise: steps of up to 8 rows would be 2 to 3 % faster by it, decoding one request at width 1,024 17.8 ms for 18.4.)
+__device__ __forceinline__ float2 columns_stats(float x) {
 #pragma clang fp contract(off)
-  const float mean = group_reduce<8>(x, SumOp()) * (1.0f / 8.0f);
+  const float mean = group_reduce<16>(x, SumOp()) * (1.0f / 16.0f);
   const float d = x - mean;
-  const float sq = d * d;
-  return float2{mean, group_reduce<8>(sq, SumOp())};
-}
-__device__ __forceinline__ float2 join_eights(float2 a, float2 b) {
-  const float mean = 0.5f * (a.x + b.x), d = a.x - mean, e = b.x - mean;
-  return float2{mean, fmaf(8.0f, fmaf(d, d, e * e), a.y + b.y)};
-}
-constexpr int ROW_ROTATE_8 = 0x128;      // (DPP: lane i of each 16 takes from lane i - 8 of the same 16)
-__device__ __forceinline__ float other_eight(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ROW_ROTATE_8, 0xf, 0xf, true));
-}
-// of the 16 columns in 16 lanes; right in the first 8 lanes
-__device__ __forceinline__ float2 sixteen_columns_stats(float x) {
-  const float2 own = eight_columns_stats(x);
-  return join_eights(own, float2{other_eight(own.x), other_eight(own.y)});
+  float sq = fmaf(d, d, dpp_move<DN_DPP_XOR1>(d * d));
+  sq += dpp_move<DN_DPP_XOR2>(sq);
+  sq += dpp_move<DN_DPP_HALF_MIRROR>(sq);
+  sq += dpp_move<DN_DPP_MIRROR>(sq);
+  return float2{mean, sq};
 }
 
 // what a kernel's last argument is (the plain kernels read none of it)
@@ -306,7 +297,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float x = epi_x[p][r] + (s[r] + epi_bias[p]);
-        const float2 stats = sixteen_columns_stats(x);
+        const float2 stats = columns_stats(x);
         const int m = row0 + mb * 16 + g * 4 + r;
         if (col == 0 && m < M)
           *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x * NB + nb) * 2) = stats;
@@ -364,7 +355,7 @@ static Late<END> late_of(const Call& c, const NormIO& nio) {
 // of its own (no barrier: a wave's LDS operations keep their order) and reads the operands from
 // there, two pairs at a time through two such pieces, so that the way into LDS and out of it is
 // waited for once per two pairs.  16 columns per workgroup, sums joined through LDS in wave order, as in gemm_kernel.
-template <int WAVES, int U, typename TC, bool KV, int NORM, bool TWO, int END = END_PLAIN, bool EIGHTS = false>
+template <int WAVES, int U, typename TC, bool KV, int NORM, bool TWO, int END = END_PLAIN, bool SHORT = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int rows, int N,
                                                              int K, const void* __restrict__ p, const float* __restrict__ bias, const void* __restrict__ q,
                                                              Late<END> late) {
@@ -389,8 +380,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   // (TWO: rows 8 .. 15 need a second load per pair)
   // NORM_IN: the rows' pairs of statistics are asked for before the operands (loads come back in the
   // order asked): wave w joins rows w, w + WAVES, ...; a lane holds up to SP pairs of a row
-  // (EIGHTS: statistics by blocks of 8 columns, 8 rows and K = 2,048 at most, so no load of a row or place that cannot be there)
-  constexpr int SP = EIGHTS ? 2 : 4, SR = (TWO ? 16 : 8) / WAVES;
+  // (SHORT: K = 2,048 at most, so no load of a place that cannot be there)
+  constexpr int SP = SHORT ? 2 : 4, SR = (TWO ? 16 : 8) / WAVES;
   __shared__ float rowstat[16][2];
   // what the epilogue will read is asked for first of all (wave 0 finishes the block)
   float epi_bias = 0.f;
@@ -411,22 +402,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
     }
   }
   // (after the epilogue's loads and before the operands': they are back before the operands are)
-  float4 st[SR][SP];      // (of 16 columns, or of each half of them)
+  float2 st[SR][SP];
   float epi_c1 = 0.f, epi_gamma = 1.f;
   if constexpr (NORM == NORM_IN) {
 #pragma unroll
     for (int t = 0; t < SR; ++t) {
       const size_t row = static_cast<size_t>(min(wave + t * WAVES, M - 1)) * blocks_in;
-      if constexpr (EIGHTS) {
 #pragma unroll
-        for (int i = 0; i < SP; ++i) st[t][i] = *reinterpret_cast<const float4*>(stats_in + (row + min(lane + 64 * i, blocks_in - 1)) * 4);
-      } else {
-#pragma unroll
-        for (int i = 0; i < SP; ++i) {
-          const float2 two = *reinterpret_cast<const float2*>(stats_in + (row + min(lane + 64 * i, blocks_in - 1)) * 2);
-          st[t][i].x = two.x, st[t][i].y = two.y;
-        }
-      }
+      for (int i = 0; i < SP; ++i) st[t][i] = *reinterpret_cast<const float2*>(stats_in + (row + min(lane + 64 * i, blocks_in - 1)) * 2);
     }
   }
   // never a conditional load; a step beyond K reads W's first block and meets zeros of A
@@ -497,15 +480,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
   if constexpr (NORM == NORM_IN) {
     // the rows' means and 1 / sqrt(var + eps) for wave 0, which meets them behind the barrier further down
     const float blocks = static_cast<float>(blocks_in);      // of 16 columns
-    if constexpr (EIGHTS) {
-#pragma unroll
-      for (int t = 0; t < SR; ++t)
-#pragma unroll
-        for (int i = 0; i < SP; ++i) {
-          const float2 both = join_eights(float2{st[t][i].x, st[t][i].y}, float2{st[t][i].z, st[t][i].w});
-          st[t][i].x = both.x, st[t][i].y = both.y;
-        }
-    }
 #pragma unroll
     for (int t = 0; t < SR; ++t) {
       const int row = wave + t * WAVES;
@@ -568,7 +542,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float x = epi_x[r] + (sm[r] + epi_bias);
-        const float2 stats = sixteen_columns_stats(x);
+        const float2 stats = columns_stats(x);
         const int m = g * 4 + r;
         if (col == 0 && m < M)
           *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(m) * nblocks + blockIdx.x) * 2) = stats;
@@ -578,12 +552,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
 }
 
 
+constexpr int ROW_ROTATE_8 = 0x128;      // (DPP: lane i of each 16 takes from lane i - 8 of the same 16)
+
 // Up to 8 rows of a product with few columns: gemm16_kernel with 8 columns a workgroup.  A CU takes 50 to 60 GB/s of what its XCD's L2 does not
 // hold, whatever it asks for ahead, so a workgroup of 16 columns waits for its own share of W (205 KB at K = 6,400) while half of the
 // CUs have none.  A pair of steps is one load of W: lanes l % 16 < 8 bring 8 columns of the first step, the others the same
 // columns of the second.  The product of the second step takes them with the halves of every 16 lanes exchanged; what columns 8 .. 15 of the
 // results add up to is nothing and is dropped.  A column's sums are gemm16_kernel's, in its order: the same bits.  A lane ends one element.
-template <int WAVES, int U, typename TC, int NORM>
+template <int WAVES, int U, typename TC>
 __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int rows, int N, int K,
                                                             const void* __restrict__ p, const float* __restrict__ bias, const void* __restrict__ q,
                                                             Late<END_PLAIN> late) {
@@ -602,7 +578,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
   const int ksteps = (K + 31) / 32, npairs = (ksteps + 1) / 2;
   const bf16_t* wblk = W + (static_cast<size_t>(blockIdx.x / 2) * ksteps * 64 + g * 16 + (blockIdx.x % 2) * 8 + col % 8) * 8;
   // what the epilogue will read is asked for first of all
-  float epi_bias = 0.f, epi_x = 0.f, epi_gamma = 1.f;
+  float epi_bias = 0.f, epi_x = 0.f;
   if (wave == 0) {
     const int c = min(nn, N - 1);
     if (bias) epi_bias = bias[c];
@@ -630,8 +606,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
   };
   if (wave < npairs) ask(wave);
   // behind the operands, as in gemm16_kernel
-  if constexpr (NORM == NORM_OUT) epi_gamma = late.gamma_out[min(nn, N - 1)];
-  late_at_hand<NORM, false>(late);
+  late_at_hand<NORM_NONE, false>(late);
   for (int p0 = wave; p0 < npairs; p0 += WAVES * U) {
     if (p0 != wave) ask(p0);
 #pragma unroll
@@ -669,18 +644,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
 #pragma unroll
   for (int w = 1; w < WAVES; ++w) sum += at[w * 64 * 4];
   const float v = sum + epi_bias;
-  if constexpr (NORM == NORM_OUT) {
-    // a row's 8 columns lie in 8 lanes side by side (N is a multiple of 16)
-    const float x = epi_x + v;
-    const float2 stats = eight_columns_stats(x);
-    if (lane % 8 == 0 && mm < M)
-      *reinterpret_cast<float2*>(late.stats_out + (static_cast<size_t>(mm) * gridDim.x + blockIdx.x) * 2) = stats;
-  }
   if (mm >= M || nn >= N) return;
   if (resid) {
     resid[static_cast<size_t>(mm) * ldr + nn] = epi_x + v;
-    if constexpr (NORM == NORM_OUT)
-      late.copy_out[static_cast<size_t>(mm) * late.ldcopy + nn] = from_float<bf16_t>((epi_x + v) * epi_gamma);
   } else {
     C[static_cast<size_t>(mm) * ldc + nn] = from_float<TC>(apply_epilogue_fast(v, late.epi));
   }
@@ -756,13 +722,13 @@ static int pairs_ahead(int K, int most) {
 template <int WAVES, int U, typename TC, bool KV, int NORM, int END>
 static void launch16_ahead(const Call& c, const NormIO& nio, hipStream_t stream) {
   const First f = first_of(c, nio, NORM);
-#define DN_L16(TWO, EIGHTS)                                                                                               \
-  hipLaunchKernelGGL((gemm16_kernel<WAVES, U, TC, KV, NORM, TWO, END, EIGHTS>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0,       \
+#define DN_L16(TWO, SHORT)                                                                                               \
+  hipLaunchKernelGGL((gemm16_kernel<WAVES, U, TC, KV, NORM, TWO, END, SHORT>), dim3((c.N + 15) / 16), dim3(WAVES * 64), 0,       \
                      stream, static_cast<const bf16_t*>(c.A), static_cast<const bf16_t*>(c.W), c.lda, f.rows, c.N, c.K,   \
                      f.p, c.bias, f.q, late_of<END>(c, nio))
   if (c.M > 8)
     DN_L16(true, false);
-  else if (NORM == NORM_IN && nio.blocks_in * 16 != c.K)
+  else if (NORM == NORM_IN && c.K <= 2048)
     DN_L16(false, NORM == NORM_IN);
   else
     DN_L16(false, false);
@@ -781,20 +747,20 @@ static void launch16_one(const Call& c, const NormIO& nio, hipStream_t stream) {
 
 // Where gemm8_kernel runs: up to 8 rows of at most 2,048 columns, whose 256 workgroups the chip has CUs for (beyond, 16 columns a workgroup
 // give every CU its own too, and read A half as often: 2,304 columns from K = 9,216 at 8 rows 13.6 us so, 16 to 17 in eights).
-bool eight_columns(int M, int N) { return M <= 8 && N <= 2048; }
+static bool eight_columns(int M, int N) { return M <= 8 && N <= 2048; }
 
 // The pairs in flight per wave are as many as make its share of K whole rounds: loads of what is not there cost as much as the others
 // (1,024 x 1,024 at 8 rows 3.1 us with 2, 3.5 with 4, 4.2 with 8; 1,024 x 4,096 5.1, 4.8, 4.8; 1,600 x 6,400 9.3, 9.2, 8.3 and 8.1 with 6).
 // gemm16_kernel -> this, with the next norm's statistics, 1 and 8 rows: 1,024 x 1,024 3.7 -> 3.0 and 4.2 -> 3.1 us, 1,600 x 1,600 3.9 -> 3.7 and 4.3 -> 3.8,
 // 1,024 x 4,096 5.0 -> 4.5 and 5.6 -> 4.8, 1,600 x 6,400 8.8 -> 7.6 and 10.1 -> 8.1, 2,048 x 8,192 10.2 -> 8.8 and 11.9 -> 9.6.
-template <int WAVES, typename TC, int NORM>
-static void launch8(const Call& c, const NormIO& nio, hipStream_t stream) {
-  const First f = first_of(c, nio, NORM);
+template <int WAVES, typename TC>
+static void launch8(const Call& c, hipStream_t stream) {
+  const First f = first_of(c, NormIO{}, NORM_NONE);
 #define DN_L8(U)                                                                                                          \
   case U:                                                                                                                 \
-    hipLaunchKernelGGL((gemm8_kernel<WAVES, U, TC, NORM>), dim3((c.N + 7) / 8), dim3(WAVES * 64), 0, stream,              \
+    hipLaunchKernelGGL((gemm8_kernel<WAVES, U, TC>), dim3((c.N + 7) / 8), dim3(WAVES * 64), 0, stream,              \
                        static_cast<const bf16_t*>(c.A), static_cast<const bf16_t*>(c.W), c.lda, f.rows, c.N, c.K, f.p,    \
-                       c.bias, f.q, late_of<END_PLAIN>(c, nio));                                                          \
+                       c.bias, f.q, late_of<END_PLAIN>(c, NormIO{}));                                                        \
     break
   switch (pairs_ahead<WAVES>(c.K, 8)) {
     DN_L8(1);
@@ -812,7 +778,6 @@ static void launch8(const Call& c, const NormIO& nio, hipStream_t stream) {
 // the same with the norm before the product (NORM_IN: bfloat16 out) or after it (NORM_OUT: into the residual stream)
 template <int WAVES>
 static void launch16_norm(const Call& c, const NormIO& nio, int norm, hipStream_t stream) {
-  if (norm == NORM_OUT && nio.blocks_in == 8) return launch8<WAVES, float, NORM_OUT>(c, nio, stream);
   if (norm == NORM_OUT) return launch16_one<WAVES, float, false, NORM_OUT>(c, nio, stream);
   if (c.kv) return launch16_one<WAVES, bf16_t, true, NORM_IN>(c, nio, stream);
   return launch16_one<WAVES, bf16_t, false, NORM_IN>(c, nio, stream);
@@ -842,8 +807,8 @@ static void launch_mb(const Call& c, hipStream_t stream) {
   // at 256, where sixteen row blocks x one column block took 7.7 and 12.6: every workgroup read all rows)
   if (mb > 4 && c.N < 2048 && c.K < 4096) return launch<4, 2, WAVES, 4>(c, stream);
   if (mb == 1 && !(c.packed & (PACKED_A | PACKED_C)) && eight_columns(c.M, c.N) && !c.kv && c.end == END_PLAIN) {
-    if (c.out_dtype == DN_BF16 && !c.resid) return launch8<WAVES, bf16_t, NORM_NONE>(c, NormIO{}, stream);
-    return launch8<WAVES, float, NORM_NONE>(c, NormIO{}, stream);
+    if (c.out_dtype == DN_BF16 && !c.resid) return launch8<WAVES, bf16_t>(c, stream);
+    return launch8<WAVES, float>(c, stream);
   }
   // (one row too, since this kernel asks for whole rounds only: 50,257 x 1,024 27.3 -> 22.1 us, 32,000 x 1,024 18.4 -> 15.1, 4,096 x 1,024 4.0 -> 3.9)
   if (mb == 1 && !(c.packed & (PACKED_A | PACKED_C))) return launch16<WAVES>(c, stream);

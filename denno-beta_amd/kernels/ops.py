@@ -113,9 +113,8 @@ def _declare(name, lib):
             "dn_gemm_plain_qkv_takes": [P, I, P, I, I, I, I],
             "dn_gemm_plain_qkv": [P, I, P, P, P, I, I, I, I, I, P, P, P, I, I, I, I, P, c_longlong, P],
             "dn_pack_matrix": [P, P, I, I, P],
-            "dn_gemm_norm_out": [P, I, P, P, P, I, I, I, I, P, P, I, P, I, P],
-            "dn_gemm_norm_block": [I, I],
-            "dn_gemm_norm_in": [P, I, P, P, P, F, P, P, I, I, I, I, I, P, P, P, I, I, I, I, I, I, I, P],
+            "dn_gemm_norm_out": [P, I, P, P, P, I, I, I, I, P, P, I, P, P],
+            "dn_gemm_norm_in": [P, I, P, P, P, F, P, P, I, I, I, I, I, P, P, P, I, I, I, I, I, I, P],
             "dn_gemm_qkv": [P, I, P, P, P, I, I, I, I, P, P, P, I, I, I, I, I, I, P],
             "dn_gemm_deferred_shares": [I, I, I],
             "dn_gemm_deferred": [P, I, P, I, I, I, I, P, c_longlong, P],
@@ -989,18 +988,13 @@ def norm_stream_takes(n_rows, width, w):
     return n_rows <= 64 and width % 32 == 0 and 1024 <= width <= 2048 and w.shape[1] >= 1024
 
 
-def norm_stream_block(n_rows, w):
-    """How many columns a pair of statistics is best about that linear_norm_out leaves for n_rows rows with the packed weight w."""
-    return _lib_quiet("gemm").dn_gemm_norm_block(n_rows, w.shape[0])
-
-
-def norm_stream_buffers(n_rows, width, device, block=16):
+def norm_stream_buffers(n_rows, width, device):
     """(copy, stats): the residual stream's rows times the next norm's weight, in bfloat16 ([n_rows,
-    width], from 17 rows on as packed rows), and, per row and block of 16 columns (or 8: norm_stream_block), the mean and
-    the sum of squared distances from it [n_rows, width / block, 2]."""
+    width], from 17 rows on as packed rows), and, per row and block of 16 columns, the mean and
+    the sum of squared distances from it [n_rows, width / 16, 2]."""
     copy = (packed_rows(n_rows, width, device) if n_rows >= PACKED_ROWS_MIN else
             torch.empty((n_rows, width), dtype=torch.bfloat16, device=device))
-    return copy, torch.empty((n_rows, width // block, 2), dtype=torch.float32, device=device)
+    return copy, torch.empty((n_rows, width // 16, 2), dtype=torch.float32, device=device)
 
 
 def norm_folded(w_rows, bias, gamma, beta, no_mean=False):
@@ -1027,18 +1021,10 @@ def _rows_or_packed(t, name, M, width):
     return _rows(t, name)
 
 
-def _stats_block(stats, n_rows, width, what):
-    """The columns that a pair of `stats` is about: 16 or 8."""
-    block = 8 if stats.dim() == 3 and stats.shape[1] == width // 8 else 16
-    _need(tuple(stats.shape) == (n_rows, width // block, 2) and width % block == 0 and stats.dtype == torch.float32 and stats.is_contiguous(),
-          lambda: f"{what}: stats")
-    return block
-
-
 def linear_norm_out(a, w, bias, residual, gamma, copy, stats):
     """residual += a @ w.T + bias (32-bit, in place), and what a LayerNorm of the updated rows with
     weight gamma needs: copy = the rows times gamma in bfloat16 (a tensor, or packed rows), stats =
-    each row's means and squared distances by blocks of 16 columns (up to 8 rows: or of 8, as stats has room for).  a: bfloat16 [M, K] in rows or
+    each row's means and squared distances by blocks of 16 columns.  a: bfloat16 [M, K] in rows or
     packed rows; w: PackedMatrix [N, K], N a multiple of 16."""
     _dev(residual, "residual", (torch.float32,), 2)
     M, K = a.shape
@@ -1046,8 +1032,8 @@ def linear_norm_out(a, w, bias, residual, gamma, copy, stats):
     _need(norm_stream_takes(M, N, w) and w.shape[1] == K and K % 8 == 0, "linear_norm_out: sizes it does not take")
     lda, ldcopy = _rows_or_packed(a, "a", M, K), _rows_or_packed(copy, "copy", M, N)
     _need(M > 16 or lda > 0, "linear_norm_out: up to 16 rows come in rows")
-    block = _stats_block(stats, M, N, "linear_norm_out")
-    _need(tuple(residual.shape) == (M, N) and (block == 16 or M <= 8), "linear_norm_out: residual or stats")
+    _need(tuple(residual.shape) == (M, N) and tuple(stats.shape) == (M, N // 16, 2) and stats.dtype == torch.float32
+          and stats.is_contiguous(), "linear_norm_out: residual or stats")
     for v, name in ((bias, "bias"), (gamma, "gamma")):
         if v is not None:
             _dev(v, name, (torch.float32,), 1)
@@ -1055,7 +1041,7 @@ def linear_norm_out(a, w, bias, residual, gamma, copy, stats):
     _need(gamma is not None, "linear_norm_out: gamma")
     _ok(_lib("gemm").dn_gemm_norm_out(a.data_ptr(), lda, w.data_ptr(), _ptr(bias), residual.data_ptr(),
                                       _rows(residual, "residual"), M, N, K, gamma.data_ptr(), copy.data_ptr(),
-                                      ldcopy, stats.data_ptr(), block, _stream()),
+                                      ldcopy, stats.data_ptr(), _stream()),
         "linear_norm_out" if _timed is None else f"linear {K} -> {N}, added into the stream, leaves the next norm's statistics")
     return residual
 
@@ -1077,8 +1063,8 @@ def linear_norm_in(copy, stats, c1, c2, eps, w, out, epilogue="none", kv=None, n
         ldc = _rows(out, "out")
     lda = _rows_or_packed(copy, "copy", M, K)
     _need(M > 16 or lda > 0, "linear_norm_in: up to 16 rows come in rows")
-    block = _stats_block(stats, M, K, "linear_norm_in")
-    _need(block == 16 or (M <= 16 and K <= 2048), "linear_norm_in: stats")
+    _need(tuple(stats.shape) == (M, K // 16, 2) and stats.dtype == torch.float32 and stats.is_contiguous(),
+          "linear_norm_in: stats")
     for v, name in ((c1, "c1"), (c2, "c2")):
         _dev(v, name, (torch.float32,), 1)
         _need(v.is_contiguous() and v.shape[0] == N, lambda: f"linear_norm_in: {name}")
@@ -1097,7 +1083,7 @@ def linear_norm_in(copy, stats, c1, c2, eps, w, out, epilogue="none", kv=None, n
         args = (slot_map.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), q_width, Hkv, dh, ps, out.shape[1])
     _ok(_lib("gemm").dn_gemm_norm_in(copy.data_ptr(), lda, stats.data_ptr(), c1.data_ptr(),
                                      c2.data_ptr(), float(eps), w.data_ptr(), out.data_ptr(), ldc,
-                                     M, N, K, EPILOGUES[epilogue], *args, int(bool(no_mean)), block, _stream()),
+                                     M, N, K, EPILOGUES[epilogue], *args, int(bool(no_mean)), _stream()),
         "linear_norm_in" if _timed is None else
         f"norm + linear {K} -> {N}" + (", cache write" if kv is not None else "") + (f", {epilogue}" if epilogue != "none" else ""))
     return out if kv is None else out[:, :kv[3]]

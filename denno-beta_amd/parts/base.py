@@ -143,8 +143,7 @@ class Part:
 
     def writes_norm_stats(self, n_rows: int) -> bool:
         """A mixer or feed-forward whose last kernel, as it adds into the residual stream, can leave
-        the statistics for the norm after it, by blocks of `stats_block(n_rows)` columns; its forward then takes `stats=` (a
-        StreamStats)."""
+        the statistics for the norm after it; its forward then takes `stats=` (a StreamStats)."""
         return False
 
     # helpers ---------------------------------------------------------------
@@ -154,7 +153,7 @@ class Part:
 
 class StreamStats:
     """What one norm of the residual stream's rows needs, left by the kernel that last added into
-    the stream: the rows times that norm's weight, rounded to bfloat16, and per row and block of 16 (or 8)
+    the stream: the rows times that norm's weight, rounded to bfloat16, and per row and block of 16
     columns the mean and the sum of squared distances from it (kernels.ops.linear_norm_out /
     linear_norm_in).  `norm` is the norm it was made for: nobody else may use it."""
 

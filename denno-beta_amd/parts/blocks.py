@@ -57,10 +57,10 @@ class PreNormBlock:
         if before is not None and not (before.written and before.norm is self.norm1
                                        and self.mixer.takes_lazy_norm(n, self.norm1)):
             before = None
-        between = (self._stats(x, self.norm2, self.mixer)
+        between = (self._stats(x, self.norm2)
                    if self.mixer.writes_norm_stats(n) and self.ffn.takes_lazy_norm(n, self.norm2) else None)
         nxt = runtime.next_norm
-        after = self._stats(x, nxt, self.ffn) if nxt is not None and self.ffn.writes_norm_stats(n) else None
+        after = self._stats(x, nxt) if nxt is not None and self.ffn.writes_norm_stats(n) else None
         runtime.stream_stats = None
         self.mixer.forward(self._normed(self.norm1, x, self.mixer, before, runtime, came), ctx, cache, accumulate_into=x,
                            **({"stats": between} if between is not None else {}),
@@ -74,11 +74,10 @@ class PreNormBlock:
         runtime.stream_deferred = end if end is not None and end.filled else None
 
     @staticmethod
-    def _stats(x, norm, part):
-        """What `part` fills for `norm`."""
+    def _stats(x, norm):
         if getattr(norm, "fused_params", None) is None:
             return None
-        return StreamStats(*ops.norm_stream_buffers(x.shape[0], x.shape[1], x.device, part.stats_block(x.shape[0])), norm)
+        return StreamStats(*ops.norm_stream_buffers(x.shape[0], x.shape[1], x.device), norm)
 
     @staticmethod
     def _normed(norm, x, part, stream, runtime, deferred=None):

@@ -70,9 +70,6 @@ class DenseMLP(Part):
     def writes_norm_stats(self, n_rows):
         return self.down.writes_norm_stats(n_rows)
 
-    def stats_block(self, n_rows):
-        return self.down.stats_block(n_rows)
-
     def defers_sum(self, n_rows):
         return self.down.defers(n_rows)
 

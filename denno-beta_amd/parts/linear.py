@@ -85,10 +85,6 @@ class Linear:
         """Whether a call with n_rows rows that adds into the residual stream can leave what the norm after it needs."""
         return ops.norm_stream_takes(n_rows, self.out_features, self.weight) and self.in_features % 8 == 0
 
-    def stats_block(self, n_rows: int) -> int:
-        """The columns that a pair of the statistics is about that a call with n_rows rows leaves (writes_norm_stats)."""
-        return ops.norm_stream_block(n_rows, self.weight)
-
     def defers(self, n_rows: int) -> bool:
         """Whether a call with n_rows rows that adds into the residual stream can leave its sum for the next norm's kernel."""
         return ops.linear_deferred_shares(n_rows, self.weight) > 0

@@ -143,9 +143,6 @@ class CausalSelfAttention(Part):
     def writes_norm_stats(self, n_rows):
         return self.out.writes_norm_stats(n_rows)
 
-    def stats_block(self, n_rows):
-        return self.out.stats_block(n_rows)
-
     def defers_sum(self, n_rows):
         return self.out.defers(n_rows)
 
