@@ -525,24 +525,22 @@ int shares_of_k(int M, int N, int K, int packed, bool kv) {
 
 // A product into the residual stream whose sum a norm's kernel adds (dn_gemm_deferred): the shares of K that it
 // is cut into, 0 if it is not worth it.  Few columns and 65 to 512 rows: the tiles are too few to fill the chip,
-// and with the shares' sums left for the next kernel to add nothing has to join them here.  Up to 256 rows: 4 where the chip takes as many
-// times the tiles of 64 x 64 at once (more means a second round for some) and each has 320 along K, since the norm reads every one of
-// them; else 2.  With the norm's kernel, weights that no cache holds, 2 shares -> 4, us: 136 rows, 1,280 columns from K = 5,120 17.2
-// -> 13.1; 256 rows, 1,024 from 4,096 14.5 -> 12.3; 256 rows, 768 from 3,072 12.5 -> 10.6; 72 rows, 1,600 from 1,600 10.2 -> 9.4, 128 rows
-// 10.7 -> 10.2.  Not: 203 rows, 1,600 from 6,400 (20.7 and 21.0), 1,280 from 5,120 (17.4 and 17.2), 256 rows, 1,024 from 1,024 (9.1 and
-// 9.3).  Left open: 3 shares, which would suit 60 to 85 tiles of a long K (203 rows, 1,280 from 5,120 14.7).
-// Beyond 256 rows: as many shares as make one round of 64 x 64 tiles, or, where that is one
+// and with the shares' sums left for the next kernel to add nothing has to join them here (1,600 x 1,600 at 128
+// and 256 rows: 4.8 and 6.2 us where the whole product takes 6.7 and 8.0; K = 6,400: the kernel that adds the
+// shares, 4.5 us, falls away).  Up to 256 rows a long K is cut as shares_of_k says, so that a row's sums do not depend on who adds the
+// shares (left open for it, with the norm's kernel, 2 shares -> 4, us: 136 rows, 1,280 columns from K = 5,120 17.2 -> 13.1; 256 rows, 1,024 from
+// 4,096 14.5 -> 12.3).  Beyond 256 rows: as many shares as make one round of 64 x 64 tiles, or, where that is one
 // share of a long K, two rounds in three shares or more (with the norm's kernel, weights that no cache holds, whole -> in shares: 320
 // rows x 1,280 columns, K = 5,120 31.6 -> 20.7 us in 2, 384 rows 31.8 -> 21.0, 512 rows 31.7 -> 24.8 in 3; 384 x 1,024, K = 4,096
 // 22.7 -> 15.5; K = 1,280 12.0 -> 11.0 at 320 rows.  Not: 512 rows x 1,600 columns, K = 6,400, 37.5 and 37.6 in 2; 512 x 1,280, K = 1,280,
 // 12.8 and 13.6).
 int deferred_shares(int M, int N, int K) {
   if (M <= 64 || M > 512 || N >= 2048 || K % 64 != 0) return 0;
-  const int tiles = ((M + 63) / 64) * ((N + 63) / 64), one = CUS / tiles, two = 2 * CUS / tiles;
   if (M <= 256) {
-    if (K >= 4096 && M <= 128) return 4;      // (at most 64 tiles)
-    return K >= 1280 && one >= 4 ? 4 : K / 64 >= 8 ? 2 : 0;
+    if (K >= 4096) return M <= 128 ? 4 : 2;
+    return K / 64 >= 8 ? 2 : 0;
   }
+  const int tiles = ((M + 63) / 64) * ((N + 63) / 64), one = CUS / tiles, two = 2 * CUS / tiles;
   if (K < 4096) return one >= 2 && K / 64 >= 16 ? 2 : 0;
   return one >= 2 ? min(one, 4) : two >= 3 ? 3 : 0;
 }

@@ -24,3 +24,16 @@ def test_shares_of_a_deferred_product(M, N, K, shares):
     w = ops.PackedMatrix(torch.empty(0, dtype=torch.bfloat16), (N, K))
     assert ops.linear_deferred_shares(M, w) == shares
     assert ops.linear_deferred_shares(M, torch.empty(0)) == 0
+
+
+@pytest.mark.parametrize("M", [65, 72, 128, 129, 136, 192, 203, 256])
+@pytest.mark.parametrize("N", [64, 768, 1024, 1280, 1600, 2032])
+def test_a_long_k_is_cut_alike_deferred_and_not(M, N):
+    """From K = 4,096 on the product that adds into the stream itself cuts K too: into the same shares, so that a row is the same bits with its
+    sum deferred and without."""
+    for K in (4096, 5120, 6400, 8192):
+        w = ops.PackedMatrix(torch.empty(0, dtype=torch.bfloat16), (N, K))
+        floats = ops._libs["gemm"].dn_gemm_work_floats(M, N, K, ops.PACKED_W)
+        assert floats == ops.linear_deferred_shares(M, w) * M * N, (M, N, K)
+    for K in (1280, 1600, 3072):      # (cut only where the sum is deferred)
+        assert ops.linear_deferred_shares(M, ops.PackedMatrix(torch.empty(0, dtype=torch.bfloat16), (N, K))) == 2
