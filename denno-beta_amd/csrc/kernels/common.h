@@ -95,6 +95,11 @@ __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf
 // log(1 + e^z), without overflow
 __device__ __forceinline__ float softplus_f(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 
+// v > 0: a v^2 + v / 2; else b (e^v - 1 - v) + v / 2
+__device__ __forceinline__ float xielu_f(float v, float a, float b) {
+  return v > 0.f ? fmaf(a * v, v, 0.5f * v) : fmaf(b, expm1f(v) - v, 0.5f * v);
+}
+
 static inline int dn_launch_status() { return static_cast<int>(hipGetLastError()); }
 
 // A packed matrix: blocks of 16 rows x 32 columns, 1 KB each and contiguous, block (r / 16, k / 32)

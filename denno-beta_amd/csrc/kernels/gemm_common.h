@@ -34,7 +34,7 @@ __device__ __forceinline__ float apply_epilogue_fast(float v, int epi) {
 }
 
 // Activations with numbers of their own (dn_gemm_act), in place of a kernel between two products; columns from `cols` on have none:
-//   EPI_XIELU             v > 0: p[0] v^2 + v / 2; else p[1] (e^v - 1 - v) + v / 2     (bfloat16 results)
+//   EPI_XIELU             xielu_f(v, p[0], p[1])     (bfloat16 results)
 //   EPI_SILU              v sigmoid(v)
 //   EPI_EXP_NEG_SOFTPLUS  exp(-p[column] log(1 + e^v))
 #define EPI_XIELU 4
@@ -53,19 +53,6 @@ struct Ends {
   int ldc2, a_shift;
 };
 
-// e^v - 1 - v for v <= 0 without its cancellation near 0: the series there (2e-7 of the result at most), the hardware's exponential
-// beyond.  Some fifteen instructions where expm1f takes several dozen, which shows in the epilogue of a product with many columns.
-__device__ __forceinline__ float xielu_fast(float v, float a, float b) {
-  float s = fmaf(v, 1.0f / 40320.0f, 1.0f / 5040.0f);
-  s = fmaf(s, v, 1.0f / 720.0f);
-  s = fmaf(s, v, 1.0f / 120.0f);
-  s = fmaf(s, v, 1.0f / 24.0f);
-  s = fmaf(s, v, 1.0f / 6.0f);
-  s = fmaf(s, v, 0.5f);
-  const float near = s * v * v, far = __builtin_amdgcn_exp2f(1.4426950408889634f * v) - 1.0f - v;
-  return v > 0.f ? fmaf(a * v, v, 0.5f * v) : fmaf(b, v > -0.5f ? near : far, 0.5f * v);
-}
-
 // the numbers that an element's activation wants, asked for before the product, and the activation
 template <typename TC, int END, typename E>
 __device__ __forceinline__ float2 end_numbers(const E& ends, int column) {
@@ -75,7 +62,7 @@ __device__ __forceinline__ float2 end_numbers(const E& ends, int column) {
 }
 template <typename TC, int END, typename E>
 __device__ __forceinline__ float end_value(float v, int epi, int column, const E& ends, const float2& n) {
-  if constexpr (END == END_ACT && sizeof(TC) == 2) return xielu_fast(v, n.x, n.y);
+  if constexpr (END == END_ACT && sizeof(TC) == 2) return xielu_f(v, n.x, n.y);
   if constexpr (END == END_ACT && sizeof(TC) == 4) return column < ends.cols ? v * sigmoid_f(v) : v;
   if constexpr (END == END_PAIR) return column < ends.cols ? expf(-n.x * softplus_f(v)) : v;
   return END == END_PLAIN ? apply_epilogue_fast(v, epi) : v;

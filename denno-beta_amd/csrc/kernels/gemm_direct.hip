@@ -349,7 +349,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
         for (int r = 0; r < 4; ++r) o[r] = apply_epilogue_fast(v[r], epi);
         *reinterpret_cast<floatx4*>(C + static_cast<size_t>(m) * ldc + n) = o;
       } else {
-        auto finish = [&](float e) { return XIELU ? xielu_fast(e, act_a, act_b) : apply_epilogue_fast(e, epi); };
+        auto finish = [&](float e) { return XIELU ? xielu_f(e, act_a, act_b) : apply_epilogue_fast(e, epi); };
         const uint2 cv = pack4(finish(v[0]), finish(v[1]), finish(v[2]), finish(v[3]));
         // (in packed rows, four columns from a multiple of 4 are 8 bytes side by side too)
         if (!KV || n < kv.c_cols)

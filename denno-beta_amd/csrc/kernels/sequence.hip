@@ -714,7 +714,7 @@ __global__ __launch_bounds__(256) void activate_kernel(const float* x, size_t ld
     if (c >= n) break;
     const float v = z[i] + b[i];
     if (kind == ACT_XIELU)
-      store_as(out, t * ldo + c, out_dt, v > 0.f ? fmaf(two[0] * v, v, 0.5f * v) : fmaf(two[1], expm1f(v) - v, 0.5f * v));
+      store_as(out, t * ldo + c, out_dt, xielu_f(v, two[0], two[1]));
     else
       store_as(out, t * ldo + c, out_dt, activation(kind, v, l[i]));
   }
@@ -729,7 +729,7 @@ __global__ __launch_bounds__(256) void activate_narrow_kernel(const float* x, si
     const float a = lower[0], b = lower[1];
     for (int c = threadIdx.x; c < n; c += 256) {
       const float z = x[t * ldx + c] + (bias ? bias[c] : 0.f);
-      store_as(out, t * ldo + c, out_dt, z > 0.f ? fmaf(a * z, z, 0.5f * z) : fmaf(b, expm1f(z) - z, 0.5f * z));
+      store_as(out, t * ldo + c, out_dt, xielu_f(z, a, b));
     }
     return;
   }

@@ -52,6 +52,19 @@ def test_xielu_of_large_infinite_and_missing_values():
         assert torch.allclose(out[both].float(), ref[both].float(), rtol=2.0 ** -7, atol=1e-30)
 
 
+@pytest.mark.parametrize("M", ROWS)
+@pytest.mark.parametrize("N,K", [(2048, 512), (4096, 1024), (100, 72), (8192, 2048)])
+def test_xielu_has_the_bits_of_two_kernels(M, N, K):
+    from denno_beta_amd.kernels import ops
+    a, w, bias, _ = _operands(M, N, K)
+    numbers = torch.tensor([0.9, 1.3], device="cuda")
+    for b in (None, bias):
+        out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        z = ops.linear(a, w, b, out=torch.empty(M, N, device="cuda"))
+        if ops.linear_act(a, w, "xielu", out, bias=b, numbers=numbers):
+            assert torch.equal(out, ops.activate(z, "xielu", torch.empty_like(out), lower=numbers))
+
+
 @pytest.mark.parametrize("M", [1, 2, 8, 9, 16, 17, 33, 64, 65, 300])
 @pytest.mark.parametrize("N,K", [(1024, 64), (3072, 1024), (56, 40)])
 def test_silu_and_decays_have_the_bits_of_two_kernels(M, N, K):
