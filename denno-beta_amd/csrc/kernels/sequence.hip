@@ -486,8 +486,9 @@ __global__ __launch_bounds__(256) void rotary_runs_kernel(const void* src, int s
         const float ang = p * freq[i];
         const float c = cosf(ang) * mag, sn = sinf(ang) * mag;
         const float x = load_as(src, a + 2 * i, src_dt), y = load_as(src, a + 2 * i + 1, src_dt);
-        store_as(u.dst, b + 2 * i, u.dst_dt, x * c - y * sn);
-        store_as(u.dst, b + 2 * i + 1, u.dst_dt, y * c + x * sn);
+        // (which of a sum's two products is rounded by itself is said here: norm_turn_write_kernel makes the same bits)
+        store_as(u.dst, b + 2 * i, u.dst_dt, fmaf(x, c, -(y * sn)));
+        store_as(u.dst, b + 2 * i + 1, u.dst_dt, fmaf(x, sn, y * c));
       } else {
         const int k = u.dims + (i - half);
         store_as(u.dst, b + k, u.dst_dt, load_as(src, a + k, src_dt));
@@ -1615,6 +1616,7 @@ struct NormTurnArgs {
   const int* slot_map;
   void *k_pool, *v_pool;
   int page_size, dt, write;
+  int as_runs;      // a pair's second result is rounded as rotary_runs_kernel rounds it (y c first), else with x s first
 };
 
 // two neighbours from an even place
@@ -1680,8 +1682,8 @@ __global__ __launch_bounds__(256) void norm_turn_write_kernel(NormTurnArgs a) {
       }
       if (i < turned) {
         const float c = cs[base + i], s = sn[base + i];
-        const float u = x * c - y * s;
-        y = y * c + x * s;
+        const float u = fmaf(x, c, -(y * s));
+        y = a.as_runs ? fmaf(x, s, y * c) : fmaf(y, c, x * s);
         x = u;
       }
       if (is_q) {
@@ -2715,7 +2717,7 @@ int dn_norm_pair_write(const float* z, long long ldz, int qw, int kw, const floa
 int dn_norm_turn_write(const float* z, long long ldz, int H, int G, int dk, int dv, const float* wq, const float* wk, const float* q_scale,
                        float pos_coef, double pos_every, float eps, const float* freq, int dims, const float* v_freq, int v_dims, const int* positions, void* q_out,
                        long long ldq, int kept, const int* slot_map, void* k_pool, void* v_pool, int T, int page_size, int dt, int write,
-                       hipStream_t stream) {
+                       int as_runs, hipStream_t stream) {
   if (!float_kind(dt)) return DN_ERR_DTYPE;
   if (H < 1 || G < 1 || dk < 1 || dv < 1 || kept > 256 || kept % 2 != 0 || dk > kept || dv > kept || dims < 0 || dims % 2 != 0 || dims > dk ||
       v_dims < 0 || v_dims % 2 != 0 || v_dims > dv || (dims > 0 && !freq) || (v_dims > 0 && !v_freq) || page_size < 1 ||
@@ -2725,7 +2727,7 @@ int dn_norm_turn_write(const float* z, long long ldz, int H, int G, int dk, int 
   if (T == 0) return 0;
   if (pos_coef != 0.f && !(pos_every > 0.0)) return DN_ERR_SHAPE;
   const NormTurnArgs a{z, static_cast<size_t>(ldz), H, G, dk, dv, wq, wk, q_scale, pos_coef, pos_every, eps, freq, dims, v_freq, v_dims, positions, q_out,
-                       static_cast<size_t>(ldq), kept, slot_map, k_pool, v_pool, page_size, dt, write};
+                       static_cast<size_t>(ldq), kept, slot_map, k_pool, v_pool, page_size, dt, write, as_runs};
   // (few rows: the vectors of a row spread over workgroups, so that a step of decoded tokens is more than a handful of them; many
   // rows: one workgroup a row, whose angles are made once.  By the sizes alone a vector has 32 or 64 lanes: the same bits either way)
   const int at_once = kept <= 64 ? 8 : 4, groups = T <= 256 ? (H + 2 * G + at_once - 1) / at_once : 1;

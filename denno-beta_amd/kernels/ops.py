@@ -155,7 +155,7 @@ def _declare(name, lib):
             "dn_streams_read": [P, c_longlong, I, P, P, F, P, I, c_longlong, P, I, I, P],
             "dn_streams_write": [P, c_longlong, I, P, P, P, c_longlong, P, c_longlong, P, P, F, P, I, P, P, F, P, I, c_longlong, I, I, P],
             "dn_norm_pair_write": [P, c_longlong, I, I, P, P, F, P, c_longlong, P, P, P, I, I, I, I, I, I, I, P],
-            "dn_norm_turn_write": [P, c_longlong, I, I, I, I, P, P, P, F, c_double, F, P, I, P, I, P, P, c_longlong, I, P, P, P, I, I, I, I, P],
+            "dn_norm_turn_write": [P, c_longlong, I, I, I, I, P, P, P, F, c_double, F, P, I, P, I, P, P, c_longlong, I, P, P, P, I, I, I, I, I, P],
             "dn_conv_turn_write": [P, c_longlong, I, I, I, I, P, I, P, c_longlong, P, P, I, P, P, F, P, I, P, P, c_longlong, I, P, P, P, I, I, I, I, I, P],
             "dn_clamped_glu": [P, c_longlong, F, F, P, I, c_longlong, I, I, P],
             "dn_post_norm": [P, c_longlong, F, P, c_longlong, P, c_longlong, P, P, F, P, P, I, I, P, P, F, P, I, c_longlong, I, I, P],
@@ -1668,13 +1668,13 @@ def norm_pair_write(z, q_width, wq, wk, eps, q_out, slot_map, k_pool, v_pool, wr
 
 
 def norm_turn_write(z, n_heads, n_kv, dk, dv, positions, q_out, slot_map, k_pool, v_pool, wq=None, wk=None, eps=None, q_scale=None,
-                    freq=None, v_freq=None, write=True, q_by_position=None):
+                    freq=None, v_freq=None, write=True, q_by_position=None, as_runs=False):
     """A row of z (32-bit) begins with [q: n_heads x dk | k: n_kv x dk | v: n_kv x dv].  Every query and key is x / sqrt(mean(x^2) + eps)
     (eps None: x) times wq or wk (dk numbers shared by the heads, or None), then its first 2 len(freq) entries are turned in pairs (2i, 2i + 1) by
     positions[t] * freq[i]; a value's first 2 len(v_freq) entries likewise.  Queries times q_scale[head] go to q_out (heads side by
     side, as wide as the pools' keys), keys to k_pool [pages, n_kv, page, width], values to v_pool [pages, n_kv, width, page];
     the columns a vector does not have are zeros.  slot_map as in norm_pair_write.  q_by_position = (coef, every): queries are also multiplied
-    by 1 + coef * ln(floor((positions[t] + 1) / every) + 1).  One launch."""
+    by 1 + coef * ln(floor((positions[t] + 1) / every) + 1).  as_runs: turned pairs are the bits of rotary_runs.  One launch."""
     _dev(z, "z", (torch.float32,), 2), _dev(q_out, "q_out", _FLOATS, 2), _dev(slot_map, "slot_map", _I32, 1), _dev(positions, "positions", _I32, 1)
     _dev(k_pool, "k_pool", (q_out.dtype,), 4), _dev(v_pool, "v_pool", (q_out.dtype,), 4)
     T = z.shape[0]
@@ -1691,7 +1691,7 @@ def norm_turn_write(z, n_heads, n_kv, dk, dv, positions, q_out, slot_map, k_pool
     _ok(_lib("sequence").dn_norm_turn_write(z.data_ptr(), _rows(z, "z"), n_heads, n_kv, dk, dv, _ptr(wq), _ptr(wk), _ptr(q_scale),
                                             coef, every, -1.0 if eps is None else float(eps), _ptr(freq), dims, _ptr(v_freq), v_dims, positions.data_ptr(), q_out.data_ptr(),
                                             _rows(q_out, "q_out"), kept, slot_map.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), T, ps,
-                                            _CODE[q_out.dtype], int(bool(write)), _stream()), "norm_turn_write")
+                                            _CODE[q_out.dtype], int(bool(write)), int(bool(as_runs)), _stream()), "norm_turn_write")
     return q_out
 
 

@@ -163,7 +163,7 @@ class CausalSelfAttention(Part):
         # factor on cos and sin, and its norm stands in front of the turn)
         if not unit and mag == 1.0:
             q = ops.norm_turn_write(z, H, G, dk, dv, ctx.positions, torch.empty((T, H * hw), dtype=act, device=dev), g.slot_map, cache.k, cache.v,
-                                    freq=freq if dims else None, write=cache.writes)
+                                    freq=freq if dims else None, write=cache.writes, as_runs=True)
         else:
             new = torch.zeros if hw != dk or hw != dv else torch.empty
             q = new((T, H * hw), dtype=act, device=dev)

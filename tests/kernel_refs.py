@@ -578,7 +578,7 @@ def _turned(x, positions, freq, sign=1.0):
 
 
 def norm_turn_write(z, n_heads, n_kv, dk, dv, positions, q_out, slot_map, k_pool, v_pool, wq=None, wk=None, eps=None, q_scale=None,
-                    freq=None, v_freq=None, write=True, q_by_position=None):
+                    freq=None, v_freq=None, write=True, q_by_position=None, as_runs=False):
     T, kept, ps = z.shape[0], k_pool.shape[3], k_pool.shape[2]
     zd = z.double()
     q = zd[:, :n_heads * dk].reshape(T, n_heads, dk)
