@@ -129,7 +129,9 @@ class Linear:
 
     def activated(self, a, kind, out_dtype, bias=None, numbers=None, cols=None):
         """ops.linear_act of the rows `a` with this weight and its bias (or the one given) as a new tensor of out_dtype, or None where
-        no kernel does both."""
+        no kernel does both (no kernel has a norm inside as well: a LazyNorm's rows are made first)."""
+        if isinstance(a, LazyNorm):
+            a = a.rows(packed=self.packed_input(a.shape[0]))
         if not isinstance(self.weight, ops.PackedMatrix) or a.dtype != self.weight.dtype:
             return None
         out = torch.empty((a.shape[0], self.out_features), dtype=out_dtype, device=a.device)

@@ -120,3 +120,28 @@ def test_matrices_that_do_not_stack():
     _, w1, _, make = _operands(1, 24, 64)      # (24 rows are one and a half blocks)
     _, w2, _, _ = _operands(1, 16, 72)
     assert ops.stacked(w1, w1) is None and ops.stacked(w2, w1) is None and ops.stacked(make(16, 64).bfloat16(), w1) is None
+
+
+@pytest.mark.parametrize("M", [1, 8, 16, 17, 64])
+def test_xielu_behind_a_norm_that_is_left_to_the_product(M):
+    """A feed-forward with xielu is handed a norm of the stream that nobody has run yet (steps of few rows): the same bits as with its rows."""
+    from denno_beta_amd.kernels import ops
+    from denno_beta_amd.parts import FEED_FORWARDS, NORMS
+    from denno_beta_amd.parts.base import LazyNorm, Runtime, StreamStats
+    W, inner = 1024, 2048
+    g = torch.Generator(device="cuda").manual_seed(M)
+    make = lambda *s: torch.randn(*s, generator=g, device="cuda")   # noqa: E731
+    tensors = dict(up=(make(inner, W) * W ** -0.5).bfloat16(), down=(make(W, inner) * inner ** -0.5).bfloat16(), numbers=make(2), gamma=1 + 0.1 * make(W))
+    runtime = Runtime(torch.bfloat16, torch.device("cuda"))
+    ffn = FEED_FORWARDS.make(("dense_mlp", dict(width=W, inner=inner, activation="xielu", up_weight="up", up_bias=None, down_weight="down", down_bias=None,
+                                                activation_params="numbers")))
+    norm = NORMS.make(("layernorm", dict(width=W, eps=1e-5, weight_name="gamma")))
+    ffn.bind(tensors, runtime), norm.bind(tensors, runtime)
+    ffn.prepare_lazy_norm(norm)
+    x, stream = make(M, W), StreamStats(*ops.norm_stream_buffers(M, W, "cuda"), norm)
+    stream.written = True
+    assert ffn.takes_lazy_norm(M, norm)
+    mine, want = x.clone(), x.clone()
+    ffn.forward(LazyNorm(norm, x, torch.bfloat16, stream), None, mine)
+    ffn.forward(norm.forward(x, torch.bfloat16), None, want)
+    assert torch.equal(mine, want) and not torch.equal(mine, x)
