@@ -93,6 +93,11 @@ __device__ __forceinline__ void late_at_hand(const Late<END>& late) {
   if constexpr (END == END_TWO) asm volatile("" ::"s"(late.ends.C2), "s"(late.ends.ldc2), "s"(late.ends.cols));
 }
 
+// What a load of W's step beyond K reads (no load is conditional): a packed block of zeros, so that the step adds nothing whatever the weights are.
+// (A block of W's own times zeros of A would do for finite weights; one infinity in it, and every column of the product is not a number.)
+__device__ uint4 zero_block[64];
+__device__ __forceinline__ const bf16_t* no_step(int lane) { return reinterpret_cast<const bf16_t*>(&zero_block[lane]); }
+
 // MB row blocks and NB column blocks of 16 per workgroup; U steps of K in flight per wave.
 template <int MB, int NB, int WAVES, int U, typename TC, bool KV, int NORM = NORM_NONE, int END = END_PLAIN>
 __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int M, int N, int K, int packed,
@@ -168,7 +173,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   }
   // Loads are never conditional and nothing uses a loaded value before all loads of a round are
   // issued (a predicated load, or a use in between, makes each load wait for the one before it).
-  // A step beyond K reads W's first block instead (finite numbers) and meets a zeroed piece of A.
+  // A step beyond K reads zeros (no_step) and meets a zeroed piece of A.
   // The first round of W is on its way while the rest of the prologue works.
   bf16x8 b[U][NB];
 #pragma unroll
@@ -176,7 +181,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
     const int ks = 2 * (wave + (u / 2) * WAVES) + u % 2;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
-      b[u][nb] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk[nb] + ks * 512 : W + lane * 8);
+      b[u][nb] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk[nb] + ks * 512 : no_step(lane));
   }
   // what the epilogue reads by arguments that do not come with the launch: behind the first round of W
 #pragma unroll
@@ -252,7 +257,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
       if (p0 != wave) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
-          b[u][nb] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk[nb] + ks * 512 : W + lane * 8);
+          b[u][nb] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk[nb] + ks * 512 : no_step(lane));
       }
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
@@ -412,7 +417,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
       for (int i = 0; i < SP; ++i) st[t][i] = *reinterpret_cast<const float2*>(stats_in + (row + min(lane + 64 * i, blocks_in - 1)) * 2);
     }
   }
-  // never a conditional load; a step beyond K reads W's first block and meets zeros of A
+  // never a conditional load; a step beyond K reads zeros and meets zeros of A
   const int lrow = lane / 8, lch = lane % 8;               // as loader: row and 16-byte chunk of the pair's 128 bytes
   const bf16_t* a0 = A + static_cast<size_t>(min(lrow, M - 1)) * lda + lch * 8;
   const bf16_t* a1 = A + static_cast<size_t>(min(lrow + 8, M - 1)) * lda + lch * 8;
@@ -428,8 +433,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm16_kernel(const bf16_t* __rest
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int p = p0 + u * WAVES, ks = 2 * p;
-      b[u][0] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk + ks * 512 : W + lane * 8);
-      b[u][1] = *reinterpret_cast<const bf16x8*>(ks + 1 < ksteps ? wblk + (ks + 1) * 512 : W + lane * 8);
+      b[u][0] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk + ks * 512 : no_step(lane));
+      b[u][1] = *reinterpret_cast<const bf16x8*>(ks + 1 < ksteps ? wblk + (ks + 1) * 512 : no_step(lane));
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -584,7 +589,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
     if (bias) epi_bias = bias[c];
     if (resid) epi_x = resid[static_cast<size_t>(min(mm, M - 1)) * ldr + c];
   }
-  // never a conditional load; a step beyond K reads W's first block and meets zeros of A, whose chunks beyond K come from the row's start
+  // never a conditional load; a step beyond K reads zeros and meets zeros of A, whose chunks beyond K come from the row's start
   const int lrow = lane / 8, lch = lane % 8;               // as loader: row and 16-byte chunk of the pair's 128 bytes
   const bf16_t* asafe = A + static_cast<size_t>(min(lrow, M - 1)) * lda;
   const bf16_t* a0 = asafe + lch * 8;
@@ -596,7 +601,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm8_kernel(const bf16_t* __restr
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int step = 2 * (p0 + u * WAVES) + second;
-      b[u] = *reinterpret_cast<const u32x4*>(step < ksteps ? wblk + static_cast<size_t>(step) * 512 : W + lane * 8);
+      b[u] = *reinterpret_cast<const u32x4*>(step < ksteps ? wblk + static_cast<size_t>(step) * 512 : no_step(lane));
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
