@@ -742,8 +742,11 @@ static void launch16_ahead(const Call& c, const NormIO& nio, hipStream_t stream)
 
 template <int WAVES, typename TC, bool KV, int NORM = NORM_NONE, int END = END_PLAIN>
 static void launch16_one(const Call& c, const NormIO& nio, hipStream_t stream) {
-  switch (pairs_ahead<WAVES>(c.K, 4)) {
-    case 1: return launch16_ahead<WAVES, 1, TC, KV, NORM, END>(c, nio, stream);
+  const int ahead = pairs_ahead<WAVES>(c.K, 4);
+  if constexpr (WAVES == 4) {      // (eight waves: K of 1,024 and more, at least two pairs each)
+    if (ahead == 1) return launch16_ahead<WAVES, 1, TC, KV, NORM, END>(c, nio, stream);
+  }
+  switch (ahead) {
     case 2: return launch16_ahead<WAVES, 2, TC, KV, NORM, END>(c, nio, stream);
     case 3: return launch16_ahead<WAVES, 3, TC, KV, NORM, END>(c, nio, stream);
     default: return launch16_ahead<WAVES, 4, TC, KV, NORM, END>(c, nio, stream);
@@ -763,19 +766,28 @@ static void launch8(const Call& c, hipStream_t stream) {
   const First f = first_of(c, NormIO{}, NORM_NONE);
 #define DN_L8(U)                                                                                                          \
   case U:                                                                                                                 \
-    hipLaunchKernelGGL((gemm8_kernel<WAVES, U, TC>), dim3((c.N + 7) / 8), dim3(WAVES * 64), 0, stream,              \
+    hipLaunchKernelGGL((gemm8_kernel<WAVES, U, TC>), dim3((c.N + 7) / 8), dim3(WAVES * 64), 0, stream,                    \
                        static_cast<const bf16_t*>(c.A), static_cast<const bf16_t*>(c.W), c.lda, f.rows, c.N, c.K, f.p,    \
-                       c.bias, f.q, late_of<END_PLAIN>(c, NormIO{}));                                                        \
+                       c.bias, f.q, late_of<END_PLAIN>(c, NormIO{}));                                                     \
     break
-  switch (pairs_ahead<WAVES>(c.K, 8)) {
-    DN_L8(1);
-    DN_L8(2);
-    DN_L8(3);
-    DN_L8(4);
-    DN_L8(5);
-    DN_L8(6);
-    DN_L8(7);
-    DN_L8(8);
+  const int ahead = pairs_ahead<WAVES>(c.K, 8);
+  if constexpr (WAVES == 4) {      // (K below 1,024: at most four pairs a wave; eight waves have at least two)
+    switch (ahead) {
+      DN_L8(1);
+      DN_L8(2);
+      DN_L8(3);
+      DN_L8(4);
+    }
+  } else {
+    switch (ahead) {
+      DN_L8(2);
+      DN_L8(3);
+      DN_L8(4);
+      DN_L8(5);
+      DN_L8(6);
+      DN_L8(7);
+      DN_L8(8);
+    }
   }
 #undef DN_L8
 }
