@@ -12,6 +12,8 @@ import math
 
 import torch
 
+from denno_beta_amd.kernels.ops import OpenPlanes
+
 
 def embed(tokens, positions, wte, wpe, out, token_scale=1.0):
     x = wte[tokens.long()].float()
@@ -291,10 +293,17 @@ def rmsnorm_add(y, weight, scale, mult, eps, x, gate=None, then=None):
 
 
 def depth_mix(hist, n, weights, out):
+    planes = hist if isinstance(hist, OpenPlanes) else None
+    if planes is not None:
+        one_kernel = planes.add is not None and planes.hist.shape[2] <= 4096 and planes.last == n - 1
+        hist = planes.close()
     acc = torch.zeros_like(hist[0])
     for j in range(n):
         acc = acc + weights[j] * hist[j]
     out.copy_(acc)
+    if planes is not None and one_kernel and planes.then is not None:      # (the norm that reads the average next)
+        _then(planes.then, out)
+        planes.normed = planes.then[2]
     return out
 
 

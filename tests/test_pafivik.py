@@ -308,6 +308,29 @@ def test_the_stream_after_every_layer(backend, folders):
         assert d < 2e-5, f"the stream behind layer {i} differs by {d:.3g} of its largest entry"
 
 
+def test_the_average_takes_the_last_result_and_hands_on_normed_rows(backend, folders, monkeypatch):
+    """With the last sublayer's result, the average and the next layer's norm in one kernel, and one after the other: the same logits."""
+    from denno_beta_amd.kernels import ops
+    from denno_beta_amd.parts.blocks import SandwichBlock
+    folder = folders("P", "float32")
+    seq = seqs_for(CONFIGS["P"][0], [19], seed=12)[0]
+    handed, real = [], ops.depth_mix
+
+    def spy(hist, n, weights, out):
+        res = real(hist, n, weights, out)
+        handed.append(isinstance(hist, ops.OpenPlanes) and hist.normed is not None)
+        return res
+    r = runner_for(folder, "float32", backend, 64)
+    monkeypatch.setattr(ops, "depth_mix", spy)
+    one = U.replay(r, U.whole_trace([seq]))
+    assert sum(handed) == len(CONFIGS["P"][0]["layers"]) - 1      # (every layer but the last has a layer's norm behind its average)
+    monkeypatch.setattr(SandwichBlock, "opens_planes", False)
+    handed.clear()
+    apart = U.replay(r, U.whole_trace([seq]))
+    assert not any(handed) and len(handed) > 1
+    assert one.keys() == apart.keys() and all(torch.equal(one[k], apart[k]) for k in one)
+
+
 # ----------------------------------------------------------------------------------------------------------------
 # far tokens: weights made so that losing one shows
 # ----------------------------------------------------------------------------------------------------------------
