@@ -29,3 +29,19 @@ def test_the_bits_of_sixteen_columns(N, K):
     want = ops.linear(a, w, bias, residual=x0.clone())
     for M in (1, 3, 8):
         assert torch.equal(ops.linear(a[:M], w, bias, residual=x0[:M].clone()), want[:M]), M
+
+
+@pytest.mark.parametrize("N,K", SIZES)
+def test_against_64_bits(N, K):
+    from denno_beta_amd.kernels import ops
+    a, w, bias, make = _case(N, K)
+    a, x0, rows = a[:8], make(8, N), w.rows().double()
+    exact, size = a.double() @ rows.t() + bias.double(), a.double().abs() @ rows.abs().t() + bias.double().abs()
+    # (sums of K products in 32 bits: every partial sum lies within the sum of the magnitudes, and K + 2 of them are rounded)
+    bound = (K + 2) * 2.0 ** -23 * size
+    for M in (1, 5, 8):
+        got = ops.linear(a[:M], w, bias, out=torch.empty(M, N, device="cuda"))
+        assert bool(((got.double() - exact[:M]).abs() <= bound[:M]).all())
+        into = ops.linear(a[:M], w, bias, residual=x0[:M].clone())
+        total = x0[:M].double() + exact[:M]
+        assert bool(((into.double() - total).abs() <= bound[:M] + 2.0 ** -23 * total.abs()).all())

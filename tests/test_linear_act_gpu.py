@@ -63,6 +63,8 @@ def test_xielu_has_the_bits_of_two_kernels(M, N, K):
         z = ops.linear(a, w, b, out=torch.empty(M, N, device="cuda"))
         if ops.linear_act(a, w, "xielu", out, bias=b, numbers=numbers):
             assert torch.equal(out, ops.activate(z, "xielu", torch.empty_like(out), lower=numbers))
+        else:
+            assert M > 64 and (M <= 256 or K % 32 != 0)
 
 
 @pytest.mark.parametrize("M", [1, 2, 8, 9, 16, 17, 33, 64, 65, 300])
@@ -94,10 +96,11 @@ def test_two_products_of_the_same_rows(M, first, rest, K):
     both, v1, v2 = ops.stacked(w1, w2)
     assert torch.equal(v1.rows(), w1.rows()) and torch.equal(v2.rows(), w2.rows()) and both.shape == (first + rest, K)
     low, z = ops.linear_two(a, both, first)
-    # (the same kernel for both lays a sum out in another order only where K is cut among more waves)
     one = ops.linear(a, both, out=torch.empty(M, first + rest, device="cuda"))
     assert torch.equal(z, one[:, first:]) and torch.equal(low, one[:, :first].bfloat16())
-    assert torch.allclose(z, ops.linear(a, w2, out=torch.empty(M, rest, device="cuda")), rtol=1e-4, atol=1e-5)
+    # (up to 64 rows the order of a sum follows from K alone: the products one after the other have the same bits)
+    assert torch.equal(z, ops.linear(a, w2, out=torch.empty(M, rest, device="cuda")))
+    assert torch.equal(low, ops.linear(a, w1, out=torch.empty(M, first, dtype=torch.bfloat16, device="cuda")))
 
 
 @pytest.mark.parametrize("M", [1, 2, 8, 9, 16, 17, 33, 64])
@@ -109,8 +112,8 @@ def test_two_products_of_neighbouring_columns(M, n1, n2, K):
     both = ops.stacked(w1, w2)[0]
     g, gate = ops.linear_pair(low, both, n1, bias, rate)
     z = ops.linear(low[:, :K], w1, out=torch.empty(M, n1, device="cuda"))
-    assert torch.allclose(g, ops.activate(z, "exp_neg_softplus", torch.empty_like(z), bias=bias[:n1], lower=rate), rtol=1e-5, atol=1e-6)
-    assert torch.allclose(gate, ops.linear(low[:, K:], w2, bias[n1:].contiguous(), out=torch.empty(M, n2, device="cuda")), rtol=1e-5, atol=1e-6)
+    assert torch.equal(g, ops.activate(z, "exp_neg_softplus", torch.empty_like(z), bias=bias[:n1].contiguous(), lower=rate))
+    assert torch.equal(gate, ops.linear(low[:, K:], w2, bias[n1:].contiguous(), out=torch.empty(M, n2, device="cuda")))
     with pytest.raises(Exception):      # (a bias for the first columns only: the kernel would read beyond it)
         ops.linear_pair(low, both, n1, bias[:n1], rate)
 
