@@ -11,6 +11,7 @@ from ..kernels import ops
 import torch
 
 from .base import ARRANGEMENTS, DeferredSum, LazyNorm, StreamStats
+from .norms import StreamRMSNorm
 
 
 @ARRANGEMENTS.register("pre_norm")
@@ -216,6 +217,20 @@ class SandwichBlock:
         part.forward(*args, accumulate_into=y)
         return y
 
+    @staticmethod
+    def _hands_on(post):
+        """Whether `post` adds into the stream as the framework's own kind does, whose kernels make a norm of the rows behind it too; of
+        another kind, or one that changes this step, nothing but add_into(y, x) is asked."""
+        return getattr(type(post), "add_into", None) is StreamRMSNorm.add_into
+
+    @classmethod
+    def _behind(cls, post, y, x, then, act):
+        """The result y goes into the stream -> the rows of the norm `then` where the same kernel made them, else None."""
+        if cls._hands_on(post):
+            return post.add_into(y, x, then=then, out_dtype=act)
+        post.add_into(y, x)
+        return None
+
     def first_norm(self):
         """The norm that reads the residual stream first in this block."""
         return self.norm1
@@ -230,14 +245,14 @@ class SandwichBlock:
         h = came[1] if came is not None and came[0] is self.norm1 else self.norm1.forward(x, act)
         y, post, nxt = self._result(self.mixer, x, h, ctx, caches[0]), self.post1, runtime.next_norm
         if self.has_ffn:
-            h = post.add_into(y, x, then=self.norm2, out_dtype=act)
+            h = self._behind(post, y, x, self.norm2, act)
             if h is None:
                 h = self.norm2.forward(x, act)
             y, post = self._result(self.ffn, x, h, ctx), self.post2
-        if runtime.average is not None:
+        if runtime.average is not None and self._hands_on(post):
             runtime.average = post.open_planes(y, *runtime.average, then=nxt, out_dtype=act)
             return
-        h = post.add_into(y, x, then=nxt, out_dtype=act)
+        h = self._behind(post, y, x, nxt, act)
         if h is not None and nxt is not None:
             runtime.normed_rows = (nxt, h)
 

@@ -331,7 +331,7 @@ class DecoderModel:
                 rt.stream_stats = rt.stream_deferred = rt.normed_rows = rt.stream_cast = None
                 if not own:
                     kept[i + 1].copy_(x)
-                planes, rt.average = rt.average, None
+                planes, rt.average = rt.average if isinstance(rt.average, ops.OpenPlanes) else None, None      # (else the block left nothing)
                 w = self.averages.get(i)
                 if w is None and planes is not None:
                     planes.close()

@@ -331,6 +331,63 @@ def test_the_average_takes_the_last_result_and_hands_on_normed_rows(backend, fol
     assert one.keys() == apart.keys() and all(torch.equal(one[k], apart[k]) for k in one)
 
 
+def test_a_norm_that_only_adds_into_the_stream_may_stand_behind_a_sublayer(backend):
+    """What an arrangement asks of the norm behind a sublayer is `add_into(y, x)`: a kind of one's own with nothing more, and one that
+    changes the framework's own, run in the model as the framework's own does, averages over depth included; and so does an
+    arrangement of one's own that goes on from the framework's and leaves nothing to the average's kernel."""
+    from denno_beta_amd.config import EngineOptions
+    from denno_beta_amd.engine import ModelRunner
+    from denno_beta_amd.models.pafivik import PafivikConfig, build_pafivik
+    from denno_beta_amd.parts import ARRANGEMENTS, NORMS
+    from denno_beta_amd.parts.blocks import SandwichBlock
+    from denno_beta_amd.parts.norms import RMSNorm, StreamRMSNorm
+    from denno_beta_amd.weights import draw_all
+
+    def add(self, y, x):
+        n = y.float() / torch.sqrt(y.float().pow(2).mean(1, keepdim=True) + self.eps) * self.weight
+        x += self.mult * (n if self.scale is None else n * self.scale)
+    if "toy_into_stream" not in NORMS:
+        NORMS.register("toy_into_stream_changed")(type("ToyChanged", (StreamRMSNorm,), {"add_into": add}))
+
+        @NORMS.register("toy_into_stream")
+        class ToyIntoStream(RMSNorm):
+            def __init__(self, width, eps, weight_name, scale_name, mult):
+                super().__init__(width, eps, weight_name)
+                self.behind = StreamRMSNorm(width, eps, weight_name, scale_name, mult)
+
+            def param_specs(self):
+                return self.behind.param_specs()
+
+            def bind(self, tensors, runtime):
+                super().bind(tensors, runtime)
+                self.behind.bind(tensors, runtime)
+                self.scale, self.mult = self.behind.scale, self.behind.mult
+            add_into = add
+
+        @ARRANGEMENTS.register("toy_on_sandwich")
+        class ToyOnSandwich(SandwichBlock):
+            def forward(self, x, ctx, caches, runtime):
+                act = runtime.act_dtype
+                self.post1.add_into(self._result(self.mixer, x, self.norm1.forward(x, act), ctx, caches[0]), x)
+                if self.has_ffn:
+                    self.post2.add_into(self._result(self.ffn, x, self.norm2.forward(x, act), ctx), x)
+    cfg = CONFIGS["P"][0]
+
+    def logits(kind, arrangement="sandwich"):
+        spec = build_pafivik(PafivikConfig.from_dict(cfg))
+        for layer in spec.layers:
+            layer.arrangement = arrangement
+            for slot in ("post1", "post2"):
+                layer.parts[slot] = (kind, layer.parts[slot][1])
+        tensors = draw_all(spec.param_specs(), 5, engine_dtype="float32", device=torch.device(backend), stored="float32")
+        r = ModelRunner(spec, tensors, EngineOptions(dtype="float32", device=backend, page_size=16, cache_tokens=64, max_live=4))
+        return U.replay(r, U.whole_trace([seqs_for(cfg, [19], seed=4)[0]]))["r0"]
+    want = logits("rmsnorm_into_stream")
+    for kind in ("toy_into_stream", "toy_into_stream_changed"):
+        U.assert_close(logits(kind), want, "float32", kind)
+    U.assert_close(logits("rmsnorm_into_stream", "toy_on_sandwich"), want, "float32", "an arrangement of one's own")
+
+
 # ----------------------------------------------------------------------------------------------------------------
 # far tokens: weights made so that losing one shows
 # ----------------------------------------------------------------------------------------------------------------
