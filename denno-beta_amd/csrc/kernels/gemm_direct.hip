@@ -117,8 +117,9 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   // its sums in part[blockIdx.y][m][n] and a second kernel adds them in order and ends with the epilogue
   // (stages of KB slabs: the host launches KB > 1 only where K is a multiple of 32 KB; split_slabs counts stages)
   const int kall = K / 32, nblocks = (N + 15) / 16;
-  // (the first 14 words of the arguments come in registers with the launch: all that the first loads need.  With the bias asked for in
-  // front, us: 203 x 4,800 x 1,600 14.2 -> 13.6, 203 x 5,120 x 1,280 12.3 -> 11.7, 203 x 1,600 x 6,400 into the stream 19.9 -> 19.4, 1,024 x 1,600 x 1,600
+  // (the first 14 words of the arguments come in registers with the launch: all that the operands' first loads need, and the slots of a cache
+  // write.  The bias' pointer stands behind them: where its load goes in front (BIAS_FIRST), that one trip to the arguments goes before the operands.  Both
+  // together, us: 203 x 4,800 x 1,600 14.2 -> 13.6, 203 x 5,120 x 1,280 12.3 -> 11.7, 203 x 1,600 x 6,400 into the stream 19.9 -> 19.4, 1,024 x 1,600 x 1,600
   // 16.4 -> 15.9, 1,024 x 3,840 x 1,280 17.0 -> 16.5)
   const int first = blockIdx.y * split_slabs;
   const int ksteps = min(split_slabs, kall / KB - first);

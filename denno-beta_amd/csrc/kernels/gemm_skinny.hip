@@ -64,7 +64,8 @@ using EndsOf = typename EndsFor<END>::type;
 // or are added to; q is the slot map (NORM_IN), else the leading dimension of p (a pointer in any case: through a pointer made from a number the
 // compiler loads by instructions that are waited for one by one, 0.5 us more).
 // In this order the operands' loads leave 0.2 to 0.5 us sooner, 8 rows: with the norm before, 3,072 x 1,024 4.3 -> 4.0 us, 5,120 x 1,280 6.6 -> 6.1,
-// 6,400 x 1,600 7.6 -> 7.2; with the norm after, 1,024 x 1,024 3.1 -> 3.0, 1,280 x 5,120 6.4 -> 6.0, 1,600 x 6,400 8.1 -> 7.6; 50,257 x 1,024 23.8 -> 23.0.
+// 6,400 x 1,600 7.6 -> 7.2; 50,257 x 1,024 23.8 -> 23.0; 8 columns a workgroup (with statistics, which that kernel left then), 1,024 x 1,024 3.1 -> 3.0,
+// 1,280 x 5,120 6.4 -> 6.0, 1,600 x 6,400 8.1 -> 7.6.  64 rows: 4,800 x 1,600 8.4 -> 8.0, with the norm before 11.4 -> 11.1; with the norm after level.
 constexpr int FIRST_ROWS = 255, FIRST_ADDS = 256;
 template <int END>
 struct Late {
@@ -758,9 +759,9 @@ static void launch16_one(const Call& c, const NormIO& nio, hipStream_t stream) {
 static bool eight_columns(int M, int N) { return M <= 8 && N <= 2048; }
 
 // The pairs in flight per wave are as many as make its share of K whole rounds: loads of what is not there cost as much as the others
-// (1,024 x 1,024 at 8 rows 3.1 us with 2, 3.5 with 4, 4.2 with 8; 1,024 x 4,096 5.1, 4.8, 4.8; 1,600 x 6,400 9.3, 9.2, 8.3 and 8.1 with 6).
-// gemm16_kernel -> this, with the next norm's statistics, 1 and 8 rows: 1,024 x 1,024 3.7 -> 3.0 and 4.2 -> 3.1 us, 1,600 x 1,600 3.9 -> 3.7 and 4.3 -> 3.8,
-// 1,024 x 4,096 5.0 -> 4.5 and 5.6 -> 4.8, 1,600 x 6,400 8.8 -> 7.6 and 10.1 -> 8.1, 2,048 x 8,192 10.2 -> 8.8 and 11.9 -> 9.6.
+// (with statistics, at 8 rows, 1,024 x 1,024 3.1 us with 2, 3.5 with 4, 4.2 with 8; 1,024 x 4,096 5.1, 4.8, 4.8; 1,600 x 6,400 9.3, 9.2, 8.3 and 8.1 with 6).
+// gemm16_kernel -> this, into the stream, 1 and 8 rows: 1,024 x 1,024 3.0 -> 2.8 and 3.6 -> 2.9 us, 1,600 x 1,600 3.6 -> 3.5 and 4.4 -> 3.7,
+// 1,024 x 4,096 5.0 -> 4.7 and 6.0 -> 5.3, 1,280 x 5,120 6.4 -> 5.4 and 7.7 -> 5.9, 1,600 x 6,400 8.4 -> 7.1 and 9.6 -> 7.9, 2,048 x 8,192 9.7 -> 9.1 and 12.7 -> 9.7.
 template <int WAVES, typename TC>
 static void launch8(const Call& c, hipStream_t stream) {
   const First f = first_of(c, NormIO{}, NORM_NONE);
