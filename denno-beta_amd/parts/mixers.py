@@ -157,6 +157,8 @@ class CausalSelfAttention(Part):
             raise TypeError(f"{type(position).__name__}: the 32-bit turn needs an encoding with a table of frequencies (rotary_pairs)")
         dims = position.dims if turns else 0
         freq = position.freq if turns else self.no_freq
+        if freq.shape[0] * 2 != dims:      # (an encoding's table may be longer than what is turned here)
+            freq = freq[:dims // 2]
         unit = self.unit_eps is not None
         mag = getattr(position, "mag", 1.0) if turns else 1.0
         # (one launch with the cache write in it: 8 rows of 16 + 8 heads of 64 5.5 -> 3.1 us, 2,136 rows 13.3 -> 9.5; it knows nothing of a

@@ -388,6 +388,21 @@ def test_a_norm_that_only_adds_into_the_stream_may_stand_behind_a_sublayer(backe
     U.assert_close(logits("rmsnorm_into_stream", "toy_on_sandwich"), want, "float32", "an arrangement of one's own")
 
 
+def test_a_table_of_frequencies_may_be_longer_than_the_turned_pairs(backend, folders, monkeypatch):
+    """The exact turn reads a table's first dims / 2 frequencies; more of them in an encoding's table change nothing."""
+    from denno_beta_amd.parts.positions import RotaryPairs
+    folder = folders("P", "float32")      # (its attention turns 8 of 16 entries)
+    seq = seqs_for(CONFIGS["P"][0], [19], seed=13)[0]
+    want = U.replay(runner_for(folder, "float32", backend, 64), U.whole_trace([seq]))["r0"]
+    bind = RotaryPairs.bind
+
+    def longer(self, tensors, runtime):
+        bind(self, tensors, runtime)
+        self.freq = torch.cat([self.freq, torch.ones(3, device=self.freq.device)])
+    monkeypatch.setattr(RotaryPairs, "bind", longer)
+    assert torch.equal(U.replay(runner_for(folder, "float32", backend, 64), U.whole_trace([seq]))["r0"], want)
+
+
 # ----------------------------------------------------------------------------------------------------------------
 # far tokens: weights made so that losing one shows
 # ----------------------------------------------------------------------------------------------------------------
