@@ -157,7 +157,9 @@ class CausalSelfAttention(Part):
             raise TypeError(f"{type(position).__name__}: the 32-bit turn needs an encoding with a table of frequencies (rotary_pairs)")
         dims = position.dims if turns else 0
         freq = position.freq if turns else self.no_freq
-        if freq.shape[0] * 2 != dims:      # (an encoding's table may be longer than what is turned here)
+        if freq.shape[0] * 2 != dims:      # (an encoding's table may be longer than what is turned here; no shorter, and pairs are whole)
+            if dims % 2 != 0 or freq.shape[0] * 2 < dims:
+                raise ops.KernelError(f"{type(position).__name__}: {freq.shape[0]} frequencies for {dims} turned entries")
             freq = freq[:dims // 2]
         unit = self.unit_eps is not None
         mag = getattr(position, "mag", 1.0) if turns else 1.0

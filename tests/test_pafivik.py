@@ -403,6 +403,26 @@ def test_a_table_of_frequencies_may_be_longer_than_the_turned_pairs(backend, fol
     assert torch.equal(U.replay(runner_for(folder, "float32", backend, 64), U.whole_trace([seq]))["r0"], want)
 
 
+@pytest.mark.parametrize("odd", [False, True])
+def test_a_table_of_frequencies_may_not_be_shorter_than_the_turned_pairs(backend, folders, monkeypatch, odd):
+    """The exact turn refuses a table that lacks a turned pair's frequency, and half a pair."""
+    from denno_beta_amd.kernels.ops import KernelError
+    from denno_beta_amd.parts.positions import RotaryPairs
+    folder = folders("P", "float32")
+    seq = seqs_for(CONFIGS["P"][0], [19], seed=13)[0]
+    bind = RotaryPairs.bind
+
+    def shorter(self, tensors, runtime):
+        bind(self, tensors, runtime)
+        if odd:
+            self.dims -= 1
+        else:
+            self.freq = self.freq[:-1].contiguous()
+    monkeypatch.setattr(RotaryPairs, "bind", shorter)
+    with pytest.raises(KernelError, match="frequencies for"):
+        U.replay(runner_for(folder, "float32", backend, 64), U.whole_trace([seq]))
+
+
 # ----------------------------------------------------------------------------------------------------------------
 # far tokens: weights made so that losing one shows
 # ----------------------------------------------------------------------------------------------------------------
