@@ -118,9 +118,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   // (stages of KB slabs: the host launches KB > 1 only where K is a multiple of 32 KB; split_slabs counts stages)
   const int kall = K / 32, nblocks = (N + 15) / 16;
   // (the first 14 words of the arguments come in registers with the launch: all that the operands' first loads need, and the slots of a cache
-  // write.  The bias' pointer stands behind them: where its load goes in front (BIAS_FIRST), that one trip to the arguments goes before the operands.  Both
-  // together, us: 203 x 4,800 x 1,600 14.2 -> 13.6, 203 x 5,120 x 1,280 12.3 -> 11.7, 203 x 1,600 x 6,400 into the stream 19.9 -> 19.4, 1,024 x 1,600 x 1,600
-  // 16.4 -> 15.9, 1,024 x 3,840 x 1,280 17.0 -> 16.5)
+  // write; the others by a trip to memory, see ARGS_EARLY)
   const int first = blockIdx.y * split_slabs;
   const int ksteps = min(split_slabs, kall / KB - first);
   // Where the 16 bytes of row lane % 16, columns 8 (lane / 16) .. of a block of A lie among its KB pieces of 1 KB (see the loads below).
@@ -149,8 +147,13 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
       for (int e = 0; e < 4; ++e) vslot[i][e] = mq + e < M ? slot_map[mq + e] : -1;
     }
   }
-  // the bias, for the epilogue, in front of the operands' loads, where a tile leaves the registers for it
-  constexpr bool BIAS_FIRST = TN <= 4;
+  // The epilogue's arguments do not come with the launch.  With a cache write, and in tiles of four waves, they are brought into registers behind
+  // the operands' first loads (ARGS_EARLY).  Elsewhere that held up the walk along K, and they come with the bias, asked for in front of the operands where
+  // a tile leaves the registers for it (BIAS_FIRST): which of the two is measured, us, arguments in their old order -> both everywhere -> as it is:
+  // four waves: GELU 65 x 1,024 x 4,096 20.1 -> 21.4 -> 19.8, 300 x 512 x 512 6.25 -> 6.36 -> 6.24; cache write: 203 x 3,840 x 1,280 10.7 -> 10.7 -> 10.4,
+  // 65 x 4,800 x 1,600 11.5 -> 11.6 -> 11.1; sixteen waves: GELU 203 x 4,800 x 1,600 13.8 -> 13.5 -> 13.3, 203 x 4,096 x 1,024 7.95 -> 8.04 -> 7.76,
+  // 1,000 x 1,024 x 1,024 8.05 -> 8.25 -> 7.79, into the stream 1,000 x 1,600 x 1,600 15.4 -> 15.0 -> 14.7.
+  constexpr bool ARGS_EARLY = KV || NW == 4, BIAS_FIRST = !ARGS_EARLY && TN <= 4;
   floatx4 bvs[TN];
   auto ask_bias = [&]() {
 #pragma clang loop unroll(full)
@@ -209,8 +212,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < ksteps) issue(s);
-  // the epilogue's arguments, which do not come with the launch: here, not at the kernel's end
-  asm volatile("" ::"s"(C), "s"(ldc), "s"(resid), "s"(ldr), "s"(epi), "s"(part));
+  // (here, not at the kernel's end)
+  if constexpr (ARGS_EARLY) asm volatile("" ::"s"(C), "s"(ldc), "s"(resid), "s"(ldr), "s"(epi), "s"(part));
   if constexpr (KV) asm volatile("" ::"s"(kv.k_pool), "s"(kv.v_pool), "s"(kv.q_width), "s"(kv.kv_width), "s"(kv.dh), "s"(kv.page_size), "s"(kv.c_cols));
   // this wave's share of a stage has landed when only its loads of the STAGES - 2 stages after it are out
   auto landed = [&](bool more) {
