@@ -2728,9 +2728,11 @@ int dn_norm_turn_write(const float* z, long long ldz, int H, int G, int dk, int 
   if (pos_coef != 0.f && !(pos_every > 0.0)) return DN_ERR_SHAPE;
   const NormTurnArgs a{z, static_cast<size_t>(ldz), H, G, dk, dv, wq, wk, q_scale, pos_coef, pos_every, eps, freq, dims, v_freq, v_dims, positions, q_out,
                        static_cast<size_t>(ldq), kept, slot_map, k_pool, v_pool, page_size, dt, write, as_runs};
-  // (few rows: the vectors of a row spread over workgroups, so that a step of decoded tokens is more than a handful of them; many
-  // rows: one workgroup a row, whose angles are made once.  By the sizes alone a vector has 32 or 64 lanes: the same bits either way)
-  const int at_once = kept <= 64 ? 8 : 4, groups = T <= 256 ? (H + 2 * G + at_once - 1) / at_once : 1;
+  // (few rows: the vectors of a row spread over workgroups, so that a step of decoded tokens is more than a handful of them; some hundreds: over as
+  // many as make four workgroups a CU (25 + 25 heads of 80 13.3 -> 8.3 us at 257 rows where one a row takes longer than two kernels, 11.8, and 24.7 -> 20.8
+  // at 1,000; twice as many gives 0.95 to 1.2 times that); many rows: one workgroup a row, whose angles are made once.  By the sizes alone a vector has 32 or 64
+  // lanes: the same bits either way)
+  const int at_once = kept <= 64 ? 8 : 4, all = (H + 2 * G + at_once - 1) / at_once, fill = (1024 + T - 1) / T, groups = T <= 256 || all < fill ? all : fill;
   const dim3 grid(T, groups < 65535 ? groups : 65535);
   if (kept <= 64) hipLaunchKernelGGL((norm_turn_write_kernel<32, 1>), grid, dim3(256), 0, stream, a);
   else if (kept <= 128) hipLaunchKernelGGL((norm_turn_write_kernel<64, 1>), grid, dim3(256), 0, stream, a);

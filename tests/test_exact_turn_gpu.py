@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("H,G,dk,dv,kept,dims,page", [(16, 8, 64, 64, 64, 64, 16), (4, 4, 48, 32, 48, 16, 32), (25, 5, 80, 80, 80, 80, 16), (3, 1, 33, 47, 48, 32, 16),
                                                       (2, 2, 128, 128, 128, 0, 16), (2, 1, 256, 200, 256, 256, 48), (8, 2, 96, 16, 96, 94, 16)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T", [1, 8, 257])
+@pytest.mark.parametrize("T", [1, 8, 257, 1023, 1025])      # (all a row's vectors at once, four workgroups a row, two, one)
 def test_one_launch_has_the_bits_of_two(H, G, dk, dv, kept, dims, page, dtype, T):
     g = torch.Generator(device="cuda").manual_seed(H * 1000 + dk + T)
     make = lambda *s: torch.randn(*s, generator=g, device="cuda")   # noqa: E731
