@@ -159,6 +159,8 @@ def _declare(name, lib):
             "dn_conv_turn_write": [P, c_longlong, I, I, I, I, P, I, P, c_longlong, P, P, I, P, P, F, P, I, P, P, c_longlong, I, P, P, P, I, I, I, I, I, P],
             "dn_clamped_glu": [P, c_longlong, F, F, P, I, c_longlong, I, I, P],
             "dn_post_norm": [P, c_longlong, F, P, c_longlong, P, c_longlong, P, P, F, P, P, I, I, P, P, F, P, I, c_longlong, I, I, P],
+            "dn_scan_chunks": [P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, P, I, P, c_longlong, P, P, I, I, I, I, I, I, P, P,
+                               c_longlong, P],
             "dn_delta_chunks": [P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, P, P, c_longlong, P, P, I, I, I, I, I, I, P, P,
                                 c_longlong, P],
             "dn_turn_back_gate": [P, I, c_longlong, I, P, c_longlong, P, P, P, I, c_longlong, I, I, I, P],
@@ -1416,12 +1418,42 @@ def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, rea
     return out
 
 
-DELTA_CHUNKS_ROWS_MIN = 32      # rows a request, on average, from which the delta rule's chunks are worth their own kernels
+# Rows a request, on average, from which a step's recurrences are walked in chunks.  A request of a chunk or two is sooner done row by row: the first of
+# the two kernels takes 8 us whatever it has to do, and with a decay per channel or head most of it in 64-bit.
+CHUNKS_ROWS_MIN, DELTA_CHUNKS_ROWS_MIN = 96, 32
 
 
-def delta_chunks_takes(T, S, dk):
-    """Whether a step of T rows of S requests is one for `delta_chunks` (portions, key heads of a size that it knows)."""
-    return T >= DELTA_CHUNKS_ROWS_MIN * S and dk % 16 == 0 and 16 <= dk <= 128
+def chunks_takes(T, S, dk, least=CHUNKS_ROWS_MIN):
+    """Whether a step of T rows of S requests is one for `scan_chunks` (`least` DELTA_CHUNKS_ROWS_MIN: for `delta_chunks`): portions, key heads of
+    a size that they know."""
+    return T >= least * S and dk % 16 == 0 and 16 <= dk <= 128
+
+
+def scan_chunks(r, k, v, w, state, row_start, slots, n_heads, dk, dv, out, beta=None, w_head=None, qk_heads=None):
+    """state_scan's delta rule with a decay per row and channel (beta given, as the sigmoid's argument; w [T, heads * dk]), or its
+    recurrence with one constant decay per head that reads after its write (w None, w_head [heads]; no beta), 16 rows of a request at a
+    time on the matrix cores in 32-bit: the same recurrence, its sums in another order, so a row's result changes by rounding with
+    the place where its portion begins.  dk: a multiple of 16 up to 128."""
+    G = n_heads if qk_heads is None else qk_heads
+    _need(G >= 1 and n_heads % G == 0, lambda: f"scan_chunks: {n_heads} heads over {G} heads of queries and keys")
+    _need((w is None) != (w_head is None) and (beta is None) == (w is None), "scan_chunks: decays per row and channel with beta, or one per head without")
+    given = ((r, "r", G * dk), (k, "k", G * dk), (v, "v", n_heads * dv), (out, "out", n_heads * dv)) \
+        + (() if w is None else ((w, "w", n_heads * dk), (beta, "beta", n_heads)))
+    T = r.shape[0]
+    for t, name, n in given:
+        _dev(t, name, (torch.float32,), 2)
+        _need(tuple(t.shape) == (T, n), lambda: f"scan_chunks: {name} {tuple(t.shape)}")
+    S = _request_tables(row_start, slots, "scan_chunks")
+    _need(dk % 16 == 0 and 16 <= dk <= 128, lambda: f"scan_chunks: {dk} key channels a head; a multiple of 16 up to 128")
+    _f32vec(w_head, "w_head", n_heads)
+    stride = _history(state, n_heads * dk * dv, "scan_chunks")
+    lib = _lib("sequence")
+    work = torch.empty(lib.dn_delta_chunks_floats(T, S, n_heads, dk, dv), dtype=torch.float32, device=r.device)
+    _ok(lib.dn_scan_chunks(r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"), _ptr(beta),
+                           _rows(beta, "beta") if beta is not None else 0, _ptr(w_head) if w is None else w.data_ptr(), 0 if w is None else _rows(w, "w"),
+                           0, 0, 2 if w is None else 0, state.data_ptr(), stride, row_start.data_ptr(), slots.data_ptr(), S, T, n_heads, G, dk, dv,
+                           work.data_ptr(), out.data_ptr(), _rows(out, "out"), _stream()), "scan_chunks")
+    return out
 
 
 def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads, dk, dv, out, qk_heads=None):

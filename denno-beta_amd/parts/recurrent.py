@@ -156,8 +156,14 @@ class Lightning(Part):
             z = self.proj(h, out_dtype=F32)
             ops.activate(z[:, :2 * qk + vw], "silu", z[:, :2 * qk + vw])
         o = torch.empty((T, vw), dtype=F32, device=h.device)
-        ops.state_scan(z[:, :qk], z[:, qk:2 * qk], z[:, 2 * qk:2 * qk + vw], None, None, cache.state, ctx.row_start, ctx.state_slots,
-                       self.n_heads, self.head_dim, self.value_dim, o, read_after=True, w_head=self.decay_t)
+        q, k, v = z[:, :qk], z[:, qk:2 * qk], z[:, 2 * qk:2 * qk + vw]
+        # (the 32-bit engine walks a request's rows in order: its logits are the same bits however a prompt is cut)
+        if act != F32 and not ctx.single_rows and ops.chunks_takes(T, ctx.S, self.head_dim):
+            ops.scan_chunks(q, k, v, None, cache.state, ctx.row_start, ctx.state_slots, self.n_heads, self.head_dim, self.value_dim, o,
+                            w_head=self.decay_t)
+        else:
+            ops.state_scan(q, k, v, None, None, cache.state, ctx.row_start, ctx.state_slots, self.n_heads, self.head_dim, self.value_dim, o,
+                           read_after=True, w_head=self.decay_t)
         y = torch.empty((T, vw), dtype=act, device=h.device)
         ops.head_norm(o, self.norm, self.eps, y, 1, gate=z[:, 2 * qk + vw:], gate_kind="sigmoid")
         if accumulate_into is None:
@@ -274,9 +280,14 @@ class ChannelDelta(Part):
                 ops.activate(g, "exp_neg_softplus", g, bias=self.dt_bias, lower=self.rate)
             gate = self.g2(g_in, out_dtype=F32)
         o = torch.empty((T, vw), dtype=F32, device=dev)
-        # (beta = sigmoid of the projection's columns behind the channels, taken inside the scan)
-        ops.state_scan(q, k, v, g, None, state, ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, beta=z[:, C:C + H],
-                       qk_heads=self.n_qk_heads, beta_logits=True)
+        # (beta = sigmoid of the projection's columns behind the channels, taken inside the scan; the 32-bit engine walks a request's rows in
+        # order: its logits are the same bits however a prompt is cut)
+        if act != F32 and not single and ops.chunks_takes(T, ctx.S, self.head_dim):
+            ops.scan_chunks(q, k, v, g, state, ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, beta=z[:, C:C + H],
+                            qk_heads=self.n_qk_heads)
+        else:
+            ops.state_scan(q, k, v, g, None, state, ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, beta=z[:, C:C + H],
+                           qk_heads=self.n_qk_heads, beta_logits=True)
         y = torch.empty((T, vw), dtype=act, device=dev)
         ops.head_norm(o, self.norm, self.eps, y, H, gate=gate, gate_kind="sigmoid")
         if accumulate_into is None:
@@ -359,7 +370,7 @@ class GatedDelta(Part):
         o = torch.empty((T, vw), dtype=F32, device=dev)
         # (beta and the decay are made from their arguments inside the scan; the 32-bit engine walks a request's rows in order: its
         # logits are the same bits however a prompt is cut)
-        if act != F32 and not single and qk % 4 == 0 and C % 4 == 0 and ops.delta_chunks_takes(T, ctx.S, self.head_dim):
+        if act != F32 and not single and qk % 4 == 0 and C % 4 == 0 and ops.chunks_takes(T, ctx.S, self.head_dim, ops.DELTA_CHUNKS_ROWS_MIN):
             ops.delta_chunks(x[:, :qk], x[:, qk:2 * qk], x[:, 2 * qk:], z[:, b:b + H], z[:, b + H:b + 2 * H], self.rate, self.dt_bias, state,
                              ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, qk_heads=self.n_qk_heads)
         else:

@@ -448,6 +448,11 @@ def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads,
                       w_rate=rate, w_bias=bias)
 
 
+def scan_chunks(r, k, v, w, state, row_start, slots, n_heads, dk, dv, out, beta=None, w_head=None, qk_heads=None):
+    return state_scan(r, k, v, w, None, state, row_start, slots, n_heads, dk, dv, out, read_after=beta is None, beta=beta, w_head=w_head, qk_heads=qk_heads,
+                      beta_logits=beta is not None)
+
+
 def head_norm(o, weight, eps, out, n_heads, gate=None, gate_kind="silu", gate_first=False, skip=None, skip_scale=None):
     T, n = o.shape
     dv = n // n_heads

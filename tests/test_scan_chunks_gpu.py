@@ -1,0 +1,72 @@
+"""The recurrences in chunks of 16 rows against the recurrence in 64 bits: sizes of heads, requests that end inside a chunk, and what is no number."""
+import pytest
+import torch
+
+import kernel_refs as R
+from test_kernels_gpu import ops, rnd
+from test_sequence_kernels_gpu import close, tables
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def operands(mode, heads, qk_heads, dk, dv, T, fade):
+    """r, k (unit vectors that point almost the same way), v, then decays and beta's arguments, as views of wider rows."""
+    C = 2 * qk_heads * dk + heads * dv
+    x = rnd(T, C + 3, seed=1)[:, 1:1 + C]      # (rows that begin at any number)
+    r, k, v = x[:, :qk_heads * dk], x[:, qk_heads * dk:2 * qk_heads * dk], x[:, 2 * qk_heads * dk:]
+    unit = lambda t: torch.nn.functional.normalize(t.reshape(T, qk_heads, dk), dim=-1).reshape(T, -1)      # noqa: E731
+    k.copy_(unit(k + 2.0 * rnd(1, qk_heads * dk, seed=2)))
+    r.copy_(unit(r) * dk ** -0.5)
+    if mode == "head":
+        return r, k, v, dict(w=None, w_head=torch.exp(-fade * torch.rand(heads, device=DEV)))
+    return r, k, v, dict(w=torch.exp(-fade * torch.rand(T, heads * dk, device=DEV)), beta=rnd(T, heads + 2, seed=4)[:, 1:1 + heads] * 2)
+
+
+@pytest.mark.parametrize("mode", ["wide", "head"])
+@pytest.mark.parametrize("dk,dv,heads,qk_heads", [(16, 16, 2, 2), (64, 128, 4, 2), (48, 33, 3, 1), (128, 40, 2, 2), (80, 7, 2, 1), (32, 64, 6, 3), (96, 16, 1, 1),
+                                                  (112, 50, 2, 2), (64, 300, 1, 1), (16, 1, 1, 1)])
+@pytest.mark.parametrize("lengths", [[40], [16, 1, 33], [1, 15, 17, 200, 3], [64, 63, 65], [2, 2, 5]])
+@pytest.mark.parametrize("fade", [0.02, 1.0, 200.0])
+def test_chunks_in_64_bits(mode, dk, dv, heads, qk_heads, lengths, fade):
+    slot_of = [4, 0, -1, 2, 1][:len(lengths)]
+    row_start, slots, T = tables(lengths, slot_of)
+    r, k, v, kw = operands(mode, heads, qk_heads, dk, dv, T, fade)
+    state = torch.randn(5, heads * dk * dv + 11, device=DEV)
+    n = heads * dk * dv
+    d = lambda t: t.cpu().double() if torch.is_tensor(t) else t      # noqa: E731
+    want_state, want = d(state), torch.zeros(T, heads * dv, dtype=torch.float64)
+    R.scan_chunks(d(r), d(k), d(v), d(kw["w"]), want_state[:, :n], row_start.cpu(), slots.cpu(), heads, dk, dv, want, qk_heads=qk_heads,
+                  **{a: d(t) for a, t in kw.items() if a != "w"})
+    got_state, got = state.clone(), torch.full((T + 1, heads * dv), 7.0, device=DEV)
+    ops().scan_chunks(r, k, v, kw["w"], got_state[:, :n], row_start, slots, heads, dk, dv, got[:T], qk_heads=qk_heads,
+                      **{a: t for a, t in kw.items() if a != "w"})
+    real = [t for s, m in enumerate(lengths) for t in range(int(row_start[s]), int(row_start[s]) + m) if slot_of[s] >= 0]
+    close(got[real], want[real]), close(got_state, want_state)
+    rest = [t for t in range(T + 1) if t not in real]
+    assert bool((got[rest] == 7.0).all()) and torch.equal(got_state[3], state[3])      # (rows and slots of no request)
+
+
+@pytest.mark.parametrize("mode", ["wide", "head"])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("which", ["v", "k", "r"])
+def test_what_is_no_number_does_not_reach_rows_before_it(mode, bad, which):
+    heads, dk, dv, T, at = 2, 64, 40, 50, 21
+    row_start, slots, _ = tables([T], [0])
+    r, k, v, kw = operands(mode, heads, heads, dk, dv, T, 0.5)
+    got = []
+    for spoilt in (False, True):
+        x = dict(r=r.clone(), k=k.clone(), v=v.clone())
+        if spoilt:
+            x[which][at, 5] = bad
+        out = torch.zeros(T, heads * dv, device=DEV)
+        ops().scan_chunks(x["r"], x["k"], x["v"], kw["w"], torch.zeros(1, heads * dk * dv, device=DEV), row_start, slots, heads, dk, dv, out,
+                          **{a: t for a, t in kw.items() if a != "w"})
+        got.append(out)
+    close(got[1][:at], got[0][:at]), close(got[1][:, dv:], got[0][:, dv:])      # (rows before it, and the other head)
+    assert not bool(torch.isfinite(got[1][at]).all())
+    if which == "v":      # (a value's column alone)
+        keep = [j for j in range(heads * dv) if j != 5]
+        close(got[1][:, keep], got[0][:, keep])
+    if which == "r":
+        close(got[1][at + 1:], got[0][at + 1:])
