@@ -293,19 +293,31 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   // in its page a value lies as [dim][offset], so four tokens whose slots follow one another from a
   // multiple of 4 are 8 bytes side by side for one dim: the four lanes of a quad, which hold four
   // tokens x four dims, exchange them (a 4 x 4 turn), and each stores four tokens of one dim.
-  int kpage[KV ? TM : 1], koff[KV ? TM : 1], vpage[KV ? TM : 1], voff[KV ? TM : 1];
+  // A place is the row's (page and offset) plus the block's (head and first dim), and the block's is the same for all lanes: worked out
+  // lane by lane, with its divisions, it was most of this epilogue.
+  long long krow[KV ? TM : 1], vrow[KV ? TM : 1];      // of the row in the pools, -1: none
+  uint32_t dh_inverse = 0;                             // 2^32 / dh, rounded up: c / dh is c times that (below 2^32 / dh)
+  int page_numbers = 0;
   if constexpr (KV) {
+    dh_inverse = 0xffffffffu / static_cast<uint32_t>(kv.dh) + 1;
+    page_numbers = kv.Hkv * kv.page_size * kv.dh;
 #pragma clang loop unroll(full)
     for (int i = 0; i < TM; ++i) {
-      page_and_offset(kv, max(kslot[i], 0), kpage[i], koff[i]);
-      if (kslot[i] < 0) kpage[i] = -1, koff[i] = 0;
+      int page, off;
+      page_and_offset(kv, max(kslot[i], 0), page, off);
+      krow[i] = kslot[i] < 0 ? -1 : static_cast<long long>(page) * page_numbers + off * kv.dh;
       const int* sq = vslot[i];
       const bool run = kv.page_size % 4 == 0 && sq[0] >= 0 && sq[0] % 4 == 0 && sq[1] == sq[0] + 1 && sq[2] == sq[0] + 2 &&
                        sq[3] == sq[0] + 3;
-      page_and_offset(kv, max(sq[0], 0), vpage[i], voff[i]);
-      if (!run) vpage[i] = -1, voff[i] = 0;
+      page_and_offset(kv, max(sq[0], 0), page, off);
+      vrow[i] = run ? static_cast<long long>(page) * page_numbers + off : -1;
     }
   }
+  // where a block of keys lies in a page, from its first column on
+  auto key_place = [&](int first_column) {
+    const uint32_t c = first_column - kv.q_width;
+    return static_cast<int>(c + __umulhi(c, dh_inverse) * (kv.page_size - 1) * kv.dh);
+  };
   if (part) {
 #pragma clang loop unroll(full)
     for (int j = 0; j < TN; ++j) {
@@ -324,25 +336,79 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   // every load of the epilogue before its first store: a wait for a load is a wait for the stores
   // issued before it as well (one counter), and a load per column block made the blocks take turns
   if constexpr (!BIAS_FIRST) ask_bias();
+  // Results of 16 bits leave through LDS, 16 rows of the wave's columns at a time: 16 bytes a lane side by side, where a lane's four columns as they lie
+  // are 32 bytes of each of 16 rows a store (2,048 x 6,400 x 64, all epilogue: 15.3 -> 11.5 us; with K = 1,600 and GELU 49.0 -> 47.1,
+  // 2,048 x 4,800 x 1,600 36.1 -> 33.2, 8,192 x 6,400 x 1,600 181 -> 170).  A row's part is 16 bytes longer in LDS, so that the
+  // rows' pieces meet different banks.  The values of a fused projection stay out of it: a store of theirs is a page's 512 bytes already
+  // (fused projections, with the places in pages by row and block as above: 2,048 x 4,800 x 1,600 43.2 -> 39.9, 6,700 x 3,840 x 1,280 88 -> 84).
+  constexpr int ROW = TN * 32 + 16, PIECES = 2 * TN;
+  constexpr bool STAGED = sizeof(TC) == 2 && TN >= 2 && NW * 16 * ROW <= STAGES * SLAB * 16;
+  bool staged = false;
+  if constexpr (STAGED) {
+    staged = !(packed & PACKED_C) && ldc % 8 == 0 && N % 8 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+    if constexpr (KV) staged = staged && kv.c_cols % 8 == 0 && reinterpret_cast<uintptr_t>(kv.k_pool) % 16 == 0;
+    if (staged) {
+      int place[KV ? TN : 1];      // of a block of keys in its page: the head's and the first dim's
+      if constexpr (KV) {
+#pragma clang loop unroll(full)
+        for (int j = 0; j < TN; ++j) place[j] = key_place(max(n0 + (wnb + j) * 16, kv.q_width));
+      }
+      char* mine = reinterpret_cast<char*>(lds) + wave * (16 * ROW);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();      // (the last stage has been read)
+      // (what the wave's columns have none of costs it nothing: keys among queries, and columns that go elsewhere)
+      const int first = n0 + wnb * 16, end = KV ? max(kv.q_width + kv.kv_width, kv.c_cols) : N;
+      const bool keys = KV && first < kv.q_width + kv.kv_width && first + TN * 16 > kv.q_width;
+#pragma clang loop unroll(full)
+      for (int i = 0; i < TM; ++i) {
+        if (first >= end) break;
+#pragma clang loop unroll(full)
+        for (int j = 0; j < TN; ++j) {
+          const floatx4 v = acc[i][j] + bvs[j];
+          auto finish = [&](float e) { return XIELU ? xielu_f(e, act_a, act_b) : apply_epilogue_fast(e, epi); };
+          *reinterpret_cast<uint2*>(mine + (lane % 16) * ROW + j * 32 + (lane / 16) * 8) = pack4(finish(v[0]), finish(v[1]), finish(v[2]), finish(v[3]));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma clang loop unroll(full)
+        for (int it = 0; it < (16 * PIECES + 63) / 64; ++it) {
+          const int u = it * 64 + lane, row = min(u / PIECES, 15), piece = u % PIECES;
+          const int m = m0 + (wmb + i) * 16 + row, n = n0 + wnb * 16 + piece * 8;
+          const u32x4 x = *reinterpret_cast<const u32x4*>(mine + row * ROW + piece * 16);
+          const bool ok = u < 16 * PIECES && m < M && n < N;
+          if (ok && (!KV || n < kv.c_cols)) *reinterpret_cast<u32x4*>(C + static_cast<size_t>(m) * ldc + n) = x;
+          if (KV && keys) {
+            const long long of_row = static_cast<long long>(static_cast<uint64_t>(static_cast<uint32_t>(__shfl(static_cast<int>(krow[i] >> 32), row))) << 32 |
+                                                            static_cast<uint32_t>(__shfl(static_cast<int>(krow[i]), row)));
+            int at = place[0];
+#pragma clang loop unroll(full)
+            for (int j = 1; j < TN; ++j) at = piece / 2 == j ? place[j] : at;
+            if (ok && of_row >= 0 && n >= kv.q_width && n < kv.q_width + kv.kv_width)
+              *reinterpret_cast<u32x4*>(kv.k_pool + of_row + at + piece % 2 * 8) = x;
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the next rows go where these lay)
+      }
+      if constexpr (!KV) return;
+    }
+  }
 #pragma clang loop unroll(full)
   for (int j = 0; j < TN; ++j) {
     const int n = n0 + (wnb + j) * 16 + (lane / 16) * 4;
     if (n >= N) continue;
     const floatx4 bv = bvs[j];
-    // the block's place among the keys or the values: head hh, dims d .. d + 3 (a block of 16 columns is
-    // all queries, all keys or all values, and of one head: the widths are multiples of 16)
+    // (a block of 16 columns is all queries, all keys or all values, and of one head: the widths are multiples of 16)
+    const int block = n0 + (wnb + j) * 16;
     bool is_key = false, is_value = false;
-    int hh = 0, d = 0;
+    int at = 0;
     if constexpr (KV) {
-      is_key = n >= kv.q_width && n < kv.q_width + kv.kv_width;
-      is_value = n >= kv.q_width + kv.kv_width;
-      const int c = n - kv.q_width - (is_value ? kv.kv_width : 0);
-      hh = c / kv.dh, d = c % kv.dh;
+      is_key = block >= kv.q_width && block < kv.q_width + kv.kv_width;
+      is_value = block >= kv.q_width + kv.kv_width;
+      at = is_value ? (block - kv.q_width - kv.kv_width) * kv.page_size : is_key ? key_place(block) : 0;
     }
 #pragma clang loop unroll(full)
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + (wmb + i) * 16 + lane % 16;
-      if (m >= M) continue;
+      if (m >= M || (STAGED && staged)) continue;
       const floatx4 v = acc[i][j] + bv;
       if (resid) {
         floatx4* x = reinterpret_cast<floatx4*>(resid + static_cast<size_t>(m) * ldr + n);
@@ -359,9 +425,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
         if (!KV || n < kv.c_cols)
           *reinterpret_cast<uint2*>(C + ((packed & PACKED_C) ? packed_index(m, n, N / 32) : static_cast<size_t>(m) * ldc + n)) = cv;
         if constexpr (KV) {
-          if (is_key && kpage[i] >= 0)
-            *reinterpret_cast<uint2*>(kv.k_pool + ((static_cast<size_t>(kpage[i]) * kv.Hkv + hh) * kv.page_size + koff[i]) * kv.dh +
-                                      d) = cv;
+          if (is_key && krow[i] >= 0) *reinterpret_cast<uint2*>(kv.k_pool + krow[i] + at + (lane / 16) * 4) = cv;
         }
       }
     }
@@ -374,9 +438,9 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
           const floatx4 v = acc[i][j] + bv;
           // token mq + e, dim d + q: lane e of the quad holds it in v[q]
           const float t0 = quad_pick<0>(v, q), t1 = quad_pick<1>(v, q), t2 = quad_pick<2>(v, q), t3 = quad_pick<3>(v, q);
-          if (vpage[i] >= 0) {
-            *reinterpret_cast<uint2*>(kv.v_pool + ((static_cast<size_t>(vpage[i]) * kv.Hkv + hh) * kv.dh + d + q) * kv.page_size +
-                                      voff[i]) = pack4(t0, t1, t2, t3);
+          const int dim = (lane / 16) * 4 + q;
+          if (vrow[i] >= 0) {
+            *reinterpret_cast<uint2*>(kv.v_pool + vrow[i] + at + dim * kv.page_size) = pack4(t0, t1, t2, t3);
           } else {
 #pragma clang loop unroll(full)
             for (int e = 0; e < 4; ++e) {
@@ -384,7 +448,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
               if (slot < 0) continue;
               int page, off;
               page_and_offset(kv, slot, page, off);
-              kv.v_pool[((static_cast<size_t>(page) * kv.Hkv + hh) * kv.dh + d + q) * kv.page_size + off] =
+              kv.v_pool[static_cast<size_t>(page) * page_numbers + at + dim * kv.page_size + off] =
                   from_float<bf16_t>(e == 0 ? t0 : e == 1 ? t1 : e == 2 ? t2 : t3);
             }
           }
@@ -581,11 +645,12 @@ int run(const Args& a, hipStream_t stream) {
     case 3:
       if (!sixteen || !two) return launch_as<4, 2, 4, 5, 4>(a, stream);
       // Eight waves in turns walk along K faster than sixteen in step and end slower, the more so the more the epilogue does: a wave
-      // has twice the blocks to finish.  So a long K takes turns: from 1,600 on where the results are 32-bit, from 2,560 where they
-      // are rounded to bfloat16 (time of turns over time in step, 1,500 x 6,400 with GELU: K = 64 1.29, 1,024 1.10, 1,600 1.05, 2,560 1.00, 4,096
-      // 0.97, 6,400 0.93; added into the stream: 1.16, 1.03, 1.00, 0.98, 0.95, 0.93), and the product with a cache write, whose
-      // epilogue is the longest, never does (2,048 x 4,800 x 1,600 46.8 us in step, 54.9 in turns).
-      if (!a.kv && a.K >= (a.out_dtype == DN_BF16 && !a.resid ? 2560 : 1600)) return launch_without_kv<4, 2, 4, 5, 3, 2, true>(a, stream);
+      // has twice the blocks to finish.  So a long K takes turns: from 1,600 on where the results are 32-bit, from 1,280 where they
+      // are rounded to bfloat16 and leave through LDS (time of turns over time in step, K = 512, 1,024, 1,280, 1,600, 2,560: 1,500 x 6,400 with GELU
+      // 1.05, 0.99, 0.98, 0.97, 0.96; 2,048 x 5,120 with GELU 1.06, 1.00, 0.99, 1.00, 0.95; 8,192 x 3,200 1.11, 1.03, 0.99, 0.98, 0.94; added into the
+      // stream, 1,500 x 6,400, K = 1,024, 1,600, 2,560, 4,096: 1.03, 1.00, 0.98, 0.95), and the product with a cache write, whose
+      // epilogue is the longest, never does (2,048 x 4,800 x 1,600 40.3 us in step, 46.6 in turns; 6,700 x 3,840 x 1,280 84 and 106).
+      if (!a.kv && a.K >= (a.out_dtype == DN_BF16 && !a.resid ? 1280 : 1600)) return launch_without_kv<4, 2, 4, 5, 3, 2, true>(a, stream);
       return launch_as<8, 2, 2, 5, 3, 2>(a, stream);
     case 4:
       if (!sixteen) return launch_as<4, 2, 4, 6, 4>(a, stream);
