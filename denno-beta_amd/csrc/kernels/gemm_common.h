@@ -195,6 +195,12 @@ int run(const void* A, int lda, const void* W, const float* bias, void* C, int l
         int N, int K, int out_dtype, int epi, const KVScatter* kv, hipStream_t stream);
 }  // namespace tiled
 
+// 16 bytes a lane from memory straight into LDS: lane l's at the wave's address + 16 l
+// not a template: the host pass must not see the builtin inside one
+__device__ __forceinline__ void load_to_lds(const void* src, void* dst) {
+  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+}
+
 namespace direct {
 struct Args {
   const void* A; int lda; const void* W; const float* bias; void* C; int ldc; float* resid; int ldr;

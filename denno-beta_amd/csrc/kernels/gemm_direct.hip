@@ -40,11 +40,6 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
 constexpr int XCDS = 8, CUS = 256, LDS_PER_CU = 160 * 1024;
 
-// not a template: the host pass must not see the builtin inside one
-__device__ __forceinline__ void load_to_lds(const void* src, void* dst) {
-  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
-}
-
 // element `which` (0..3, the lane's own choice) of the vector that lane E of this lane's quad holds
 template <int E>
 __device__ __forceinline__ float quad_pick(const floatx4& v, int which) {

@@ -22,7 +22,7 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 // so the product itself runs on rows that are not normalised, and the norm is two numbers per row in
 // the epilogue.  NORM_OUT: a product that adds into the residual stream also stores the updated rows
 // times gamma (the next norm's), rounded to bfloat16, and, for each row, the mean and the sum of
-// squared distances from it of its 16 columns.  NORM_IN: A is such a copy; each wave joins two rows'
+// squared distances from it of its 16 columns.  NORM_IN: A is such a copy; each wave joins two to eight rows'
 // N / 16 pairs (means are averaged; the squares add up with 16 times the squared distance of each
 // block's mean from the row's: exact, and as stable as two passes over the row) while the operands
 // travel, and wave 0 applies them at the end.  The rows are rounded to bfloat16 before the mean is
@@ -111,7 +111,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   TC* C = static_cast<TC*>(late.C);
   constexpr int BLOCKS = MB * NB;                          // 16 x 16 blocks of C in this workgroup
   constexpr int PASSES = (BLOCKS + WAVES - 1) / WAVES;     // wave w finishes blocks w, w + WAVES, ...
-  __shared__ floatx4 red[WAVES][BLOCKS][64];
+  constexpr int SP = 2, SR = NORM == NORM_IN ? MB * 16 / WAVES : 0;      // (statistics: up to 64 SP pairs a row, SR rows a wave)
+  __shared__ floatx4 red[WAVES][SR > BLOCKS ? SR : BLOCKS][64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;   // (a scalar: what follows from it is the scalar unit's work)
   const int col = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * (16 * NB);
@@ -158,32 +159,42 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
       }
     }
   }
-  // NORM_IN: wave w joins the statistics of rows w, w + WAVES, ...: their pairs are asked for now, before
-  // the operands (up to SP * 64 blocks of 16 columns a row)
-  constexpr int SP = 2, SR = MB * 16 / WAVES;
+  // NORM_IN: wave w joins the statistics of rows SR w .. SR w + SR - 1.  Their pairs are asked for now, before the operands, and go
+  // straight into LDS, a row's 1 KB where this wave's sums will lie at the end, so no barrier stands between.  In registers they stood beside a round's
+  // operands (with all else as it is here, 64 rows of 4,800 x 1,600 with a cache write 12.0 us for 11.0, 5,120 x 1,280 9.1 for 8.0).
   __shared__ float rowstat[NORM == NORM_IN ? MB * 16 : 1][2];
-  float2 st[NORM == NORM_IN ? SR : 1][SP];
   if constexpr (NORM == NORM_IN) {
+    if (blocks_in % 2 == 0 && reinterpret_cast<uintptr_t>(stats_in) % 16 == 0) {
 #pragma unroll
-    for (int t = 0; t < SR; ++t) {
-      const int row = min(row0 + wave + t * WAVES, M - 1);
+      for (int t = 0; t < SR; ++t) {
+        const int row = min(row0 + wave * SR + t, M - 1);
+        load_to_lds(stats_in + (static_cast<size_t>(row) * blocks_in + min(2 * lane, blocks_in - 2)) * 2, red[wave][t]);
+      }
+    } else {      // (rows of an odd number of pairs are no multiples of 16 bytes)
 #pragma unroll
-      for (int i = 0; i < SP; ++i)
-        st[t][i] = *reinterpret_cast<const float2*>(stats_in + (static_cast<size_t>(row) * blocks_in + min(lane + 64 * i, blocks_in - 1)) * 2);
+      for (int t = 0; t < SR; ++t) {
+        const float* row = stats_in + static_cast<size_t>(min(row0 + wave * SR + t, M - 1)) * blocks_in * 2;
+#pragma unroll
+        for (int i = 0; i < SP; ++i)
+          reinterpret_cast<float2*>(red[wave][t])[lane + 64 * i] = *reinterpret_cast<const float2*>(row + min(lane + 64 * i, blocks_in - 1) * 2);
+      }
     }
   }
   // Loads are never conditional and nothing uses a loaded value before all loads of a round are
   // issued (a predicated load, or a use in between, makes each load wait for the one before it).
   // A step beyond K reads zeros (no_step) and meets a zeroed piece of A.
   // The first round of W is on its way while the rest of the prologue works.
-  bf16x8 b[U][NB];
+  bf16x8 b[U][NB], a[U][MB];
+  auto ask_w = [&](int p0) {
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int ks = 2 * (wave + (u / 2) * WAVES) + u % 2;
+    for (int u = 0; u < U; ++u) {
+      const int ks = 2 * (p0 + (u / 2) * WAVES) + u % 2;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-      b[u][nb] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk[nb] + ks * 512 : no_step(lane));
-  }
+      for (int nb = 0; nb < NB; ++nb)
+        b[u][nb] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk[nb] + ks * 512 : no_step(lane));
+    }
+  };
+  ask_w(wave);
   // what the epilogue reads by arguments that do not come with the launch: behind the first round of W
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) {
@@ -217,29 +228,56 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   }
   // NORM_IN: the rows' means and 1 / sqrt(var + eps), joined while the first round of operands travels (a
   // wave does it in its first turn of the loop below, which every wave has: K >= 1024); the finishing
-  // waves meet them behind the barrier further down
+  // waves meet them behind the barrier further down.  The sums of several rows go through the lanes side by side, with no branch between them, and the
+  // last steps are lane t's for the wave's row t.  Row by row, each with divisions, a square root and stores of its own, a wave's eight rows took longer than
+  // the operands (before -> with the statistics in LDS and the later rounds' loads together, 24, 40 and 64 rows: 4,800 x 1,600 with a cache write 9.2 -> 8.5,
+  // 10.7 -> 9.7, 13.0 -> 11.0 us; 6,400 x 1,600 with GELU 8.7 -> 7.8, 10.1 -> 8.8, 11.4 -> 9.8; 3,840 x 1,280 7.7 -> 7.2, 9.0 -> 8.2, 11.3 -> 9.3; 4,096 x
+  // 1,024 5.9 -> 5.4, 7.4 -> 6.2, 9.1 -> 7.2).
   auto join_stats = [&]() {
     const float blocks = static_cast<float>(blocks_in);      // pairs of statistics a row, 16 columns a pair
+    // The first round's U (MB + NB) loads are behind the statistics' and in front of this wait (the wave asked for both already), so with that many
+    // out the statistics are there; no load may move across.  The compiler sets no wait of its own between such loads and reads of LDS.
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(U * (MB + NB)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int TOGETHER = SR % 4 == 0 ? 4 : 3;      // rows whose sums go through the lanes side by side
+    float row_mean = 0.f, row_sq = 0.f;                // (lane t: of the wave's row t)
 #pragma unroll
-    for (int t = 0; t < SR; ++t) {
-      const int row = wave + t * WAVES;
-      float sm = 0.f;
+    for (int t0 = 0; t0 < SR; t0 += TOGETHER) {
+      float2 st[TOGETHER][SP];
+      float mean[TOGETHER], sq[TOGETHER];
 #pragma unroll
-      for (int i = 0; i < SP; ++i)
-        if (lane + 64 * i < blocks_in) sm += st[t][i].x;
-      const float mean = late.no_mean ? 0.f : wave_sum(sm) / blocks;      // (without it the squares are taken about 0)
-      float sq = 0.f;
+      for (int t = 0; t < TOGETHER; ++t)
 #pragma unroll
-      for (int i = 0; i < SP; ++i)
-        if (lane + 64 * i < blocks_in) {
-          const float d = st[t][i].x - mean;
-          sq += st[t][i].y + 16.f * d * d;
-        }
-      const float var = wave_sum(sq) / (16.f * blocks);
-      if (lane == 0) {
-        rowstat[row][0] = row0 + row < M ? mean : 0.f;
-        rowstat[row][1] = row0 + row < M ? 1.0f / sqrtf(var + late.eps) : 0.f;
+        for (int i = 0; i < SP; ++i) st[t][i] = reinterpret_cast<const float2*>(red[wave][t0 + t])[lane + 64 * i];
+#pragma unroll
+      for (int t = 0; t < TOGETHER; ++t) {
+        mean[t] = sq[t] = 0.f;
+#pragma unroll
+        for (int i = 0; i < SP; ++i) mean[t] += lane + 64 * i < blocks_in ? st[t][i].x : 0.f;
       }
+#pragma unroll
+      for (int t = 0; t < TOGETHER; ++t) mean[t] = wave_sum(mean[t]);
+#pragma unroll
+      for (int t = 0; t < TOGETHER; ++t) {
+        mean[t] = late.no_mean ? 0.f : mean[t] / blocks;      // (without it the squares are taken about 0)
+#pragma unroll
+        for (int i = 0; i < SP; ++i) {
+          const float d = st[t][i].x - mean[t];
+          const float more = sq[t] + (st[t][i].y + 16.f * d * d);
+          sq[t] = lane + 64 * i < blocks_in ? more : sq[t];
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < TOGETHER; ++t) sq[t] = wave_sum(sq[t]);
+#pragma unroll
+      for (int t = 0; t < TOGETHER; ++t)
+        if (lane == t0 + t) row_mean = mean[t], row_sq = sq[t];
+    }
+    if (lane < SR) {
+      const int row = wave * SR + lane;
+      rowstat[row][0] = row0 + row < M ? row_mean : 0.f;
+      rowstat[row][1] = row0 + row < M ? 1.0f / sqrtf(row_sq / (16.f * blocks) + late.eps) : 0.f;
     }
   };
   floatx4 acc[MB][NB];
@@ -249,24 +287,17 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = floatx4{0.f, 0.f, 0.f, 0.f};
   // the steps go to the waves in pairs: wave w takes steps 2w, 2w + 1, 2 (w + WAVES), ... (the same
   // shares as in gemm16_kernel, so that both sum in the same order)
-  for (int p0 = wave; 2 * p0 < ksteps; p0 += WAVES * (U / 2)) {
-    bf16x8 a[U][MB];
+  auto ask_a = [&](int p0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int ks = 2 * (p0 + (u / 2) * WAVES) + u % 2;
       const bool ok = ks < ksteps && ks * 32 + g * 8 < K;
-      if (p0 != wave) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          b[u][nb] = *reinterpret_cast<const bf16x8*>(ks < ksteps ? wblk[nb] + ks * 512 : no_step(lane));
-      }
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
         a[u][mb] = *reinterpret_cast<const bf16x8*>(ok ? arow[mb] + ks * astep : asafe[mb]);
     }
-    if constexpr (NORM == NORM_IN) {
-      if (p0 == wave) join_stats();
-    }
+  };
+  auto use = [&](int p0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int ks = 2 * (p0 + (u / 2) * WAVES) + u % 2;
@@ -282,6 +313,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
           acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][mb], b[u][nb], acc[mb][nb], 0, 0, 0);
+  };
+  // A later round's loads of W stand together behind one branch: a branch for each step, among A's loads, made each of them wait for every load
+  // before it.
+  for (int p0 = wave; 2 * p0 < ksteps; p0 += WAVES * (U / 2)) {
+    if (p0 != wave) ask_w(p0);
+    ask_a(p0);
+    if constexpr (NORM == NORM_IN) {
+      if (p0 == wave) join_stats();
+    }
+    use(p0);
   }
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
@@ -677,12 +718,14 @@ static void launch_norm(const Call& c, const NormIO& nio, int norm, hipStream_t 
   hipLaunchKernelGGL((gemm_kernel<MB, NB, WAVES, U, TC, KV, NORM>), grid, block, 0, stream,                       \
                      static_cast<const bf16_t*>(c.A), static_cast<const bf16_t*>(c.W), c.lda, c.M, c.N, c.K, c.packed, c.ldr, \
                      NORM == NORM_IN ? static_cast<const void*>(nio.stats_in) : c.resid, c.bias, late_of<END_PLAIN>(c, nio))
-  if (norm == NORM_OUT)
+  if (norm == NORM_OUT) {
     DN_LN(float, false, NORM_OUT);
-  else if (c.kv)
-    DN_LN(bf16_t, true, NORM_IN);
-  else
-    DN_LN(bf16_t, false, NORM_IN);
+  } else if constexpr (U <= 8) {      // (K of 2,048 at most: four pairs a wave)
+    if (c.kv)
+      DN_LN(bf16_t, true, NORM_IN);
+    else
+      DN_LN(bf16_t, false, NORM_IN);
+  }
 #undef DN_LN
 }
 
@@ -691,14 +734,15 @@ void launch_mb_norm(const Call& c, const NormIO& nio, int norm, hipStream_t stre
   const int mb = (c.M + 15) / 16;
   if (c.N >= 2560) {
     switch (mb) {
-      // (four steps in flight a wave: with six, the norm's sums beside them no longer fit the registers, and the
-      // product that also scatters keys and values took 24 us where it takes 13)
+      // (four steps in flight a wave; with six and the statistics in LDS, 64 rows of 3,840 x 1,280 9.3 -> 10.3 us, 4,800 x 1,600 level)
       case 2: return launch_norm<2, 2, 8, 4>(c, nio, norm, stream);
       case 3: return launch_norm<3, 2, 8, 4>(c, nio, norm, stream);
       default: return launch_norm<4, 2, 8, 4>(c, nio, norm, stream);
     }
   }
   // (few columns: the rows in two halves, so that there are workgroups for all CUs)
+  // A wave's share of K in whole rounds of five pairs where it is that many (64 rows of 1,280 x 5,120, two rounds for three: 10.7 -> 9.5 us), else in rounds of four.
+  if (norm == NORM_OUT && ((c.K + 63) / 64 + 7) / 8 % 5 == 0) return launch_norm<2, 1, 8, 10>(c, nio, norm, stream);
   return launch_norm<2, 1, 8, 8>(c, nio, norm, stream);
 }
 
