@@ -87,7 +87,7 @@ static int act_route(const void* A, int lda, const void* W, const float* bias, c
   if (kind < EPI_XIELU || kind > EPI_EXP_NEG_SOFTPLUS || out_dtype != (kind == EPI_XIELU ? DN_BF16 : DN_F32)) return 0;
   const bool few = skinny::takes(A, lda, W, M, K, packed);
   const bool many = direct::takes(A, lda, W, bias, C, ldc, nullptr, 0, N, K, out_dtype, packed);
-  if (many && (!few || direct::beats_few_rows(M, N, K))) return kind == EPI_XIELU ? 2 : 0;
+  if (many && (!few || direct::beats_few_rows(M, N, K)) && (kind == EPI_XIELU || M > 64)) return kind == EPI_XIELU ? 2 : 0;
   return few && M <= 64 ? 1 : 0;
 }
 

@@ -38,6 +38,7 @@ namespace direct {
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+typedef floatx4 floatx4_at_4 __attribute__((aligned(4)));
 constexpr int XCDS = 8, CUS = 256, LDS_PER_CU = 160 * 1024;
 
 // element `which` (0..3, the lane's own choice) of the vector that lane E of this lane's quad holds
@@ -409,10 +410,18 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
         floatx4* x = reinterpret_cast<floatx4*>(resid + static_cast<size_t>(m) * ldr + n);
         *x = *x + v;
       } else if constexpr (sizeof(TC) == 4) {
+        // (rows of any length and place, see `takes`: 16 bytes at a multiple of 4, a row's last one to three columns by themselves)
         floatx4 o;
 #pragma clang loop unroll(full)
         for (int r = 0; r < 4; ++r) o[r] = apply_epilogue_fast(v[r], epi);
-        *reinterpret_cast<floatx4*>(C + static_cast<size_t>(m) * ldc + n) = o;
+        TC* to = C + static_cast<size_t>(m) * ldc + n;
+        if (n + 4 <= N) {
+          *reinterpret_cast<floatx4_at_4*>(to) = o;
+        } else {
+#pragma clang loop unroll(full)
+          for (int r = 0; r < 3; ++r)
+            if (n + r < N) to[r] = o[r];
+        }
       } else {
         auto finish = [&](float e) { return XIELU ? xielu_f(e, act_a, act_b) : apply_epilogue_fast(e, epi); };
         const uint2 cv = pack4(finish(v[0]), finish(v[1]), finish(v[2]), finish(v[3]));
@@ -453,14 +462,18 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   }
 }
 
-// everything 16 bytes at a time: slabs of 32 along K, rows of A and C (or the residual) and the bias
+// Everything 16 bytes at a time: slabs of 32 along K, rows of A and C (or the residual) and the bias.  32-bit results without a bias may have
+// rows of any length and place: a vocabulary's logits (203 rows of 50,257 x 1,280 in the few-rows kernel, which took them, 279 us, here 48;
+// 65 rows 81 and 36; 1,024 rows, in the tiled kernel before, 200).
 bool takes(const void* A, int lda, const void* W, const float* bias, const void* C, int ldc, const float* resid,
                   int ldr, int N, int K, int out_dtype, int packed) {
   auto aligned = [](const void* p, int a) { return reinterpret_cast<uintptr_t>(p) % a == 0; };
-  if (K % 32 != 0 || N % 4 != 0 || !aligned(A, 16) || !aligned(W, 16) || !aligned(bias, 16)) return false;
+  const bool any_rows = out_dtype == DN_F32 && !resid && !bias && !(packed & PACKED_C);
+  if (K % 32 != 0 || (N % 4 != 0 && !any_rows) || !aligned(A, 16) || !aligned(W, 16) || !aligned(bias, 16)) return false;
   if (!(packed & PACKED_A) && lda % 8 != 0) return false;
   if (resid) return ldr % 4 == 0 && aligned(resid, 16);
   if (packed & PACKED_C) return N % 32 == 0 && out_dtype == DN_BF16 && aligned(C, 8);
+  if (any_rows) return aligned(C, 4);
   return ldc % 4 == 0 && aligned(C, out_dtype == DN_F32 ? 16 : 8);
 }
 
@@ -567,11 +580,19 @@ bool mid_rows(int M, int N, int K) {
   return M <= 256;
 }
 
+// 17 to 64 rows of so many columns that tiles of 64 x 64 give most CUs one (a vocabulary): a workgroup of the few-rows kernel reads all rows anew for
+// every 32 or 64 columns, and its waves wait for the rows.  Few-rows kernel -> here, packed rows, K = 1,024, 1,600 and 2,048: 17 rows of 12,288 columns 8.3 ->
+// 7.3, 12.8 -> 11.9, 16.3 -> 14.0 us, of 50,257 30.5 -> 23.8, 44.9 -> 36.5, 54.2 -> 41.9; 64 rows 11.0 -> 7.9, 16.0 -> 13.7, 20.3 -> 15.1 and 43.5 ->
+// 26.2, 63.4 -> 39.2, 74.1 -> 45.2; 8,192 columns stay (64 rows 7.1, 7.6 here; 17 rows 5.9, 7.1).  Where those tiles are more than
+// the CUs, tiles of 64 x 128 (64 rows of 24,576 x 1,600 22.4 -> 20.3, of 20,480 x 1,024 13.9 -> 13.2).  A short K: 40 rows of 50,257 x 512 19.6 -> 16.7, of
+// 12,288 x 512 6.7 -> 5.7; up to 32 rows level from 576 to 832 (17 rows x 50,257 x 768 20.6 and 20.7) and slower below (512 14.9, 15.7).
+bool wide_few(int M, int N, int K) { return M > 16 && M <= 64 && N >= 12288 && K >= (M > 32 ? 512 : 1024) && K % 64 == 0; }
+
 // Up to 256 rows the few-rows kernel takes the product too (both read and write packed rows): it stays ahead,
 // or level, where the product has few columns and a short K; everywhere else from 65 rows on this kernel is
 // the faster (`mid_rows`), and beyond 256 rows it is the only one.
 bool beats_few_rows(int M, int N, int K) {
-  return mid_rows(M, N, K) || (M > 104 && N >= 4096) || (M > 208 && N >= 2048);
+  return wide_few(M, N, K) || mid_rows(M, N, K) || (M > 104 && N >= 4096) || (M > 208 && N >= 2048);
 }
 
 // A long K beside few columns and few rows: the tiles are few and each walks all of K, a slab at a time,
@@ -611,9 +632,15 @@ int deferred_shares(int M, int N, int K) {
 static bool wide_mid(int M, int N) { return N >= 2048 && M <= 256; }
 static long tiles_of(int M, int N, int bm, int bn) { return static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 static long mid_tiles_64(int M, int N) { return tiles_of(M, N, 64, 64); }
+// Whether `mid_rows` has its tiles: wide products only while one round of tiles of 128 x 64 covers them; beyond, `pick`'s larger ones read the rows less
+// often (these -> those: 203 rows of 9,216 x 1,600 26.5 -> 16.9 us, of 16,384 29.0 -> 23.1, 50,257 x 1,280 78 -> 48; 128 rows of 20,480 x
+// 1,024 20.8 -> 16.1, and of 16,384, one round, 12.3 and 12.1; 256 rows of 8,192 x 1,600, one round, 14.9 and 14.6).
+static bool mid_tiles(int M, int N, int K) { return mid_rows(M, N, K) && (N < 2048 || tiles_of(M, N, 128, 64) <= CUS); }
 
 int run(const Args& a, hipStream_t stream) {
-  if (mid_rows(a.M, a.N, a.K) || (a.part && a.N < 2048 && a.K % 64 == 0)) {
+  if (wide_few(a.M, a.N, a.K) && !a.part)
+    return mid_tiles_64(a.M, a.N) <= CUS ? launch_mid<4, 4, 1, 1, 4, 2>(a, stream) : launch_as<4, 4, 1, 2, 4, 2>(a, stream);
+  if (mid_tiles(a.M, a.N, a.K) || (a.part && a.N < 2048 && a.K % 64 == 0)) {
     // Wide products: sixteen waves a workgroup, four a SIMD, each with one 16 x 16 block of a 64 x 64 tile (a wave
     // of such a product waits on a counter for more than half of its life, and with one wave a SIMD nothing else
     // runs meanwhile: 16.0 -> 13.9 and 12.8 -> 11.3 us for 4,800 and 6,400 columns at 128 rows); where those tiles
@@ -665,7 +692,8 @@ int run(const Args& a, hipStream_t stream) {
 
 // the tile that a product of these sizes gets: rows * 1000 + columns
 int tile_of(int M, int N, int K, bool kv) {
-  if (mid_rows(M, N, K)) return wide_mid(M, N) && mid_tiles_64(M, N) > CUS ? 128064 : 64064;
+  if (wide_few(M, N, K)) return mid_tiles_64(M, N) <= CUS ? 64064 : 64128;
+  if (mid_tiles(M, N, K)) return wide_mid(M, N) && mid_tiles_64(M, N) > CUS ? 128064 : 64064;
   const Shape& s = SHAPES[pick(M, N, K, kv)];
   return s.bm * 1000 + s.bn;
 }
