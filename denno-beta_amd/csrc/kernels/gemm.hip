@@ -22,7 +22,9 @@
 
 // the tile that a product of these sizes gets from the kernel above: rows * 1000 + columns
 extern "C" int dn_gemm_tile(int M, int N, int K) { return direct::tile_of(M, N, K); }
-// the same for a fused projection that writes the cache (some tiles are not on offer to it)
+// the tile that stands before it for 65 to 512 rows of a wide product, 0: none
+extern "C" int dn_gemm_wide_tile(int M, int N, int K) { return direct::wide_tile_of(M, N, K); }
+// dn_gemm_tile for a fused projection that writes the cache (some tiles are not on offer to it)
 extern "C" int dn_gemm_tile_qkv(int M, int N, int K) { return direct::tile_of(M, N, K, true); }
 
 // packed: bit flags.  W in rows of K elements (the plain kernel, any dtype), or packed bfloat16

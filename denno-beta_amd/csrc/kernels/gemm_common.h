@@ -218,4 +218,5 @@ int shares_of_k(int M, int N, int K, int packed, bool kv);
 int deferred_shares(int M, int N, int K);
 int run(const Args& a, hipStream_t stream);
 int tile_of(int M, int N, int K, bool kv = false);
+int wide_tile_of(int M, int N, int K);
 }  // namespace direct

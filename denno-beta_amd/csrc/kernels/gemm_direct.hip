@@ -573,7 +573,7 @@ int pick(int M, int N, int K, bool kv) {
 // four products of a layer 1,600 wide (rows and weights that no cache holds; us, before -> now):
 //   128 rows: 4,800 columns 18.7 -> 15.7, 6,400 columns 15.3 -> 12.3, 1,600 columns from K = 6,400 19.4 -> 15.2
 //   256 rows: 25.6 -> 23.2, 19.3 -> 18.0, 25.6 -> 21.4;  512 rows, 1,600 columns: K = 1,600 12.6 -> 10.7, K = 6,400 38.7 -> 35.4
-// -> whether this kernel takes the product with those tiles (else `pick` chooses, or the few-rows kernel runs)
+// -> whether this kernel takes the product for its rows (wide ones in `wide_mid`'s tiles; else `pick` chooses, or the few-rows kernel runs)
 bool mid_rows(int M, int N, int K) {
   if (M <= 64 || M > 512 || K % 64 != 0) return false;
   if (N < 2048) return K >= 4096 || M > 256;      // (few columns and a short K up to 256 rows: the few-rows kernel)
@@ -629,27 +629,38 @@ int deferred_shares(int M, int N, int K) {
   return one >= 2 ? min(one, 4) : two >= 3 ? 3 : 0;
 }
 
-static bool wide_mid(int M, int N) { return N >= 2048 && M <= 256; }
 static long tiles_of(int M, int N, int bm, int bn) { return static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 static long mid_tiles_64(int M, int N) { return tiles_of(M, N, 64, 64); }
-// Whether `mid_rows` has its tiles: wide products only while one round of tiles of 128 x 64 covers them; beyond, `pick`'s larger ones read the rows less
-// often (these -> those: 203 rows of 9,216 x 1,600 26.5 -> 16.9 us, of 16,384 29.0 -> 23.1, 50,257 x 1,280 78 -> 48; 128 rows of 20,480 x
-// 1,024 20.8 -> 16.1, and of 16,384, one round, 12.3 and 12.1; 256 rows of 8,192 x 1,600, one round, 14.9 and 14.6).
-static bool mid_tiles(int M, int N, int K) { return mid_rows(M, N, K) && (N < 2048 || tiles_of(M, N, 128, 64) <= CUS); }
+// The tile of 65 to 512 rows of a wide product: the first of 64 x 64, 64 x 96 and 128 x 64 of which one round covers the product, 0 (`pick` chooses) where none
+// does: beyond, larger tiles read the rows less often.  Sixteen waves a workgroup, eight for 64 x 96, each tile's walk along K being what a round takes.
+// us, 64 x 96 for what ran before (128 x 64, beyond 256 rows what `pick` has): 203 and 256 rows of 4,800 x 1,600 with a cache write 15.3 -> 13.6 and
+// 15.7 -> 13.9, of 5,120 x 1,280 with GELU 11.8 -> 11.0 and 12.0 -> 11.2, 136 of 6,400 x 1,600 13.7 -> 12.5; 320 of 3,840 x 1,280 13.1 -> 11.9, 384 of 3,072 x
+// 1,024 11.5 -> 10.3; where 64 x 64 is one round, 203 of 3,840 x 1,280, 9.5 stays (11.6 so); where 64 x 96 is two, 288 of 5,120 x 1,280,
+// 128 x 64 11.9 and 64 x 96 13.1.  128 x 64 beyond 256 rows: 320 of 5,120 x 1,280 12.5 -> 11.6, 448 of 4,096 x 1,024 10.5 -> 10.1.  Two rounds of
+// 128 x 64 for what `pick` has: 203 rows of 9,216 x 1,600 26.5 and 16.9 us, 16,384 x 1,600 29.0 and 23.1, 50,257 x 1,280 78 and 48; 128 rows of
+// 20,480 x 1,024 20.8 and 16.1, of 16,384, one round, 12.3 and 12.1.
+static int wide_mid(int M, int N, int K) {
+  if (M <= 64 || M > 512 || N < 2048 || K % 64 != 0) return 0;
+  if (mid_tiles_64(M, N) <= CUS) return 64064;
+  if (tiles_of(M, N, 64, 96) <= CUS) return 64096;
+  return tiles_of(M, N, 128, 64) <= CUS ? 128064 : 0;
+}
 
 int run(const Args& a, hipStream_t stream) {
   if (wide_few(a.M, a.N, a.K) && !a.part)
     return mid_tiles_64(a.M, a.N) <= CUS ? launch_mid<4, 4, 1, 1, 4, 2>(a, stream) : launch_as<4, 4, 1, 2, 4, 2>(a, stream);
-  if (mid_tiles(a.M, a.N, a.K) || (a.part && a.N < 2048 && a.K % 64 == 0)) {
-    // Wide products: sixteen waves a workgroup, four a SIMD, each with one 16 x 16 block of a 64 x 64 tile (a wave
-    // of such a product waits on a counter for more than half of its life, and with one wave a SIMD nothing else
-    // runs meanwhile: 16.0 -> 13.9 and 12.8 -> 11.3 us for 4,800 and 6,400 columns at 128 rows); where those tiles
-    // are more than the chip has CUs, tiles of 128 x 64 with two blocks a wave (at 256 rows 23.3 -> 20.2 and
-    // 18.1 -> 15.2 us).  The narrow ones, whose K is shared out, take neither way faster: four waves as before.
-    if (wide_mid(a.M, a.N) && !a.part)
-      return mid_tiles_64(a.M, a.N) <= CUS ? launch_mid<4, 4, 1, 1, 4, 2>(a, stream) : launch_mid<4, 4, 2, 1, 4, 2>(a, stream);
-    return launch_mid<2, 2, 2, 2, 4, 2>(a, stream);
+  // Wide products: sixteen waves a workgroup, four a SIMD, each with one 16 x 16 block of a 64 x 64 tile (a wave
+  // of such a product waits on a counter for more than half of its life, and with one wave a SIMD nothing else
+  // runs meanwhile: 16.0 -> 13.9 and 12.8 -> 11.3 us for 4,800 and 6,400 columns at 128 rows), or tiles with more blocks a wave (`wide_mid`).
+  // The narrow ones, whose K is shared out, take no such way faster: four waves.
+  if (!a.part) {
+    switch (wide_mid(a.M, a.N, a.K)) {
+      case 64064: return launch_mid<4, 4, 1, 1, 4, 2>(a, stream);
+      case 64096: return launch_mid<4, 2, 1, 3, 4, 2>(a, stream);
+      case 128064: return launch_mid<4, 4, 2, 1, 4, 2>(a, stream);
+    }
   }
+  if (((a.part || a.N < 2048) && mid_rows(a.M, a.N, a.K)) || (a.part && a.N < 2048 && a.K % 64 == 0)) return launch_mid<2, 2, 2, 2, 4, 2>(a, stream);
   // Tiles of 128 and 256 rows: sixteen waves a workgroup, four a SIMD, as 8 x 2 (a wave: 32 rows x a half of the
   // tile's columns) or 4 x 4, where eight waves as 4 x 2 with twice the rows each left the SIMDs waiting (a wave
   // waits on a counter for more than half of its life and the matrix cores were busy 30 % of the time).  At 2,048
@@ -690,11 +701,13 @@ int run(const Args& a, hipStream_t stream) {
   }
 }
 
-// the tile that a product of these sizes gets: rows * 1000 + columns
+// the tile that a product of these sizes gets: rows * 1000 + columns; beyond 256 rows the one that the list has for it, before which `wide_tile_of` is asked
 int tile_of(int M, int N, int K, bool kv) {
   if (wide_few(M, N, K)) return mid_tiles_64(M, N) <= CUS ? 64064 : 64128;
-  if (mid_tiles(M, N, K)) return wide_mid(M, N) && mid_tiles_64(M, N) > CUS ? 128064 : 64064;
+  if (N < 2048 && mid_rows(M, N, K)) return 64064;
+  if (const int tile = wide_mid(M, N, K); tile && M <= 256) return tile;
   const Shape& s = SHAPES[pick(M, N, K, kv)];
   return s.bm * 1000 + s.bn;
 }
+int wide_tile_of(int M, int N, int K) { return wide_mid(M, N, K); }
 }  // namespace direct
