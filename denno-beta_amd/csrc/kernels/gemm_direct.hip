@@ -289,12 +289,15 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   // in its page a value lies as [dim][offset], so four tokens whose slots follow one another from a
   // multiple of 4 are 8 bytes side by side for one dim: the four lanes of a quad, which hold four
   // tokens x four dims, exchange them (a 4 x 4 turn), and each stores four tokens of one dim.
-  // A place is the row's (page and offset) plus the block's (head and first dim), and the block's is the same for all lanes: worked out
-  // lane by lane, with its divisions, it was most of this epilogue.
+  // A place is the row's (page and offset) plus the column's (head and dim); the latter without a division.  Only where a head is a
+  // multiple of 16 dims, and keys and values begin at one, does a block of 16 columns have one place (`whole_blocks`: the keys of the staged way
+  // below); elsewhere a lane's four columns have theirs, which are one head's and of one kind since all of these are multiples of 4.
   long long krow[KV ? TM : 1], vrow[KV ? TM : 1];      // of the row in the pools, -1: none
   uint32_t dh_inverse = 0;                             // 2^32 / dh, rounded up: c / dh is c times that (below 2^32 / dh)
   int page_numbers = 0;
+  bool whole_blocks = false;
   if constexpr (KV) {
+    whole_blocks = kv.dh % 16 == 0 && kv.q_width % 16 == 0;
     dh_inverse = 0xffffffffu / static_cast<uint32_t>(kv.dh) + 1;
     page_numbers = kv.Hkv * kv.page_size * kv.dh;
 #pragma clang loop unroll(full)
@@ -309,9 +312,9 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
       vrow[i] = run ? static_cast<long long>(page) * page_numbers + off : -1;
     }
   }
-  // where a block of keys lies in a page, from its first column on
-  auto key_place = [&](int first_column) {
-    const uint32_t c = first_column - kv.q_width;
+  // where keys lie in a page from this column on, to the end of their head
+  auto key_place = [&](int column) {
+    const uint32_t c = column - kv.q_width;
     return static_cast<int>(c + __umulhi(c, dh_inverse) * (kv.page_size - 1) * kv.dh);
   };
   if (part) {
@@ -342,7 +345,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
   bool staged = false;
   if constexpr (STAGED) {
     staged = !(packed & PACKED_C) && ldc % 8 == 0 && N % 8 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
-    if constexpr (KV) staged = staged && kv.c_cols % 8 == 0 && reinterpret_cast<uintptr_t>(kv.k_pool) % 16 == 0;
+    if constexpr (KV) staged = staged && whole_blocks && kv.c_cols % 8 == 0 && reinterpret_cast<uintptr_t>(kv.k_pool) % 16 == 0;
     if (staged) {
       int place[KV ? TN : 1];      // of a block of keys in its page: the head's and the first dim's
       if constexpr (KV) {
@@ -392,14 +395,14 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
     const int n = n0 + (wnb + j) * 16 + (lane / 16) * 4;
     if (n >= N) continue;
     const floatx4 bv = bvs[j];
-    // (a block of 16 columns is all queries, all keys or all values, and of one head: the widths are multiples of 16)
+    // (what a block has none of is known to the whole wave)
     const int block = n0 + (wnb + j) * 16;
-    bool is_key = false, is_value = false;
-    int at = 0;
+    bool keys = false, values = false;
+    int at = 0;      // of the block's first column among the values of a page
     if constexpr (KV) {
-      is_key = block >= kv.q_width && block < kv.q_width + kv.kv_width;
-      is_value = block >= kv.q_width + kv.kv_width;
-      at = is_value ? (block - kv.q_width - kv.kv_width) * kv.page_size : is_key ? key_place(block) : 0;
+      keys = block + 16 > kv.q_width && block < kv.q_width + kv.kv_width;
+      values = block + 16 > kv.q_width + kv.kv_width;
+      at = (block - kv.q_width - kv.kv_width) * kv.page_size;
     }
 #pragma clang loop unroll(full)
     for (int i = 0; i < TM; ++i) {
@@ -429,12 +432,16 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
         if (!KV || n < kv.c_cols)
           *reinterpret_cast<uint2*>(C + ((packed & PACKED_C) ? packed_index(m, n, N / 32) : static_cast<size_t>(m) * ldc + n)) = cv;
         if constexpr (KV) {
-          if (is_key && krow[i] >= 0) *reinterpret_cast<uint2*>(kv.k_pool + krow[i] + at + (lane / 16) * 4) = cv;
+          // (with the place of whole blocks the scalar unit's: lane by lane for all of them the wide tiles' registers don't reach)
+          if (keys && krow[i] >= 0 && n >= kv.q_width && n < kv.q_width + kv.kv_width) {
+            const int place = whole_blocks ? key_place(block) + (lane / 16) * 4 : key_place(n);
+            *reinterpret_cast<uint2*>(kv.k_pool + krow[i] + place) = cv;
+          }
         }
       }
     }
     if constexpr (KV) {
-      if (is_value) {
+      if (values) {
         const int q = lane % 4;       // this lane's dim of the four after the turn
 #pragma clang loop unroll(full)
         for (int i = 0; i < TM; ++i) {
@@ -443,6 +450,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(const bf16_t* __rest
           // token mq + e, dim d + q: lane e of the quad holds it in v[q]
           const float t0 = quad_pick<0>(v, q), t1 = quad_pick<1>(v, q), t2 = quad_pick<2>(v, q), t3 = quad_pick<3>(v, q);
           const int dim = (lane / 16) * 4 + q;
+          if (n < kv.q_width + kv.kv_width) continue;
           if (vrow[i] >= 0) {
             *reinterpret_cast<uint2*>(kv.v_pool + vrow[i] + at + dim * kv.page_size) = pack4(t0, t1, t2, t3);
           } else {

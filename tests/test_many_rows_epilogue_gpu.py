@@ -54,3 +54,65 @@ def test_queries_and_keys_of_many_rows_go_to_their_places(M, heads, kv_heads, dh
         q = ops().linear_qkv(a, w, bias, out, slots, k1, v1, qw)
         assert torch.equal(q, plain[:, :qw]) and torch.equal(k1, k0) and torch.equal(v1, v0)
         assert wide == qw or torch.equal(out, plain)
+
+
+def into_cache(M, heads, kv_heads, dh, ps, beyond, q_more=0, K=128):
+    """The fused projection's queries and pages against the product alone with its keys and values put into the pages by torch, bit for bit."""
+    qw, kvw = heads * dh + q_more, kv_heads * dh
+    N, pages = qw + 2 * kvw, M // ps + 4
+    a, w, bias = operands(M, N, K)
+    slot = torch.arange(M) + 3
+    order = torch.cat([torch.randperm(pages - 1, generator=torch.Generator().manual_seed(4)), torch.tensor([pages - 1])])      # (the last page is nobody's)
+    slots = (order[slot // ps] * ps + slot % ps).to(torch.int32)
+    slots[5::97] = -1
+    plain = torch.empty(M, N, dtype=BF, device=DEV)
+    ops().linear(a, w, bias, out=plain)
+    new = lambda: (torch.full((pages, kv_heads, ps, dh), 7.0, dtype=BF, device=DEV), torch.full((pages, kv_heads, dh, ps), 7.0, dtype=BF, device=DEV))      # noqa: E731
+    k0, v0 = new()
+    has = (slots >= 0).nonzero()[:, 0].to(DEV)
+    page, off = slots.to(DEV).long()[has] // ps, slots.to(DEV).long()[has] % ps
+    k0[page, :, off] = plain[has, qw:qw + kvw].view(-1, kv_heads, dh)
+    v0[page, :, :, off] = plain[has, qw + kvw:].view(-1, kv_heads, dh)
+    for wide in (qw, N):
+        k1, v1 = new()
+        rows = torch.full((M + 1, wide + beyond), 7.0, dtype=BF, device=DEV)
+        q = ops().linear_qkv(a, w, bias, rows[:M, :wide], slots.to(DEV), k1, v1, qw)
+        assert torch.equal(q, plain[:, :qw]) and torch.equal(k1, k0) and torch.equal(v1, v0)
+        assert bool((rows[M] == 7.0).all()) and bool((rows[:M, wide:] == 7.0).all())
+        assert wide == qw or torch.equal(rows[:M, :wide], plain)
+
+
+# (dims that are multiples of 4 alone, of 8, of 16; widths of queries, and of keys, that end inside a block of 16 columns)
+HEADS = [(8, 8, 40, 16), (16, 16, 24, 16), (16, 16, 20, 24), (5, 3, 20, 16), (6, 2, 20, 32), (8, 8, 72, 64), (8, 2, 104, 16), (3, 1, 100, 16), (9, 9, 4, 16),
+         (7, 3, 12, 48), (4, 4, 64, 16), (4, 2, 48, 24)]
+
+
+@pytest.mark.parametrize("M", [16, 64, 257, 513, 2049])
+@pytest.mark.parametrize("heads,kv_heads,dh,ps", HEADS)
+@pytest.mark.parametrize("beyond", [0, 4])
+def test_heads_of_any_multiple_of_four(M, heads, kv_heads, dh, ps, beyond):
+    """A block of 16 columns may hold the end of one head and the beginning of the next, or queries and keys, or keys and values."""
+    into_cache(M, heads, kv_heads, dh, ps, beyond)
+
+
+@pytest.mark.parametrize("M", [65, 203, 257, 300])
+@pytest.mark.parametrize("heads,kv_heads,dh,ps", [(40, 40, 20, 16), (30, 30, 24, 24), (24, 24, 40, 16), (12, 12, 100, 16), (29, 3, 72, 32), (60, 20, 36, 16), (25, 25, 64, 16)])
+@pytest.mark.parametrize("beyond", [0, 4])
+def test_wide_heads_of_any_multiple_of_four(M, heads, kv_heads, dh, ps, beyond):
+    """2,048 columns and more: the tiles of 65 to 512 rows."""
+    into_cache(M, heads, kv_heads, dh, ps, beyond)
+
+
+@pytest.mark.parametrize("M", [64, 300, 2049])
+@pytest.mark.parametrize("q_more", [4, 8, 12])
+@pytest.mark.parametrize("dh", [40, 64])
+def test_queries_that_end_inside_a_block(M, q_more, dh):
+    """Whole heads of 16 dims behind queries that are no whole blocks."""
+    into_cache(M, 10, 10, dh, 16, 0, q_more)
+
+
+@pytest.mark.parametrize("M", [1100, 2049])
+@pytest.mark.parametrize("heads,kv_heads,dh,K", [(40, 40, 40, 1280), (16, 16, 100, 96), (64, 64, 20, 64), (25, 25, 64, 1280)])
+def test_large_tiles_with_heads_of_any_multiple_of_four(M, heads, kv_heads, dh, K):
+    """Thousands of columns: the tiles of 128 and 256 rows, in both widths of a stage."""
+    into_cache(M, heads, kv_heads, dh, 16, 0, K=K)
