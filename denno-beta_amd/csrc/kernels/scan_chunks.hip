@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256, 4) void chunk_parts_kernel(ChunkArgs a) {
       asm volatile("" : "+v"(x[L - 1]), "+v"(x[j + 1])::"memory");
     }
 #pragma unroll
-    for (int t = 0; t < L; ++t) X[t][n] = static_cast<float>(x[t] * beta[n]);
+    for (int t = 0; t < L; ++t) X[t][n] = t >= n ? static_cast<float>(x[t] * beta[n]) : 0.f;      // (a later row's beta may be no number)
   } else if (tid >= 64 && tid - 64 < DK) {
     const int i = tid - 64, b = i / 16;
     double f = 1.0;

@@ -70,3 +70,40 @@ def test_what_is_no_number_does_not_reach_rows_before_it(mode, bad, which):
         close(got[1][:, keep], got[0][:, keep])
     if which == "r":
         close(got[1][at + 1:], got[0][at + 1:])
+
+
+def per_row(heads, qk_heads, dk, dv, T, fade):
+    """The operands of the delta rule with one decay a row: beta's and the decay's arguments, rate and bias."""
+    r, k, v, kw = operands("wide", heads, qk_heads, dk, dv, T, fade)
+    return r, k, v, dict(beta=kw["beta"], w=rnd(T, heads, seed=6)), rnd(heads, seed=7).abs() * fade, rnd(heads, seed=8)
+
+
+def chunks(mode, r, k, v, kw, state, row_start, slots, heads, dk, dv, qk_heads=None):
+    out = torch.zeros(len(r), heads * dv, device=DEV)
+    if mode == "rows":
+        kw, rate, bias = kw
+        ops().delta_chunks(r, k, v, kw["beta"], kw["w"], rate, bias, state, row_start, slots, heads, dk, dv, out, qk_heads)
+    else:
+        ops().scan_chunks(r, k, v, kw["w"], state, row_start, slots, heads, dk, dv, out, qk_heads=qk_heads, **{a: t for a, t in kw.items() if a != "w"})
+    return out
+
+
+@pytest.mark.parametrize("mode,which", [("wide", "beta"), ("wide", "w"), ("rows", "beta"), ("rows", "w"), ("rows", "v"), ("rows", "k"), ("rows", "r")])
+@pytest.mark.parametrize("at", [0, 15, 16, 21, 49])
+def test_no_number_among_the_numbers_of_a_row(mode, which, at):
+    """Beta's argument, decays and the operands of the rule with one decay a row: rows before it and other heads have none of it."""
+    heads, dk, dv, T = 2, 64, 40, 50
+    row_start, slots, _ = tables([T], [0])
+    r, k, v, kw = operands("wide", heads, heads, dk, dv, T, 0.5)
+    if mode == "rows":
+        r, k, v, kw, rate, bias = per_row(heads, heads, dk, dv, T, 0.5)
+    got = []
+    for spoilt in (False, True):
+        x = dict(r=r.clone(), k=k.clone(), v=v.clone(), **{a: t.clone() for a, t in kw.items()})
+        if spoilt:
+            x[which][at, 0] = float("nan")      # (of head 0)
+        numbers = {a: x[a] for a in kw}
+        got.append(chunks(mode, x["r"], x["k"], x["v"], (numbers, rate, bias) if mode == "rows" else numbers, torch.zeros(1, heads * dk * dv, device=DEV),
+                          row_start, slots, heads, dk, dv))
+    close(got[1][:at], got[0][:at]), close(got[1][:, dv:], got[0][:, dv:])
+    assert not bool(torch.isfinite(got[1][at, :dv]).all())
