@@ -419,7 +419,9 @@ __global__ __launch_bounds__((Walk<DB>::WAVES + 1) * 64) void chunk_walk_kernel(
         for (int i = 0; i < 4; ++i) x = mfma(q.kt[b][i], E[i], x);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float y = fmaf(S[b][i], q.hi[b][i], fmaf(S[b][i], q.lo[b][i], x[i]));
+          // (Without the delta rule, which makes of an infinity what is no number, it stays one: as it is, times what the decay's rounding left, which may be
+          // nothing or less, it would not.  The largest number in its place in that product: three requests of 2,136 rows 41.1 -> 42.4 us.)
+          const float rest = DELTA ? S[b][i] : __builtin_amdgcn_fmed3f(S[b][i], -__FLT_MAX__, __FLT_MAX__), y = fmaf(S[b][i], q.hi[b][i], fmaf(rest, q.lo[b][i], x[i]));
           S[b][i] = mine[b] ? y : 0.f;
         }
       }

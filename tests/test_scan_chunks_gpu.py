@@ -107,3 +107,23 @@ def test_no_number_among_the_numbers_of_a_row(mode, which, at):
                           row_start, slots, heads, dk, dv))
     close(got[1][:at], got[0][:at]), close(got[1][:, dv:], got[0][:, dv:])
     assert not bool(torch.isfinite(got[1][at, :dv]).all())
+
+
+@pytest.mark.parametrize("T", [1, 16, 40, 200])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf")])
+def test_an_infinite_state_stays_infinite(T, bad):
+    """Constant decays: as row after row, an entry that has overflowed stays what it is, and so do its column's results."""
+    heads, dk, dv = 2, 64, 40
+    row_start, slots, _ = tables([T], [0])
+    r, k, v, kw = operands("head", heads, heads, dk, dv, T, 0.1)
+    state = torch.randn(1, heads * dv * dk, device=DEV)
+    state.view(heads, dv, dk)[1, 7, 3] = bad
+    one, many = state.clone(), state.clone()
+    want = torch.zeros(T, heads * dv, device=DEV)
+    ops().state_scan(r, k, v, None, None, one, row_start, slots, heads, dk, dv, want, read_after=True, w_head=kw["w_head"])
+    got = chunks("head", r, k, v, kw, many, row_start, slots, heads, dk, dv)
+    for a, b in ((got, want), (many, one)):
+        fine = torch.isfinite(b)
+        assert torch.equal(a[~fine], b[~fine])
+        close(a[fine], b[fine])
+    assert int((~torch.isfinite(many)).sum()) == 1 and bool(torch.isinf(want[:, dv + 7]).all())
