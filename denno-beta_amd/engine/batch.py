@@ -103,16 +103,18 @@ def plan_rows(entries: Sequence[StepEntry], starts: Sequence[int], vocab: int, m
             row_start, tiles, wide)
 
 
-def build_context(entries: Sequence[StepEntry], cache, vocab: int, max_positions: int, device) -> StepContext:
+def build_context(entries: Sequence[StepEntry], cache, vocab: int, max_positions: int, device, logit_rows_min: int = 0) -> StepContext:
     """Reserves pages for the entries' tokens (raising cache.OutOfPages; pages taken for
     earlier entries stay with their requests) and builds the step's tables.  The cache manager is
-    asked once per table for the whole step, not once per request."""
+    asked once per table for the whole step, not once per request.  logit_rows_min: row 0's logits are wanted behind the wanted
+    places until there are so many."""
     mgr = cache.manager
     rids = np.asarray([e.rid for e in entries], dtype=np.int64)
     counts = np.asarray([len(e.tokens) for e in entries], dtype=np.int32)
     starts_a = mgr.lengths(rids)
     starts = starts_a.tolist()
     tokens, positions, logit_rows, row_start, tiles, wide = plan_rows(entries, starts, vocab, max_positions)
+    logit_rows = logit_rows + [0] * (logit_rows_min - len(logit_rows))
     slots_a = mgr.reserve_step(rids, starts_a + counts)
     T, S, R = len(tokens), len(entries), len(logit_rows)
     slots = slots_a.tolist()

@@ -167,6 +167,28 @@ def _bucket(n, sizes):
     return None
 
 
+def portion_bucket(entries: Sequence[StepEntry]):
+    """(T, S, R) of the bucket that a step of these entries falls into, or None if none takes it."""
+    rows, wanted = sum(len(e.tokens) for e in entries), sum(len(e.want) for e in entries)
+    T, S = _bucket(rows, PORTION_ROWS), _bucket(len(entries), PORTION_REQUESTS)
+    if T is None or S is None or rows < 1:
+        return None
+    return (T, S, S if wanted <= S else T)
+
+
+def wanted_rows(entries: Sequence[StepEntry], max_live: int) -> int:
+    """The rows whose logits a captured step of these entries computes, 0 if they want none; the wanted places themselves where no graph takes such a
+    step.  A vocabulary's product sums in another order from 17 rows on than up to 16 (csrc/kernels/gemm_direct.hip), so a step kernel by kernel
+    computes as many: its logits are then the same bits."""
+    wanted = sum(len(e.want) for e in entries)
+    if wanted == 0:
+        return 0
+    if all(len(e.tokens) == 1 for e in entries):
+        return max(wanted, batch_bucket(len(entries), max_live))
+    bucket = portion_bucket(entries)
+    return wanted if bucket is None else max(wanted, bucket[2])
+
+
 class PortionGraph:
     def __init__(self, runner, T: int, S: int, R: int):
         from .batch import TILE_ROWS, WIDE_TILE_ROWS
@@ -352,11 +374,7 @@ class DecodeGraphs:
         runner = self.runner
         if not runner.model.graph_safe or not runner.options.graph_portions:
             return None
-        rows, wanted = sum(len(e.tokens) for e in entries), sum(len(e.want) for e in entries)
-        T, S = _bucket(rows, PORTION_ROWS), _bucket(len(entries), PORTION_REQUESTS)
-        if T is None or S is None or rows < 1:
-            return None
-        return (T, S, S if wanted <= S else T)
+        return portion_bucket(entries)
 
     def takes_portions(self, entries: Sequence[StepEntry]) -> bool:
         """Whether this step is replayed from a captured graph: its bucket has been met before (and is captured

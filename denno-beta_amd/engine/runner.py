@@ -16,6 +16,7 @@ from ..config import EngineOptions, load_config
 from ..parts import Runtime
 from ..weights import draw_all, load_checkpoint
 from .batch import StepEntry, build_context
+from .graphs import DecodeGraphs, wanted_rows
 
 _ACT = {"bfloat16": torch.bfloat16, "float32": torch.float32}
 
@@ -46,7 +47,6 @@ class ModelRunner:
         self.steps_run = 0
         self.graphs = None
         if options.use_graphs and self.device.type == "cuda":
-            from .graphs import DecodeGraphs
             self.graphs = DecodeGraphs(self)
 
     # -- construction --------------------------------------------------------------------
@@ -108,8 +108,14 @@ class ModelRunner:
         if self.graphs is not None and self.graphs.takes_portions(entries):
             self.steps_run += 1
             return self.graphs.step_portions(entries, borrow)
-        ctx = build_context(entries, self.cache, self.spec.vocab, self.spec.max_positions, self.device)
+        # (as many rows as a captured step of these entries has: see wanted_rows; the 32-bit products are the same bits for any number of rows)
+        rows = 0
+        if self.device.type == "cuda" and self.model.graph_safe and self.runtime.act_dtype != torch.float32:
+            rows = wanted_rows(entries, self.options.max_live)
+        ctx = build_context(entries, self.cache, self.spec.vocab, self.spec.max_positions, self.device, rows)
         logits = self.model.forward(ctx, self.cache)
+        if rows:
+            logits = logits[:sum(len(e.want) for e in entries)]
         self.cache.manager.commit_step(
             np.asarray(ctx.rids, dtype=np.int64),
             np.asarray([start + len(e.tokens) for e, start in zip(entries, ctx.host_first_pos)], dtype=np.int32))
