@@ -48,7 +48,7 @@ struct ChunkArgs {
   float* state;
   size_t slot_stride;
   const int *row_start, *slots;
-  int S, H, G, dk, dv, chunks;
+  int S, H, G, dk, dv, chunks, rows_min;      // (requests of fewer than rows_min rows are another kernel's)
   float* work;
   float* out;
   size_t ldo;
@@ -114,8 +114,8 @@ __global__ __launch_bounds__(256, 4) void chunk_parts_kernel(ChunkArgs a) {
     if (before != ~0ull) break;
   }
   if (s < 0) return;
-  const int base = chunk_base(a.row_start, s), row0 = a.row_start[s] + L * (id - base), rows = min(L, a.row_start[s + 1] - row0);
-  if (rows <= 0 || a.slots[s] < 0) return;
+  const int base = chunk_base(a.row_start, s), begin = a.row_start[s], end = a.row_start[s + 1], row0 = begin + L * (id - base), rows = min(L, end - row0);
+  if (rows <= 0 || end - begin < a.rows_min || a.slots[s] < 0) return;
   const int hq = h / (a.H / a.G), dv = a.dv, vblocks = (dv + 15) / 16;
   float* rec = a.work + (static_cast<size_t>(id) * a.H + h) * Rec::floats(dv);
   // rows beyond the last: r = 0, k = 0, w = 1, beta = 0, which change nothing
@@ -337,7 +337,7 @@ __global__ __launch_bounds__((Walk<DB>::WAVES + 1) * 64) void chunk_walk_kernel(
   const int slot = a.slots[s];
   if (slot < 0) return;
   const int row0 = a.row_start[s], row1 = a.row_start[s + 1];
-  if (row0 >= row1) return;
+  if (row0 >= row1 || row1 - row0 < a.rows_min) return;
   const int dv = a.dv, col = blockIdx.y * 16 + n;
   const bool live = col < dv;
   const int chunks = (row1 - row0 + L - 1) / L;
@@ -551,15 +551,15 @@ long long dn_delta_chunks_floats(int T, int S, int H, int dk, int dv) {
 // 2: a constant decay per head, w [H], no delta rule (zb none).
 int dn_scan_chunks(const float* r, long long ldr, const float* k, long long ldk, const float* v, long long ldv, const float* zb, long long ldb,
                    const float* w, long long ldw, const float* rate, const float* bias, int mode, float* state, long long slot_stride,
-                   const int* row_start, const int* slots, int S, int T, int H, int G, int dk, int dv, float* work, float* out, long long ldo,
-                   hipStream_t stream) {
+                   const int* row_start, const int* slots, int S, int T, int H, int G, int dk, int dv, int rows_min, float* work, float* out,
+                   long long ldo, hipStream_t stream) {
   if (dk < 16 || dk > 128 || dk % 16 != 0 || dv < 1 || H < 1 || G < 1 || H % G != 0 || S < 1 || S > 65535 || H > 65535 || (dv + 15) / 16 > 65535 ||
       reinterpret_cast<uintptr_t>(work) % 16 != 0 || slot_stride < static_cast<long long>(H) * dk * dv || ldo >= (1LL << 24) || mode < DELTA_WIDE || mode > FADE_HEAD ||
       !w || (mode != FADE_HEAD) != (zb != nullptr) || (mode == DELTA_ROWS) != (rate != nullptr))
     return DN_ERR_SHAPE;
   if (T == 0) return 0;
   const ChunkArgs a{r, k, v, zb, w, rate, bias, static_cast<size_t>(ldr), static_cast<size_t>(ldk), static_cast<size_t>(ldv), static_cast<size_t>(ldb),
-                    static_cast<size_t>(ldw), state, static_cast<size_t>(slot_stride), row_start, slots, S, H, G, dk, dv, T / L + S, work, out,
+                    static_cast<size_t>(ldw), state, static_cast<size_t>(slot_stride), row_start, slots, S, H, G, dk, dv, T / L + S, rows_min, work, out,
                     static_cast<size_t>(ldo)};
   if (mode == DELTA_WIDE) return launch_of<DELTA_WIDE>(a, stream);
   if (mode == DELTA_ROWS) return launch_of<DELTA_ROWS>(a, stream);
@@ -569,12 +569,12 @@ int dn_scan_chunks(const float* r, long long ldr, const float* k, long long ldk,
 // mode 1 alone, rows of r and k at multiples of 16 bytes
 int dn_delta_chunks(const float* r, long long ldr, const float* k, long long ldk, const float* v, long long ldv, const float* zb, long long ldb,
                     const float* zw, long long ldw, const float* rate, const float* bias, float* state, long long slot_stride,
-                    const int* row_start, const int* slots, int S, int T, int H, int G, int dk, int dv, float* work, float* out,
+                    const int* row_start, const int* slots, int S, int T, int H, int G, int dk, int dv, int rows_min, float* work, float* out,
                     long long ldo, hipStream_t stream) {
   auto by16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (ldr % 4 != 0 || ldk % 4 != 0 || !by16(r) || !by16(k)) return DN_ERR_SHAPE;
-  return dn_scan_chunks(r, ldr, k, ldk, v, ldv, zb, ldb, zw, ldw, rate, bias, DELTA_ROWS, state, slot_stride, row_start, slots, S, T, H, G, dk, dv, work,
-                        out, ldo, stream);
+  return dn_scan_chunks(r, ldr, k, ldk, v, ldv, zb, ldb, zw, ldw, rate, bias, DELTA_ROWS, state, slot_stride, row_start, slots, S, T, H, G, dk, dv, rows_min,
+                        work, out, ldo, stream);
 }
 
 }  // extern "C"

@@ -809,7 +809,7 @@ struct ScanArgs {
   float* state;
   size_t slot_stride;
   const int *row_start, *slots;
-  int H, dk, dv, read_after, key_from_decay, beta_logits, w_rows;
+  int H, dk, dv, read_after, key_from_decay, beta_logits, w_rows, rows_below;      // (requests of rows_below rows and more are another kernel's; 0: none are)
   float* out;
   size_t ldo;
 };
@@ -840,7 +840,7 @@ __global__ __launch_bounds__(64) void scan_kernel(ScanArgs a) {
   const int slot = a.slots[s];
   if (slot < 0) return;
   const int row0 = a.row_start[s], row1 = a.row_start[s + 1];
-  if (row0 >= row1) return;
+  if (row0 >= row1 || (a.rows_below > 0 && row1 - row0 >= a.rows_below)) return;
   const bool live = j < a.dv;
   const int dk = a.dk, dv = a.dv;
   // the state lies [head][value column][key channel]: a lane's channels side by side, a column's lanes too
@@ -2544,8 +2544,8 @@ int dn_gated(const void* x, int x_dt, long long ldx, const float* g, long long l
 int dn_state_scan(const float* r, long long ldr, const float* k, long long ldk, const float* v, long long ldv, const float* w,
                   long long ldw, const float* u, const float* beta, long long ldb, const float* w_head, int G, float* state,
                   long long slot_stride, const int* row_start, const int* slots, int S, int T, int H, int dk, int dv, int mode,
-                  int key_from_decay, int beta_logits, int w_rows, const float* w_rate, const float* w_bias, float* out, long long ldo,
-                  hipStream_t stream) {
+                  int key_from_decay, int beta_logits, int w_rows, const float* w_rate, const float* w_bias, int rows_below, float* out,
+                  long long ldo, hipStream_t stream) {
   if (dk < 1 || dk > 256 || dv < 1 || H < 1 || G < 1 || H % G != 0) return DN_ERR_SHAPE;
   if ((!key_from_decay && k == nullptr) || (w_rows && (w == nullptr || key_from_decay))) return DN_ERR_SHAPE;
   if (mode < SCAN_BEFORE || mode > SCAN_DELTA || (mode == SCAN_DELTA && beta == nullptr) || (w == nullptr) == (w_head == nullptr))
@@ -2554,7 +2554,7 @@ int dn_state_scan(const float* r, long long ldr, const float* k, long long ldk, 
   if (S == 0) return 0;
   const int read_after = mode;
   ScanArgs a{r, k, v, w, u, beta, w_head, w_rate, w_bias, static_cast<size_t>(ldr), static_cast<size_t>(ldk), static_cast<size_t>(ldv),
-             static_cast<size_t>(ldw), static_cast<size_t>(ldb), G, state, static_cast<size_t>(slot_stride), row_start, slots, H, dk, dv, read_after, key_from_decay, beta_logits, w_rows, out,
+             static_cast<size_t>(ldw), static_cast<size_t>(ldb), G, state, static_cast<size_t>(slot_stride), row_start, slots, H, dk, dv, read_after, key_from_decay, beta_logits, w_rows, rows_below, out,
              static_cast<size_t>(ldo)};
   // (the parts of a column's sum by the head's size alone, never by the step: a row's bits are the same in every step)
   const dim3 few((dv + 15) / 16, H, S), many((dv + 3) / 4, H, S);

@@ -148,7 +148,7 @@ def _declare(name, lib):
             "dn_activate": [P, c_longlong, P, P, I, P, I, c_longlong, I, I, P],
             "dn_gated": [P, I, c_longlong, P, c_longlong, I, P, I, c_longlong, I, I, P],
             "dn_state_scan": [P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, P, c_longlong, P, I, P, c_longlong, P, P,
-                              I, I, I, I, I, I, I, I, I, P, P, P, c_longlong, P],
+                              I, I, I, I, I, I, I, I, I, P, P, I, P, c_longlong, P],
             "dn_head_norm": [P, c_longlong, P, I, F, P, c_longlong, I, I, P, c_longlong, P, I, P, I, c_longlong, I, I, I, P],
             "dn_step_sizes": [P, c_longlong, P, P, P, c_longlong, I, I, I, P, c_longlong, P, c_longlong, P],
             "dn_gate_scan": [P, c_longlong, P, c_longlong, P, c_longlong, P, P, P, c_longlong, P, P, I, I, I, P, I, c_longlong, P],
@@ -159,9 +159,9 @@ def _declare(name, lib):
             "dn_conv_turn_write": [P, c_longlong, I, I, I, I, P, I, P, c_longlong, P, P, I, P, P, F, P, I, P, P, c_longlong, I, P, P, P, I, I, I, I, I, P],
             "dn_clamped_glu": [P, c_longlong, F, F, P, I, c_longlong, I, I, P],
             "dn_post_norm": [P, c_longlong, F, P, c_longlong, P, c_longlong, P, P, F, P, P, I, I, P, P, F, P, I, c_longlong, I, I, P],
-            "dn_scan_chunks": [P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, P, I, P, c_longlong, P, P, I, I, I, I, I, I, P, P,
+            "dn_scan_chunks": [P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, P, I, P, c_longlong, P, P, I, I, I, I, I, I, I, P, P,
                                c_longlong, P],
-            "dn_delta_chunks": [P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, P, P, c_longlong, P, P, I, I, I, I, I, I, P, P,
+            "dn_delta_chunks": [P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, P, P, c_longlong, P, P, I, I, I, I, I, I, I, P, P,
                                 c_longlong, P],
             "dn_turn_back_gate": [P, I, c_longlong, I, P, c_longlong, P, P, P, I, c_longlong, I, I, I, P],
             "dn_poly_norm": [P, c_longlong, P, F, P, I, c_longlong, I, I, P],
@@ -1376,7 +1376,7 @@ def gated(x, g, kind, out):
 
 
 def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, read_after=False, key_from_decay=False, beta=None,
-               w_head=None, qk_heads=None, beta_logits=False, w_rows=False, w_rate=None, w_bias=None):
+               w_head=None, qk_heads=None, beta_logits=False, w_rows=False, w_rate=None, w_bias=None, rows_below=0):
     """The recurrence of a matrix state per head, S [dk, dv], over each request's rows of this step in order:
       a = 1 - w if key_from_decay else k
       read_after:  S <- diag(w) S + a v^T ;  o = S^T r
@@ -1387,7 +1387,8 @@ def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, rea
     w_head: 32-bit [heads], one decay per head for every row and channel;
     w_rate (and w_bias): 32-bit [heads], with w_rows in the delta rule: w holds z and the decay is exp(-w_rate log(1 + e^(z + w_bias)));
     v, out: 32-bit [T, heads * dv]; beta: 32-bit [T, heads] (beta_logits: it holds z, and beta is 1 / (1 + e^-z)); state: 32-bit [slots, heads * dv * dk] (a head's state
-    held [value column][key channel]), read and written at the requests' slots."""
+    held [value column][key channel]), read and written at the requests' slots.  rows_below: requests of that many rows and more are left alone
+    (0: none are), for `scan_chunks` and `delta_chunks` with the same number."""
     G = n_heads if qk_heads is None else qk_heads
     _need(G >= 1 and n_heads % G == 0, lambda: f"state_scan: {n_heads} heads over {G} heads of queries and keys")
     _need((w is None) != (w_head is None), "state_scan: a decay per row and channel (w) or one per head (w_head)")
@@ -1412,28 +1413,31 @@ def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, rea
                                        _rows(w, "w") if w is not None else 0, _ptr(u), _ptr(beta),
                                        _rows(beta, "beta") if beta is not None else 0, _ptr(w_head), G, state.data_ptr(), stride,
                                        row_start.data_ptr(), slots.data_ptr(), S, T, n_heads, dk, dv, mode, int(key_from_decay),
-                                       int(bool(beta_logits)), int(bool(w_rows)), _ptr(w_rate), _ptr(w_bias), out.data_ptr(),
+                                       int(bool(beta_logits)), int(bool(w_rows)), _ptr(w_rate), _ptr(w_bias), int(rows_below), out.data_ptr(),
                                        _rows(out, "out"), _stream()),
         "state_scan" if beta is None else "state_scan (delta rule)")
     return out
 
 
-# Rows a request, on average, from which a step's recurrences are walked in chunks.  A request of a chunk or two is sooner done row by row: the first of
-# the two kernels takes 8 us whatever it has to do, and with a decay per channel or head most of it in 64-bit.
+# Rows of a request in a step from which its recurrences are walked in chunks.  A request of a chunk or two is sooner done row by row: the first of
+# the two kernels takes 8 us whatever it has to do, and with a decay per channel or head most of it in 64-bit (us, 8 heads of 64 x 128, chunks and by
+# rows: a decay per channel 64 rows 15.3 and 10.6, 96 16.3 and 15.0, 128 17.6 and 18.9; per head 64 9.7 and 8.4, 96 10.5 and 11.4; one a row 32 10.9 and 6.6, 80
+# 12.4 and 12.6: for these, less, because chunks are the nearer to 64 bits, 1.1e-7 and 1.7e-7 at 32 rows).  By the request's own rows, whatever else is
+# in the step: its bits then depend neither on that nor on a captured step's padding, and a prompt beside decoded rows goes in chunks (1,024 rows and ten
+# of one: 160 us by rows, 60 in both kernels; where the others are no single rows but 60 and 90 beside 350 they take longer, 29 -> 45).
 CHUNKS_ROWS_MIN, DELTA_CHUNKS_ROWS_MIN = 96, 32
 
 
-def chunks_takes(T, S, dk, least=CHUNKS_ROWS_MIN):
-    """Whether a step of T rows of S requests is one for `scan_chunks` (`least` DELTA_CHUNKS_ROWS_MIN: for `delta_chunks`): portions, key heads of
-    a size that they know."""
-    return T >= least * S and dk % 16 == 0 and 16 <= dk <= 128
+def chunks_take(dk):
+    """Whether key heads are of a size that `scan_chunks` and `delta_chunks` know."""
+    return dk % 16 == 0 and 16 <= dk <= 128
 
 
-def scan_chunks(r, k, v, w, state, row_start, slots, n_heads, dk, dv, out, beta=None, w_head=None, qk_heads=None):
+def scan_chunks(r, k, v, w, state, row_start, slots, n_heads, dk, dv, out, beta=None, w_head=None, qk_heads=None, rows_min=0):
     """state_scan's delta rule with a decay per row and channel (beta given, as the sigmoid's argument; w [T, heads * dk]), or its
     recurrence with one constant decay per head that reads after its write (w None, w_head [heads]; no beta), 16 rows of a request at a
     time on the matrix cores in 32-bit: the same recurrence, its sums in another order, so a row's result changes by rounding with
-    the place where its portion begins.  dk: a multiple of 16 up to 128."""
+    the place where its portion begins.  dk: a multiple of 16 up to 128.  rows_min: requests of fewer rows are left alone."""
     G = n_heads if qk_heads is None else qk_heads
     _need(G >= 1 and n_heads % G == 0, lambda: f"scan_chunks: {n_heads} heads over {G} heads of queries and keys")
     _need((w is None) != (w_head is None) and (beta is None) == (w is None), "scan_chunks: decays per row and channel with beta, or one per head without")
@@ -1452,14 +1456,15 @@ def scan_chunks(r, k, v, w, state, row_start, slots, n_heads, dk, dv, out, beta=
     _ok(lib.dn_scan_chunks(r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"), _ptr(beta),
                            _rows(beta, "beta") if beta is not None else 0, _ptr(w_head) if w is None else w.data_ptr(), 0 if w is None else _rows(w, "w"),
                            0, 0, 2 if w is None else 0, state.data_ptr(), stride, row_start.data_ptr(), slots.data_ptr(), S, T, n_heads, G, dk, dv,
-                           work.data_ptr(), out.data_ptr(), _rows(out, "out"), _stream()), "scan_chunks")
+                           int(rows_min), work.data_ptr(), out.data_ptr(), _rows(out, "out"), _stream()), "scan_chunks")
     return out
 
 
-def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads, dk, dv, out, qk_heads=None):
+def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads, dk, dv, out, qk_heads=None, rows_min=0):
     """state_scan's delta rule with one decay per row and head (beta_logits, w_rows, w_rate = rate, w_bias = bias), 16 rows of a
     request at a time on the matrix cores in 32-bit: the same recurrence, its sums in another order, so a row's result changes by
-    rounding with the place where its portion begins.  dk: a multiple of 16 up to 128; rows of r and k at multiples of 16 bytes."""
+    rounding with the place where its portion begins.  dk: a multiple of 16 up to 128; rows of r and k at multiples of 16 bytes.
+    rows_min: requests of fewer rows are left alone."""
     G = n_heads if qk_heads is None else qk_heads
     _need(G >= 1 and n_heads % G == 0, lambda: f"delta_chunks: {n_heads} heads over {G} heads of queries and keys")
     given = ((r, "r", G * dk), (k, "k", G * dk), (v, "v", n_heads * dv), (out, "out", n_heads * dv), (beta, "beta", n_heads), (w, "w", n_heads))
@@ -1476,7 +1481,7 @@ def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads,
     work = torch.empty(lib.dn_delta_chunks_floats(T, S, n_heads, dk, dv), dtype=torch.float32, device=r.device)
     _ok(lib.dn_delta_chunks(r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"), beta.data_ptr(), _rows(beta, "beta"),
                             w.data_ptr(), _rows(w, "w"), rate.data_ptr(), _ptr(bias), state.data_ptr(), stride, row_start.data_ptr(), slots.data_ptr(),
-                            S, T, n_heads, G, dk, dv, work.data_ptr(), out.data_ptr(), _rows(out, "out"), _stream()), "delta_chunks")
+                            S, T, n_heads, G, dk, dv, int(rows_min), work.data_ptr(), out.data_ptr(), _rows(out, "out"), _stream()), "delta_chunks")
     return out
 
 

@@ -12,6 +12,24 @@ from .linear import Linear
 F32 = torch.float32
 
 
+def walk(ctx, dk, rows_min, in_chunks, by_rows):
+    """A step's recurrences, each request's by its own rows: in_chunks(rows_min) for those of that many and more, by_rows(rows_below) for the others
+    (0: for all).  What no request of the step needs is not launched.  A captured step's rows stand in its tables alone, which a replay
+    fills: it has both, if it has room for such a request."""
+    starts = ctx.host_row_start
+    if starts and starts[-1] == ctx.T:
+        rows = [b - a for a, b in zip(starts, starts[1:])]
+        fewest, most = min(rows, default=0), max(rows, default=0)
+    else:
+        fewest, most = 0, ctx.T
+    if most < rows_min or not ops.chunks_take(dk):
+        by_rows(0)
+    elif fewest >= rows_min:
+        in_chunks(0)
+    else:
+        in_chunks(rows_min), by_rows(rows_min)
+
+
 @MIXERS.register("wkv")
 class WKV(Part):
     """Every projection reads its own blend of the token's row and the row before it, h + (h' - h) mu.  r, k, v are
@@ -157,13 +175,19 @@ class Lightning(Part):
             ops.activate(z[:, :2 * qk + vw], "silu", z[:, :2 * qk + vw])
         o = torch.empty((T, vw), dtype=F32, device=h.device)
         q, k, v = z[:, :qk], z[:, qk:2 * qk], z[:, 2 * qk:2 * qk + vw]
-        # (the 32-bit engine walks a request's rows in order: its logits are the same bits however a prompt is cut)
-        if act != F32 and not ctx.single_rows and ops.chunks_takes(T, ctx.S, self.head_dim):
+
+        def in_chunks(least):
             ops.scan_chunks(q, k, v, None, cache.state, ctx.row_start, ctx.state_slots, self.n_heads, self.head_dim, self.value_dim, o,
-                            w_head=self.decay_t)
-        else:
+                            w_head=self.decay_t, rows_min=least)
+
+        def by_rows(below):
             ops.state_scan(q, k, v, None, None, cache.state, ctx.row_start, ctx.state_slots, self.n_heads, self.head_dim, self.value_dim, o,
-                           read_after=True, w_head=self.decay_t)
+                           read_after=True, w_head=self.decay_t, rows_below=below)
+        # (the 32-bit engine walks a request's rows in order: its logits are the same bits however a prompt is cut)
+        if act != F32 and not ctx.single_rows:
+            walk(ctx, self.head_dim, ops.CHUNKS_ROWS_MIN, in_chunks, by_rows)
+        else:
+            by_rows(0)
         y = torch.empty((T, vw), dtype=act, device=h.device)
         ops.head_norm(o, self.norm, self.eps, y, 1, gate=z[:, 2 * qk + vw:], gate_kind="sigmoid")
         if accumulate_into is None:
@@ -280,14 +304,20 @@ class ChannelDelta(Part):
                 ops.activate(g, "exp_neg_softplus", g, bias=self.dt_bias, lower=self.rate)
             gate = self.g2(g_in, out_dtype=F32)
         o = torch.empty((T, vw), dtype=F32, device=dev)
-        # (beta = sigmoid of the projection's columns behind the channels, taken inside the scan; the 32-bit engine walks a request's rows in
-        # order: its logits are the same bits however a prompt is cut)
-        if act != F32 and not single and ops.chunks_takes(T, ctx.S, self.head_dim):
+
+        # (beta = sigmoid of the projection's columns behind the channels, taken inside the scan)
+        def in_chunks(least):
             ops.scan_chunks(q, k, v, g, state, ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, beta=z[:, C:C + H],
-                            qk_heads=self.n_qk_heads)
-        else:
+                            qk_heads=self.n_qk_heads, rows_min=least)
+
+        def by_rows(below):
             ops.state_scan(q, k, v, g, None, state, ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, beta=z[:, C:C + H],
-                           qk_heads=self.n_qk_heads, beta_logits=True)
+                           qk_heads=self.n_qk_heads, beta_logits=True, rows_below=below)
+        # (the 32-bit engine walks a request's rows in order: its logits are the same bits however a prompt is cut)
+        if act != F32 and not single:
+            walk(ctx, self.head_dim, ops.CHUNKS_ROWS_MIN, in_chunks, by_rows)
+        else:
+            by_rows(0)
         y = torch.empty((T, vw), dtype=act, device=dev)
         ops.head_norm(o, self.norm, self.eps, y, H, gate=gate, gate_kind="sigmoid")
         if accumulate_into is None:
@@ -368,15 +398,21 @@ class GatedDelta(Part):
             ops.history_update(z[:, :C], past, ctx.row_start, ctx.state_slots)
         gate, b = C, C + vw
         o = torch.empty((T, vw), dtype=F32, device=dev)
-        # (beta and the decay are made from their arguments inside the scan; the 32-bit engine walks a request's rows in order: its
-        # logits are the same bits however a prompt is cut)
-        if act != F32 and not single and qk % 4 == 0 and C % 4 == 0 and ops.chunks_takes(T, ctx.S, self.head_dim, ops.DELTA_CHUNKS_ROWS_MIN):
+
+        # (beta and the decay are made from their arguments inside the scan)
+        def in_chunks(least):
             ops.delta_chunks(x[:, :qk], x[:, qk:2 * qk], x[:, 2 * qk:], z[:, b:b + H], z[:, b + H:b + 2 * H], self.rate, self.dt_bias, state,
-                             ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, qk_heads=self.n_qk_heads)
-        else:
+                             ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, qk_heads=self.n_qk_heads, rows_min=least)
+
+        def by_rows(below):
             ops.state_scan(x[:, :qk], x[:, qk:2 * qk], x[:, 2 * qk:], z[:, b + H:b + 2 * H], None, state, ctx.row_start, ctx.state_slots, H,
                            self.head_dim, self.value_dim, o, beta=z[:, b:b + H], qk_heads=self.n_qk_heads, beta_logits=True, w_rows=True,
-                           w_rate=self.rate, w_bias=self.dt_bias)
+                           w_rate=self.rate, w_bias=self.dt_bias, rows_below=below)
+        # (the 32-bit engine walks a request's rows in order: its logits are the same bits however a prompt is cut)
+        if act != F32 and not single and qk % 4 == 0 and C % 4 == 0:
+            walk(ctx, self.head_dim, ops.DELTA_CHUNKS_ROWS_MIN, in_chunks, by_rows)
+        else:
+            by_rows(0)
         y = torch.empty((T, vw), dtype=act, device=dev)
         ops.head_norm(o, self.norm, self.eps, y, H, gate=z[:, gate:gate + vw], gate_kind="silu")
         if accumulate_into is None:
