@@ -179,6 +179,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
           reinterpret_cast<float2*>(red[wave][t])[lane + 64 * i] = *reinterpret_cast<const float2*>(row + min(lane + 64 * i, blocks_in - 1) * 2);
       }
     }
+    // (no load of the first round in front of these: `join_stats` counts on their order)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
   }
   // Loads are never conditional and nothing uses a loaded value before all loads of a round are
   // issued (a predicated load, or a use in between, makes each load wait for the one before it).
@@ -235,8 +238,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   // 1,024 5.9 -> 5.4, 7.4 -> 6.2, 9.1 -> 7.2).
   auto join_stats = [&]() {
     const float blocks = static_cast<float>(blocks_in);      // pairs of statistics a row, 16 columns a pair
-    // The first round's U (MB + NB) loads are behind the statistics' and in front of this wait (the wave asked for both already), so with that many
-    // out the statistics are there; no load may move across.  The compiler sets no wait of its own between such loads and reads of LDS.
+    // The first round's U (MB + NB) loads are behind the statistics' (a barrier to the compiler stands between) and in front of this wait (the wave asked
+    // for both already), so with that many out the statistics are there; no load may move across.  The compiler sets no wait of its own between such loads and reads of LDS.
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(U * (MB + NB)) : "memory");
     __builtin_amdgcn_sched_barrier(0);
