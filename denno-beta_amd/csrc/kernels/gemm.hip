@@ -20,9 +20,10 @@
 // columns beyond N and K are zeros.
 #include "gemm_common.h"
 
-// the tile that a product of these sizes gets from the kernel above: rows * 1000 + columns
+// The tile that a product of these sizes gets from the many-rows kernel, rows * 1000 + columns; beyond 256 rows the one on its list, which is what
+// runs where dn_gemm_wide_tile is 0.
 extern "C" int dn_gemm_tile(int M, int N, int K) { return direct::tile_of(M, N, K); }
-// the tile that stands before it for 65 to 512 rows of a wide product, 0: none
+// the tile that goes before the list's for 65 to 512 rows of a wide product, 0: none does
 extern "C" int dn_gemm_wide_tile(int M, int N, int K) { return direct::wide_tile_of(M, N, K); }
 // dn_gemm_tile for a fused projection that writes the cache (some tiles are not on offer to it)
 extern "C" int dn_gemm_tile_qkv(int M, int N, int K) { return direct::tile_of(M, N, K, true); }

@@ -709,7 +709,7 @@ int run(const Args& a, hipStream_t stream) {
   }
 }
 
-// the tile that a product of these sizes gets: rows * 1000 + columns; beyond 256 rows the one that the list has for it, before which `wide_tile_of` is asked
+// the tile that a product of these sizes gets: rows * 1000 + columns; beyond 256 rows the one on the list, which runs where `wide_tile_of` is 0
 int tile_of(int M, int N, int K, bool kv) {
   if (wide_few(M, N, K)) return mid_tiles_64(M, N) <= CUS ? 64064 : 64128;
   if (N < 2048 && mid_rows(M, N, K)) return 64064;

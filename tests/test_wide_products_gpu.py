@@ -78,6 +78,9 @@ def test_one_round_of_wide_products(M, N, tile, K):
     within(exact, a, w)
     ops().linear(a, wp, bias, out=rounded[:M])
     assert torch.equal(rounded[:M], (exact + bias).to(BF)) and bool((rounded[M] == 7.0).all())
+    ops().linear(a, wp, bias, out=rounded[:M], epilogue="gelu_tanh")
+    # (half a unit of 8 bits, and what the kernel's tanh is off by)
+    assert torch.allclose(rounded[:M].float(), torch.nn.functional.gelu(exact + bias, approximate="tanh"), rtol=2.0 ** -8, atol=2e-6)
     x = x0.clone()
     ops().linear(a, wp, bias, residual=x)
     assert (x - (x0 + (exact + bias))).abs().max().item() <= 2.0 ** -20      # (one more rounding of sums below 16)
