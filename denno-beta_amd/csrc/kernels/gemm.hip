@@ -80,7 +80,9 @@ extern "C" int dn_gemm(const void* A, int lda, const void* W, const float* bias,
 // C [M, N] = act(A . W^T + bias) for an activation with numbers of its own (EPI_XIELU and on, see gemm_common.h), packed W: in the
 // epilogue of the kernel that dn_gemm would run, where it has that activation: the few-rows kernels with up to 64 rows have all
 // three, the many-rows kernel EPI_XIELU.  A kernel between the products is a launch (2 to 3 us of a decode step), and with many rows
-// a pass over the product's 32-bit result; the epilogue calls the same function, so the bits are those of the two kernels (EPI_XIELU, K = 1,024, two
+// a pass over the product's 32-bit result; the epilogue calls the same function, so the bits are those of the two kernels (but for EPI_SILU and
+// EPI_EXP_NEG_SOFTPLUS of 17 to 64 rows and 12,288 columns or more, `direct::wide_few`: the product alone is then the many-rows kernel's, whose sums stand in
+// another order; so it is with dn_gemm_two and dn_gemm_pair; EPI_XIELU, K = 1,024, two
 // kernels -> one: 8 rows of 4,096 columns 7.2 -> 4.6 us, 64 12.7 -> 9.7, 2,136 36.0 -> 28.7; a series and the hardware's exponential there would
 // take 0.1 us off few rows and 0.9 off many, and round otherwise).
 static int act_route(const void* A, int lda, const void* W, const float* bias, const void* C, int ldc, int M, int N, int K, int out_dtype,
