@@ -56,11 +56,12 @@ def test_queries_and_keys_of_many_rows_go_to_their_places(M, heads, kv_heads, dh
         assert wide == qw or torch.equal(out, plain)
 
 
-def into_cache(M, heads, kv_heads, dh, ps, beyond, q_more=0, K=128):
+def into_cache(M, heads, kv_heads, dh, ps, beyond, q_more=0, K=128, packed=False):
     """The fused projection's queries and pages against the product alone with its keys and values put into the pages by torch, bit for bit."""
     qw, kvw = heads * dh + q_more, kv_heads * dh
     N, pages = qw + 2 * kvw, M // ps + 4
     a, w, bias = operands(M, N, K)
+    a = ops().pack_matrix(a) if packed else a
     slot = torch.arange(M) + 3
     order = torch.cat([torch.randperm(pages - 1, generator=torch.Generator().manual_seed(4)), torch.tensor([pages - 1])])      # (the last page is nobody's)
     slots = (order[slot // ps] * ps + slot % ps).to(torch.int32)
@@ -116,3 +117,12 @@ def test_queries_that_end_inside_a_block(M, q_more, dh):
 def test_large_tiles_with_heads_of_any_multiple_of_four(M, heads, kv_heads, dh, K):
     """Thousands of columns: the tiles of 128 and 256 rows, in both widths of a stage."""
     into_cache(M, heads, kv_heads, dh, 16, 0, K=K)
+
+
+@pytest.mark.parametrize("M,K", [(17, 1024), (32, 1088), (33, 512), (64, 576)])
+@pytest.mark.parametrize("heads,kv_heads,dh", [(64, 64, 64), (65, 64, 64), (128, 128, 64), (103, 103, 40), (200, 4, 64), (131, 129, 64)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_few_rows_of_very_many_columns_write_the_cache(M, K, heads, kv_heads, dh, packed):
+    """Few rows and 12,288 columns or more: tiles of 64 x 64, and of 64 x 128 where those are more than the CUs."""
+    assert ops()._lib_quiet("gemm").dn_gemm_tile(M, (heads + 2 * kv_heads) * dh, K) == (64064 if (heads + 2 * kv_heads) * dh <= 16384 else 64128)
+    into_cache(M, heads, kv_heads, dh, 16, 0, K=K, packed=packed)
