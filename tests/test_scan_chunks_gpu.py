@@ -127,3 +127,25 @@ def test_an_infinite_state_stays_infinite(T, bad):
         assert torch.equal(a[~fine], b[~fine])
         close(a[fine], b[fine])
     assert int((~torch.isfinite(many)).sum()) == 1 and bool(torch.isinf(want[:, dv + 7]).all())
+
+
+@pytest.mark.parametrize("mode", ["wide", "rows", "head"])
+@pytest.mark.parametrize("S", [63, 64, 65, 128, 130, 200])
+def test_many_requests(mode, S):
+    """A chunk finds its request among 64 at a time: empty requests, ones that end inside a chunk, and ones without a slot among them."""
+    heads, dk, dv = 2, 16, 20
+    lengths = [[17, 0, 5, 40, 16, 1, 33, 0, 3][i % 9] for i in range(S)]
+    row_start, slots, T = tables(lengths, [-1 if i % 7 == 3 else S - 1 - i for i in range(S)])
+    r, k, v, kw = operands("wide" if mode == "rows" else mode, heads, heads, dk, dv, T, 0.5)
+    if mode == "rows":
+        r, k, v, kw, rate, bias = per_row(heads, heads, dk, dv, T, 0.5)
+        r, k = r.contiguous(), k.contiguous()
+    state = torch.randn(S, heads * dk * dv, device=DEV)
+    one, many, want = state.clone(), state.clone(), torch.zeros(T, heads * dv, device=DEV)
+    how = dict(head=dict(read_after=True, w_head=kw.get("w_head")), wide=dict(beta=kw.get("beta"), beta_logits=True),
+               rows=dict(beta=kw.get("beta"), beta_logits=True, w_rows=True))[mode]
+    if mode == "rows":
+        how.update(w_rate=rate, w_bias=bias)
+    ops().state_scan(r, k, v, kw["w"], None, one, row_start, slots, heads, dk, dv, want, **how)
+    got = chunks(mode, r, k, v, (kw, rate, bias) if mode == "rows" else kw, many, row_start, slots, heads, dk, dv)
+    close(got, want), close(many, one)
