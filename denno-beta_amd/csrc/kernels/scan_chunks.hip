@@ -541,12 +541,12 @@ int launch_of(const ChunkArgs& a, hipStream_t stream) {
 
 extern "C" {
 
-// floats of scratch that dn_scan_chunks and dn_delta_chunks need for a step of T rows of S requests
-long long dn_delta_chunks_floats(int T, int S, int H, int dk, int dv) {
+// floats of scratch that dn_scan_chunks needs for a step of T rows of S requests
+long long dn_scan_chunks_floats(int T, int S, int H, int dk, int dv) {
   return (static_cast<long long>(T) / L + S) * H * record_floats(dk, dv);
 }
 
-// r, k [T, G dk], v, out [T, H dv], 32-bit; dk a multiple of 16 up to 128; work: dn_delta_chunks_floats floats, at a multiple of 16 bytes.
+// r, k [T, G dk], v, out [T, H dv], 32-bit; dk a multiple of 16 up to 128; work: dn_scan_chunks_floats floats, at a multiple of 16 bytes.
 // mode 0: the delta rule, beta = sigmoid(zb [T, H]), decays w [T, H dk]; 1: the same, log decay = -rate softplus(w [T, H] + bias);
 // 2: a constant decay per head, w [H], no delta rule (zb none).
 int dn_scan_chunks(const float* r, long long ldr, const float* k, long long ldk, const float* v, long long ldv, const float* zb, long long ldb,
@@ -564,17 +564,6 @@ int dn_scan_chunks(const float* r, long long ldr, const float* k, long long ldk,
   if (mode == DELTA_WIDE) return launch_of<DELTA_WIDE>(a, stream);
   if (mode == DELTA_ROWS) return launch_of<DELTA_ROWS>(a, stream);
   return launch_of<FADE_HEAD>(a, stream);
-}
-
-// mode 1 alone, rows of r and k at multiples of 16 bytes
-int dn_delta_chunks(const float* r, long long ldr, const float* k, long long ldk, const float* v, long long ldv, const float* zb, long long ldb,
-                    const float* zw, long long ldw, const float* rate, const float* bias, float* state, long long slot_stride,
-                    const int* row_start, const int* slots, int S, int T, int H, int G, int dk, int dv, int rows_min, float* work, float* out,
-                    long long ldo, hipStream_t stream) {
-  auto by16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  if (ldr % 4 != 0 || ldk % 4 != 0 || !by16(r) || !by16(k)) return DN_ERR_SHAPE;
-  return dn_scan_chunks(r, ldr, k, ldk, v, ldv, zb, ldb, zw, ldw, rate, bias, DELTA_ROWS, state, slot_stride, row_start, slots, S, T, H, G, dk, dv, rows_min,
-                        work, out, ldo, stream);
 }
 
 }  // extern "C"

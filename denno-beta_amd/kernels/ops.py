@@ -161,8 +161,6 @@ def _declare(name, lib):
             "dn_post_norm": [P, c_longlong, F, P, c_longlong, P, c_longlong, P, P, F, P, P, I, I, P, P, F, P, I, c_longlong, I, I, P],
             "dn_scan_chunks": [P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, P, I, P, c_longlong, P, P, I, I, I, I, I, I, I, P, P,
                                c_longlong, P],
-            "dn_delta_chunks": [P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, c_longlong, P, P, P, c_longlong, P, P, I, I, I, I, I, I, I, P, P,
-                                c_longlong, P],
             "dn_turn_back_gate": [P, I, c_longlong, I, P, c_longlong, P, P, P, I, c_longlong, I, I, I, P],
             "dn_poly_norm": [P, c_longlong, P, F, P, I, c_longlong, I, I, P],
             "dn_head_gate": [P, I, c_longlong, I, P, c_longlong, P, I, c_longlong, I, I, I, P],
@@ -192,8 +190,8 @@ def _declare(name, lib):
         f.argtypes = args
         f.restype = c_int
     if name == "sequence":
-        lib.dn_delta_chunks_floats.argtypes = [I, I, I, I, I]
-        lib.dn_delta_chunks_floats.restype = c_longlong
+        lib.dn_scan_chunks_floats.argtypes = [I, I, I, I, I]
+        lib.dn_scan_chunks_floats.restype = c_longlong
     if name == "attention":
         lib.dn_attention_rows_part_floats.argtypes = [P, P, I, I, I, I, I, I, I]
         lib.dn_attention_rows_part_floats.restype = c_longlong
@@ -1451,20 +1449,15 @@ def scan_chunks(r, k, v, w, state, row_start, slots, n_heads, dk, dv, out, beta=
     _need(dk % 16 == 0 and 16 <= dk <= 128, lambda: f"scan_chunks: {dk} key channels a head; a multiple of 16 up to 128")
     _f32vec(w_head, "w_head", n_heads)
     stride = _history(state, n_heads * dk * dv, "scan_chunks")
-    lib = _lib("sequence")
-    work = torch.empty(lib.dn_delta_chunks_floats(T, S, n_heads, dk, dv), dtype=torch.float32, device=r.device)
-    _ok(lib.dn_scan_chunks(r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"), _ptr(beta),
-                           _rows(beta, "beta") if beta is not None else 0, _ptr(w_head) if w is None else w.data_ptr(), 0 if w is None else _rows(w, "w"),
-                           0, 0, 2 if w is None else 0, state.data_ptr(), stride, row_start.data_ptr(), slots.data_ptr(), S, T, n_heads, G, dk, dv,
-                           int(rows_min), work.data_ptr(), out.data_ptr(), _rows(out, "out"), _stream()), "scan_chunks")
+    _chunks(r, k, v, beta, w_head if w is None else w, None, None, 2 if w is None else 0, state, stride, row_start, slots, S, n_heads, G, dk, dv, rows_min, out,
+            "scan_chunks")
     return out
 
 
 def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads, dk, dv, out, qk_heads=None, rows_min=0):
     """state_scan's delta rule with one decay per row and head (beta_logits, w_rows, w_rate = rate, w_bias = bias), 16 rows of a
     request at a time on the matrix cores in 32-bit: the same recurrence, its sums in another order, so a row's result changes by
-    rounding with the place where its portion begins.  dk: a multiple of 16 up to 128; rows of r and k at multiples of 16 bytes.
-    rows_min: requests of fewer rows are left alone."""
+    rounding with the place where its portion begins.  dk: a multiple of 16 up to 128.  rows_min: requests of fewer rows are left alone."""
     G = n_heads if qk_heads is None else qk_heads
     _need(G >= 1 and n_heads % G == 0, lambda: f"delta_chunks: {n_heads} heads over {G} heads of queries and keys")
     given = ((r, "r", G * dk), (k, "k", G * dk), (v, "v", n_heads * dv), (out, "out", n_heads * dv), (beta, "beta", n_heads), (w, "w", n_heads))
@@ -1477,12 +1470,22 @@ def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads,
     _need(rate is not None, "delta_chunks: rate")
     _f32vec(rate, "rate", n_heads), _f32vec(bias, "bias", n_heads)
     stride = _history(state, n_heads * dk * dv, "delta_chunks")
-    lib = _lib("sequence")
-    work = torch.empty(lib.dn_delta_chunks_floats(T, S, n_heads, dk, dv), dtype=torch.float32, device=r.device)
-    _ok(lib.dn_delta_chunks(r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"), beta.data_ptr(), _rows(beta, "beta"),
-                            w.data_ptr(), _rows(w, "w"), rate.data_ptr(), _ptr(bias), state.data_ptr(), stride, row_start.data_ptr(), slots.data_ptr(),
-                            S, T, n_heads, G, dk, dv, int(rows_min), work.data_ptr(), out.data_ptr(), _rows(out, "out"), _stream()), "delta_chunks")
+    _chunks(r, k, v, beta, w, rate, bias, 1, state, stride, row_start, slots, S, n_heads, G, dk, dv, rows_min, out, "delta_chunks")
     return out
+
+
+def _chunks(r, k, v, beta, w, rate, bias, mode, state, stride, row_start, slots, S, n_heads, G, dk, dv, rows_min, out, what):
+    T = r.shape[0]
+    # (the kernel reaches rows of results that begin fewer than 2^24 numbers apart; others are filled in rows of their own width)
+    near = out if _rows(out, "out") < 1 << 24 else out.clone(memory_format=torch.contiguous_format)
+    lib = _lib("sequence")
+    work = torch.empty(lib.dn_scan_chunks_floats(T, S, n_heads, dk, dv), dtype=torch.float32, device=r.device)
+    _ok(lib.dn_scan_chunks(r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"), _ptr(beta),
+                           _rows(beta, "beta") if beta is not None else 0, w.data_ptr(), _rows(w, "w") if w.dim() == 2 else 0, _ptr(rate), _ptr(bias), mode,
+                           state.data_ptr(), stride, row_start.data_ptr(), slots.data_ptr(), S, T, n_heads, G, dk, dv, int(rows_min), work.data_ptr(),
+                           near.data_ptr(), _rows(near, "out"), _stream()), what)
+    if near is not out:
+        out.copy_(near)
 
 
 def head_norm(o, weight, eps, out, n_heads, gate=None, gate_kind="silu", gate_first=False, skip=None, skip_scale=None):

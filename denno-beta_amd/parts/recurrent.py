@@ -409,7 +409,7 @@ class GatedDelta(Part):
                            self.head_dim, self.value_dim, o, beta=z[:, b:b + H], qk_heads=self.n_qk_heads, beta_logits=True, w_rows=True,
                            w_rate=self.rate, w_bias=self.dt_bias, rows_below=below)
         # (the 32-bit engine walks a request's rows in order: its logits are the same bits however a prompt is cut)
-        if act != F32 and not single and qk % 4 == 0 and C % 4 == 0:
+        if act != F32 and not single:
             walk(ctx, self.head_dim, ops.DELTA_CHUNKS_ROWS_MIN, in_chunks, by_rows)
         else:
             by_rows(0)

@@ -59,7 +59,7 @@ def test_each_request_has_the_bits_it_has_alone(mode, lengths, padding):
     row_start, slots, T = tables(lengths + [0] * (padding > 0), [i if i != 1 else 7 for i in range(len(lengths))] + [-1] * (padding > 0))
     if mode == "rows":
         r, k, v, kw, rate, bias = per_row(heads, heads, dk, dv, T + padding, 0.5)
-        r, k, numbers = r.contiguous(), k.contiguous(), dict(kw, rate=rate, bias=bias)
+        numbers = dict(kw, rate=rate, bias=bias)
     else:
         r, k, v, kw = operands(mode, heads, heads, dk, dv, T + padding, 0.5)
         numbers = dict(kw)

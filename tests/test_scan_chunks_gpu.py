@@ -139,7 +139,6 @@ def test_many_requests(mode, S):
     r, k, v, kw = operands("wide" if mode == "rows" else mode, heads, heads, dk, dv, T, 0.5)
     if mode == "rows":
         r, k, v, kw, rate, bias = per_row(heads, heads, dk, dv, T, 0.5)
-        r, k = r.contiguous(), k.contiguous()
     state = torch.randn(S, heads * dk * dv, device=DEV)
     one, many, want = state.clone(), state.clone(), torch.zeros(T, heads * dv, device=DEV)
     how = dict(head=dict(read_after=True, w_head=kw.get("w_head")), wide=dict(beta=kw.get("beta"), beta_logits=True),
@@ -149,3 +148,40 @@ def test_many_requests(mode, S):
     ops().state_scan(r, k, v, kw["w"], None, one, row_start, slots, heads, dk, dv, want, **how)
     got = chunks(mode, r, k, v, (kw, rate, bias) if mode == "rows" else kw, many, row_start, slots, heads, dk, dv)
     close(got, want), close(many, one)
+
+
+@pytest.mark.parametrize("dk,heads,qk_heads", [(64, 4, 2), (48, 3, 1), (16, 2, 2)])
+@pytest.mark.parametrize("lengths", [[1, 15, 40], [200]])
+def test_one_decay_a_row_from_rows_that_begin_anywhere(dk, heads, qk_heads, lengths):
+    """Rows of r and k that begin at no multiple of 16 bytes: the bits of rows that do."""
+    dv = 24
+    row_start, slots, T = tables(lengths, [2, 0, 1][:len(lengths)])
+    r, k, v, kw, rate, bias = per_row(heads, qk_heads, dk, dv, T, 0.5)
+    assert r.data_ptr() % 16 != 0 and r.stride(0) % 4 != 0
+    state = torch.randn(3, heads * dk * dv, device=DEV)
+    one, many = state.clone(), state.clone()
+    want = chunks("rows", r.contiguous(), k.contiguous(), v.contiguous(), (kw, rate, bias), one, row_start, slots, heads, dk, dv, qk_heads)
+    got = chunks("rows", r, k, v, (kw, rate, bias), many, row_start, slots, heads, dk, dv, qk_heads)
+    assert torch.equal(got, want) and torch.equal(many, one)
+
+
+@pytest.mark.parametrize("mode", ["wide", "rows", "head"])
+@pytest.mark.parametrize("T", [1, 20])
+def test_results_whose_rows_lie_far_apart(mode, T):
+    """Rows 2^24 numbers apart and more, another request's left as they are."""
+    heads, dk, dv, far = 2, 16, 20, (1 << 24) + 4
+    row_start, slots, rows = tables([T, 1], [0, 1])
+    r, k, v, kw = operands("wide" if mode == "rows" else mode, heads, heads, dk, dv, rows, 0.5)
+    if mode == "rows":
+        r, k, v, kw, rate, bias = per_row(heads, heads, dk, dv, rows, 0.5)
+    held = torch.full((rows * far,), 7.0, device=DEV)
+    out, near = held.as_strided((rows, heads * dv), (far, 1)), torch.full((rows, heads * dv), 7.0, device=DEV)
+    state = torch.zeros(2, heads * dk * dv, device=DEV)
+    for to in (out, near):
+        if mode == "rows":
+            ops().delta_chunks(r, k, v, kw["beta"], kw["w"], rate, bias, state.clone(), row_start, slots, heads, dk, dv, to, rows_min=T if T > 1 else 0)
+        else:
+            ops().scan_chunks(r, k, v, kw["w"], state.clone(), row_start, slots, heads, dk, dv, to, **{a: t for a, t in kw.items() if a != "w"},
+                              rows_min=T if T > 1 else 0)
+    assert torch.equal(out, near) and bool((held.view(rows, far)[:, heads * dv:] == 7.0).all())
+    assert T == 1 or bool((near[T] == 7.0).all())
