@@ -9,7 +9,7 @@ session (:60-73); here a step takes any mix of both.
 from __future__ import annotations
 
 from dataclasses import dataclass, field
-from typing import List, Optional, Sequence
+from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -55,6 +55,7 @@ class StepContext:
     host_slots: List[int] = field(default_factory=list)
     rids: List[int] = field(default_factory=list)
     single_rows: bool = False      # every request brings one row (a pure decode step)
+    rows_of_requests: Optional[Tuple[int, int]] = None      # the fewest and the most rows of a request; None: only row_start has them (a captured step)
 
 
 class BatchError(ValueError):
@@ -164,4 +165,5 @@ def build_context(entries: Sequence[StepEntry], cache, vocab: int, max_positions
     return StepContext(
         T=T, S=S, R=R, tokens=view("tokens"), positions=view("positions"), logit_rows=view("logit_rows"),
         state_slots=view("state_slots"), row_start=view("row_start"), groups=groups,
-        host_row_start=row_start, host_first_pos=starts, host_slots=slots, rids=[e.rid for e in entries], single_rows=single)
+        host_row_start=row_start, host_first_pos=starts, host_slots=slots, rids=[e.rid for e in entries], single_rows=single,
+        rows_of_requests=(int(counts.min()), int(counts.max())))

@@ -16,12 +16,7 @@ def walk(ctx, dk, rows_min, in_chunks, by_rows):
     """A step's recurrences, each request's by its own rows: in_chunks(rows_min) for those of that many and more, by_rows(rows_below) for the others
     (0: for all).  What no request of the step needs is not launched.  A captured step's rows stand in its tables alone, which a replay
     fills: it has both, if it has room for such a request."""
-    starts = ctx.host_row_start
-    if starts and starts[-1] == ctx.T:
-        rows = [b - a for a, b in zip(starts, starts[1:])]
-        fewest, most = min(rows, default=0), max(rows, default=0)
-    else:
-        fewest, most = 0, ctx.T
+    fewest, most = ctx.rows_of_requests or (0, ctx.T)
     if most < rows_min or not ops.chunks_take(dk):
         by_rows(0)
     elif fewest >= rows_min:

@@ -13,7 +13,7 @@ def routes(lengths, padding=None, rows_min=96, dk=64):
     for n in lengths:
         starts.append(starts[-1] + n)
     T, S = padding or (starts[-1], len(lengths))
-    ctx = SimpleNamespace(T=T, S=S, host_row_start=[0] * (S + 1) if padding else starts)
+    ctx = SimpleNamespace(T=T, S=S, rows_of_requests=None if padding else (min(lengths), max(lengths)))
     got, launches = [""] * len(lengths), []
 
     def in_chunks(least):
