@@ -503,3 +503,28 @@ def test_steps_with_portions_are_replayed_from_graphs(model_folders, dtype):
                 assert torch.equal(got[True][f"r{i}"], got[False][f"r{i}"]), (kind, i)
             else:
                 U.assert_close(got[True][f"r{i}"], got[False][f"r{i}"], dtype, f"graphs against kernel by kernel, {kind}, request {i}")
+
+
+HEADS_BETWEEN = {
+    "sixteen heads of 40": _cfg(2, 640, 16, 1280, 301, 360),      # a block of 16 columns holds the end of a head and the beginning of the next
+    "sixteen heads of 20": _cfg(2, 320, 16, 640, 301, 360),
+    "eight heads of 72": _cfg(2, 576, 8, 1152, 301, 360),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(HEADS_BETWEEN))
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_many_rows_of_heads_that_are_no_multiple_of_16(tmp_path, name, dtype):
+    """Prompts of some hundreds of rows, whose keys the product's own kernel puts into the pages, and tokens decoded from there."""
+    from denno_beta_amd.weights import write_model_folder
+    cfg, folder = HEADS_BETWEEN[name], str(tmp_path)
+    write_model_folder(folder, cfg, 11, dtype)
+    seqs = [seeded_tokens(50 + i, n, cfg["vocab_size"]) for i, n in enumerate((330, 356, 290))]
+    want = plain_logits(folder, seqs)
+    for kind, steps in (("whole", U.whole_trace(seqs)), ("tail", U.tail_decode_trace(seqs, 24)), ("chunks", U.chunk_trace(seqs, sizes=(300, 2, 290, 7)))):
+        r = runner_for(folder, dtype, "cuda:0", cache_tokens=U.max_live_tokens(steps))
+        got = U.replay(r, steps)
+        r.cache.manager.check()
+        for i in range(len(seqs)):
+            U.assert_close(got[f"r{i}"], want[i], dtype, f"{name} {dtype} {kind} request {i}")
