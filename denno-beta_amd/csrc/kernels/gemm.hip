@@ -57,7 +57,8 @@ extern "C" int dn_gemm(const void* A, int lda, const void* W, const float* bias,
       plain::join_shares(work, shares, bias, resid, ldr, M, N, stream);
       return dn_launch_status();
     }
-    if (many && (!few || direct::beats_few_rows(M, N, K))) {
+    const bool any_rows = out_dtype == DN_F32 && !resid && (N % 4 != 0 || ldc % 4 != 0 || reinterpret_cast<uintptr_t>(C) % 16 != 0);
+    if (many && (!few || direct::beats_few_rows(M, N, K, any_rows))) {
       int rc = direct::run(direct::Args{A, lda, W, bias, C, ldc, resid, ldr, M, N, K, out_dtype, epilogue, packed, nullptr}, stream);
       return rc != 0 ? rc : dn_launch_status();
     }

@@ -118,3 +118,15 @@ def test_tiles_of_64_by_128_beyond_512_rows(K):
     out = torch.empty(M, N, device=DEV)
     o.linear(a, o.pack_matrix(w), None, out=out)
     within(out, a, w)
+
+
+@pytest.mark.parametrize("M", [64, 65, 128, 129, 256])
+@pytest.mark.parametrize("N,K", [(3001, 1024), (4095, 512), (4097, 512), (1001, 4096), (2050, 1056)])
+def test_some_rows_of_any_length(M, N, K):
+    """Up to 128 rows of fewer than 4,096 columns, no multiple of 4, and those on the other side of each border, from packed rows and from rows."""
+    a, w = rnd(M, K, seed=M, dtype=BF), rnd(N, K, seed=N + 1000, dtype=BF, scale=K ** -0.5)
+    wp = ops().pack_matrix(w)
+    got = [torch.full((M + 1, N), 7.0, device=DEV) for _ in range(2)]
+    ops().linear(a, wp, None, out=got[0][:M]), ops().linear(ops().pack_matrix(a), wp, None, out=got[1][:M])
+    within(got[0][:M], a, w)
+    assert torch.equal(got[0], got[1]) and bool((got[0][M] == 7.0).all())
