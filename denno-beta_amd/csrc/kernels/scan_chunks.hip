@@ -541,6 +541,12 @@ int launch_of(const ChunkArgs& a, hipStream_t stream) {
 
 extern "C" {
 
+int dn_state_scan(const float* r, long long ldr, const float* k, long long ldk, const float* v, long long ldv, const float* w,
+                  long long ldw, const float* u, const float* beta, long long ldb, const float* w_head, int G, float* state,
+                  long long slot_stride, const int* row_start, const int* slots, int S, int T, int H, int dk, int dv, int mode,
+                  int key_from_decay, int beta_logits, int w_rows, const float* w_rate, const float* w_bias, int rows_below, float* out,
+                  long long ldo, hipStream_t stream);      // (sequence.hip)
+
 // floats of scratch that dn_scan_chunks needs for a step of T rows of S requests
 long long dn_scan_chunks_floats(int T, int S, int H, int dk, int dv) {
   return (static_cast<long long>(T) / L + S) * H * record_floats(dk, dv);
@@ -548,22 +554,25 @@ long long dn_scan_chunks_floats(int T, int S, int H, int dk, int dv) {
 
 // r, k [T, G dk], v, out [T, H dv], 32-bit; dk a multiple of 16 up to 128; work: dn_scan_chunks_floats floats, at a multiple of 16 bytes.
 // mode 0: the delta rule, beta = sigmoid(zb [T, H]), decays w [T, H dk]; 1: the same, log decay = -rate softplus(w [T, H] + bias);
-// 2: a constant decay per head, w [H], no delta rule (zb none).
+// 2: a constant decay per head, w [H], no delta rule (zb none).  Requests of fewer than rows_min rows are walked row by row (0: none are) by a launch of
+// dn_state_scan's kernel: in this call, since a call of its own for them cost a step outside the graphs 30 us a layer, most of it in checks on the host.
 int dn_scan_chunks(const float* r, long long ldr, const float* k, long long ldk, const float* v, long long ldv, const float* zb, long long ldb,
                    const float* w, long long ldw, const float* rate, const float* bias, int mode, float* state, long long slot_stride,
                    const int* row_start, const int* slots, int S, int T, int H, int G, int dk, int dv, int rows_min, float* work, float* out,
                    long long ldo, hipStream_t stream) {
   if (dk < 16 || dk > 128 || dk % 16 != 0 || dv < 1 || H < 1 || G < 1 || H % G != 0 || S < 1 || S > 65535 || H > 65535 || (dv + 15) / 16 > 65535 ||
-      reinterpret_cast<uintptr_t>(work) % 16 != 0 || slot_stride < static_cast<long long>(H) * dk * dv || ldo >= (1LL << 24) || mode < DELTA_WIDE || mode > FADE_HEAD ||
+      reinterpret_cast<uintptr_t>(work) % 16 != 0 || slot_stride < static_cast<long long>(H) * dk * dv || ldo >= (1LL << 24) || rows_min < 0 || mode < DELTA_WIDE || mode > FADE_HEAD ||
       !w || (mode != FADE_HEAD) != (zb != nullptr) || (mode == DELTA_ROWS) != (rate != nullptr))
     return DN_ERR_SHAPE;
   if (T == 0) return 0;
   const ChunkArgs a{r, k, v, zb, w, rate, bias, static_cast<size_t>(ldr), static_cast<size_t>(ldk), static_cast<size_t>(ldv), static_cast<size_t>(ldb),
                     static_cast<size_t>(ldw), state, static_cast<size_t>(slot_stride), row_start, slots, S, H, G, dk, dv, T / L + S, rows_min, work, out,
                     static_cast<size_t>(ldo)};
-  if (mode == DELTA_WIDE) return launch_of<DELTA_WIDE>(a, stream);
-  if (mode == DELTA_ROWS) return launch_of<DELTA_ROWS>(a, stream);
-  return launch_of<FADE_HEAD>(a, stream);
+  const int rc = mode == DELTA_WIDE ? launch_of<DELTA_WIDE>(a, stream) : mode == DELTA_ROWS ? launch_of<DELTA_ROWS>(a, stream) : launch_of<FADE_HEAD>(a, stream);
+  if (rc != 0 || rows_min == 0) return rc;
+  const bool head = mode == FADE_HEAD;
+  return dn_state_scan(r, ldr, k, ldk, v, ldv, head ? nullptr : w, ldw, nullptr, zb, ldb, head ? w : nullptr, G, state, slot_stride, row_start, slots, S, T, H, dk,
+                       dv, head ? 1 : 2, 0, !head, mode == DELTA_ROWS, rate, bias, rows_min, out, ldo, stream);
 }
 
 }  // extern "C"

@@ -1374,7 +1374,7 @@ def gated(x, g, kind, out):
 
 
 def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, read_after=False, key_from_decay=False, beta=None,
-               w_head=None, qk_heads=None, beta_logits=False, w_rows=False, w_rate=None, w_bias=None, rows_below=0):
+               w_head=None, qk_heads=None, beta_logits=False, w_rows=False, w_rate=None, w_bias=None):
     """The recurrence of a matrix state per head, S [dk, dv], over each request's rows of this step in order:
       a = 1 - w if key_from_decay else k
       read_after:  S <- diag(w) S + a v^T ;  o = S^T r
@@ -1385,8 +1385,7 @@ def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, rea
     w_head: 32-bit [heads], one decay per head for every row and channel;
     w_rate (and w_bias): 32-bit [heads], with w_rows in the delta rule: w holds z and the decay is exp(-w_rate log(1 + e^(z + w_bias)));
     v, out: 32-bit [T, heads * dv]; beta: 32-bit [T, heads] (beta_logits: it holds z, and beta is 1 / (1 + e^-z)); state: 32-bit [slots, heads * dv * dk] (a head's state
-    held [value column][key channel]), read and written at the requests' slots.  rows_below: requests of that many rows and more are left alone
-    (0: none are), for `scan_chunks` and `delta_chunks` with the same number."""
+    held [value column][key channel]), read and written at the requests' slots."""
     G = n_heads if qk_heads is None else qk_heads
     _need(G >= 1 and n_heads % G == 0, lambda: f"state_scan: {n_heads} heads over {G} heads of queries and keys")
     _need((w is None) != (w_head is None), "state_scan: a decay per row and channel (w) or one per head (w_head)")
@@ -1411,7 +1410,7 @@ def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, rea
                                        _rows(w, "w") if w is not None else 0, _ptr(u), _ptr(beta),
                                        _rows(beta, "beta") if beta is not None else 0, _ptr(w_head), G, state.data_ptr(), stride,
                                        row_start.data_ptr(), slots.data_ptr(), S, T, n_heads, dk, dv, mode, int(key_from_decay),
-                                       int(bool(beta_logits)), int(bool(w_rows)), _ptr(w_rate), _ptr(w_bias), int(rows_below), out.data_ptr(),
+                                       int(bool(beta_logits)), int(bool(w_rows)), _ptr(w_rate), _ptr(w_bias), 0, out.data_ptr(),
                                        _rows(out, "out"), _stream()),
         "state_scan" if beta is None else "state_scan (delta rule)")
     return out
@@ -1435,7 +1434,8 @@ def scan_chunks(r, k, v, w, state, row_start, slots, n_heads, dk, dv, out, beta=
     """state_scan's delta rule with a decay per row and channel (beta given, as the sigmoid's argument; w [T, heads * dk]), or its
     recurrence with one constant decay per head that reads after its write (w None, w_head [heads]; no beta), 16 rows of a request at a
     time on the matrix cores in 32-bit: the same recurrence, its sums in another order, so a row's result changes by rounding with
-    the place where its portion begins.  dk: a multiple of 16 up to 128.  rows_min: requests of fewer rows are left alone."""
+    the place where its portion begins.  dk: a multiple of 16 up to 128.  rows_min: requests of fewer rows are walked row by row, with the bits
+    that state_scan gives them."""
     G = n_heads if qk_heads is None else qk_heads
     _need(G >= 1 and n_heads % G == 0, lambda: f"scan_chunks: {n_heads} heads over {G} heads of queries and keys")
     _need((w is None) != (w_head is None) and (beta is None) == (w is None), "scan_chunks: decays per row and channel with beta, or one per head without")
@@ -1457,7 +1457,8 @@ def scan_chunks(r, k, v, w, state, row_start, slots, n_heads, dk, dv, out, beta=
 def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads, dk, dv, out, qk_heads=None, rows_min=0):
     """state_scan's delta rule with one decay per row and head (beta_logits, w_rows, w_rate = rate, w_bias = bias), 16 rows of a
     request at a time on the matrix cores in 32-bit: the same recurrence, its sums in another order, so a row's result changes by
-    rounding with the place where its portion begins.  dk: a multiple of 16 up to 128.  rows_min: requests of fewer rows are left alone."""
+    rounding with the place where its portion begins.  dk: a multiple of 16 up to 128.  rows_min: requests of fewer rows are walked row by row, with the bits
+    that state_scan gives them."""
     G = n_heads if qk_heads is None else qk_heads
     _need(G >= 1 and n_heads % G == 0, lambda: f"delta_chunks: {n_heads} heads over {G} heads of queries and keys")
     given = ((r, "r", G * dk), (k, "k", G * dk), (v, "v", n_heads * dv), (out, "out", n_heads * dv), (beta, "beta", n_heads), (w, "w", n_heads))

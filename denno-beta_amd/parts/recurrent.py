@@ -13,16 +13,14 @@ F32 = torch.float32
 
 
 def walk(ctx, dk, rows_min, in_chunks, by_rows):
-    """A step's recurrences, each request's by its own rows: in_chunks(rows_min) for those of that many and more, by_rows(rows_below) for the others
-    (0: for all).  What no request of the step needs is not launched.  A captured step's rows stand in its tables alone, which a replay
-    fills: it has both, if it has room for such a request."""
+    """A step's recurrences, each request's by its own rows: in chunks those of rows_min and more.  in_chunks(rows_min) walks the others row by row in the
+    same call, in_chunks(0) has none such, by_rows() walks all row by row: what no request of the step needs is not launched.  A captured step's rows
+    stand in its tables alone, which a replay fills: it has both, if it has room for a request of rows_min."""
     fewest, most = ctx.rows_of_requests or (0, ctx.T)
     if most < rows_min or not ops.chunks_take(dk):
-        by_rows(0)
-    elif fewest >= rows_min:
-        in_chunks(0)
+        by_rows()
     else:
-        in_chunks(rows_min), by_rows(rows_min)
+        in_chunks(0 if fewest >= rows_min else rows_min)
 
 
 @MIXERS.register("wkv")
@@ -175,14 +173,14 @@ class Lightning(Part):
             ops.scan_chunks(q, k, v, None, cache.state, ctx.row_start, ctx.state_slots, self.n_heads, self.head_dim, self.value_dim, o,
                             w_head=self.decay_t, rows_min=least)
 
-        def by_rows(below):
+        def by_rows():
             ops.state_scan(q, k, v, None, None, cache.state, ctx.row_start, ctx.state_slots, self.n_heads, self.head_dim, self.value_dim, o,
-                           read_after=True, w_head=self.decay_t, rows_below=below)
+                           read_after=True, w_head=self.decay_t)
         # (the 32-bit engine walks a request's rows in order: its logits are the same bits however a prompt is cut)
         if act != F32 and not ctx.single_rows:
             walk(ctx, self.head_dim, ops.CHUNKS_ROWS_MIN, in_chunks, by_rows)
         else:
-            by_rows(0)
+            by_rows()
         y = torch.empty((T, vw), dtype=act, device=h.device)
         ops.head_norm(o, self.norm, self.eps, y, 1, gate=z[:, 2 * qk + vw:], gate_kind="sigmoid")
         if accumulate_into is None:
@@ -305,14 +303,14 @@ class ChannelDelta(Part):
             ops.scan_chunks(q, k, v, g, state, ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, beta=z[:, C:C + H],
                             qk_heads=self.n_qk_heads, rows_min=least)
 
-        def by_rows(below):
+        def by_rows():
             ops.state_scan(q, k, v, g, None, state, ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, beta=z[:, C:C + H],
-                           qk_heads=self.n_qk_heads, beta_logits=True, rows_below=below)
+                           qk_heads=self.n_qk_heads, beta_logits=True)
         # (the 32-bit engine walks a request's rows in order: its logits are the same bits however a prompt is cut)
         if act != F32 and not single:
             walk(ctx, self.head_dim, ops.CHUNKS_ROWS_MIN, in_chunks, by_rows)
         else:
-            by_rows(0)
+            by_rows()
         y = torch.empty((T, vw), dtype=act, device=dev)
         ops.head_norm(o, self.norm, self.eps, y, H, gate=gate, gate_kind="sigmoid")
         if accumulate_into is None:
@@ -399,15 +397,15 @@ class GatedDelta(Part):
             ops.delta_chunks(x[:, :qk], x[:, qk:2 * qk], x[:, 2 * qk:], z[:, b:b + H], z[:, b + H:b + 2 * H], self.rate, self.dt_bias, state,
                              ctx.row_start, ctx.state_slots, H, self.head_dim, self.value_dim, o, qk_heads=self.n_qk_heads, rows_min=least)
 
-        def by_rows(below):
+        def by_rows():
             ops.state_scan(x[:, :qk], x[:, qk:2 * qk], x[:, 2 * qk:], z[:, b + H:b + 2 * H], None, state, ctx.row_start, ctx.state_slots, H,
                            self.head_dim, self.value_dim, o, beta=z[:, b:b + H], qk_heads=self.n_qk_heads, beta_logits=True, w_rows=True,
-                           w_rate=self.rate, w_bias=self.dt_bias, rows_below=below)
+                           w_rate=self.rate, w_bias=self.dt_bias)
         # (the 32-bit engine walks a request's rows in order: its logits are the same bits however a prompt is cut)
         if act != F32 and not single:
             walk(ctx, self.head_dim, ops.DELTA_CHUNKS_ROWS_MIN, in_chunks, by_rows)
         else:
-            by_rows(0)
+            by_rows()
         y = torch.empty((T, vw), dtype=act, device=dev)
         ops.head_norm(o, self.norm, self.eps, y, H, gate=z[:, gate:gate + vw], gate_kind="silu")
         if accumulate_into is None:

@@ -412,7 +412,7 @@ def gated(x, g, kind, out):
 
 
 def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, read_after=False, key_from_decay=False, beta=None,
-               w_head=None, qk_heads=None, beta_logits=False, w_rows=False, w_rate=None, w_bias=None, rows_below=0, rows_min=0):
+               w_head=None, qk_heads=None, beta_logits=False, w_rows=False, w_rate=None, w_bias=None):
     H = n_heads
     if w_rate is not None:
         w = torch.exp(-w_rate * torch.nn.functional.softplus(w + (w_bias if w_bias is not None else 0.0)))
@@ -421,8 +421,6 @@ def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, rea
     G = H if qk_heads is None else qk_heads
     spread = lambda x: x.view(G, dk).repeat_interleave(H // G, dim=0)      # noqa: E731  (head h reads head h // (H // G))
     for slot, a, b in _requests(row_start, slots):
-        if b - a < rows_min or (rows_below and b - a >= rows_below):
-            continue
         S = state[slot].view(H, dv, dk).transpose(1, 2).clone()      # (held [head][value column][key channel])
         for t in range(a, b):
             rt, vt = spread(r[t]), v[t].view(H, dv)
@@ -447,12 +445,12 @@ def state_scan(r, k, v, w, u, state, row_start, slots, n_heads, dk, dv, out, rea
 
 def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads, dk, dv, out, qk_heads=None, rows_min=0):
     return state_scan(r, k, v, w, None, state, row_start, slots, n_heads, dk, dv, out, beta=beta, qk_heads=qk_heads, beta_logits=True, w_rows=True,
-                      w_rate=rate, w_bias=bias, rows_min=rows_min)
+                      w_rate=rate, w_bias=bias)
 
 
 def scan_chunks(r, k, v, w, state, row_start, slots, n_heads, dk, dv, out, beta=None, w_head=None, qk_heads=None, rows_min=0):
     return state_scan(r, k, v, w, None, state, row_start, slots, n_heads, dk, dv, out, read_after=beta is None, beta=beta, w_head=w_head, qk_heads=qk_heads,
-                      beta_logits=beta is not None, rows_min=rows_min)
+                      beta_logits=beta is not None)
 
 
 def head_norm(o, weight, eps, out, n_heads, gate=None, gate_kind="silu", gate_first=False, skip=None, skip_scale=None):

@@ -17,16 +17,14 @@ def routes(lengths, padding=None, rows_min=96, dk=64):
     got, launches = [""] * len(lengths), []
 
     def in_chunks(least):
-        launches.append("chunks")
+        launches.extend(["chunks", "rows"] if least else ["chunks"])
         for i, n in enumerate(lengths):
-            if n >= least:
-                got[i] += "chunks"
+            got[i] += "chunks" if n >= least else "rows"
 
-    def by_rows(below):
+    def by_rows():
         launches.append("rows")
-        for i, n in enumerate(lengths):
-            if not below or n < below:
-                got[i] += "rows"
+        for i in range(len(lengths)):
+            got[i] += "rows"
     walk(ctx, dk, rows_min, in_chunks, by_rows)
     return got, launches
 
@@ -64,32 +62,29 @@ def test_each_request_has_the_bits_it_has_alone(mode, lengths, padding):
         r, k, v, kw = operands(mode, heads, heads, dk, dv, T + padding, 0.5)
         numbers = dict(kw)
 
-    def step(rows, state, row_start, slots, how, below):
+    def step(rows, state, row_start, slots, how, least=0):
         out = torch.full((rows.stop - rows.start, heads * dv), 7.0, device=DEV)
         n = {a: t[rows] if t is not None and t.dim() == 2 else t for a, t in numbers.items()}
         a = (state, row_start, slots, heads, dk, dv, out)
         if how == "chunks" and mode == "rows":
-            ops().delta_chunks(r[rows], k[rows], v[rows], n["beta"], n["w"], n["rate"], n["bias"], *a, rows_min=below)
+            ops().delta_chunks(r[rows], k[rows], v[rows], n["beta"], n["w"], n["rate"], n["bias"], *a, rows_min=least)
         elif how == "chunks":
-            ops().scan_chunks(r[rows], k[rows], v[rows], n["w"], *a, **{x: t for x, t in n.items() if x != "w"}, rows_min=below)
+            ops().scan_chunks(r[rows], k[rows], v[rows], n["w"], *a, **{x: t for x, t in n.items() if x != "w"}, rows_min=least)
         elif mode == "head":
-            ops().state_scan(r[rows], k[rows], v[rows], None, None, *a, read_after=True, w_head=n["w_head"], rows_below=below)
+            ops().state_scan(r[rows], k[rows], v[rows], None, None, *a, read_after=True, w_head=n["w_head"])
         elif mode == "wide":
-            ops().state_scan(r[rows], k[rows], v[rows], n["w"], None, *a, beta=n["beta"], beta_logits=True, rows_below=below)
+            ops().state_scan(r[rows], k[rows], v[rows], n["w"], None, *a, beta=n["beta"], beta_logits=True)
         else:
-            ops().state_scan(r[rows], k[rows], v[rows], n["w"], None, *a, beta=n["beta"], beta_logits=True, w_rows=True, w_rate=n["rate"], w_bias=n["bias"],
-                             rows_below=below)
+            ops().state_scan(r[rows], k[rows], v[rows], n["w"], None, *a, beta=n["beta"], beta_logits=True, w_rows=True, w_rate=n["rate"], w_bias=n["bias"])
         return out
     first = torch.randn(9, heads * dk * dv, device=DEV)
     together = first.clone()
-    in_chunks = step(slice(0, T + padding), together, row_start, slots, "chunks", least)
-    by_rows = step(slice(0, T + padding), together, row_start, slots, "rows", least)
+    got = step(slice(0, T + padding), together, row_start, slots, "chunks", least)
     alone = first.clone()
     for s, n in enumerate(lengths):
         rows = slice(int(row_start[s]), int(row_start[s + 1]))
         table, slot = torch.tensor([0, n], dtype=torch.int32, device=DEV), slots[s:s + 1].contiguous()
-        want = step(rows, alone, table, slot, "chunks" if n >= least else "rows", 0)
-        mine, other = (in_chunks, by_rows) if n >= least else (by_rows, in_chunks)
-        assert torch.equal(mine[rows], want) and bool((other[rows] == 7.0).all())
+        want = step(rows, alone, table, slot, "chunks" if n >= least else "rows")
+        assert torch.equal(got[rows], want)
     assert torch.equal(together, alone)
-    assert bool((in_chunks[T:] == 7.0).all()) and bool((by_rows[T:] == 7.0).all())
+    assert bool((got[T:] == 7.0).all())

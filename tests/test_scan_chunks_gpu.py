@@ -168,7 +168,7 @@ def test_one_decay_a_row_from_rows_that_begin_anywhere(dk, heads, qk_heads, leng
 @pytest.mark.parametrize("mode", ["wide", "rows", "head"])
 @pytest.mark.parametrize("T", [1, 20])
 def test_results_whose_rows_lie_far_apart(mode, T):
-    """Rows 2^24 numbers apart and more, another request's left as they are."""
+    """Rows 2^24 numbers apart and more; with 20 rows the other request's one is walked row by row."""
     heads, dk, dv, far = 2, 16, 20, (1 << 24) + 4
     row_start, slots, rows = tables([T, 1], [0, 1])
     r, k, v, kw = operands("wide" if mode == "rows" else mode, heads, heads, dk, dv, rows, 0.5)
@@ -184,4 +184,3 @@ def test_results_whose_rows_lie_far_apart(mode, T):
             ops().scan_chunks(r, k, v, kw["w"], state.clone(), row_start, slots, heads, dk, dv, to, **{a: t for a, t in kw.items() if a != "w"},
                               rows_min=T if T > 1 else 0)
     assert torch.equal(out, near) and bool((held.view(rows, far)[:, heads * dv:] == 7.0).all())
-    assert T == 1 or bool((near[T] == 7.0).all())
