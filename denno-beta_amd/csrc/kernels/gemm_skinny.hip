@@ -318,11 +318,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
           acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][mb], b[u][nb], acc[mb][nb], 0, 0, 0);
   };
   // A later round's loads of W stand together behind one branch: a branch for each step, among A's loads, made each of them wait for every load
-  // before it.  Not so in workgroups of four waves with four column blocks (very many columns, K below 1,024), where several share a CU and the second round is
-  // the last: 17 and 32 rows of 50,304 x 768 21.4 -> 20.3 and 22.4 -> 21.2 us with a branch a step, of 50,304 x 640 18.8 -> 18.0 and 19.9 -> 19.2, of 50,304 x
-  // 512, one round, 14.3 -> 14.7.
+  // before it.  Not so (`BY_STEP`) where a round's loads of W are many, so that a first step waits long for the last step's: with four column blocks (together ->
+  // a branch a step: 17 and 32 rows of 50,304 x 768 21.4 -> 20.3 and 22.4 -> 21.2 us; 24 of 33,000 x 2,080 41.2 -> 37.8, 64 56.4 -> 50.1), with two and four
+  // steps (250 rows of 1,600 x 3,104 11.6 -> 11.0), and with twelve row blocks (160 rows of 1,600 x 4,128 19.9 -> 18.5; of 4,800 x 1,632, where K is no
+  // multiple of 32, 11.9 -> 13.1).
+  constexpr bool BY_STEP = NORM == NORM_NONE && (NB == 4 || (NB == 2 && U == 4) || (MB == 12 && WAVES == 8));
   for (int p0 = wave; 2 * p0 < ksteps; p0 += WAVES * (U / 2)) {
-    if constexpr (WAVES == 4 && NB == 4) {
+    if constexpr (BY_STEP) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int ks = 2 * (p0 + (u / 2) * WAVES) + u % 2;
