@@ -599,12 +599,12 @@ bool wide_few(int M, int N, int K) { return M > 16 && M <= 64 && N >= 12288 && K
 // Up to 256 rows the few-rows kernel takes the product too (both read and write packed rows): it stays ahead,
 // or level, where the product has few columns and a short K; everywhere else from 65 rows on this kernel is
 // the faster (`mid_rows`), and beyond 256 rows it is the only one.
-// any_rows: 32-bit rows that only `takes`' allowance lets in (no multiple of 4 columns, or not at 16 bytes), up to 128 of them of fewer than 4,096 columns, stay
-// with the few-rows kernel, whose waves share K (there -> here: 65 rows of 2,049 x 1,024 5.0 and 6.7 us, of 3,001 x 2,048 7.1 and 10.1, of 257 x 4,096 10.0 and 18.2,
-// 128 of 3,001 x 1,600 7.4 and 8.8, of 1,601 x 5,120 21.2 and 23.1; 65 of 4,099 x 1,024 7.9 and 6.7; 160 of 2,049 x 1,600 9.6 and 8.9, of 257 x 4,096 17.2 and 18.2,
-// of 1,001 x 8,192 40.9 and 33.5).
+// any_rows: 32-bit rows that only `takes`' allowance lets in (no multiple of 4 columns, or not at 16 bytes), up to 128 of them of fewer than 4,096 columns and up to
+// 192, the few-rows kernel's next border, of up to 1,024, stay with the few-rows kernel, whose waves share K (there -> here: 65 rows of 2,049 x 1,024 5.0 and 6.7 us, of 3,001 x 2,048 7.1 and 10.1, of 257 x 4,096 10.0 and 18.2,
+// 128 of 3,001 x 1,600 7.4 and 8.8, of 1,601 x 5,120 21.2 and 23.1; 65 of 4,099 x 1,024 7.9 and 6.7; 160 of 2,049 x 1,600 9.6 and 8.9; 129
+// of 257 x 4,096 16.6 and 18.4, 192 of 1,001 x 4,096 18.3 and 18.6, of 257 x 8,192 31.2 and 33.1, of 1,999 x 8,192 45.8 and 37.1, 208 of 257 x 4,096 22.6 and 18.4).
 bool beats_few_rows(int M, int N, int K, bool any_rows) {
-  if (any_rows && M <= 128 && N < 4096) return false;
+  if (any_rows && (M <= 128 ? N < 4096 : M <= 192 && N <= 1024)) return false;
   return wide_few(M, N, K) || mid_rows(M, N, K) || (M > 104 && N >= 4096) || (M > 208 && N >= 2048);
 }
 

@@ -120,10 +120,10 @@ def test_tiles_of_64_by_128_beyond_512_rows(K):
     within(out, a, w)
 
 
-@pytest.mark.parametrize("M", [64, 65, 128, 129, 256])
-@pytest.mark.parametrize("N,K", [(3001, 1024), (4095, 512), (4097, 512), (1001, 4096), (2050, 1056)])
+@pytest.mark.parametrize("M", [64, 65, 128, 129, 192, 193, 256])
+@pytest.mark.parametrize("N,K", [(3001, 1024), (4095, 512), (4097, 512), (1001, 4096), (1023, 4160), (1025, 4096), (2050, 1056)])
 def test_some_rows_of_any_length(M, N, K):
-    """Up to 128 rows of fewer than 4,096 columns, no multiple of 4, and those on the other side of each border, from packed rows and from rows."""
+    """Up to 128 rows of fewer than 4,096 columns, no multiple of 4, up to 192 of up to 1,024, and those on the other side of each border, from packed rows and from rows."""
     a, w = rnd(M, K, seed=M, dtype=BF), rnd(N, K, seed=N + 1000, dtype=BF, scale=K ** -0.5)
     wp = ops().pack_matrix(w)
     got = [torch.full((M + 1, N), 7.0, device=DEV) for _ in range(2)]
