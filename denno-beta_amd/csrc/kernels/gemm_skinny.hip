@@ -321,8 +321,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const bf16_t* __restri
   // before it.  Not so (`BY_STEP`) where a round's loads of W are many, so that a first step waits long for the last step's: with four column blocks (together ->
   // a branch a step: 17 and 32 rows of 50,304 x 768 21.4 -> 20.3 and 22.4 -> 21.2 us; 24 of 33,000 x 2,080 41.2 -> 37.8, 64 56.4 -> 50.1), with two and four
   // steps (250 rows of 1,600 x 3,104 11.6 -> 11.0), and with twelve row blocks (160 rows of 1,600 x 4,128 19.9 -> 18.5; of 4,800 x 1,632, where K is no
-  // multiple of 32, 11.9 -> 13.1).
-  constexpr bool BY_STEP = NORM == NORM_NONE && (NB == 4 || (NB == 2 && U == 4) || (MB == 12 && WAVES == 8));
+  // multiple of 32, 11.9 -> 13.1).  Nor, with eight steps, where the norm's statistics are left (33 rows of 1,600 x 4,096 8.4 -> 8.1, of 1,024 x 4,096 6.5 -> 6.4, no other K differs).
+  constexpr bool BY_STEP = (NORM == NORM_OUT && U == 8) || (NORM == NORM_NONE && (NB == 4 || (NB == 2 && U == 4) || (MB == 12 && WAVES == 8)));
   for (int p0 = wave; 2 * p0 < ksteps; p0 += WAVES * (U / 2)) {
     if constexpr (BY_STEP) {
 #pragma unroll
