@@ -696,7 +696,9 @@ int run(const Args& a, hipStream_t stream) {
       // 1.05, 0.99, 0.98, 0.97, 0.96; 2,048 x 5,120 with GELU 1.06, 1.00, 0.99, 1.00, 0.95; 8,192 x 3,200 1.11, 1.03, 0.99, 0.98, 0.94; added into the
       // stream, 1,500 x 6,400, K = 1,024, 1,600, 2,560, 4,096: 1.03, 1.00, 0.98, 0.95), and the product with a cache write, whose
       // epilogue is the longest, never does (2,048 x 4,800 x 1,600 40.3 us in step, 46.6 in turns; 6,700 x 3,840 x 1,280 84 and 106).
-      if (!a.kv && a.K >= (a.out_dtype == DN_BF16 && !a.resid ? 1280 : 1600)) return launch_without_kv<4, 2, 4, 5, 3, 2, true>(a, stream);
+      // GELU with the error function, the longest of the others', from 2,304 (in turns and in step: 2,048 x 5,120, K = 1,280 and 1,600 40.0 and 38.0, 44.4 and
+      // 42.3 us; 3,000 x 3,072, K = 1,280, 2,048, 2,304 and 2,496 40.2 and 37.6, 49.1 and 47.4, 52.8 and 52.7, 55.5 and 56.8).
+      if (!a.kv && a.K >= (a.out_dtype != DN_BF16 || a.resid ? 1600 : a.epi == EPI_GELU_ERF ? 2304 : 1280)) return launch_without_kv<4, 2, 4, 5, 3, 2, true>(a, stream);
       return launch_as<8, 2, 2, 5, 3, 2>(a, stream);
     case 4:
       if (!sixteen) return launch_as<4, 2, 4, 6, 4>(a, stream);

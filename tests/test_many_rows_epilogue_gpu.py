@@ -126,3 +126,16 @@ def test_few_rows_of_very_many_columns_write_the_cache(M, K, heads, kv_heads, dh
     """Few rows and 12,288 columns or more: tiles of 64 x 64, and of 64 x 128 where those are more than the CUs."""
     assert ops()._lib_quiet("gemm").dn_gemm_tile(M, (heads + 2 * kv_heads) * dh, K) == (64064 if (heads + 2 * kv_heads) * dh <= 16384 else 64128)
     into_cache(M, heads, kv_heads, dh, 16, 0, K=K, packed=packed)
+
+
+@pytest.mark.parametrize("K", [1216, 1280, 2240, 2304])
+@pytest.mark.parametrize("epilogue", ["gelu_tanh", "gelu_erf"])
+def test_tiles_of_256_by_160_in_step_and_in_turns(K, epilogue):
+    """On both sides of the borders from which their waves take turns: the results in 32-bit, rounded."""
+    M, N = 1500, 6400
+    assert ops()._lib("gemm").dn_gemm_tile(M, N, K) == 256160
+    a, w, bias = operands(M, N, K)
+    got, exact = torch.full((M + 1, N), 7.0, dtype=BF, device=DEV), torch.empty(M, N, device=DEV)
+    ops().linear(a, w, bias, out=got[:M], epilogue=epilogue)
+    ops().linear(a, w, bias, out=exact, epilogue=epilogue)
+    assert bool(((got[:M].float() - exact).abs() <= 2.0 ** -8 * exact.abs() + 1e-30).all()) and bool((got[M] == 7.0).all())
