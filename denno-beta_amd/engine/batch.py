@@ -111,7 +111,8 @@ def build_context(entries: Sequence[StepEntry], cache, vocab: int, max_positions
     places until there are so many."""
     mgr = cache.manager
     rids = np.asarray([e.rid for e in entries], dtype=np.int64)
-    counts = np.asarray([len(e.tokens) for e in entries], dtype=np.int32)
+    lengths = [len(e.tokens) for e in entries]
+    counts = np.asarray(lengths, dtype=np.int32)
     starts_a = mgr.lengths(rids)
     starts = starts_a.tolist()
     tokens, positions, logit_rows, row_start, tiles, wide = plan_rows(entries, starts, vocab, max_positions)
@@ -166,4 +167,4 @@ def build_context(entries: Sequence[StepEntry], cache, vocab: int, max_positions
         T=T, S=S, R=R, tokens=view("tokens"), positions=view("positions"), logit_rows=view("logit_rows"),
         state_slots=view("state_slots"), row_start=view("row_start"), groups=groups,
         host_row_start=row_start, host_first_pos=starts, host_slots=slots, rids=[e.rid for e in entries], single_rows=single,
-        rows_of_requests=(int(counts.min()), int(counts.max())))
+        rows_of_requests=(min(lengths), max(lengths)))

@@ -180,11 +180,13 @@ def wanted_rows(entries: Sequence[StepEntry], max_live: int) -> int:
     """The rows whose logits a captured step of these entries computes, 0 if they want none; the wanted places themselves where no graph takes such a
     step.  A vocabulary's product sums in another order from 17 rows on than up to 16 (csrc/kernels/gemm_direct.hip), so a step kernel by kernel
     computes as many: its logits are then the same bits."""
-    wanted = sum(len(e.want) for e in entries)
+    wanted, rows = sum([len(e.want) for e in entries]), sum([len(e.tokens) for e in entries])
     if wanted == 0:
         return 0
-    if all(len(e.tokens) == 1 for e in entries):
+    if rows == len(entries) and all(len(e.tokens) == 1 for e in entries):
         return max(wanted, batch_bucket(len(entries), max_live))
+    if rows > PORTION_ROWS[-1]:
+        return wanted
     bucket = portion_bucket(entries)
     return wanted if bucket is None else max(wanted, bucket[2])
 

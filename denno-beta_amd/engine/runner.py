@@ -114,8 +114,8 @@ class ModelRunner:
             rows = wanted_rows(entries, self.options.max_live)
         ctx = build_context(entries, self.cache, self.spec.vocab, self.spec.max_positions, self.device, rows)
         logits = self.model.forward(ctx, self.cache)
-        if rows:
-            logits = logits[:sum(len(e.want) for e in entries)]
+        if rows and rows > (wanted := sum([len(e.want) for e in entries])):
+            logits = logits[:wanted]
         self.cache.manager.commit_step(
             np.asarray(ctx.rids, dtype=np.int64),
             np.asarray([start + len(e.tokens) for e, start in zip(entries, ctx.host_first_pos)], dtype=np.int32))

@@ -1478,13 +1478,16 @@ def delta_chunks(r, k, v, beta, w, rate, bias, state, row_start, slots, n_heads,
 def _chunks(r, k, v, beta, w, rate, bias, mode, state, stride, row_start, slots, S, n_heads, G, dk, dv, rows_min, out, what):
     T = r.shape[0]
     # (the kernel reaches rows of results that begin fewer than 2^24 numbers apart; others are filled in rows of their own width)
-    near = out if _rows(out, "out") < 1 << 24 else out.clone(memory_format=torch.contiguous_format)
+    near, ld = out, _rows(out, "out")
+    if ld >= 1 << 24:
+        near = out.clone(memory_format=torch.contiguous_format)
+        ld = _rows(near, "out")
     lib = _lib("sequence")
     work = torch.empty(lib.dn_scan_chunks_floats(T, S, n_heads, dk, dv), dtype=torch.float32, device=r.device)
     _ok(lib.dn_scan_chunks(r.data_ptr(), _rows(r, "r"), k.data_ptr(), _rows(k, "k"), v.data_ptr(), _rows(v, "v"), _ptr(beta),
                            _rows(beta, "beta") if beta is not None else 0, w.data_ptr(), _rows(w, "w") if w.dim() == 2 else 0, _ptr(rate), _ptr(bias), mode,
                            state.data_ptr(), stride, row_start.data_ptr(), slots.data_ptr(), S, T, n_heads, G, dk, dv, int(rows_min), work.data_ptr(),
-                           near.data_ptr(), _rows(near, "out"), _stream()), what)
+                           near.data_ptr(), ld, _stream()), what)
     if near is not out:
         out.copy_(near)
 
